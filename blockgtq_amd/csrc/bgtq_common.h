@@ -33,3 +33,7 @@ __device__ static inline float bgtq_h2f(uint16_t h) {
 __device__ static inline uint16_t bgtq_f2h(float f) {
     return __half_as_ushort(__float2half_rn(f));
 }
+// fp16 bits of an input value that is stored as fp16 or (bf16 != 0, uniform) as bf16
+__device__ static inline uint16_t bgtq_in16(uint16_t x, int bf16) {
+    return bf16 ? bgtq_f2h(__uint_as_float((uint32_t)x << 16)) : x;
+}

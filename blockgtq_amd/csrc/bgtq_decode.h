@@ -40,3 +40,6 @@ struct DecodeArgs {
 // Returns BGTQ_EUNSUPPORTED when the arguments do not meet its layout
 // requirements, in which case the caller takes the layout-agnostic kernel.
 int bgtq_launch_decode_seg(const DecodeArgs& a, hipStream_t stream);
+
+// The preparation part of bgtq_decode_step (bgtq_encode.hip).  kv_fp16: k and v are fp16 whatever x_dtype says.
+int bgtq_step_prepare(const bgtq_step& s, bool kv_fp16, hipStream_t st);

@@ -395,7 +395,7 @@ __global__ __launch_bounds__(RT_THREADS) void lse_reduce_kernel(
 // ---- dense fp16 partial over the sink + recent-window tokens ------------------
 constexpr int WT = 256;
 __global__ __launch_bounds__(WT) void window_attn_generic_kernel(
-    const uint16_t* q, int64_t q_sb, int64_t q_sh,
+    const uint16_t* q, int64_t q_sb, int64_t q_sh, int bf16,
     const uint16_t* kbuf, const uint16_t* vbuf, int64_t w_sb, int64_t w_sh, int64_t w_st,
     const int32_t* lens, int W, int n_q, int gqa, float scale, float* part_out, float* part_lse) {
     extern __shared__ float wlog[];            // [W] logits, then weights
@@ -405,7 +405,7 @@ __global__ __launch_bounds__(WT) void window_attn_generic_kernel(
     const int hq = blockIdx.x, b = blockIdx.y, h = hq / gqa;
     const int n = lens ? min(lens[b], W) : W;
     const size_t row = (size_t)b * n_q + hq;
-    if (tid < D) q_s[tid] = bgtq_h2f(q[b * q_sb + hq * q_sh + tid]);
+    if (tid < D) q_s[tid] = bgtq_h2f(bgtq_in16(q[b * q_sb + hq * q_sh + tid], bf16));
     __syncthreads();
     const uint16_t* kb = kbuf + b * w_sb + h * w_sh;
     const uint16_t* vb = vbuf + b * w_sb + h * w_sh;
@@ -459,7 +459,7 @@ __device__ __forceinline__ float row16_sum(float x) {
 
 template <int HG>
 __global__ __launch_bounds__(WT) void window_attn_kernel(
-    const uint16_t* q, int64_t q_sb, int64_t q_sh,
+    const uint16_t* q, int64_t q_sb, int64_t q_sh, int bf16,
     const uint16_t* kbuf, const uint16_t* vbuf, int64_t w_sb, int64_t w_sh, int64_t w_st,
     const int32_t* lens, int W, int n_q, int gqa, float scale, float* part_out, float* part_lse) {
     extern __shared__ float wlog[];            // [HG][W]
@@ -503,8 +503,8 @@ __global__ __launch_bounds__(WT) void window_attn_kernel(
             const uint32_t ws[4] = {w4.x, w4.y, w4.z, w4.w};
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                qf[g][2 * i] = bgtq_h2f((uint16_t)(ws[i] & 0xFFFFu)) * scale;
-                qf[g][2 * i + 1] = bgtq_h2f((uint16_t)(ws[i] >> 16)) * scale;
+                qf[g][2 * i] = bgtq_h2f(bgtq_in16((uint16_t)(ws[i] & 0xFFFFu), bf16)) * scale;
+                qf[g][2 * i + 1] = bgtq_h2f(bgtq_in16((uint16_t)(ws[i] >> 16), bf16)) * scale;
             }
         }
         uint4 kc[SB], kn[SB];
@@ -602,19 +602,43 @@ __global__ __launch_bounds__(WT) void window_attn_kernel(
 // [0, W) moves nothing and leaves zeros in the outputs.
 __global__ __launch_bounds__(D) void window_swap_kernel(
     uint16_t* kbuf, uint16_t* vbuf, int64_t w_sb, int64_t w_sh, int64_t w_st,
-    const uint16_t* new_k, const uint16_t* new_v, int64_t n_sb, int64_t n_sh,
+    const uint16_t* new_k, const uint16_t* new_v, int64_t nk_sb, int64_t nk_sh, int64_t nv_sb, int64_t nv_sh, int bf16,
     const int32_t* slot, int W, int n_kv, uint16_t* old_k, uint16_t* old_v) {
     const int j = threadIdx.x, h = blockIdx.x, b = blockIdx.y;
     const int sl = slot[b];
     const int64_t o = ((int64_t)b * n_kv + h) * D + j;
     if (sl < 0 || sl >= W) { old_k[o] = 0; old_v[o] = 0; return; }
     const int64_t at = b * w_sb + h * w_sh + (int64_t)sl * w_st + j;
-    const int64_t nw = b * n_sb + h * n_sh + j;
-    const uint16_t nk = new_k[nw], nv = new_v[nw];
+    const uint16_t nk = bgtq_in16(new_k[b * nk_sb + h * nk_sh + j], bf16), nv = bgtq_in16(new_v[b * nv_sb + h * nv_sh + j], bf16);
     old_k[o] = kbuf[at];
     old_v[o] = vbuf[at];
     kbuf[at] = nk;
     vbuf[at] = nv;
+}
+
+int launch_window_attn(const void* q, int64_t q_sb, int64_t q_sh, int bf16, const void* kbuf, const void* vbuf,
+                       int64_t w_sb, int64_t w_sh, int64_t w_st, const int32_t* lens, int W,
+                       int B, int n_kv, int gqa, float scale, float* part_out, float* part_lse, hipStream_t st) {
+    const size_t wbytes = (size_t)(W > 0 ? W : 1) * sizeof(float);
+    // rows and query vectors on 16-byte boundaries: one work-group per (row, KV head)
+    const bool wide = (((uintptr_t)q | (uintptr_t)kbuf | (uintptr_t)vbuf) & 15) == 0 &&
+                      ((q_sb | q_sh | w_sb | w_sh | w_st) & 7) == 0;
+    auto kern = !wide ? window_attn_generic_kernel
+                      : gqa > 1 && 4 * wbytes <= 48 * 1024 ? window_attn_kernel<4> : window_attn_kernel<1>;
+    const dim3 grid((unsigned)(wide ? n_kv : n_kv * gqa), (unsigned)B);
+    hipLaunchKernelGGL(kern, grid, dim3(WT), kern == window_attn_kernel<4> ? 4 * wbytes : wbytes, st,
+                       (const uint16_t*)q, q_sb, q_sh, bf16, (const uint16_t*)kbuf, (const uint16_t*)vbuf, w_sb, w_sh, w_st,
+                       lens, W, n_kv * gqa, gqa, scale, part_out, part_lse);
+    return bgtq_launch_status();
+}
+
+int launch_window_swap(void* kbuf, void* vbuf, int64_t w_sb, int64_t w_sh, int64_t w_st,
+                       const void* new_k, const void* new_v, int64_t nk_sb, int64_t nk_sh, int64_t nv_sb, int64_t nv_sh,
+                       int bf16, const int32_t* slot, int W, int B, int n_kv, void* old_k, void* old_v, hipStream_t st) {
+    hipLaunchKernelGGL(window_swap_kernel, dim3((unsigned)n_kv, (unsigned)B), dim3(D), 0, st,
+                       (uint16_t*)kbuf, (uint16_t*)vbuf, w_sb, w_sh, w_st, (const uint16_t*)new_k, (const uint16_t*)new_v,
+                       nk_sb, nk_sh, nv_sb, nv_sh, bf16, slot, W, n_kv, (uint16_t*)old_k, (uint16_t*)old_v);
+    return bgtq_launch_status();
 }
 
 }  // namespace
@@ -795,30 +819,8 @@ int bgtq_window_attn(const void* q, int64_t q_sb, int64_t q_sh,
     BGTQ_CHECK_ARG(B >= 0 && n_kv >= 0 && gqa >= 1 && W >= 0);
     if (W > 8192) return BGTQ_ELIMIT;
     if (B == 0 || n_kv == 0) return BGTQ_OK;
-    const size_t wbytes = (size_t)(W > 0 ? W : 1) * sizeof(float);
-    // rows and query vectors on 16-byte boundaries: one work-group per (row, KV head)
-    const bool wide = (((uintptr_t)q | (uintptr_t)kbuf | (uintptr_t)vbuf) & 15) == 0 &&
-                      ((q_sb | q_sh | w_sb | w_sh | w_st) & 7) == 0;
-    if (wide) {
-        dim3 grid((unsigned)n_kv, (unsigned)B);
-        if (gqa > 1 && 4 * wbytes <= 48 * 1024)
-            hipLaunchKernelGGL((window_attn_kernel<4>), grid, dim3(WT), 4 * wbytes,
-                               (hipStream_t)stream, (const uint16_t*)q, q_sb, q_sh,
-                               (const uint16_t*)kbuf, (const uint16_t*)vbuf, w_sb, w_sh, w_st,
-                               lens, W, n_kv * gqa, gqa, scale, part_out, part_lse);
-        else
-            hipLaunchKernelGGL((window_attn_kernel<1>), grid, dim3(WT), wbytes,
-                               (hipStream_t)stream, (const uint16_t*)q, q_sb, q_sh,
-                               (const uint16_t*)kbuf, (const uint16_t*)vbuf, w_sb, w_sh, w_st,
-                               lens, W, n_kv * gqa, gqa, scale, part_out, part_lse);
-        return bgtq_launch_status();
-    }
-    dim3 grid((unsigned)(n_kv * gqa), (unsigned)B);
-    hipLaunchKernelGGL(window_attn_generic_kernel, grid, dim3(WT), wbytes,
-                       (hipStream_t)stream, (const uint16_t*)q, q_sb, q_sh,
-                       (const uint16_t*)kbuf, (const uint16_t*)vbuf, w_sb, w_sh, w_st,
-                       lens, W, n_kv * gqa, gqa, scale, part_out, part_lse);
-    return bgtq_launch_status();
+    return launch_window_attn(q, q_sb, q_sh, 0, kbuf, vbuf, w_sb, w_sh, w_st, lens, W, B, n_kv, gqa, scale,
+                              part_out, part_lse, (hipStream_t)stream);
 }
 
 int bgtq_window_swap(void* kbuf, void* vbuf, int64_t w_sb, int64_t w_sh, int64_t w_st,
@@ -828,11 +830,44 @@ int bgtq_window_swap(void* kbuf, void* vbuf, int64_t w_sb, int64_t w_sh, int64_t
     BGTQ_CHECK_ARG(kbuf && vbuf && new_k && new_v && slot && old_k && old_v);
     BGTQ_CHECK_ARG(B >= 0 && n_kv >= 0 && W >= 1);
     if (B == 0 || n_kv == 0) return BGTQ_OK;
-    hipLaunchKernelGGL(window_swap_kernel, dim3((unsigned)n_kv, (unsigned)B), dim3(D), 0, (hipStream_t)stream,
-                       (uint16_t*)kbuf, (uint16_t*)vbuf, w_sb, w_sh, w_st,
-                       (const uint16_t*)new_k, (const uint16_t*)new_v, n_sb, n_sh, slot, W, n_kv,
-                       (uint16_t*)old_k, (uint16_t*)old_v);
-    return bgtq_launch_status();
+    return launch_window_swap(kbuf, vbuf, w_sb, w_sh, w_st, new_k, new_v, n_sb, n_sh, n_sb, n_sh, 0, slot, W, B, n_kv,
+                              old_k, old_v, (hipStream_t)stream);
+}
+
+int bgtq_decode_step(const bgtq_step* step, void* stream) {
+    BGTQ_CHECK_ARG(step);
+    bgtq_step s = *step;
+    hipStream_t st = (hipStream_t)stream;
+    BGTQ_CHECK_ARG(s.B >= 0 && s.n_kv >= 0 && s.S >= 0 && s.gqa >= 1 && s.q && s.out);
+    if (s.B == 0 || s.n_kv == 0) return BGTQ_OK;
+    const int n_q = s.n_kv * s.gqa;
+    const bool windowed = s.win_k != nullptr;
+    if (windowed) {
+        BGTQ_CHECK_ARG(s.S == 1 && s.q_rot && s.win_v && s.win_slot && s.win_lens && s.win_old && s.win_out && s.win_lse);
+        BGTQ_CHECK_ARG(s.k && s.v && s.win_W >= 1);
+        if (s.win_W > 8192) return BGTQ_ELIMIT;
+        uint16_t *old_k = (uint16_t*)s.win_old, *old_v = old_k + (size_t)s.B * s.n_kv * D;
+        int rc = launch_window_swap(s.win_k, s.win_v, s.w_sb, s.w_sh, s.w_st, s.k, s.v, s.k_sb, s.k_sh, s.v_sb, s.v_sh,
+                                    s.x_dtype == BGTQ_X_BF16, s.win_slot, s.win_W, s.B, s.n_kv, old_k, old_v, st);
+        if (rc != BGTQ_OK) return rc;
+        rc = launch_window_attn(s.q, s.q_sb, s.q_sh, s.x_dtype == BGTQ_X_BF16, s.win_k, s.win_v, s.w_sb, s.w_sh, s.w_st,
+                                s.win_lens, s.win_W, s.B, s.n_kv, s.gqa, s.scale, s.win_out, s.win_lse, st);
+        if (rc != BGTQ_OK) return rc;
+        s.k = old_k; s.v = old_v;
+        s.k_sb = s.v_sb = (int64_t)s.n_kv * D; s.k_sh = s.v_sh = D; s.k_ss = s.v_ss = D;
+    }
+    int rc = bgtq_step_prepare(s, windowed && s.x_dtype == BGTQ_X_BF16, st);
+    if (rc != BGTQ_OK) return rc;
+    const void* q = s.q_rot ? s.q_rot : s.q;
+    rc = bgtq_decode_attn(s.plans, q, s.q_rot ? (int64_t)n_q * D : s.q_sb, s.q_rot ? D : s.q_sh,
+                          s.k_packed, s.kp_sb, s.kp_sh, s.kp_st, s.k_row_width, s.k_norms, s.kn_sb, s.kn_sh, s.kn_st,
+                          s.v_packed, s.vp_sb, s.vp_sh, s.vp_st, s.v_row_width, s.v_norms, s.vn_sb, s.vn_sh, s.vn_st,
+                          s.seq_lens, s.T, s.B, s.n_kv, s.gqa, s.n_splits, s.partial_out, s.partial_lse,
+                          s.k_layout, s.v_layout, s.scale, stream);
+    if (rc != BGTQ_OK) return rc;
+    return bgtq_lse_reduce(s.plans, s.partial_out, s.partial_lse, s.n_splits, windowed ? s.win_out : nullptr,
+                           windowed ? s.win_lse : nullptr, windowed ? 1 : 0, s.B, s.n_kv, s.gqa, 1,
+                           s.out, (int64_t)n_q * D, D, nullptr, stream);
 }
 
 size_t bgtq_plan_sizeof(void) { return sizeof(bgtq_head_plan); }

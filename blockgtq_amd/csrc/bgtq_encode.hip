@@ -15,7 +15,7 @@
 // registers; rows are staged in LDS so the k-loop reads them as broadcasts.
 #include <type_traits>
 
-#include "bgtq_common.h"
+#include "bgtq_decode.h"
 
 namespace {
 
@@ -42,6 +42,7 @@ struct EncodeArgs {
     uint8_t* codes_out;         // [N][128] unpacked codes, or nullptr
     float* norms_f32_out;       // K: [N][norm_width] fp32; or nullptr
     int corrected;              // K codes path: emit corrected norms
+    int bf16;                   // x holds bf16: rounded to fp16 as it is read
 };
 
 // One byte of the LSB-first stream of bw-bit codes (bw <= 4) covers the codes first .. first + n - 1,
@@ -254,11 +255,11 @@ __device__ __forceinline__ void encode_rows(const EncodeArgs& a, const int bx, c
     // ---- 1. rows to LDS, next tile's rows on their way, gather by head_perm (K) -------------
     if constexpr (IS_V) {              // (no gather: a thread converts its own value)
 #pragma unroll
-        for (int r = 0; r < ROWS; r++) xs[r][j] = bgtq_h2f(xr[r]);
+        for (int r = 0; r < ROWS; r++) xs[r][j] = bgtq_h2f(bgtq_in16(xr[r], a.bf16));
         if (tile + tile_stride < n_tiles) fetch_rows(tile + tile_stride);
     } else {
 #pragma unroll
-        for (int r = 0; r < ROWS; r++) xraw[r][j] = xr[r];
+        for (int r = 0; r < ROWS; r++) xraw[r][j] = bgtq_in16(xr[r], a.bf16);
         __syncthreads();
         if (tile + tile_stride < n_tiles) fetch_rows(tile + tile_stride);
 #pragma unroll
@@ -585,6 +586,7 @@ struct RotQArgs {
     uint16_t* q_rot;    int64_t qr_sr, qr_sh;
     int n_rows, n_q, gqa;
     int group;          // query heads per work-group: 1 or 4
+    int bf16;           // q holds bf16
 };
 
 // QG query heads (h_first ..) of one (row, KV head): the rotation is fetched and parked once for
@@ -623,7 +625,7 @@ __device__ __forceinline__ void rotate_q_group(const RotQArgs& a, const int64_t 
     if (!compact) park_rotation(rot_s, j, rst);
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < QG; r++) xs[r][j] = bgtq_h2f(qraw[r][src]);
+    for (int r = 0; r < QG; r++) xs[r][j] = bgtq_h2f(bgtq_in16(qraw[r][src], a.bf16));
     __syncthreads();
     float acc[QG];
 #pragma unroll
@@ -765,9 +767,68 @@ int fill_v_args(EncodeArgs& a, const bgtq_head_plan* plans,
     return BGTQ_OK;
 }
 
+int launch_rotate_q(const bgtq_head_plan* plans, const void* q, int64_t q_sr, int64_t q_sh, int bf16,
+                    void* q_rot, int64_t qr_sr, int64_t qr_sh, int n_rows, int n_kv, int gqa, hipStream_t st) {
+    const int group = rotate_q_group_size(n_rows, n_kv * gqa);
+    RotQArgs a{plans, (const uint16_t*)q, q_sr, q_sh, (uint16_t*)q_rot, qr_sr, qr_sh, n_rows, n_kv * gqa, gqa, group, bf16};
+    hipLaunchKernelGGL(rotate_q_kernel, dim3(rotate_q_blocks(n_rows, n_kv, gqa, group)), dim3(NT), 0, st, a);
+    return bgtq_launch_status();
+}
+
+// K and V appended and (q not null) the queries rotated: one launch for the few rows of a decode step
+int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, int64_t q_sr, int64_t q_sh, int q_bf16,
+                   void* q_rot, int64_t qr_sr, int64_t qr_sh, int gqa, hipStream_t st) {
+    const int B = ak.B, n_kv = ak.n_kv;
+    const int64_t N = (int64_t)B * ak.S;
+    if (N > 64) {          // prefill-sized append: the three stages are big enough on their own
+        int rc = launch_encode<false>(ak, st);
+        if (rc != BGTQ_OK) return rc;
+        rc = launch_encode<true>(av, st);
+        if (rc != BGTQ_OK || !q) return rc;
+        return launch_rotate_q(ak.plans, q, q_sr, q_sh, q_bf16, q_rot, qr_sr, qr_sh, B, n_kv, gqa, st);
+    }
+    const int group = rotate_q_group_size(B, n_kv * gqa);
+    RotQArgs aq{ak.plans, (const uint16_t*)q, q_sr, q_sh, (uint16_t*)q_rot, qr_sr, qr_sh, B, n_kv * gqa, gqa, group, q_bf16};
+    const int tiles = (int)((N + PREP_ROWS - 1) / PREP_ROWS);
+    const unsigned blocks = (unsigned)(2 * tiles * n_kv) + (q ? rotate_q_blocks(B, n_kv, gqa, group) : 0u);
+    hipLaunchKernelGGL(prepare_kernel, dim3(blocks), dim3(NT), 0, st, ak, av, aq, tiles, tiles);
+    return bgtq_launch_status();
+}
+
+int fill_step_args(const bgtq_step& s, EncodeArgs& ak, EncodeArgs& av) {
+    BGTQ_CHECK_ARG(s.x_dtype == BGTQ_X_FP16 || s.x_dtype == BGTQ_X_BF16);
+    int rc = fill_k_args(ak, s.plans, s.k, s.k_sb, s.k_sh, s.k_ss, s.B, s.n_kv, s.S, s.k_packed, s.kp_sb, s.kp_sh, s.kp_st,
+                         s.k_row_width, s.k_norms, s.kn_sb, s.kn_sh, s.kn_st, s.norm_width, s.t_pos, s.t_pos_scalar, s.max_T,
+                         s.k_layout, s.quant_mode);
+    if (rc != BGTQ_OK) return rc;
+    rc = fill_v_args(av, s.plans, s.v, s.v_sb, s.v_sh, s.v_ss, s.B, s.n_kv, s.S, s.v_packed, s.vp_sb, s.vp_sh, s.vp_st,
+                     s.v_row_width, s.v_norms, s.vn_sb, s.vn_sh, s.vn_st, s.t_pos, s.t_pos_scalar, s.max_T, s.v_layout);
+    ak.bf16 = av.bf16 = s.x_dtype == BGTQ_X_BF16;
+    return rc;
+}
+
 }  // namespace
 
+int bgtq_step_prepare(const bgtq_step& s, bool kv_fp16, hipStream_t st) {
+    EncodeArgs ak{}, av{};
+    const int rc = fill_step_args(s, ak, av);
+    if (rc != BGTQ_OK) return rc;
+    const int q_bf16 = ak.bf16;
+    if (kv_fp16) ak.bf16 = av.bf16 = 0;
+    return launch_prepare(ak, av, s.q_rot ? s.q : nullptr, s.q_sb, s.q_sh, q_bf16, s.q_rot,
+                          (int64_t)s.n_kv * s.gqa * D, D, s.gqa, st);
+}
+
 extern "C" {
+
+int bgtq_encode_kv(const bgtq_step* step, void* stream) {
+    BGTQ_CHECK_ARG(step && step->B >= 0 && step->n_kv >= 0 && step->S >= 0);
+    if (step->B == 0 || step->n_kv == 0 || step->S == 0) return BGTQ_OK;
+    EncodeArgs ak{}, av{};
+    const int rc = fill_step_args(*step, ak, av);
+    if (rc != BGTQ_OK) return rc;
+    return launch_prepare(ak, av, nullptr, 0, 0, 0, nullptr, 0, 0, 1, (hipStream_t)stream);
+}
 
 int bgtq_encode_k(const bgtq_head_plan* plans,
                   const void* k, int64_t k_sb, int64_t k_sh, int64_t k_ss,
@@ -834,11 +895,7 @@ int bgtq_rotate_q(const bgtq_head_plan* plans,
     BGTQ_CHECK_ARG(plans && q && q_rot);
     BGTQ_CHECK_ARG(n_rows >= 0 && n_kv >= 0 && gqa >= 1);
     if (n_rows == 0 || n_kv == 0) return BGTQ_OK;
-    const int group = rotate_q_group_size(n_rows, n_kv * gqa);
-    RotQArgs a{plans, (const uint16_t*)q, q_sr, q_sh, (uint16_t*)q_rot, qr_sr, qr_sh, n_rows, n_kv * gqa, gqa, group};
-    hipLaunchKernelGGL(rotate_q_kernel, dim3(rotate_q_blocks(n_rows, n_kv, gqa, group)), dim3(NT), 0,
-                       (hipStream_t)stream, a);
-    return bgtq_launch_status();
+    return launch_rotate_q(plans, q, q_sr, q_sh, 0, q_rot, qr_sr, qr_sh, n_rows, n_kv, gqa, (hipStream_t)stream);
 }
 
 int bgtq_decode_prepare(const bgtq_head_plan* plans,
@@ -863,21 +920,7 @@ int bgtq_decode_prepare(const bgtq_head_plan* plans,
                      v_norms, vn_sb, vn_sh, vn_st, t_pos, t_pos_scalar, max_T, v_layout);
     if (rc != BGTQ_OK) return rc;
     BGTQ_CHECK_ARG((q == nullptr) == (q_rot == nullptr));     // both, or neither (queries rotated elsewhere)
-    const bool with_q = q != nullptr;
-    const int64_t N = (int64_t)B * S;
-    if (N > 64) {          // prefill-sized append: the three stages are big enough on their own
-        rc = launch_encode<false>(ak, (hipStream_t)stream);
-        if (rc != BGTQ_OK) return rc;
-        rc = launch_encode<true>(av, (hipStream_t)stream);
-        if (rc != BGTQ_OK || !with_q) return rc;
-        return bgtq_rotate_q(plans, q, q_sr, q_sh, q_rot, qr_sr, qr_sh, B, n_kv, gqa, stream);
-    }
-    const int group = rotate_q_group_size(B, n_kv * gqa);
-    RotQArgs aq{plans, (const uint16_t*)q, q_sr, q_sh, (uint16_t*)q_rot, qr_sr, qr_sh, B, n_kv * gqa, gqa, group};
-    const int tiles = (int)((N + PREP_ROWS - 1) / PREP_ROWS);
-    const unsigned blocks = (unsigned)(2 * tiles * n_kv) + (with_q ? rotate_q_blocks(B, n_kv, gqa, group) : 0u);
-    hipLaunchKernelGGL(prepare_kernel, dim3(blocks), dim3(NT), 0, (hipStream_t)stream, ak, av, aq, tiles, tiles);
-    return bgtq_launch_status();
+    return launch_prepare(ak, av, q, q_sr, q_sh, 0, q_rot, qr_sr, qr_sh, gqa, (hipStream_t)stream);
 }
 
 

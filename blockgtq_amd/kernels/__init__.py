@@ -13,7 +13,7 @@ import weakref
 import numpy as np
 import torch
 
-from .. import ops, plan as _plan
+from .. import _host, ops, plan as _plan
 
 # id(codebook_flat tensor object) -> (weak reference to that tensor, weak reference to the quantizer
 # that produced it via build_kernel_args()).  The tensor OBJECT is the key, not its address: memory
@@ -82,7 +82,6 @@ def _plan_from_args(codebook_flat, segments, v_lut, v_rotation, v_bits, device):
     return _plan.upload_plans(p.reshape(1), device)
 
 
-@torch.no_grad()
 def fused_blockgtq_decode_attention(
     q, k_packed, k_norms, codebook_flat, lut_offset, norm_group, segments,
     v_codes, v_norms, v_lut,
@@ -128,14 +127,19 @@ def fused_blockgtq_decode_attention(
                                 int(v_bits) if not v_nibble else max(int(v_bits), 1), q.device)
     if v_norms.dim() == 4:
         v_norms = v_norms[..., 0]
-    q3 = q.reshape(B, n_q, D).to(torch.float16).contiguous()
+    n_splits = max(1, min(int(t_splits), 512))
+    k_layout = _plan.K_MIXED if k_nibble else _plan.K_BITPACKED
+    v_layout = _plan.V_NIBBLE if v_nibble else _plan.V_BITPACKED
+    scale = (1.0 / math.sqrt(D)) if scale is None else float(scale)
+    if not return_lse:
+        out = _host.module().attend(plans, q, k_packed, k_norms, v_codes, v_norms, T, n_splits, k_layout, v_layout,
+                                    scale, int(v_rotation is not None), ops._default_ws)
+        if out is not None:
+            return out
+    q3 = q.detach().reshape(B, n_q, D).to(torch.float16).contiguous()
     res = ops.decode_attention(
-        plans, q3, k_packed, k_norms, v_codes, v_norms, T,
-        n_splits=max(1, min(int(t_splits), 512)),
-        k_layout=_plan.K_MIXED if k_nibble else _plan.K_BITPACKED,
-        v_layout=_plan.V_NIBBLE if v_nibble else _plan.V_BITPACKED,
-        scale=(1.0 / math.sqrt(D)) if scale is None else scale,
-        unrotate=v_rotation is not None, return_lse=return_lse)
+        plans, q3, k_packed, k_norms, v_codes, v_norms, T, n_splits=n_splits, k_layout=k_layout, v_layout=v_layout,
+        scale=scale, unrotate=v_rotation is not None, return_lse=return_lse)
     if return_lse:
         return res[0].unsqueeze(2), res[1]
     return res.unsqueeze(2)

@@ -60,6 +60,21 @@ def last_decode_path() -> int:
     return _capi.lib().bgtq_last_decode_path()
 
 
+def _note_path(n_kv, gqa, k_stride, v_stride, norm_stride, k_layout, v_layout):
+    """After an attention launch: remember which kernel took this cache geometry, warn the first time it
+    was the generic one."""
+    key = (n_kv, gqa, k_stride, v_stride, norm_stride, k_layout, v_layout)
+    if key in _paths_seen:
+        return
+    _paths_seen[key] = path = _capi.lib().bgtq_last_decode_path()
+    if path == GENERIC_PATH:
+        warnings.warn(f"bgtq_decode_attn runs its generic kernel (several times slower than the matrix-core "
+                      f"one) for n_kv={n_kv}, gqa={gqa}, K rows {k_stride} B, V rows "
+                      f"{v_stride} B: the fast kernel takes gqa <= 16, K rows that follow each "
+                      f"other at a multiple of 4 bytes (4..128), V rows of 16..64 bytes at most 4 bytes apart",
+                      RuntimeWarning, stacklevel=3)
+
+
 @torch.no_grad()
 def decode_attention(plans: torch.Tensor, q_rot: torch.Tensor,
                      k_packed: torch.Tensor, k_norms: torch.Tensor,
@@ -114,15 +129,7 @@ def decode_attention(plans: torch.Tensor, q_rot: torch.Tensor,
         _capi.ptr(seq_lens), int(T), B, n_kv, gqa, n_splits,
         _capi.ptr(part_out), _capi.ptr(part_lse), k_layout, v_layout, scale, st),
         "bgtq_decode_attn")
-    shape_key = (n_kv, gqa, k_packed.stride(2), v_packed.stride(2), k_norms.stride(2), k_layout, v_layout)
-    if shape_key not in _paths_seen:
-        _paths_seen[shape_key] = path = L.bgtq_last_decode_path()
-        if path == GENERIC_PATH:
-            warnings.warn(f"bgtq_decode_attn runs its generic kernel (several times slower than the matrix-core "
-                          f"one) for n_kv={n_kv}, gqa={gqa}, K rows {k_packed.stride(2)} B, V rows "
-                          f"{v_packed.stride(2)} B: the fast kernel takes gqa <= 16, K rows that follow each "
-                          f"other at a multiple of 4 bytes (4..128), V rows of 16..64 bytes at most 4 bytes apart",
-                          RuntimeWarning, stacklevel=2)
+    _note_path(n_kv, gqa, k_packed.stride(2), v_packed.stride(2), k_norms.stride(2), k_layout, v_layout)
     out = torch.empty((B, n_q, D), dtype=torch.float16, device=q_rot.device)
     lse = torch.empty((B, n_q), dtype=torch.float32, device=q_rot.device) if return_lse else None
     n_extra = 0

@@ -25,7 +25,7 @@ import math
 
 import torch
 
-from . import ops, plan as _plan
+from . import _host, ops, plan as _plan
 from .quantizer import (BlockGTQQuantizer, build_batched_encode_args,
                         encode_k_into, encode_v_into)
 from .v_packing import packed_v_bytes
@@ -69,6 +69,7 @@ class BlockGTQKVManager:
             raise ValueError("n_sink needs recent_window > 0")
         self._buf_k = self._buf_v = None
         self._step_src, self._step_idx = None, None     # per-step index tensors of the buffered append
+        self._layers = [None] * n_layers                # (native handle, rotation folded into q_proj) per layer
 
     # ------------------------------------------------------------ calibration
     def calibrate(self, layer_idx: int, q_data: torch.Tensor, k_data: torch.Tensor):
@@ -101,6 +102,7 @@ class BlockGTQKVManager:
 
     def _finish_layer(self, li):
         self._batched_args[li] = build_batched_encode_args(self.quantizers[li], device=self.device)
+        self._layers[li] = None
 
     # ---------------------------------------------------------------- storage
     def _ensure_storage(self):
@@ -126,6 +128,19 @@ class BlockGTQKVManager:
             self._buf_k = torch.zeros(bshape, dtype=torch.float16, device=dev)
             self._buf_v = torch.zeros(bshape, dtype=torch.float16, device=dev)
 
+    def _native(self, li):
+        """The layer's native handle (None off the GPU)."""
+        baked = self.quantizers[li][0]._q_perm_baked
+        entry = self._layers[li]
+        if entry is None or entry[1] != baked:
+            self._ensure_storage()
+            entry = (_host.layer(self._batched_args[li]['plans'], self._k_packed[li], self._k_norms[li], self._v_packed[li],
+                                 self._v_norms[li], self._k_rows[li], self._k_norms.shape[-1], self._vpb, self.n_q,
+                                 _plan.K_BITPACKED, _plan.V_BITPACKED, self.scale, baked,
+                                 self._buf_k[li] if self.buffered else None, self._buf_v[li] if self.buffered else None), baked)
+            self._layers[li] = entry
+        return entry[0]
+
     def set_seq_lens(self, seq_lens):
         """Per-row visible lengths (ragged batch); ``None`` returns to one shared length."""
         if seq_lens is None:
@@ -138,7 +153,9 @@ class BlockGTQKVManager:
 
     def _encode_kv(self, layer_idx: int, k: torch.Tensor, v: torch.Tensor, t_pos):
         """Encode k, v (B, n_kv, S, D) into the cache at ``t_pos`` (int or int32 (B,))."""
-        self._ensure_storage()
+        native = self._native(layer_idx)
+        if native is not None and native.encode(k, v, t_pos, _plan.QUANT_LUT256):
+            return
         li = layer_idx
         plans = self._batched_args[li]['plans']
         k16 = k if k.dtype == torch.float16 else k.to(torch.float16)
@@ -216,11 +233,17 @@ class BlockGTQKVManager:
     @torch.no_grad()
     def _append_and_attend_buffered(self, li, q, k_new, v_new):
         assert k_new.shape[2] == 1, "with-buffer decode appends one token per sequence"
-        self._ensure_storage()
+        native = self._native(li)
         if self._seq_lens is None:
             self.set_seq_lens([self.seq_len] * self.B)
         assert self.seq_len + 1 - self.n_sink - self.window < self.max_T - 1
         ar, slot, t_flush, packed_len, buf_len = self._buffered_step_indices()
+        T = max(self.seq_len + 1 - self.n_sink - self.window, 1)
+        if native is not None:
+            out = native.step_window(q, k_new, v_new, slot, t_flush, packed_len, buf_len, T, self.n_splits,
+                                     _plan.QUANT_LUT256, self._ws)
+            if out is not None:
+                return out
         plans = self._batched_args[li]['plans']
         B = q.shape[0]
         q3 = q.reshape(B, self.n_q, self.hd).to(torch.float16).contiguous()
@@ -233,7 +256,6 @@ class BlockGTQKVManager:
             self._v_packed[li], self._v_norms[li], t_flush, self._k_rows[li],
             self._k_norms.shape[-1], self._vpb, self.n_kv, _plan.K_BITPACKED, _plan.V_BITPACKED)
         ext_out, ext_lse = ops.window_attention(q3, bk, bv, buf_len, self.n_kv, self.scale)
-        T = max(self.seq_len + 1 - self.n_sink - self.window, 1)
         out = ops.decode_attention(
             plans, q_rot, self._k_packed[li], self._k_norms[li],
             self._v_packed[li], self._v_norms[li], T, seq_lens=packed_len, n_splits=self.n_splits,
@@ -243,13 +265,31 @@ class BlockGTQKVManager:
         return out.unsqueeze(2)
 
     # ----------------------------------------------------------------- decode
-    @torch.no_grad()
     def append_and_attend(self, layer_idx: int, q: torch.Tensor,
                           k_new: torch.Tensor, v_new: torch.Tensor) -> torch.Tensor:
         """q (B, n_q, 1, D), k_new / v_new (B, n_kv, S, D) -> (B, n_q, 1, D) fp16."""
         if self.buffered:
             return self._append_and_attend_buffered(layer_idx, q, k_new, v_new)
-        li = layer_idx
+        native = self._native(layer_idx)
+        if native is not None:
+            S = k_new.shape[2]
+            rows = self._seq_lens
+            out = native.step(q, k_new, v_new, self.seq_len if rows is None else rows, self.seq_len + S,
+                              None if rows is None else self._visible_lens(S), self.n_splits,
+                              _plan.QUANT_LUT256, self._ws)
+            if out is not None:
+                return out
+        return self._append_and_attend_general(layer_idx, q, k_new, v_new)
+
+    def _visible_lens(self, S):
+        """Per-row lengths once this step's S tokens are in (one add per step, not per layer)."""
+        if self._lens_src is not self._seq_lens or self._lens_S != S:
+            self._lens_src, self._lens_S, self._lens_plus = self._seq_lens, S, self._seq_lens + S
+        return self._lens_plus
+
+    @torch.no_grad()
+    def _append_and_attend_general(self, li, q, k_new, v_new):
+        """The same for inputs the native step does not take: converted and made contiguous first."""
         S = k_new.shape[2]
         t_pos = self._seq_lens if self._seq_lens is not None else self.seq_len
         T = self.seq_len + S
@@ -271,11 +311,7 @@ class BlockGTQKVManager:
                 plans, k16, v16, q3.contiguous(), self._k_packed[li], self._k_norms[li],
                 self._v_packed[li], self._v_norms[li], t_pos, self._k_rows[li],
                 self._k_norms.shape[-1], self._vpb, self.n_kv, _plan.K_BITPACKED, _plan.V_BITPACKED)
-        lens = None
-        if self._seq_lens is not None:
-            if self._lens_src is not self._seq_lens or self._lens_S != S:   # one add per step, not per layer
-                self._lens_src, self._lens_S, self._lens_plus = self._seq_lens, S, self._seq_lens + S
-            lens = self._lens_plus
+        lens = None if self._seq_lens is None else self._visible_lens(S)
         out = ops.decode_attention(
             plans, q3.contiguous(), self._k_packed[li], self._k_norms[li],
             self._v_packed[li], self._v_norms[li], T, seq_lens=lens, n_splits=self.n_splits,

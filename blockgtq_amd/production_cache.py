@@ -15,7 +15,7 @@ import math
 
 import torch
 
-from . import ops, plan as _plan
+from . import _host, ops, plan as _plan
 from .quantizer import encode_k_into, encode_v_into
 from .v_packing import packed_v_bytes
 
@@ -60,10 +60,27 @@ class BlockGTQProductionCache:
         # K cell search: the reference's 256-bin table (blockgtq/quantizer.py:841-850);
         # plan.QUANT_EXACT gives the nearest centroid of the unpacked torch path
         self.quant_mode = _plan.QUANT_LUT256
+        self._layers = [None] * n_layers    # native handle per layer and what it was made from
+
+    def _native(self, li):
+        """The layer's native handle (None off the GPU), made anew when the storage, the plans or the
+        folding of the query rotation have changed."""
+        plans, baked = self.batched_args[li]['plans'], self.quantizers[li][0]._q_perm_baked
+        e = self._layers[li]
+        if (e is None or e[1] is not plans or e[2] != baked or e[3] is not self.k_packed or e[4] is not self.k_norms
+                or e[5] is not self.v_packed or e[6] is not self.v_norms):
+            e = (_host.layer(plans, self.k_packed[li], self.k_norms[li], self.v_packed[li], self.v_norms[li],
+                             self.k_bytes_per_tok, self.max_ng, self.vpb, self.nq, self._k_layout, self._v_layout,
+                             self.scale, baked), plans, baked, self.k_packed, self.k_norms, self.v_packed, self.v_norms)
+            self._layers[li] = e
+        return e[0]
 
     # ---------------------------------------------------------------- encode
     def _encode_batched(self, layer_idx, k, v, t_pos):
         """Encode k, v (B, n_kv, S, D) into positions ``[t_pos, t_pos + S)``."""
+        native = self._native(layer_idx)
+        if native is not None and native.encode(k, v, t_pos, self.quant_mode):
+            return
         li = layer_idx
         plans = self.batched_args[li]['plans']
         k16 = k if k.dtype == torch.float16 else k.to(torch.float16)
@@ -97,7 +114,7 @@ class BlockGTQProductionCache:
         single-token step attends over).  Both advance together, so a step launches no arithmetic
         on the lengths."""
         self._lens2 = torch.stack([lens.to(torch.int32), lens.to(torch.int32) + 1]).contiguous()
-        self._seq_lens = self._lens2[0]
+        self._seq_lens, self._lens_next = self._lens2[0], self._lens2[1]
 
     def use_device_lengths(self):
         """Keep the lengths on the device only, so that a decode step contains no
@@ -110,10 +127,23 @@ class BlockGTQProductionCache:
         self._static_T = self.max_T
 
     # ---------------------------------------------------------------- decode
-    @torch.no_grad()
     def encode_and_attend(self, layer_idx, q, k, v):
         """q (B, n_q, 1, hd), k / v (B, n_kv, S, hd) post-RoPE -> (B, n_q, 1, hd) fp16."""
-        li = layer_idx
+        native = self._native(layer_idx)
+        if native is not None:
+            S = k.shape[2]
+            rows = self._seq_lens
+            lens = None if rows is None else self._lens_next if S == 1 else rows + S
+            out = native.step(q, k, v, self.seq_len if rows is None else rows,
+                              self.seq_len + S if self._static_T is None else self._static_T, lens, self.n_splits,
+                              self.quant_mode, self._ws)
+            if out is not None:
+                return out
+        return self._encode_and_attend_general(layer_idx, q, k, v)
+
+    @torch.no_grad()
+    def _encode_and_attend_general(self, li, q, k, v):
+        """The same for inputs the native step does not take: converted and made contiguous first."""
         S = k.shape[2]
         t_pos = self._seq_lens if self._seq_lens is not None else self.seq_len
         T = self._static_T if self._static_T is not None else self.seq_len + S
@@ -133,7 +163,7 @@ class BlockGTQProductionCache:
                 plans, k16, v16, q3.contiguous(), self.k_packed[li], self.k_norms[li],
                 self.v_packed[li], self.v_norms[li], t_pos, self.k_bytes_per_tok, self.max_ng,
                 self.vpb, self.nkv, self._k_layout, self._v_layout, self.quant_mode)
-        lens = None if self._seq_lens is None else self._lens2[1] if S == 1 else self._seq_lens + S
+        lens = None if self._seq_lens is None else self._lens_next if S == 1 else self._seq_lens + S
         out = ops.decode_attention(
             plans, q3.contiguous(), self.k_packed[li], self.k_norms[li],
             self.v_packed[li], self.v_norms[li], T, seq_lens=lens, n_splits=self.n_splits,

@@ -434,6 +434,63 @@ int bgtq_decode_attend_static(const bgtq_head_plan* plans,
                               void* out, int64_t o_sb, int64_t o_sh, float* lse_out, void* stream);
 
 /*
+ * One decode step of one layer in one call: append K and V, rotate the queries, attend over the
+ * packed cache, merge the partitions - what bgtq_decode_prepare, bgtq_decode_attn and
+ * bgtq_lse_reduce (and, with a buffer, bgtq_window_swap and bgtq_window_attn) do one after the
+ * other, with the same results.  The arguments that a layer keeps from step to step come in a
+ * struct, and the new tokens and queries may be fp16 or bf16 (x_dtype): bf16 values are rounded to
+ * fp16 as they are read, as a caller converting them first would have them.
+ * BlockGTQKVManager.append_and_attend (blockgtq/packed_kv_manager.py:269-330) and
+ * BlockGTQProductionCache.encode_and_attend (blockgtq/production_cache.py:207-262) are one such
+ * call per layer here.
+ *   k, v, q    [B][n_kv][S][128] (q: [B][n_kv*gqa][128]) of x_dtype, strides in elements, dim contiguous
+ *   q_rot      fp16 [B][n_kv*gqa][128] scratch for the rotated queries; NULL: q holds rotated fp16 queries
+ *              already (rotation folded into the projection)
+ *   win_k, win_v  NULL, or the fp16 buffer of the with-buffer mode ([B][n_kv][win_W][128], common strides):
+ *              then S is 1, the token in slot win_slot[b] leaves the buffer and is appended at t_pos[b],
+ *              the new token takes its place, and the win_lens[b] buffered tokens join the attention;
+ *              win_old (fp16 [2][B][n_kv][128]), win_out (fp32 [B][n_q][128]) and win_lse (fp32 [B][n_q])
+ *              are scratch
+ *   partial_out, partial_lse  as for bgtq_decode_attn
+ *   out        fp16 [B][n_kv*gqa][128] contiguous
+ */
+#define BGTQ_X_FP16 0
+#define BGTQ_X_BF16 1
+typedef struct bgtq_step {
+    const bgtq_head_plan* plans;
+    int32_t B, n_kv, gqa, S;
+    int32_t x_dtype, k_layout, v_layout, quant_mode;
+    const void *k, *v, *q;
+    int64_t k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, q_sb, q_sh;
+    void* q_rot;
+    void *k_packed, *k_norms, *v_packed, *v_norms;
+    int64_t kp_sb, kp_sh, kp_st, kn_sb, kn_sh, kn_st, vp_sb, vp_sh, vp_st, vn_sb, vn_sh, vn_st;
+    int32_t k_row_width, norm_width, v_row_width, max_T;
+    const int32_t* t_pos;
+    int32_t t_pos_scalar, T;
+    const int32_t* seq_lens;
+    int32_t n_splits;
+    float scale;
+    float *partial_out, *partial_lse;
+    void* out;
+    void *win_k, *win_v;
+    int64_t w_sb, w_sh, w_st;
+    const int32_t *win_slot, *win_lens;
+    int32_t win_W, reserved;
+    void* win_old;
+    float *win_out, *win_lse;
+} bgtq_step;
+
+int bgtq_decode_step(const bgtq_step* step, void* stream);
+
+/*
+ * bgtq_encode_k and bgtq_encode_v of the same tokens in one call (one launch where the sizes
+ * allow it), from fp16 or bf16 inputs.  Uses the fields of bgtq_step that describe k, v, the cache
+ * and the positions.
+ */
+int bgtq_encode_kv(const bgtq_step* step, void* stream);
+
+/*
  * Dense fp16 attention partial for the with-buffer setting: sink tokens and a
  * recent window are kept as plain fp16 K/V (post-RoPE, unrotated) next to the
  * packed cache.  The partial lives in the ORIGINAL value space and feeds

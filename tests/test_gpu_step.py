@@ -1,0 +1,66 @@
+"""GPU: the one-call decode step and append (native layer handles) against the general path.
+
+Both launch the same kernels on the same values (bf16 inputs are rounded to fp16 where they are
+read, as ``.to(torch.float16)`` rounds them), so caches and outputs must agree bit for bit."""
+import pytest
+import torch
+
+from blockgtq_amd import workloads as wl
+from blockgtq_amd.production_cache import BlockGTQProductionCache
+from blockgtq_amd.quantizer import build_batched_encode_args
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _inputs(w, energies, T, dtype):
+    k, v = wl.draw_kv(w, energies[0], 1, 321, DEV, pos0=T)
+    q = wl.draw_q(w, 0, DEV, T)
+    # as a projection leaves them: heads behind tokens in memory
+    return [t.to(dtype).transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("batch,context,ragged,window", [(1, 1, False, 0), (3, 130, True, 0), (2, 200, True, 64), (40, 70, False, 0)])
+def test_manager_step_equals_general_path(dtype, batch, context, ragged, window):
+    lens = [max(context - 3 * b, window + 5, 1) for b in range(batch)] if ragged else None
+    w = wl.Workload("t", 1, 8, 2, batch, context, 1e6, seq_lens=lens, n_sink=4 if window else 0, window=window, seed=31)
+    mgrs = []
+    for _ in range(2):
+        mgr, energies = wl.build_manager(w, DEV)
+        wl.fill_cache(mgr, w, energies, DEV)
+        mgrs.append(mgr)
+    q, k, v = _inputs(w, energies, context, dtype)
+    fast = mgrs[0].append_and_attend(0, q, k, v)
+    general = mgrs[1]
+    general._native = lambda li: general._ensure_storage()          # (no handle: every call goes the general way)
+    slow = general.append_and_attend(0, q, k, v)
+    assert fast.shape == (batch, 8, 1, 128) and fast.abs().max() > 0
+    assert torch.equal(fast, slow)
+    for name in ("_k_packed", "_k_norms", "_v_packed", "_v_norms") + (("_buf_k", "_buf_v") if window else ()):
+        assert torch.equal(getattr(mgrs[0], name)[0], getattr(general, name)[0]), name
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("nibble,device_lengths,tokens", [(True, False, 1), (False, True, 1), (False, False, 65), (True, False, 200)])
+def test_production_cache_step_and_append_equal_general_path(dtype, nibble, device_lengths, tokens):
+    w = wl.Workload("t", 1, 12, 4, 2, 300, 1e6, seed=32)
+    qs, e = wl.calibrate_layer(w, 0, DEV)
+    k0, v0 = wl.draw_kv(w, e, tokens, 5, DEV)
+    k0, v0 = k0.to(dtype), v0.to(dtype)
+    caches = []
+    for fast in (True, False):
+        c = BlockGTQProductionCache([qs], [build_batched_encode_args(qs, device=DEV)], [[q.build_kernel_args() for q in qs]],
+                                    1, 4, 12, 128, 320, k_nibble=nibble, v_nibble=nibble, device=DEV, batch_size=2)
+        if not fast:
+            c._native = lambda li: None
+        c._encode_batched(0, k0, v0, 0)
+        c.seq_len = tokens
+        if device_lengths:
+            c.use_device_lengths()
+        caches.append(c)
+    q, k, v = _inputs(w, [e], tokens, dtype)
+    outs = [c.encode_and_attend(0, q, k, v) for c in caches]
+    assert torch.equal(*outs) and outs[0].abs().max() > 0
+    for name in ("k_packed", "k_norms", "v_packed", "v_norms"):
+        assert torch.equal(getattr(caches[0], name), getattr(caches[1], name)), name
