@@ -24,7 +24,7 @@ COMMON = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-std=c++17",
 # evaluation order, so nothing in that file may be contracted into an fma
 # behind the author's back.
 SOURCES = {
-    "bgtq_encode.hip": ["-ffp-contract=off"],
+    "bgtq_encode.hip": ["-ffp-contract=off", "-fno-strict-aliasing"],
     "bgtq_decode.hip": ["-fno-strict-aliasing"],
     # LDS tiles are written as 128-bit / 16-bit words and read back as 32-bit words
     "bgtq_decode_seg.hip": ["-fno-strict-aliasing"],

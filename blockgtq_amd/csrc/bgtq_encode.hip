@@ -8,14 +8,14 @@
 // y = xhat, when the group's rotation block is the identity).  This file is
 // compiled with floating-point contraction off so nothing else fuses.
 //
-// One work-group of 128 threads encodes ROWS token rows of one KV head:
-// thread j owns packed dim j during normalise / rotate / quantise and output
-// byte j while packing.  The rotation matrix is read once per work-group
-// (coalesced across j, served from L2) and reused for all ROWS rows out of
-// registers; rows are staged in LDS so the k-loop reads them as broadcasts.
+// Two encoders keep it: a work-group of 128 threads for every row of a decode append (encode_rows: thread j
+// owns packed dim j during normalise / rotate / quantise and output byte j while packing), and blocks of 16
+// rows on the matrix cores for anything larger (encode_blocks).
+#include <algorithm>
 #include <type_traits>
 
 #include "bgtq_decode.h"
+#include "bgtq_lds.h"
 
 namespace {
 
@@ -49,13 +49,8 @@ struct EncodeArgs {
 // the first of them from its bit `skip` on.  None of this depends on the row: the plan holds it per
 // record byte (enc_byte, enc_vbyte).
 struct StreamSlot { int first, n, skip; };
-__device__ inline unsigned stream_byte(const uint8_t* codes, StreamSlot s, int bw) {
-    unsigned w = 0;
-    for (int i = 0; i < s.n; i++) w |= (unsigned)codes[s.first + i] << (i * bw);
-    return (w >> s.skip) & 0xFFu;
-}
-// The same byte with all (at most 8) code reads issued at once: for the latency-bound append of
-// a few rows, where one LDS round trip per code is what the loop above would cost.
+// All (at most 8) code reads are issued at once: the append of a few rows is bound by latency, one LDS
+// round trip per code is what a loop would cost.
 __device__ inline unsigned stream_byte_batched(const uint8_t* codes, StreamSlot s, int bw) {
     unsigned c[8];
 #pragma unroll
@@ -386,35 +381,6 @@ __device__ __forceinline__ void encode_rows(const EncodeArgs& a, const int bx, c
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        constexpr int RB = IS_V ? 32 : 16;
-        for (int k0 = (STAGED || PF > 0) ? ge : gs; k0 < ge; k0 += RB) {
-            float rt[RB];
-#pragma unroll
-            for (int i = 0; i < RB; i++) rt[i] = RT[min(k0 + i, ge - 1) * D + j];
-            if (IS_V) {
-                // dense rotation: the range is the whole row, so the row values can be
-                // read four at a time (same chain order)
-#pragma unroll
-                for (int i = 0; i < RB; i += 4) {
-#pragma unroll
-                    for (int r = 0; r < ROWS; r++) {
-                        const float4 x4 = *(const float4*)&xs[r][k0 + i];
-                        y[r] = __builtin_fmaf(x4.x, rt[i], y[r]);
-                        y[r] = __builtin_fmaf(x4.y, rt[i + 1], y[r]);
-                        y[r] = __builtin_fmaf(x4.z, rt[i + 2], y[r]);
-                        y[r] = __builtin_fmaf(x4.w, rt[i + 3], y[r]);
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < RB; i++) {
-                    if (k0 + i < ge) {
-#pragma unroll
-                        for (int r = 0; r < ROWS; r++) y[r] = __builtin_fmaf(xs[r][k0 + i], rt[i], y[r]);
-                    }
-                }
-            }
-        }
     }
 
     // ---- 5. scalar quantise ---------------------------------------------------
@@ -531,7 +497,7 @@ __device__ __forceinline__ void encode_rows(const EncodeArgs& a, const int bx, c
             int64_t t = ROWS <= 2 ? tcur[r & 1] : (a.t_pos ? a.t_pos[b] : a.t_pos_scalar) + s;
             if (t < 0 || t >= a.max_T) continue;
             unsigned v = 0;
-            if (mode == 1)      v = ROWS <= 2 ? stream_byte_batched(&cds[r][c0], slot, bw) : stream_byte(&cds[r][c0], slot, bw);
+            if (mode == 1)      v = stream_byte_batched(&cds[r][c0], slot, bw);
             else if (mode == 2) v = cds[r][c0];
             a.packed[b * a.p_sb + h * a.p_sh + t * a.p_st + j] = (uint8_t)v;
         }
@@ -546,36 +512,535 @@ __global__ __launch_bounds__(NT) void encode_kernel(EncodeArgs a) {
     __shared__ __align__(16) float rot_s[(ROWS <= 2 && !IS_V) ? D * D : 4];
     encode_rows<ROWS, IS_V>(a, blockIdx.x, blockIdx.y, (N + ROWS - 1) / ROWS, gridDim.x, rot_s);
 }
-// The prefill-sized encoder is throughput bound: at least 4 waves per SIMD (128 registers a
-// lane), which the register allocator does not aim for by itself.
-template <bool IS_V>
-__global__ __launch_bounds__(NT, 4) void encode_kernel16(EncodeArgs a) {
+// ================================================================================================
+// Prompt-sized encoder: blocks of 16 rows, every chain of the contract on the fp32 matrix cores.
+//
+// v_mfma_f32_16x16x4_f32 adds its four products to the accumulator one after the other, each as one fused
+// multiply-add rounded to nearest with subnormals kept: such instructions over ascending k are the contract's
+// fmaf chain bit for bit.  Terms outside a dim's own segment are x * 0 and leave its sum as it is (x finite; a
+// block whose norms are not all finite takes scalar chains instead).
+//
+// A block stays in one wave from the raw rows to the codes: lane (li, lg) of 16 x 4 holds dims k = 4 kk + lg
+// of row li in 32 registers, which is the A operand of step kk as it is.
+//   norms    X X^T: A and B are the same registers, the diagonal holds the 16 sums of squares (15 of 16 products
+//            are thrown away, but no lane waits for another's chain: lane = row chains left 48 lanes idle
+//            and took as long as the rotation)
+//   xhat     x / norm from the norm's rounded reciprocal, in registers (div_by below)
+//   rotate   16 columns at a time against the rotation in LDS, stored in operand order (one 16-byte read a lane
+//            feeds four steps, no bank conflicts); K takes only the steps its columns' segments reach
+//   codes    four rows of one column per lane, straight from the accumulator
+//   corrected norms  the centroids of the codes, once more X X^T
+//   packing  a lane makes four bytes of a record: a byte is a dot product of four code bytes with powers of two
+//
+// CS 1: 16 waves share a rotation, each walks blocks of its own and no barrier is met on the way.  CS 4 (few
+// rows): the 4 waves of a work-group split the columns of one block, which quarters its longest stage.
+// Bound by the matrix cores: 320 instructions of 32 clocks a V block.  65 536 records each of K and V (4 x 8192
+// tokens, 2 heads, K3V3): 135 us as two launches of 16-row tiles on the vector units (there the dense V rotation
+// alone is 55 us of FMA), 65 us here in one.
+// ================================================================================================
+constexpr int RROW = D * 2 + 16;        // bytes from one raw row to the next: rows 4 banks apart
+constexpr int CROW = D + 8;             // bytes from one row of codes to the next (a byte's window of codes may reach 8 past the last)
+
+struct TileArgs { EncodeArgs k, v; int k_groups, v_groups; };      // work-groups per head of each kind (0: none)
+
+template <int CS>
+struct EncodeLds {
+    static constexpr int NW = CS == 1 ? 16 : 4;               // waves at most
+    static constexpr int NB = NW / CS;                        // blocks at a time
+    float rot[D / 4][D][4];             // the rotation, [step][column][k % 4]
+    alignas(16) uint8_t raw[NB][16 * RROW];                   // raw rows [row][k % 4][k / 4] fp16, later the codes
+    float2 nrm[NB][BGTQ_MAX_SEGMENTS][16];                    // (norm, its reciprocal) per group and row
+    int64_t dst[NB][16], ndst[NB][16];  // a row's record and norm offsets, -1: dropped
+    uint4 pack[D];                      // per record byte: first code, its bits (offset | width << 8), dot weights of the next ones
+    float cent[BGTQ_MAX_SEGMENTS * 32];
+    uint8_t lut[BGTQ_MAX_SEGMENTS * BGTQ_LUT_BINS];
+    int2 span[D / 16];                  // per 16 columns: first and last + 1 group of four steps
+    int hdr[56];
+    float2 bin[D];                      // K cell search of a packed dim
+    int8_t group[D];                    // its group, -1: a 0-bit dim
+    alignas(16) uint16_t place[D];      // source dim -> byte offset in a raw row
+};
+
+// x / d correctly rounded from y = RN(1 / d) (Markstein: a quotient within one unit in the last place and a
+// correctly rounded reciprocal give the rounded quotient after one residual step; the first step brings x * y
+// within that unit).  For finite x, and d and y normal.
+__device__ __forceinline__ float div_by(float x, float2 dy) {
+    float q = x * dy.y;
+    q = __builtin_fmaf(__builtin_fmaf(-dy.x, q, x), dy.y, q);
+    return __builtin_fmaf(__builtin_fmaf(-dy.x, q, x), dy.y, q);
+}
+
+template <int CS, bool IS_V>
+__device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, const int first, const int stride, EncodeLds<CS>& L) {
+    const int NW = CS == 1 ? (int)blockDim.x >> 6 : 4, NTHR = NW * 64, NB = NW / CS;       // (at least 4 waves)
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lg = lane >> 4;
+    const bgtq_head_plan& P = a.plans[h];
     const int64_t N = (int64_t)a.B * a.S;
-    encode_rows<16, IS_V>(a, blockIdx.x, blockIdx.y, (N + 15) / 16, gridDim.x, nullptr);
+    const int n_blocks = (int)((N + 15) / 16);
+    const bool need_cent = IS_V || a.layout == BGTQ_K_MIXED || a.corrected;
+
+    // ---- once per work-group: tables and the rotation (64 KB, straight from the plan into LDS).  Everything is
+    // requested in one burst; the dims' table is parked where the first raw rows go later
+    {
+        const uint32_t dst = (uint32_t)(uintptr_t)(lds_ptr_t)(uint8_t*)&L.rot[0][0][0];
+        if constexpr (IS_V) {                                 // (the plan holds it in this order)
+            const uint8_t* src = (const uint8_t*)&P.v_rot_T4[0][0][0];
+            for (int c = wave * 4; c < 64; c += NW * 4) dma_full<4>((uint32_t)lane * 16, uniform_ptr(src + c * 1024), dst + c * 1024);
+        } else {                                              // four rows interleaved on the way: lane = (column, row) of 16 x 4
+            const uint32_t off = (uint32_t)((lane & 3) * D + (lane >> 2)) * 4;
+            for (int c = wave; c < 256; c += NW) {            // (k_rot_T is zero outside a column's own segment)
+                const uint8_t* src = uniform_ptr((const uint8_t*)P.k_rot_T + (c >> 3) * (4 * D * 4) + (c & 7) * 64);
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1\n"
+                             :: "v"(off), "s"(src), "s"(dst + c * 256) : "memory", "m0");
+            }
+        }
+    }
+    int n_seg = 1, v_bits = 0, n_zero = 0;
+    float bd[15];                                             // V boundaries (+inf past the last)
+    uint2 byte_of = {0u, 0u};
+    int4* dims = (int4*)&L.raw[0][0];
+    static_assert(sizeof(int4) * D <= sizeof(L.raw[0]), "the dims' table fits one block's rows");
+    if constexpr (IS_V) {
+        v_bits = P.v_bits;
+#pragma unroll
+        for (int b = 0; b < 15; b++) bd[b] = P.v_boundaries[b];
+        if (tid < 16) L.cent[tid] = P.v_centroids[tid];
+        if (tid < D / 2) byte_of = *(const uint2*)P.enc_vbyte[a.layout == BGTQ_V_NIBBLE ? 1 : 0][tid];
+    } else {
+        n_seg = P.n_seg;
+        n_zero = P.n_zero_dims;
+        if (tid < 56) L.hdr[tid] = ((const int*)&P)[tid];
+        for (int i = tid; i < BGTQ_MAX_SEGMENTS * BGTQ_LUT_BINS / 4; i += NTHR) ((uint32_t*)L.lut)[i] = ((const uint32_t*)&P.code_lut[0][0])[i];
+        if (tid < BGTQ_MAX_SEGMENTS * 32) L.cent[tid] = P.k_centroids[tid >> 5][tid & 31];
+        if (tid < D) {
+            dims[tid] = *(const int4*)P.enc_dim[tid];
+            L.bin[tid] = float2{P.lut_offset[tid], P.lut_inv_scale[tid]};
+            byte_of = *(const uint2*)P.enc_byte[a.layout == BGTQ_K_MIXED ? 1 : 0][tid];
+        }
+    }
+    if constexpr (!IS_V) __syncthreads();
+    uint32_t seg_of[4] = {0, 0, 0, 0};                        // group of dim 4 kk + lg, 4 bits each
+    if constexpr (!IS_V) {
+#pragma unroll
+        for (int kk = 0; kk < D / 4; kk++) seg_of[kk >> 3] |= (uint32_t)max(dims[4 * kk + lg].x, 0) << (4 * (kk & 7));
+        if (tid < D / 16) {
+            int lo = D, hi = 0;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int4 dim = dims[16 * tid + i];
+                lo = min(lo, dim.x >= 0 ? dim.y : D);
+                hi = max(hi, dim.x >= 0 ? dim.z : 0);
+            }
+            L.span[tid] = int2{lo >> 4, (hi + 15) >> 4};
+        }
+    }
+    if (tid < D) {
+        const int k = tid;                                    // packed dim k lies at [k % 4][k / 4] of a raw row
+        int src = k;
+        if constexpr (!IS_V) { src = dims[k].w >> 8; L.group[k] = (int8_t)dims[k].x; }
+        L.place[src] = (uint16_t)(((k & 3) * (D / 4) + (k >> 2)) * 2);
+    }
+    const int lpr = a.row_width > 64 ? 32 : 16;               // packing: lanes per row, lane = record dword dw
+    const int dw = lane & (lpr - 1);
+    const bool dwords = ((a.row_width | a.p_st | a.p_sb | a.p_sh) & 3) == 0 && ((uintptr_t)a.packed & 3) == 0;
+    if (tid < D) {
+        // byte = (code 0 >> skip) + sum over the next codes of code << (its position in the byte)
+        const uint2 e = a.packed && tid < a.row_width ? byte_of : uint2{0u, 0u};
+        const int mode = (int)(e.x & 3u), bw = (int)((e.x >> 2) & 15u), skip = (int)((e.x >> 6) & 3u), n = (int)(e.x >> 8);
+        uint4 p = {e.y, 0u, 0u, 0u};
+        if (mode == 2 || (mode == 1 && n > 0)) p.y = (uint32_t)skip | ((8u - skip) << 8);
+        if (mode == 1)
+            for (int c = 1; c < n; c++) {
+                const uint32_t w = 1u << (c * bw - skip);
+                if (c < 4) p.z |= w << (8 * c);
+                else p.w |= (w >> 4) << (8 * (c - 4));        // (1-bit codes only: the second four make a nibble of their own)
+            }
+        L.pack[tid] = p;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // this wave's share of the rotation
+    __syncthreads();
+    // (a stream of 1-bit codes; groups are in ascending width)
+    const bool two_dots = IS_V ? v_bits == 1 && a.layout == BGTQ_V_BITPACKED : P.seg_bw[0] == 1 && a.layout == BGTQ_K_BITPACKED;
+
+    // ---- this wave's (CS 1) or this work-group's (CS 4) blocks
+    const int slot = CS == 1 ? wave : 0;
+    uint8_t* raw = L.raw[slot];
+    const bool wide = ((a.x_sb | a.x_sh | a.x_ss) & 7) == 0 && ((uintptr_t)a.x & 15) == 0;
+    auto meet = [&]() {
+        asm volatile("" ::: "memory");
+        if (CS > 1) __syncthreads();
+        else __builtin_amdgcn_wave_barrier();                 // (a wave's LDS accesses keep their order)
+        asm volatile("" ::: "memory");
+    };
+    // (CS 1: neighbouring blocks to the waves of one work-group)
+    for (int blk = CS == 1 ? first * NW + wave : first; blk < n_blocks; blk += stride * NB) {
+        const unsigned n0 = (unsigned)blk * 16u;
+        const int b0 = (int)(n0 / (unsigned)a.S), s0 = (int)(n0 - (unsigned)b0 * (unsigned)a.S);
+        auto row_of = [&](int r, int& b, int& s) {            // (batch row, step) of the block's row r
+            b = b0;
+            s = s0 + r;
+            if (s >= a.S) { const unsigned q = (unsigned)s / (unsigned)a.S; b += (int)q; s -= (int)q * a.S; }
+        };
+        // ---- raw rows to LDS: 16 lanes a row, 8 values each
+        {
+            constexpr int PASS = 4 / CS;
+            const int rc = lane & 15;
+            uint4 x4[PASS];
+#pragma unroll
+            for (int p = 0; p < PASS; p++) {
+                const int r = (CS == 1 ? 4 * p : 4 * wave) + (lane >> 4);
+                x4[p] = uint4{0, 0, 0, 0};
+                if ((int64_t)n0 + r < N) {
+                    int b, s;
+                    row_of(r, b, s);
+                    const uint16_t* src = a.x + b * a.x_sb + h * a.x_sh + s * a.x_ss + rc * 8;
+                    if (wide) x4[p] = *(const uint4*)src;
+                    else {
+                        uint32_t w[4];
+#pragma unroll
+                        for (int i = 0; i < 4; i++) w[i] = (uint32_t)src[2 * i] | ((uint32_t)src[2 * i + 1] << 16);
+                        x4[p] = uint4{w[0], w[1], w[2], w[3]};
+                    }
+                }
+            }
+            const uint4 at = *(const uint4*)&L.place[rc * 8];
+            const uint32_t at2[4] = {at.x, at.y, at.z, at.w};
+            if (lane < 16 && (CS == 1 || wave == 0)) {        // where the rows go
+                int64_t dst = -1, nd = -1;
+                if ((int64_t)n0 + lane < N) {
+                    int b, s;
+                    row_of(lane, b, s);
+                    const int64_t t = (int64_t)(a.t_pos ? a.t_pos[b] : a.t_pos_scalar) + s;
+                    if (a.codes_out) dst = nd = (int64_t)n0 + lane;
+                    else if (t >= 0 && t < a.max_T) {
+                        dst = b * a.p_sb + h * a.p_sh + t * a.p_st;
+                        nd = b * a.n_sb + h * a.n_sh + t * a.n_st;
+                    }
+                }
+                L.dst[slot][lane] = dst;
+                L.ndst[slot][lane] = nd;
+            }
+#pragma unroll
+            for (int p = 0; p < PASS; p++) {
+                uint8_t* row = raw + ((CS == 1 ? 4 * p : 4 * wave) + (lane >> 4)) * RROW;
+                uint32_t w[4] = {x4[p].x, x4[p].y, x4[p].z, x4[p].w};
+                if (a.bf16) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        w[i] = (uint32_t)bgtq_in16((uint16_t)w[i], 1) | ((uint32_t)bgtq_in16((uint16_t)(w[i] >> 16), 1) << 16);
+                }
+                if constexpr (IS_V) {                         // dims 8 rc + g and 8 rc + 4 + g are neighbours
+#pragma unroll
+                    for (int g = 0; g < 4; g++)
+                        *(uint32_t*)(row + g * (D / 2) + rc * 4) =
+                            __builtin_amdgcn_perm(w[2 + (g >> 1)], w[g >> 1], g & 1 ? 0x07060302u : 0x05040100u);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 8; i++)
+                        *(uint16_t*)(row + ((at2[i >> 1] >> (16 * (i & 1))) & 0xFFFFu)) = (uint16_t)(w[i >> 1] >> (16 * (i & 1)));
+                }
+            }
+        }
+        meet();
+        // ---- A operands (K reads them once its norms are known)
+        const uint8_t* arow = raw + li * RROW + lg * (D / 2);
+        float A[D / 4];
+        auto load_a = [&](int q) {                            // dims 32 q + 4 i + lg
+            const half8 v = *(const half8*)(arow + 16 * q);
+#pragma unroll
+            for (int i = 0; i < 8; i++) A[8 * q + i] = (float)v[i];
+        };
+        if constexpr (IS_V) {
+#pragma unroll
+            for (int q = 0; q < D / 32; q++) load_a(q);
+        }
+        // ---- norms: the diagonal of X X^T; lane (li, lg) holds (row 4 lg + r, row li) in register r
+        bool finite = true;
+        auto put_norm = [&](int g, const float4v& sum) {
+            const float ss = li & 2 ? (li & 1 ? sum[3] : sum[2]) : (li & 1 ? sum[1] : sum[0]);
+            const float n = __builtin_sqrtf(ss + 1e-30f);
+            const bool diag = (li >> 2) == lg;
+            finite = finite && (!diag || n < INFINITY);
+            if (diag) L.nrm[slot][g][li] = float2{n, 1.0f / n};
+        };
+        if constexpr (IS_V) {
+            float4v sum = {0, 0, 0, 0};
+#pragma unroll
+            for (int kk = 0; kk < D / 4; kk++) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(A[kk], A[kk], sum, 0, 0, 0);
+            put_norm(0, sum);
+        } else {
+            // (CS 4: the groups are dealt to the waves)
+            for (int g = CS == 1 ? 0 : wave; g < n_seg; g += CS == 1 ? 1 : CS) {
+                const int s = L.hdr[H_START + g], e = s + L.hdr[H_LEN + g];
+                float4v sum = {0, 0, 0, 0};
+                for (int q = s >> 4; q < (e + 15) >> 4; q++) {
+                    const uint2 w = *(const uint2*)(arow + 8 * q);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const int k = 16 * q + 4 * i + lg;
+                        const float x = k >= s && k < e ? bgtq_h2f((uint16_t)((i < 2 ? w.x : w.y) >> (16 * (i & 1)))) : 0.f;
+                        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(x, x, sum, 0, 0, 0);
+                    }
+                }
+                put_norm(g, sum);
+            }
+        }
+        bool scalar_chain = !IS_V && __builtin_amdgcn_ballot_w64(!finite) != 0;           // (uniform)
+        if (CS == 1 || IS_V) asm volatile("" ::: "memory");   // (V: every wave of a work-group has written the same norms)
+        else scalar_chain = __syncthreads_or(scalar_chain) != 0;
+        // ---- xhat.  (The contract divides by 1 where the norm is at most 1e-10, for V 1e-8: a non-zero fp16 value alone
+        // makes it 6e-8, so those norms belong to rows of zeros, which stay zeros whatever they are divided by.  An
+        // infinite or NaN norm of V makes every value of its row NaN, as the dense rotation would.)
+        if constexpr (IS_V) {
+            const float2 dy = L.nrm[slot][0][li];
+#pragma unroll
+            for (int kk = 0; kk < D / 4; kk++) A[kk] = div_by(A[kk], dy);
+        } else {
+#pragma unroll
+            for (int q = 0; q < D / 32; q++) {
+                load_a(q);
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const int kk = 8 * q + i;
+                    A[kk] = div_by(A[kk], L.nrm[slot][(seg_of[q] >> (4 * i)) & 15u][li]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (n_zero) {                                     // (uniform) 0-bit dims come first
+#pragma unroll
+                for (int kk = 0; kk < D / 4; kk++) A[kk] = 4 * kk + lg < n_zero ? 0.f : A[kk];
+            }
+        }
+        // codes of rows 4 lg .. + 3 from the values of column j
+        auto quantise = [&](const float4v& y, int j, int g) -> uint32_t {
+            uint32_t code[4] = {0, 0, 0, 0};
+            if constexpr (IS_V) {
+                auto count = [&](auto lo, auto hi) {           // (by halving: more instructions in the end, the choices cost as much)
+#pragma unroll
+                    for (int b = decltype(lo)::value; b < decltype(hi)::value; b++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) code[r] += y[r] > bd[b] ? 1u : 0u;
+                };
+                count(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
+                if (v_bits > 1) count(std::integral_constant<int, 1>{}, std::integral_constant<int, 3>{});      // (uniform)
+                if (v_bits > 2) count(std::integral_constant<int, 3>{}, std::integral_constant<int, 7>{});
+                if (v_bits > 3) count(std::integral_constant<int, 7>{}, std::integral_constant<int, 15>{});
+            } else if (a.quant_mode == BGTQ_QUANT_EXACT) {
+                const int nb = g >= 0 ? (1 << L.hdr[H_BW + g]) - 1 : 0;
+#pragma unroll 1
+                for (int b = 0; b < nb; b++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) code[r] += P.k_boundaries[g][b] < y[r] ? 1u : 0u;
+            } else {
+                const float off = L.bin[j].x, scale = L.bin[j].y;
+                const uint8_t* lut = &L.lut[max(g, 0) * BGTQ_LUT_BINS];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    float t = (y[r] - off) * scale;
+                    t = fminf(fmaxf(t, 0.0f), (float)(BGTQ_LUT_BINS - 1));
+                    code[r] = lut[(int)t];
+                }
+                if (n_zero) {                                 // (uniform)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) code[r] = g < 0 ? 0u : code[r];
+                }
+            }
+            return code[0] | (code[1] << 8) | (code[2] << 16) | (code[3] << 24);
+        };
+        uint32_t odd_codes[D / 16 / CS];                      // of a block with infinities or NaNs: scalar chains over the raw rows
+        if (!IS_V && scalar_chain) {
+#pragma unroll 1
+            for (int c = 0; c < D / 16 / CS; c++) {
+                const int j = 16 * (CS == 1 ? c : wave * (D / 16 / CS) + c) + li;
+                const int4 dim = *(const int4*)P.enc_dim[j];
+                float4v y = {0, 0, 0, 0};
+#pragma unroll 1
+                for (int r = 0; r < 4; r++) {
+                    const int row = 4 * lg + r;
+                    const float n = L.nrm[slot][max(dim.x, 0)][row].x, safe = n > 1e-10f ? n : 1.0f;
+                    float t = 0.f;
+                    for (int k = dim.w & 0xFF ? j : dim.y; dim.x >= 0 && k < (dim.w & 0xFF ? j + 1 : dim.z); k++) {
+                        const float x = bgtq_h2f(*(const uint16_t*)(raw + row * RROW + ((k & 3) * (D / 4) + (k >> 2)) * 2)) / safe;
+                        t = dim.w & 0xFF ? x : __builtin_fmaf(x, P.k_rot_T[k * D + j], t);
+                    }
+                    y[r] = t;
+                }
+                odd_codes[c] = quantise(y, j, dim.x);
+            }
+        }
+        // ---- rotate and quantise 16 columns at a time; codes of rows 4 lg .. + 3, column 16 cb + li
+        uint32_t codes[D / 16 / CS];
+#pragma unroll
+        for (int c = 0; c < D / 16 / CS; c++) {
+            const int cb = CS == 1 ? c : wave * (D / 16 / CS) + c;
+            const int j = 16 * cb + li;
+            float4v y = {0, 0, 0, 0};
+            const float* rot = &L.rot[0][j][lg];              // + step * 4 D: two steps a read
+            int g = 0;
+            if constexpr (IS_V) {
+#pragma unroll
+                for (int q = 0; q < D / 16; q++) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) y = __builtin_amdgcn_mfma_f32_16x16x4f32(A[4 * q + i], rot[(4 * q + i) * 4 * D], y, 0, 0, 0);
+                }
+            } else {
+                g = L.group[j];
+                if (scalar_chain) {
+                    codes[c] = odd_codes[c];
+                    continue;
+                }
+                {
+                    const int q_lo = __builtin_amdgcn_readfirstlane(L.span[cb].x), q_hi = __builtin_amdgcn_readfirstlane(L.span[cb].y);
+#pragma unroll
+                    for (int q = 0; q < D / 16; q++)
+                        if (q >= q_lo && q < q_hi) {          // (uniform)
+#pragma unroll
+                            for (int i = 0; i < 4; i++) y = __builtin_amdgcn_mfma_f32_16x16x4f32(A[4 * q + i], rot[(4 * q + i) * 4 * D], y, 0, 0, 0);
+                        }
+                }
+            }
+            codes[c] = quantise(y, j, g);
+            __builtin_amdgcn_sched_barrier(0);                // (operands of later columns would be read ahead and spill)
+        }
+        meet();                                               // (the raw rows are read)
+#pragma unroll
+        for (int c = 0; c < D / 16 / CS; c++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                raw[(4 * lg + r) * CROW + 16 * (CS == 1 ? c : wave * (D / 16 / CS) + c) + li] = (uint8_t)(codes[c] >> (8 * r));
+        meet();
+        // ---- norms to store
+        auto store_norm = [&](int g, int row, float out) {
+            const int64_t nd = L.ndst[slot][row];
+            if (nd < 0) return;
+            if (a.codes_out && !IS_V) { if (a.norms_f32_out && g < a.norm_width) a.norms_f32_out[nd * a.norm_width + g] = out; }
+            else if (g < (IS_V ? 1 : a.norm_width) && a.norms) a.norms[nd + g] = bgtq_f2h(out);
+        };
+        if (CS == 1 || wave == 0) {
+            if (need_cent) {
+                for (int g = 0; g < n_seg; g++) {
+                    int s = 0, e = D, bw = 0;
+                    if constexpr (!IS_V) { s = L.hdr[H_START + g]; e = s + L.hdr[H_LEN + g]; bw = L.hdr[H_BW + g]; }
+                    float4v sum = {0, 0, 0, 0};
+#pragma unroll 1
+                    for (int q = s >> 4; q < (e + 15) >> 4; q++) {
+                        const uint32_t* cw = (const uint32_t*)&raw[li * CROW + 16 * q];
+                        float c[4];
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            const int k = 16 * q + 4 * i + lg;
+                            const uint32_t code = (cw[i] >> (8 * lg)) & 0xFFu;
+                            if constexpr (IS_V) c[i] = L.cent[code & 15u];
+                            else {
+                                c[i] = bw > 5 ? P.k_centroids[g][code] : L.cent[g * 32 + (code & 31u)];
+                                if (k < s || k >= e) c[i] = 0.f;
+                            }
+                        }
+#pragma unroll
+                        for (int i = 0; i < 4; i++) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(c[i], c[i], sum, 0, 0, 0);
+                    }
+                    const float cs = li & 2 ? (li & 1 ? sum[3] : sum[2]) : (li & 1 ? sum[1] : sum[0]);
+                    if ((li >> 2) == lg) {
+                        const float n = L.nrm[slot][g][li].x;
+                        if constexpr (IS_V) {
+                            const float cn = __builtin_sqrtf(cs + 1e-20f);
+                            store_norm(0, li, n / (cn > 1e-10f ? cn : 1.0f));
+                        } else {
+                            store_norm(g, li, n / fmaxf(__builtin_sqrtf(cs), 1e-10f));
+                        }
+                    }
+                }
+                if (!IS_V)
+                    for (int i = lane; i < (BGTQ_MAX_SEGMENTS - n_seg) * 16; i += 64) store_norm(n_seg + (i >> 4), i & 15, 0.f);
+            } else {
+                for (int i = lane; i < BGTQ_MAX_SEGMENTS * 16; i += 64) {
+                    const int g = i & 7, row = i >> 3;
+                    store_norm(g, row, g < n_seg ? L.nrm[slot][g][row].x : 0.f);
+                }
+            }
+        }
+        // ---- records
+        if (a.codes_out) {
+            for (int i = CS == 1 ? lane : tid; i < 16 * (D / 4); i += 64 * CS) {
+                const int64_t n = L.dst[slot][i >> 5];
+                if (n >= 0) *(uint32_t*)&a.codes_out[n * D + 4 * (i & 31)] = *(const uint32_t*)&raw[(i >> 5) * CROW + 4 * (i & 31)];
+            }
+        } else if (4 * dw < a.row_width) {
+            const int rows = 64 / lpr;
+#pragma unroll 2
+            for (int r = lane / lpr + (CS == 1 ? 0 : wave * rows); r < 16; r += rows * CS) {
+                const int64_t dst = L.dst[slot][r];
+                if (dst < 0) continue;
+                uint32_t byte[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const uint4 p = L.pack[4 * dw + i];
+                    const uint32_t* c = (const uint32_t*)&raw[r * CROW + (p.x & ~3u)];
+                    const uint32_t c0 = c[0], c1 = c[1];
+                    const uint32_t x = __builtin_amdgcn_alignbyte(c1, c0, p.x & 3u);
+                    byte[i] = __builtin_amdgcn_udot4(x, p.z, __builtin_amdgcn_ubfe(x, p.y & 0xFFu, p.y >> 8), false);
+                    if (two_dots) byte[i] += __builtin_amdgcn_udot4(__builtin_amdgcn_alignbyte(c[2], c1, p.x & 3u), p.w, 0u, false) << 4;
+                }
+                const uint32_t w = __builtin_amdgcn_perm(byte[1], byte[0], 0x0C0C0400u) | __builtin_amdgcn_perm(byte[3], byte[2], 0x04000C0Cu);
+                if (dwords) *(uint32_t*)(a.packed + dst + 4 * dw) = w;
+                else
+                    for (int i = 0; i < 4; i++)
+                        if (4 * dw + i < a.row_width) a.packed[dst + 4 * dw + i] = (uint8_t)(w >> (8 * i));
+            }
+        }
+        meet();                                               // the next block's rows overwrite codes and offsets
+    }
+}
+
+template <int CS>
+__global__ __launch_bounds__(EncodeLds<CS>::NW * 64) void encode_blocks_kernel(TileArgs t) {
+    __shared__ __align__(16) EncodeLds<CS> L;
+    int bid = blockIdx.x;
+    const int nv = t.v_groups * t.v.n_kv;                     // (V blocks, the longer ones, go out first)
+    if (bid < nv) encode_blocks<CS, true>(t.v, bid % t.v.n_kv, bid / t.v.n_kv, t.v_groups, L);
+    else {
+        bid -= nv;
+        encode_blocks<CS, false>(t.k, bid % t.k.n_kv, bid / t.k.n_kv, t.k_groups, L);
+    }
+}
+
+// K and / or V rows in blocks; either pointer may be null
+int launch_blocks(const EncodeArgs* k, const EncodeArgs* v, hipStream_t st) {
+    const EncodeArgs& any = k ? *k : *v;
+    const int64_t N = (int64_t)any.B * any.S;
+    if (N > INT32_MAX - 64) return BGTQ_EINVAL;               // the kernels index rows with 32 bits
+    const int kinds = (k ? 1 : 0) + (v ? 1 : 0);
+    TileArgs t{};
+    if (k) t.k = *k;
+    if (v) t.v = *v;
+    const int64_t blocks = (N + 15) / 16;
+    if (blocks * any.n_kv * kinds <= 512) {                   // (two work-groups fit a compute unit: one round)
+        t.k_groups = k ? (int)blocks : 0;
+        t.v_groups = v ? (int)blocks : 0;
+        hipLaunchKernelGGL(encode_blocks_kernel<4>, dim3((unsigned)(blocks * any.n_kv * kinds)), dim3(256), 0, st, t);
+        return bgtq_launch_status();
+    }
+    // One work-group of up to 16 waves a compute unit, in equal shares over kinds and heads, each wave the same
+    // number of blocks; with fewer than 16 blocks a work-group, that many waves.
+    const int64_t most = std::max<int64_t>(1, 256 / (any.n_kv * kinds));
+    const int64_t share = (blocks + most - 1) / most, rounds = (share + 15) / 16;
+    const int nw = (int)std::max<int64_t>(4, (share + rounds - 1) / rounds);
+    const int groups = (int)((blocks + nw * rounds - 1) / (nw * rounds));
+    t.k_groups = k ? groups : 0;
+    t.v_groups = v ? groups : 0;
+    hipLaunchKernelGGL(encode_blocks_kernel<1>, dim3((unsigned)(groups * kinds * any.n_kv)), dim3(nw * 64), 0, st, t);
+    return bgtq_launch_status();
 }
 
 template <bool IS_V>
 int launch_encode(const EncodeArgs& a, hipStream_t st) {
-    int64_t N = (int64_t)a.B * a.S;
+    const int64_t N = (int64_t)a.B * a.S;
     if (N == 0 || a.n_kv == 0) return BGTQ_OK;
-    if (N > INT32_MAX) return BGTQ_EINVAL;        // the kernels index rows with 32 bits
-    // Few rows (decode append): small tiles so every row gets its own work-group
-    // and the step stays latency-bound; many rows (prefill): 16-row tiles so the
-    // rotation matrix is amortised.
-    if (N <= 32) {               // one row a work-group: the shortest chain of dependent stages
-        dim3 grid((unsigned)N, (unsigned)a.n_kv);
-        hipLaunchKernelGGL((encode_kernel<1, IS_V>), grid, dim3(NT), 0, st, a);
-    } else if (N <= 64) {
-        dim3 grid((unsigned)((N + 1) / 2), (unsigned)a.n_kv);
-        hipLaunchKernelGGL((encode_kernel<2, IS_V>), grid, dim3(NT), 0, st, a);
-    } else {
-        // a work-group stages its head's plan once and walks several tiles: about 10
-        // work-groups per CU in total
-        int64_t tiles = (N + 15) / 16;
-        int64_t want = (256 * 10 + a.n_kv - 1) / a.n_kv;
-        dim3 grid((unsigned)(tiles < want ? tiles : want), (unsigned)a.n_kv);
-        hipLaunchKernelGGL((encode_kernel16<IS_V>), grid, dim3(NT), 0, st, a);
-    }
+    // few rows (a decode append): one row a work-group, the shortest chain of dependent stages
+    if (N > 32) return IS_V ? launch_blocks(nullptr, &a, st) : launch_blocks(&a, nullptr, st);
+    hipLaunchKernelGGL((encode_kernel<1, IS_V>), dim3((unsigned)N, (unsigned)a.n_kv), dim3(NT), 0, st, a);
     return bgtq_launch_status();
 }
 
@@ -781,9 +1246,7 @@ int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, in
     const int B = ak.B, n_kv = ak.n_kv;
     const int64_t N = (int64_t)B * ak.S;
     if (N > 64) {          // prefill-sized append: the three stages are big enough on their own
-        int rc = launch_encode<false>(ak, st);
-        if (rc != BGTQ_OK) return rc;
-        rc = launch_encode<true>(av, st);
+        const int rc = launch_blocks(&ak, &av, st);
         if (rc != BGTQ_OK || !q) return rc;
         return launch_rotate_q(ak.plans, q, q_sr, q_sh, q_bf16, q_rot, qr_sr, qr_sh, B, n_kv, gqa, st);
     }

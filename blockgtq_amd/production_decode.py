@@ -24,8 +24,11 @@ def production_prefill(model, input_ids, cache, chunk_encode=64):
     """Prefill with the model's own attention, then pack its fp16 K/V.
 
     Runs the HF forward with a ``DynamicCache``, reads the post-RoPE K/V of
-    every layer back and encodes them into ``cache`` in slices of
-    ``chunk_encode`` tokens.  Returns the prompt logits.
+    every layer back and encodes them into ``cache``, one launch per layer.
+    ``chunk_encode`` bounded the reference encoder's temporaries by slicing the
+    prompt; rows are encoded independently and without temporaries here, so it
+    changes nothing and is ignored (a 2001-token prompt of 8 KV heads: 374 us in
+    slices of 64, host bound, 50 us whole).  Returns the prompt logits.
     """
     from transformers import DynamicCache
 
@@ -35,9 +38,7 @@ def production_prefill(model, input_ids, cache, chunk_encode=64):
     out = model(input_ids, position_ids=position_ids, past_key_values=hf_cache, use_cache=True)
     for li in range(cache.n_layers):
         k, v = _layer_kv(hf_cache, li)
-        for lo in range(0, prompt_len, chunk_encode):
-            hi = min(lo + chunk_encode, prompt_len)
-            cache._encode_batched(li, k[:, :, lo:hi], v[:, :, lo:hi], lo)
+        cache._encode_batched(li, k, v, 0)
     cache.seq_len = prompt_len
     del hf_cache
     return out.logits
