@@ -82,6 +82,17 @@ _SIGNATURES = {
                                 c_i, c_i, c_i, c_i, c_i, c_i, c_i,
                                 c_i, c_i, ctypes.c_float, c_i,
                                 c_p, c_i64, c_i64, c_i64, c_p]),
+    "bgtq_decode_step": (c_i, [c_p, c_p]),
+    "bgtq_encode_kv": (c_i, [c_p, c_p]),
+    "bgtq_prompt_workspace_bytes": (ctypes.c_size_t, [c_i, c_i, c_i, c_i, c_i]),
+    "bgtq_prompt_attn": (c_i, [c_p, c_p, c_i, c_i, c_i64, c_i64, c_i64,
+                               c_p, c_i64, c_i64, c_i64, c_i,
+                               c_p, c_i64, c_i64, c_i64,
+                               c_p, c_i64, c_i64, c_i64, c_i,
+                               c_p, c_i64, c_i64, c_i64,
+                               c_i, c_i, c_i, c_i, c_i, c_i, c_i,
+                               c_i, c_i, c_f, c_i, c_p, ctypes.c_size_t,
+                               c_p, c_i64, c_i64, c_i64, c_p]),
     "bgtq_lse_reduce": (c_i, [c_p, c_p, c_p, c_i, c_p, c_p, c_i,
                               c_i, c_i, c_i, c_i, c_p, c_i64, c_i64, c_p, c_p]),
 }

@@ -30,6 +30,7 @@ SOURCES = {
     "bgtq_decode_seg.hip": ["-fno-strict-aliasing"],
     "bgtq_dequant.hip": [],
     "bgtq_prefill.hip": ["-fno-strict-aliasing"],
+    "bgtq_prompt.hip": ["-fno-strict-aliasing"],
 }
 
 

@@ -333,6 +333,49 @@ PyObject* attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return THPVariable_Wrap(std::move(out));
 }
 
+// ------------------------------------------------------------------------------------------ prompt phase
+// prompt(plans, q (B, n_q, S, D), rotate_q, k_packed, k_norms, v_packed, v_norms, T, k_row_width, v_row_width,
+//        q_pos_offset, is_causal, k_layout, v_layout, scale, unrotate) -> (B, n_q, S, D) fp16, or None
+PyObject* prompt(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    int64_t rotate, T, kw, vw, off, causal, kl, vl, unrotate;
+    if (n != 16 || !as_int(a[2], rotate) || !as_int(a[7], T) || !as_int(a[8], kw) || !as_int(a[9], vw) || !as_int(a[10], off) ||
+        !as_int(a[11], causal) || !as_int(a[12], kl) || !as_int(a[13], vl) || !PyFloat_Check(a[14]) || !as_int(a[15], unrotate)) Py_RETURN_NONE;
+    const at::Tensor* t[6];
+    const int at6[6] = {0, 1, 3, 4, 5, 6};
+    for (int i = 0; i < 6; i++) {
+        t[i] = tensor(a[at6[i]]);
+        if (!t[i] || !t[i]->is_cuda()) Py_RETURN_NONE;
+    }
+    const at::Tensor &plans = *t[0], &q = *t[1], &kp = *t[2], &kn = *t[3], &vp = *t[4], &vn = *t[5];
+    for (int i = 0; i < 6; i++)
+        if (t[i]->get_device() != q.get_device()) Py_RETURN_NONE;
+    if (q.dim() != 4 || !is_x(q, q.get_device()) || q.size(3) != D || (!rotate && q.scalar_type() != at::kHalf)) Py_RETURN_NONE;
+    if (kp.dim() != 4 || kn.dim() != 4 || vp.dim() != 4 || vn.dim() != 3 || kp.scalar_type() != at::kByte || vp.scalar_type() != at::kByte ||
+        kn.scalar_type() != at::kHalf || vn.scalar_type() != at::kHalf || kp.stride(3) != 1 || vp.stride(3) != 1 || kn.stride(3) != 1) Py_RETURN_NONE;
+    const int64_t B = q.size(0), n_q = q.size(1), S = q.size(2), n_kv = kp.size(1);
+    if (n_kv < 1 || n_q % n_kv || kp.size(2) < T || vp.size(2) < T || kn.size(2) < T || vn.size(2) < T || T < 0 || kp.size(0) < B) Py_RETURN_NONE;
+    const size_t bytes = bgtq_prompt_workspace_bytes((int)B, (int)n_kv, (int)(n_q / n_kv), (int)S, (int)T);
+    // (the allocator hands the same block out again from call to call, and to nobody else before the launches are done)
+    at::Tensor ws = at::empty({(int64_t)bytes}, q.options().dtype(at::kByte));
+    at::Tensor out = at::empty({B, n_q, S, D}, q.options().dtype(at::kHalf));
+    void* st = stream_of(q);
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = bgtq_prompt_attn((const bgtq_head_plan*)plans.data_ptr(), q.data_ptr(), q.scalar_type() == at::kBFloat16 ? BGTQ_X_BF16 : BGTQ_X_FP16,
+                          (int)rotate, q.stride(0), q.stride(1), q.stride(2),
+                          kp.data_ptr(), kp.stride(0), kp.stride(1), kp.stride(2), (int)kw,
+                          kn.data_ptr(), kn.stride(0), kn.stride(1), kn.stride(2),
+                          vp.data_ptr(), vp.stride(0), vp.stride(1), vp.stride(2), (int)vw,
+                          vn.data_ptr(), vn.stride(0), vn.stride(1), vn.stride(2),
+                          (int)B, (int)n_kv, (int)(n_q / n_kv), (int)S, (int)T, (int)off, (int)causal, (int)kl, (int)vl,
+                          (float)PyFloat_AS_DOUBLE(a[14]), (int)unrotate, ws.data_ptr(), bytes,
+                          out.data_ptr(), out.stride(0), out.stride(1), out.stride(2), st);
+    Py_END_ALLOW_THREADS
+    if (rc == BGTQ_EUNSUPPORTED) Py_RETURN_NONE;
+    if (rc != BGTQ_OK) return fail("bgtq_prompt_attn", rc);
+    return THPVariable_Wrap(std::move(out));
+}
+
 PyObject* setup(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 2) { PyErr_SetString(PyExc_TypeError, "setup(error class, path hook)"); return nullptr; }
     Py_INCREF(a[0]);
@@ -346,6 +389,7 @@ PyObject* setup(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 PyMethodDef module_methods[] = {
     {"attend", (PyCFunction)(void*)attend, METH_FASTCALL, "decode attention over packed records, or None"},
+    {"prompt", (PyCFunction)(void*)prompt, METH_FASTCALL, "prompt-phase attention over packed records, or None"},
     {"setup", (PyCFunction)(void*)setup, METH_FASTCALL, "hand over the error class and the hook that notes which kernel ran"},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -31,7 +31,7 @@
 // driver blockgtq/prefill.py:66-101.
 #include <atomic>
 
-#include "bgtq_lds.h"
+#include "bgtq_dequant_tile.h"
 
 namespace {
 
@@ -42,13 +42,10 @@ constexpr int MT = 64;                       // tokens per tile
 constexpr int NWAVES = 8;                    // (4 waves and 128 rows: 13 % slower, the tile is dequantised twice as often per row)
 constexpr int ROWS = 32 * NWAVES;            // query rows per work-group (32 per wave)
 constexpr int NTHR = 64 * NWAVES;
-constexpr int V_UNITS_PER_THREAD = 16 * 32 / NTHR;   // V tile: 32 token pairs x 16 units over the threads
-constexpr int MAX_UNITS = BGTQ_MAX_UNITS;
 constexpr int MAX_KN = 8;
-constexpr int UPW = (MAX_UNITS + NWAVES - 1) / NWAVES;   // K units per wave
 constexpr float REFRESH = 4.0f;
-constexpr int KROW = D * 2 + 16;             // bytes of a K tile row: rows 4 banks apart
-constexpr int VTROW = MT * 2 + 16;           // bytes of a transposed V tile row (one dim, 64 tokens)
+constexpr int KROW = DQ_KROW, VTROW = DQ_VTROW;
+static_assert(MT == DQ_MT && NWAVES == DQ_WAVES, "");
 
 // LDS layout (bytes): [V table | K tables | 2 x (raw K | K norms | V norms | raw V) | 2 x (K tile | V^T tile)]
 constexpr int VTAB_OFF = 0;
@@ -79,11 +76,6 @@ __host__ __device__ inline int raw_bytes(int krow, int vstride, int kn_st, int& 
     return kt + knr + vnr + vt;
 }
 
-__device__ __forceinline__ uint32_t pk_mul_f16(uint32_t a, uint32_t b) {
-    uint32_t r;
-    asm("v_pk_mul_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
 __device__ __forceinline__ uint32_t cvt_pk_f16(float lo, float hi) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
     h2 r = {(_Float16)lo, (_Float16)hi};
@@ -104,8 +96,6 @@ __global__ __launch_bounds__(NTHR, 8 / NWAVES) void prefill_mfma_kernel(PrefillA
     const int qb = (int)gridDim.z - 1 - (int)blockIdx.z;
     const int s0 = qb * BQ;
     const int krow = a.k_row_width, vrow = a.v_stride, kn_st = (int)a.kn_st;
-    const int vbw = vnib ? 4 : (int)P.v_bits;                    // bits of a V code as stored
-    const bool vrep = !vnib && vbw <= 3;                         // V pair table replicated over the banks
 
     // ---- the tiles this work-group walks
     const int s_last = min(s0 + BQ, a.S) - 1;
@@ -128,23 +118,7 @@ __global__ __launch_bounds__(NTHR, 8 / NWAVES) void prefill_mfma_kernel(PrefillA
 
     // ---- tables into LDS
     const uint32_t voff = (uint32_t)lane * 16;
-    {
-        const uint8_t* vimg = (const uint8_t*)P.vlut_image[vnib ? 1 : 0];
-        const uint8_t* kimg = (const uint8_t*)P.lut_image[kl];
-        const int vbytes = (vnib || vbw == 4) ? 1024 : (1 << (2 * vbw)) * 128;
-        const int kbytes = kl == BGTQ_K_MIXED ? BGTQ_LUTM_KEND : BGTQ_LUT_KEND;
-        const int vch = (vbytes + 1023) >> 10, kch = (kbytes + 1023) >> 10;
-        for (int cc = wave; cc < vch + kch; cc += NTHR / 64) {
-            const uint8_t* src;
-            uint32_t dst;
-            int left;
-            if (cc < vch) { src = vimg + cc * 1024; dst = VTAB_OFF + cc * 1024; left = vbytes - cc * 1024; }
-            else { src = kimg + (cc - vch) * 1024; dst = KTAB_OFF + (cc - vch) * 1024; left = kbytes - (cc - vch) * 1024; }
-            dma16(voff, src, __builtin_amdgcn_readfirstlane(dst), __builtin_amdgcn_ballot_w64((int)voff < left));
-        }
-    }
-    const int n_units = min(P.n_units[kl], MAX_UNITS), n_pair = min(P.n_pair_units[kl], n_units);
-    const uint32_t kend = P.kend[kl], kfirst0 = P.kfirst[kl][0], kfirst1 = P.kfirst[kl][1];
+    dq_load_tables(P, kl, vnib, vnib ? 4 : (int)P.v_bits, wave, voff);
     const int n_zero = min(max(P.n_zero_dims, 0), D);
 
     // ---- the wave's queries as B operands: lane (query li, half lg) holds dims 16 kk + 8 lg .. + 7 of step kk
@@ -188,135 +162,20 @@ __global__ __launch_bounds__(NTHR, 8 / NWAVES) void prefill_mfma_kernel(PrefillA
     }
 
     const float c2 = a.scale * 1.44269504088896340736f;        // scores in log2 units
-    const uint32_t rep = ((uint32_t)lane & 31u) * 4u;
     float16v O[4];                                              // O^T: block db = dims 32 db .., reg r -> dim 32 db + 8 (r / 4) + 4 lg + r % 4
 #pragma unroll
     for (int db = 0; db < 4; db++) O[db] = (float16v){0};
     float m_ref = -INFINITY, l_part = 0.f;                       // per query (this half's share of the denominator)
 
-    // K dequantisation: lane = token, wave w takes units w, w + NWAVES, ... (parameters: ku[] below)
     const uint32_t krow_l0 = RAW_OFF + kph + (uint32_t)lane * krow;                    // set 0; + raw_set for set 1
     const uint32_t knrow_l0 = RAW_OFF + a.kt + knph + (uint32_t)lane * kn_st * 2;
-    // V dequantisation: thread (token pair tp, unit up); code pair e of a unit's raw word is brought to
-    // the table-index position by a rotation (the V table sits at LDS address 0).  Neighbouring lanes take
-    // neighbouring units of one token pair: a half-wave then reads 16 token pairs (records 96 bytes apart fall on
-    // 8 banks) instead of 32
-    const int tp = (tid >> 1) & 31, up = 2 * (tid >> 6) + (tid & 1);
-    // Column order of the V^T tile: inside every group of 16 tokens, token x sits at position
-    // 8 ((x >> 2) & 1) + 4 (x >> 3) + (x & 3), so that the 8 tokens {4 g + i, 8 + 4 g + i} a half-wave g contracts in
-    // one MFMA step are 16 contiguous bytes.  Tokens 2 tp and 2 tp + 1 stay neighbours: byte offset of their dword
-    const uint32_t vcol = (uint32_t)(8 * (tp >> 3) + 4 * ((tp >> 1) & 1) + 2 * ((tp >> 2) & 1) + (tp & 1)) * 4;
-    const int vtsh = vrep ? 7 : 2;
-    uint32_t vrot[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) vrot[e] = (uint32_t)(2 * vbw * e - vtsh) & 31u;
-    const uint32_t vfmask = ((1u << (2 * vbw)) - 1u) << vtsh, vbase = vrep ? rep : 0u;
-
-    // The K units of this wave (w, w + NWAVES, then the third round shifted by half): their parameters stay in scalar registers for the
-    // whole walk.  A unit the wave does not have reads valid addresses and stores nothing (len 0).
-    struct KUnit { uint32_t rot[4], mask, tab, repm, off, d0x2, seg2; int len; bool raw; };
-    KUnit ku[UPW];
-#pragma unroll
-    for (int i = 0; i < UPW; i++) {
-        // the third round starts at wave NWAVES / 2: the first waves also issue the tile loads
-        const int u = i < 2 ? wave + i * NWAVES : i * NWAVES + (wave + NWAVES / 2) % NWAVES;
-        const bool have = u < n_units;
-        const int uu = have ? u : 0;
-        const uint32_t dsc = P.kunit[kl][uu];
-        ku[i].len = have ? (int)(dsc >> 8) & 0xFF : 0;
-        ku[i].d0x2 = (dsc & 0xFF) * 2;
-        ku[i].raw = have && ku[i].len > 0 && u >= n_pair;
-        const bool pair = have && ku[i].len > 0 && u < n_pair;
-#pragma unroll
-        for (int e = 0; e < 4; e++) ku[i].rot[e] = pair ? P.kprog[kl][uu][e] : 0u;
-        ku[i].mask = pair ? P.kprog[kl][uu][4] : 0u;
-        ku[i].tab = ku[i].len > 0 ? P.kprog[kl][uu][5] : (uint32_t)KTAB_OFF;
-        ku[i].repm = pair ? P.kprog[kl][uu][6] : 0u;
-        ku[i].off = ku[i].len == 0 ? 0u : uu == 0 ? kfirst0 : uu == 1 ? kfirst1 : P.kprog[kl][uu - 2][7];
-        ku[i].seg2 = ku[i].len == 0 ? 0u : 2u * (uint32_t)__builtin_popcount(kend & ((1u << uu) - 1u));
-    }
-
+    TileDequant dq;
+    dq.init(P, kl, vnib, tid);
     // Dequantise raw tile `tile` (set tile & 1) into the K and V^T tiles of the same set.
     auto dequant_tile = [&](int tile) {
-        const int nt = min(MT, t_end - tile * MT);               // records of this tile; the rows behind them hold stale bytes
-        const uint32_t set = (uint32_t)(tile & 1);
-        const uint32_t krow_l = krow_l0 + set * raw_set, knrow_l = knrow_l0 + set * raw_set;
-        const uint32_t vnraw = RAW_OFF + set * raw_set + a.kt + a.knr, vraw = vnraw + a.vnr;
-        const uint32_t ktile = tiles0 + set * tile_set, vtile = ktile + MT * KROW;
-        // K tile [token][dim] (packed-dim order) and V^T tile [dim][token], both fp16(centroid * norm).  K: lane =
-        // token, the wave's own units; V: thread = tokens 2 tp, 2 tp + 1 of V_UNITS_PER_THREAD units.  Both go
-        // through the same three stages together, without a branch between them, so that all LDS round trips
-        // of a stage overlap: codes and norms, table lookups, products and stores.
-        uint32_t nn[UPW], kw[UPW][4];
-        uint2v rr[UPW];
-        uint32_t nrm[2], vr[V_UNITS_PER_THREAD][2], vw[V_UNITS_PER_THREAD][2][4];
-        // ---- stage 1
-#pragma unroll
-        for (int i = 0; i < UPW; i++) {
-            // rows past the tile's last record get norm 0: their products must stay finite (P is 0 there)
-            const uint32_t n16 = lds_at<uint16_t>(knrow_l + ku[i].seg2);
-            nn[i] = lane < nt ? n16 | (n16 << 16) : 0u;
-            rr[i] = lds_codes8(krow_l + ku[i].off);
-        }
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const uint32_t n16 = lds_at<uint16_t>(vnraw + vnph + (uint32_t)(2 * tp + j) * 2);
-            nrm[j] = 2 * tp + j < nt ? n16 | (n16 << 16) : 0u;
-        }
-#pragma unroll
-        for (int uu = 0; uu < V_UNITS_PER_THREAD; uu++)
-#pragma unroll
-            for (int j = 0; j < 2; j++)
-                vr[uu][j] = lds_codes4(vraw + vph + (uint32_t)(2 * tp + j) * vrow + (uint32_t)((V_UNITS_PER_THREAD * up + uu) * vbw));
-        // ---- stage 2
-#pragma unroll
-        for (int i = 0; i < UPW; i++) {
-            const uint32_t r = rr[i].x;
-            const uint32_t base = and_or(rep, ku[i].repm, ku[i].tab);
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                kw[i][e] = lds_at<uint32_t>(and_or(__builtin_amdgcn_alignbit(r, r, ku[i].rot[e]), ku[i].mask, base));
-        }
-#pragma unroll
-        for (int uu = 0; uu < V_UNITS_PER_THREAD; uu++)
-#pragma unroll
-            for (int j = 0; j < 2; j++)
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    vw[uu][j][e] = lds_at<uint32_t>(and_or_v(__builtin_amdgcn_alignbit(vr[uu][j], vr[uu][j], vrot[e]), vfmask, vbase));
-#pragma unroll
-        for (int i = 0; i < UPW; i++) {
-            if (ku[i].raw) {                                     // (wave-uniform) one byte per code, one fp16 per table entry
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const uint32_t x = e < 2 ? rr[i].x : rr[i].y;
-                    const uint32_t c0 = ku[i].tab + ((x >> ((e & 1) * 16)) & 0xFF) * 2;
-                    const uint32_t c1 = ku[i].tab + ((x >> ((e & 1) * 16 + 8)) & 0xFF) * 2;
-                    kw[i][e] = (uint32_t)lds_at<uint16_t>(c0) | ((uint32_t)lds_at<uint16_t>(c1) << 16);
-                }
-            }
-        }
-        // ---- stage 3.  A dim pair past the unit's last dim goes to the 16 spare bytes at the end of the lane's
-        // K tile row, which nothing reads.
-        const uint32_t krow_t = ktile + (uint32_t)lane * KROW;
-#pragma unroll
-        for (int i = 0; i < UPW; i++)
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                lds_put<uint32_t>(krow_t + (2 * e < ku[i].len ? ku[i].d0x2 + e * 4 : (uint32_t)(D * 2)), pk_mul_f16(kw[i][e], nn[i]));
-#pragma unroll
-        for (int uu = 0; uu < V_UNITS_PER_THREAD; uu++) {
-            const int u = V_UNITS_PER_THREAD * up + uu;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const uint32_t w0 = pk_mul_f16(vw[uu][0][e], nrm[0]), w1 = pk_mul_f16(vw[uu][1][e], nrm[1]);
-                // (dim 8u + 2e of both tokens), (dim 8u + 2e + 1 of both tokens)
-                const uint32_t lo = __builtin_amdgcn_perm(w1, w0, 0x05040100u);
-                const uint32_t hi = __builtin_amdgcn_perm(w1, w0, 0x07060302u);
-                lds_put<uint32_t>(vtile + (uint32_t)(8 * u + 2 * e) * VTROW + vcol, lo);
-                lds_put<uint32_t>(vtile + (uint32_t)(8 * u + 2 * e + 1) * VTROW + vcol, hi);
-            }
-        }
+        const uint32_t set = (uint32_t)(tile & 1), raw0 = set * raw_set, ktile = tiles0 + set * tile_set;
+        const uint32_t vn0 = RAW_OFF + raw0 + a.kt + a.knr;
+        dq.run(krow_l0 + raw0, knrow_l0 + raw0, vn0 + vnph, vn0 + a.vnr + vph, vrow, min(MT, t_end - tile * MT), ktile, ktile + MT * KROW);
     };
 
     // Pipeline: while the products of tile i run, tile i + 1 is dequantised into the other set of tiles and the

@@ -1,0 +1,645 @@
+// Prompt-phase attention with a workspace (gfx950): records staged once, then a plain matrix-core attention.
+//
+// bgtq_prefill_attn dequantises every tile in every work-group that sees it, 128 times over for an 8k prompt of 8
+// query heads a KV head, and that is half of its time.  Here three kernels share the work:
+//
+//   stage   every 64-token tile is dequantised once into 32 KB of the workspace, already in the order in which
+//           the attention's waves read their matrix operands (a fragment is 64 lanes x 16 bytes that follow each
+//           other), so that a tile travels to LDS as it lies and every LDS read is a contiguous kilobyte.  The
+//           query rotation and the value un-rotation of a head are split here into fp16 (bf16 for bf16 queries)
+//           parts in operand order, too.
+//   attend  NW waves, 32 query rows each: 32 NW / gqa tokens of every query head of the group.  The rows
+//           are rotated at the start and un-rotated at the end inside the kernel, on the same matrix cores.
+//           S^T = K Q^T puts one query in each lane, so softmax statistics stay in the lane, and P goes from the
+//           score registers straight into O^T = V^T P^T.  Where an accumulator serves as an operand again (rotated
+//           queries, probabilities, outputs), the contraction index is permuted: slot 16 s + 8 g + e of a 32-block
+//           holds index 16 s + 8 (e / 4) + 4 g + e % 4, which is where half-wave g keeps its register 8 s + e.
+//   merge   only where a few query rows meet a long context: the tiles of a query block are dealt to several
+//           work-groups, whose unnormalised sums this kernel adds and un-rotates.
+//
+// Arithmetic as in bgtq_prefill_attn: fp16(centroid * norm) records, fp16 rotated queries and probabilities, fp32
+// sums; rotations from parts that hold 22 (fp16) or 24 (bf16) bits of the fp32 matrices, summed in fp32.
+//
+// Reference behaviour: blockgtq/prefill.py:66-101, blockgtq/kernels/fused_packed_attention.py:1876-2594.
+#include <algorithm>
+#include <atomic>
+
+#include "bgtq_dequant_tile.h"
+
+namespace {
+
+typedef float float16v __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int D = BGTQ_D;
+constexpr int MT = DQ_MT;
+constexpr int PROMPT_BIG = 2048;             // work-groups of 256 rows from which on they are taken
+constexpr int MAX_GQA_ROWS = 128;            // query rows of the smaller work-group, the most query heads of a group
+constexpr int TILE = 2 * MT * D * 2;         // bytes of a staged tile: K fragments, then V fragments
+constexpr int PART = D * D * 2;              // bytes of one 16-bit part of a rotation
+constexpr float REFRESH = 4.0f;
+
+// rotation parts of a head: the query rotation (3 bf16 or 2 fp16 parts), then the un-rotation (2 fp16 parts)
+constexpr int Q_PARTS_MAX = 3, HEAD_PARTS = Q_PARTS_MAX + 2;
+
+__device__ __forceinline__ uint32_t cvt_pk_f16(float lo, float hi) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    h2 r = {(_Float16)lo, (_Float16)hi};
+    return __builtin_bit_cast(uint32_t, r);
+}
+
+// ---- stage ------------------------------------------------------------------------------------------------
+struct StageArgs {
+    const bgtq_head_plan* plans;
+    const uint8_t* kp;  int64_t kp_sb, kp_sh;
+    const uint16_t* kn; int64_t kn_sb, kn_sh; int kn_st;
+    const uint8_t* vp;  int64_t vp_sb, vp_sh;
+    const uint16_t* vn; int64_t vn_sb, vn_sh;
+    int n_kv, T, n_tiles, per_wg, tile_stride;   // tiles of a (row, head), how many of them a work-group takes, the workspace's room
+    int k_layout, v_layout, k_row_width, v_stride;
+    int kt, knr, vnr, vt;                    // raw tile areas in LDS
+    int bf16, rotate_q;                      // parts of the query rotation: three bf16 / two fp16 / none
+    int tile_wgs;                            // work-groups that stage tiles; ROT_WGS per head follow
+    uint8_t *rot, *tiles;
+};
+
+__host__ __device__ inline int raw_bytes(int krow, int vstride, int kn_st, int& kt, int& knr, int& vnr, int& vt) {
+    kt = (MT * krow + 32 + 15) & ~15;
+    knr = (MT * kn_st * 2 + 16 + 15) & ~15;
+    vnr = MT * 2 + 16;
+    vt = (MT * vstride + 32 + 15) & ~15;
+    return kt + knr + vnr + vt;
+}
+constexpr int ROT_WGS = D * D / 8 / DQ_THR;   // work-groups per head that split its rotations
+constexpr int RAW_OFF = BGTQ_VLUT_BYTES + BGTQ_LUT_IMAGE_BYTES;
+
+// One head's rotation parts.  A fragment (rows 32 ob .., step kk) holds, for lane (li, lg), row 32 ob + li and
+// slots 16 kk + 8 lg + e.  Query rotation: row = packed dim, slot = original dim.  Un-rotation: row = output dim,
+// slot s = rotated dim in the permuted order.
+__device__ __forceinline__ void stage_rotations(const StageArgs& a, int wg, int tid, uint8_t* smem) {
+    const int h = wg / ROT_WGS;
+    const bgtq_head_plan& P = a.plans[h];
+    int* inv = (int*)smem;                   // original dim -> packed dim
+    if (tid < D) inv[P.head_perm[tid]] = tid;
+    __syncthreads();
+    uint8_t* dst = a.rot + (size_t)h * HEAD_PARTS * PART;
+    {
+        const int i = (wg - h * ROT_WGS) * DQ_THR + tid;           // piece of 8 slots
+        const int lane = i & 63, kk = (i >> 6) & 7, ob = i >> 9, li = lane & 31, lg = lane >> 5;
+        const int row = 32 * ob + li;
+        if (a.rotate_q) {
+            uint16_t part[3][8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float x = P.k_rot_T[inv[16 * kk + 8 * lg + e] * D + row];
+                if (a.bf16) {
+                    const __bf16 p0 = (__bf16)x, p1 = (__bf16)(x - (float)p0), p2 = (__bf16)(x - (float)p0 - (float)p1);
+                    part[0][e] = __builtin_bit_cast(uint16_t, p0);
+                    part[1][e] = __builtin_bit_cast(uint16_t, p1);
+                    part[2][e] = __builtin_bit_cast(uint16_t, p2);
+                } else {
+                    const _Float16 p0 = (_Float16)x, p1 = (_Float16)(x - (float)p0);
+                    part[0][e] = __builtin_bit_cast(uint16_t, p0);
+                    part[1][e] = __builtin_bit_cast(uint16_t, p1);
+                    part[2][e] = 0;
+                }
+            }
+            for (int p = 0; p < (a.bf16 ? 3 : 2); p++) *(uint4v*)(dst + p * PART + i * 16) = *(const uint4v*)part[p];
+        }
+        uint16_t hi[8], lo[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float x = P.v_rot[(16 * kk + 8 * (e >> 2) + 4 * lg + (e & 3)) * D + row];
+            const _Float16 p0 = (_Float16)x, p1 = (_Float16)(x - (float)p0);
+            hi[e] = __builtin_bit_cast(uint16_t, p0);
+            lo[e] = __builtin_bit_cast(uint16_t, p1);
+        }
+        *(uint4v*)(dst + Q_PARTS_MAX * PART + i * 16) = *(const uint4v*)hi;
+        *(uint4v*)(dst + (Q_PARTS_MAX + 1) * PART + i * 16) = *(const uint4v*)lo;
+    }
+}
+
+__global__ __launch_bounds__(DQ_THR) void prompt_stage_kernel(StageArgs a) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if ((int)blockIdx.x >= a.tile_wgs) { stage_rotations(a, (int)blockIdx.x - a.tile_wgs, tid, smem); return; }
+    const int wgs_per = (a.n_tiles + a.per_wg - 1) / a.per_wg;
+    const int pair = blockIdx.x / wgs_per, tile0 = ((int)blockIdx.x - pair * wgs_per) * a.per_wg;
+    const int tile1 = min(tile0 + a.per_wg, a.n_tiles);
+    const int b = pair / a.n_kv, h = pair - b * a.n_kv;
+    const bgtq_head_plan& P = a.plans[h];
+    const bool vnib = a.v_layout == BGTQ_V_NIBBLE;
+    const int krow = a.k_row_width, vrow = a.v_stride, kn_st = a.kn_st;
+    const uint32_t voff = (uint32_t)lane * 16;
+    const uint32_t raw_set = (uint32_t)(a.kt + a.knr + a.vnr + a.vt), ktile = RAW_OFF + 2 * raw_set, vtile = ktile + MT * DQ_KROW;
+    const uint8_t* kp_base = a.kp + b * a.kp_sb + h * a.kp_sh;
+    const uint8_t* vp_base = a.vp + b * a.vp_sb + h * a.vp_sh;
+    const uint8_t* kn_base = (const uint8_t*)(a.kn + b * a.kn_sb + h * a.kn_sh);
+    const uint8_t* vn_base = (const uint8_t*)(a.vn + b * a.vn_sb + h * a.vn_sh);
+    const uint32_t kph = (uint32_t)((uintptr_t)kp_base & 15), vph = (uint32_t)((uintptr_t)vp_base & 15);
+    const uint32_t knph = (uint32_t)((uintptr_t)kn_base & 15), vnph = (uint32_t)((uintptr_t)vn_base & 15);
+    // wave 0 fetches the K records, wave 1 the V records, wave 2 both norm arrays
+    auto issue = [&](int tile) {
+        const int t = tile * MT, nt = min(MT, a.T - t);
+        const uint32_t kraw = RAW_OFF + (uint32_t)(tile & 1) * raw_set, knraw = kraw + a.kt, vnraw = knraw + a.knr, vraw = vnraw + a.vnr;
+        if (wave == 0) {
+            dma_region<9>(kp_base - kph + (int64_t)t * krow, kraw, dma_shape((int)kph + nt * krow, voff), voff);
+        } else if (wave == 1) {
+            dma_region<9>(vp_base - vph + (int64_t)t * vrow, vraw, dma_shape((int)vph + nt * vrow, voff), voff);
+        } else if (wave == 2) {
+            dma_region<2>(kn_base - knph + (int64_t)t * kn_st * 2, knraw, dma_shape((int)knph + nt * kn_st * 2, voff), voff);
+            dma_region<1>(vn_base - vnph + (int64_t)t * 2, vnraw, dma_shape((int)vnph + nt * 2, voff), voff);
+        }
+    };
+    issue(tile0);
+    dq_load_tables(P, a.k_layout, vnib, vnib ? 4 : (int)P.v_bits, wave, voff);
+    TileDequant dq;
+    dq.init(P, a.k_layout, vnib, tid);
+    // the K tile's columns of 0-bit dims are never written: zero them once
+    const int n_zero = min(max(P.n_zero_dims, 0), D);
+    for (int i = tid; i < MT * (n_zero / 2); i += DQ_THR) {
+        const int t = i / (n_zero / 2), c = i - t * (n_zero / 2);
+        lds_put<uint32_t>(ktile + (uint32_t)t * DQ_KROW + c * 4, 0u);
+    }
+    const int li = lane & 31, lg = lane >> 5;
+    uint8_t* out = a.tiles + (size_t)pair * a.tile_stride * TILE + voff;
+    for (int tile = tile0; tile < tile1; tile++) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();                     // raw tile (and tables) complete; the tile buffers have been read
+        const uint32_t raw0 = RAW_OFF + (uint32_t)(tile & 1) * raw_set, vn0 = raw0 + a.kt + a.knr;
+        if (tile + 1 < tile1) issue(tile + 1);
+        dq.run(raw0 + kph + (uint32_t)lane * krow, raw0 + a.kt + knph + (uint32_t)lane * kn_st * 2, vn0 + vnph, vn0 + a.vnr + vph, vrow,
+               min(MT, a.T - tile * MT), ktile, vtile);
+        __syncthreads();
+        uint8_t* o = out + (size_t)tile * TILE;
+#pragma unroll
+        for (int c = 0; c < 2; c++) {        // K fragment (token block tb, step kk = wave); dims in the permuted order
+            const uint32_t src = ktile + (uint32_t)(32 * c + li) * DQ_KROW + (uint32_t)(16 * wave + 4 * lg) * 2;
+            const uint2v x0 = lds_at<uint2v>(src), x1 = lds_at<uint2v>(src + 16);
+            *(uint4v*)(o + (8 * c + wave) * 1024) = (uint4v){x0.x, x0.y, x1.x, x1.y};
+        }
+#pragma unroll
+        for (int c = 0; c < 2; c++) {        // V fragment f = (16-token group f / 4, dims 32 (f % 4) ..)
+            const int f = 2 * wave + c;
+            *(uint4v*)(o + 16384 + f * 1024) = lds_at<uint4v>(vtile + (uint32_t)(32 * (f & 3) + li) * DQ_VTROW + (uint32_t)(16 * (f >> 2) + 8 * lg) * 2);
+        }
+    }
+}
+
+// ---- attend -----------------------------------------------------------------------------------------------
+struct PromptArgs {
+    const uint8_t *rot, *tiles;
+    const uint16_t* q; int64_t q_sb, q_sh, q_ss;
+    int n_kv, gqa, S, T, n_tiles, q_pos_offset, causal, n_splits;
+    float scale;
+    int rotate_q, unrotate;
+    int rows;                                // query rows per work-group (32 a wave)
+    float *part_o, *part_ml;                 // n_splits > 1: sums [wg][wave][register][lane], (reference, denominator) [wg][wave][row]
+    uint16_t* out; int64_t o_sb, o_sh, o_ss;
+};
+
+// LDS of the attention: two staged tiles; two parts of a rotation take their place before and after the walk
+constexpr size_t PROMPT_LDS = 2 * TILE;
+static_assert(2 * PART <= PROMPT_LDS, "");
+
+// Which rows a wave holds: row r = wave * 32 + (lane & 31) of the block is head r / BQ, token s0 + r % BQ.
+struct RowOf {
+    int hq, sq, s0;
+    bool ok;
+    __device__ __forceinline__ RowOf(const PromptArgs& a, int qb, int wave, int lane) {
+        const int BQ = a.rows / a.gqa, row = wave * 32 + (lane & 31);
+        s0 = qb * BQ;
+        hq = row / BQ;
+        sq = s0 + row - hq * BQ;
+        ok = hq < a.gqa && sq < a.S;
+    }
+};
+
+// n consecutive rotation parts from the workspace to LDS address 0: each wave its share
+template <int NW>
+__device__ __forceinline__ void load_parts(const uint8_t* src, int n, int wave, uint32_t voff) {
+    for (int c = wave; c < n * (PART / 4096); c += NW) dma_full<4>(voff, uniform_ptr(src + c * 4096), (uint32_t)c * 4096);
+}
+
+// Normalise, un-rotate (out^T = R^T O^T: both factors split into fp16 head and remainder, the product of the
+// remainders left out) and store.  The parts lie in LDS.
+__device__ __forceinline__ void finish_rows(const PromptArgs& a, float16v (&O)[4], float l_tot, const RowOf& row, int b, int h, int lane) {
+    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+#pragma unroll
+    for (int db = 0; db < 4; db++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) O[db][r] *= inv;
+    const int lg = lane >> 5;
+    uint32_t frag = (uint32_t)lane * 16;
+    asm("" : "+v"(frag));
+    if (a.unrotate) {
+        half8 Bh[8], Bl[8];
+#pragma unroll
+        for (int db = 0; db < 4; db++)
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                uint32_t hi[4], lo[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float x0 = O[db][8 * s + 2 * j], x1 = O[db][8 * s + 2 * j + 1];
+                    const _Float16 h0 = (_Float16)x0, h1 = (_Float16)x1;
+                    hi[j] = cvt_pk_f16((float)h0, (float)h1);
+                    lo[j] = cvt_pk_f16(x0 - (float)h0, x1 - (float)h1);
+                }
+                Bh[2 * db + s] = __builtin_bit_cast(half8, (uint4v){hi[0], hi[1], hi[2], hi[3]});
+                Bl[2 * db + s] = __builtin_bit_cast(half8, (uint4v){lo[0], lo[1], lo[2], lo[3]});
+            }
+#pragma unroll
+        for (int ob = 0; ob < 4; ob++) O[ob] = (float16v){0};
+#pragma unroll
+        for (int st = 0; st < 8; st++) {                       // four independent accumulators per pass
+            half8 Ah[4], Al[4];
+#pragma unroll
+            for (int ob = 0; ob < 4; ob++) {
+                Ah[ob] = lds_at<half8>(frag + (8 * ob + st) * 1024);
+                Al[ob] = lds_at<half8>(frag + PART + (8 * ob + st) * 1024);
+            }
+#pragma unroll
+            for (int ob = 0; ob < 4; ob++) O[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Ah[ob], Bh[st], O[ob], 0, 0, 0);
+#pragma unroll
+            for (int ob = 0; ob < 4; ob++) O[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Al[ob], Bh[st], O[ob], 0, 0, 0);
+#pragma unroll
+            for (int ob = 0; ob < 4; ob++) O[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Ah[ob], Bl[st], O[ob], 0, 0, 0);
+        }
+    }
+    if (row.ok) {
+        uint16_t* orow = a.out + b * a.o_sb + ((int64_t)h * a.gqa + row.hq) * a.o_sh + (int64_t)row.sq * a.o_ss;
+#pragma unroll
+        for (int ob = 0; ob < 4; ob++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint2v w = {cvt_pk_f16(O[ob][4 * j], O[ob][4 * j + 1]), cvt_pk_f16(O[ob][4 * j + 2], O[ob][4 * j + 3])};
+                *(uint2v*)(orow + 32 * ob + 8 * j + 4 * lg) = w;
+            }
+    }
+}
+
+template <bool BF16, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    constexpr int Q_PARTS = BF16 ? 3 : 2;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = blockIdx.x, b = blockIdx.y;
+    // the query block that sees most tokens first, so that the short blocks fill the tail of the launch
+    const int nz = (int)gridDim.z - 1 - (int)blockIdx.z, qb = nz / a.n_splits, c = nz - qb * a.n_splits;
+    const RowOf row(a, qb, wave, lane);
+    const int lg = lane >> 5;
+    const int s_last = min(row.s0 + a.rows / a.gqa, a.S) - 1;
+    const int t_end = a.causal ? min(a.T, a.q_pos_offset + s_last + 1) : a.T;
+    const int n_all = (t_end + MT - 1) / MT;
+    const int tile0 = (int)((int64_t)n_all * c / a.n_splits), tile1 = (int)((int64_t)n_all * (c + 1) / a.n_splits);
+    const int lim = !row.ok ? 0 : a.causal ? min(a.T, a.q_pos_offset + row.sq + 1) : a.T;    // tokens t < lim are visible to this row
+    const bool live = __builtin_amdgcn_ballot_w64(row.ok) != 0;                              // (a wave without rows only moves data)
+
+    const uint32_t voff = (uint32_t)lane * 16;
+    const uint8_t* rot_h = a.rot + (size_t)h * HEAD_PARTS * PART;
+    const uint8_t* tiles = a.tiles + (size_t)(b * a.n_kv + h) * a.n_tiles * TILE + wave * (TILE / NW);
+    auto issue = [&](int tile) {
+        const uint8_t* src = uniform_ptr(tiles + (size_t)tile * TILE);
+        const uint32_t dst = (uint32_t)(tile & 1) * TILE + wave * (TILE / NW);
+#pragma unroll
+        for (int c = 0; c < TILE / NW; c += 4096) dma_full<4>(voff, src + c, dst + c);
+    };
+
+    // ---- queries as B operands of S^T = K Q^T, in the permuted order of the staged dims
+    half8 Qb[8];
+    const uint16_t* qrow = a.q + b * a.q_sb + ((int64_t)h * a.gqa + (row.ok ? row.hq : 0)) * a.q_sh + (int64_t)(row.ok ? row.sq : 0) * a.q_ss;
+    if (a.rotate_q) {
+        // the last two parts fit LDS at a time; three (bf16) come as the two small ones, then the head
+        load_parts<NW>(rot_h + (Q_PARTS - 2) * PART, 2, wave, voff);
+        uint4v qv[8];                                            // lane: dims 16 kk + 8 lg .. + 7 of its query
+#pragma unroll
+        for (int kk = 0; kk < 8; kk++) {
+            qv[kk] = (uint4v){0, 0, 0, 0};
+            if (row.ok) qv[kk] = *(const uint4v*)(qrow + 16 * kk + 8 * lg);
+        }
+        float16v R[4];                                           // packed dims 32 ob ..
+#pragma unroll
+        for (int ob = 0; ob < 4; ob++) R[ob] = (float16v){0};
+        auto add_part = [&](uint32_t at) {
+            asm("" : "+v"(at));
+#pragma unroll
+            for (int kk = 0; kk < 8; kk++)
+#pragma unroll
+                for (int ob = 0; ob < 4; ob++) {
+                    if constexpr (BF16)
+                        R[ob] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lds_at<bf16x8>(at + (8 * ob + kk) * 1024), __builtin_bit_cast(bf16x8, qv[kk]), R[ob], 0, 0, 0);
+                    else
+                        R[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lds_at<half8>(at + (8 * ob + kk) * 1024), __builtin_bit_cast(half8, qv[kk]), R[ob], 0, 0, 0);
+                }
+        };
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (live) { add_part(PART + voff); add_part(voff); }     // (the small parts first)
+        __syncthreads();
+        if (BF16) {
+            load_parts<NW>(rot_h, 1, wave, voff);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (live) add_part(voff);
+            __syncthreads();
+        }
+        if (tile0 < tile1) issue(tile0);
+#pragma unroll
+        for (int ob = 0; ob < 4; ob++)
+#pragma unroll
+            for (int s = 0; s < 2; s++)
+                Qb[2 * ob + s] = __builtin_bit_cast(half8, (uint4v){cvt_pk_f16(R[ob][8 * s], R[ob][8 * s + 1]), cvt_pk_f16(R[ob][8 * s + 2], R[ob][8 * s + 3]),
+                                                                    cvt_pk_f16(R[ob][8 * s + 4], R[ob][8 * s + 5]), cvt_pk_f16(R[ob][8 * s + 6], R[ob][8 * s + 7])});
+    } else {
+#pragma unroll
+        for (int kk = 0; kk < 8; kk++) {
+            uint2v x0 = {0, 0}, x1 = {0, 0};
+            if (row.ok) { x0 = *(const uint2v*)(qrow + 16 * kk + 4 * lg); x1 = *(const uint2v*)(qrow + 16 * kk + 8 + 4 * lg); }
+            Qb[kk] = __builtin_bit_cast(half8, (uint4v){x0.x, x0.y, x1.x, x1.y});
+        }
+        if (tile0 < tile1) issue(tile0);
+    }
+
+    const float c2 = a.scale * 1.44269504088896340736f;        // scores in log2 units
+    float16v O[4];                                              // O^T: block db = dims 32 db .., reg r -> dim 32 db + 8 (r / 4) + 4 lg + r % 4
+#pragma unroll
+    for (int db = 0; db < 4; db++) O[db] = (float16v){0};
+    float m_ref = -INFINITY, l_part = 0.f;                       // per query (this half's share of the denominator)
+
+    for (int tile = tile0; tile < tile1; tile++) {
+        const int t0 = tile * MT;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // this wave's share of the tile
+        __syncthreads();                                         // the tile is complete; everyone is done with the one before
+        if (tile + 1 < tile1) issue(tile + 1);
+        if (!live) continue;
+        uint32_t kf = (uint32_t)(tile & 1) * TILE + voff;
+        asm("" : "+v"(kf));                                      // (fragments at immediate offsets: left alone, every address gets an instruction)
+        const uint32_t vf = kf + 16384;
+
+        // ---- S^T = K Q^T for the wave's 32 queries: 2 token blocks x 8 steps of 16 dims, K fragments read 8 ahead
+        float16v Sc[2];
+        {
+            half8 A[16];
+#pragma unroll
+            for (int i = 0; i < 16; i++) A[i] = lds_at<half8>(kf + (8 * (i & 1) + (i >> 1)) * 1024);
+            Sc[0] = Sc[1] = (float16v){0};
+#pragma unroll
+            for (int i = 0; i < 16; i++) Sc[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[i], Qb[i >> 1], Sc[i & 1], 0, 0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+        }
+        // ---- softmax, lane = query; reg r of block tb is token t0 + 32 tb + 8 (r / 4) + 4 lg + r % 4
+        // (raw scores stay in the registers; the scale goes into the exponent's multiply-add)
+        float mx = -INFINITY;
+        if (__builtin_amdgcn_ballot_w64(t0 + MT > lim)) {        // (wave-uniform) some row of the wave has masked tokens in this tile
+#pragma unroll
+            for (int tb = 0; tb < 2; tb++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    if (t0 + 32 * tb + 8 * (r >> 2) + 4 * lg + (r & 3) >= lim) Sc[tb][r] = -INFINITY;
+                    mx = fmaxf(mx, Sc[tb][r]);
+                }
+        } else {
+#pragma unroll
+            for (int tb = 0; tb < 2; tb++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) mx = fmaxf(mx, Sc[tb][r]);
+        }
+        mx *= c2;                                                // c2 > 0: the maximum commutes with the scale
+        if (__builtin_amdgcn_ballot_w64(mx > m_ref)) {           // wave-uniform, rare after the first tiles
+            const float other = __shfl_xor(mx, 32, 64);
+            const float top = fmaxf(mx, other);
+            const float m_new = top > m_ref ? top + REFRESH : m_ref;
+            const float alpha = (m_ref == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_ref - m_new);
+            l_part *= alpha;
+#pragma unroll
+            for (int db = 0; db < 4; db++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) O[db][r] *= alpha;
+            m_ref = m_new;
+        }
+        // rows that have seen no record yet keep every exponential at 0 (no inf - inf)
+        const float mneg = m_ref == -INFINITY ? 0.f : -m_ref;
+        uint32_t Pw[2][8];                                        // fp16 pairs: Pw[tb][j] = regs 2j, 2j + 1
+#pragma unroll
+        for (int tb = 0; tb < 2; tb++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const float p0 = __builtin_amdgcn_exp2f(fmaf(Sc[tb][2 * j], c2, mneg));
+                const float p1 = __builtin_amdgcn_exp2f(fmaf(Sc[tb][2 * j + 1], c2, mneg));
+                Pw[tb][j] = cvt_pk_f16(p0, p1);
+                // (the denominator adds the probabilities the values are weighted with: two a dot product)
+                l_part = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, Pw[tb][j]), (half2v){(_Float16)1.f, (_Float16)1.f}, l_part, false);
+            }
+        // ---- O^T += V^T P^T: 16-token group 2 tb + hf
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const uint4v pw = {Pw[g >> 1][4 * (g & 1)], Pw[g >> 1][4 * (g & 1) + 1], Pw[g >> 1][4 * (g & 1) + 2], Pw[g >> 1][4 * (g & 1) + 3]};
+            const half8 Bp = __builtin_bit_cast(half8, pw);
+#pragma unroll
+            for (int db = 0; db < 4; db++)
+                O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lds_at<half8>(vf + (4 * g + db) * 1024), Bp, O[db], 0, 0, 0);
+        }
+    }
+
+    const float l_tot = l_part + __shfl_xor(l_part, 32, 64);
+    if (a.n_splits == 1) {
+        if (a.unrotate) {
+            __syncthreads();                                     // every wave is done with the tiles
+            load_parts<NW>(rot_h + Q_PARTS_MAX * PART, 2, wave, voff);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+        }
+        if (live) finish_rows(a, O, l_tot, row, b, h, lane);
+    } else if (live) {
+        const size_t wg = ((size_t)(b * a.n_kv + h) * (gridDim.z / a.n_splits) + qb) * a.n_splits + c;
+        float* po = a.part_o + (wg * NW + wave) * 64 * 64 + lane;
+#pragma unroll
+        for (int db = 0; db < 4; db++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) po[(16 * db + r) * 64] = O[db][r];
+        if (lane < 32) *(float2*)(a.part_ml + ((wg * NW + wave) * 32 + lane) * 2) = float2{m_ref, l_tot};
+    }
+}
+
+// ---- merge ------------------------------------------------------------------------------------------------
+// A work-group of 8 waves adds the partial sums of 32 rows (one wave of the attention): each wave takes every eighth
+// partition, then the eight meet in LDS.  (One wave walking all partitions took 43 us for 62 of them.)
+constexpr int MERGE_WAVES = 8;
+constexpr size_t MERGE_LDS = 2 * PART + 4 * (64 * 64 + 64) * sizeof(float);
+__global__ __launch_bounds__(64 * MERGE_WAVES) void prompt_merge_kernel(PromptArgs a) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nw = a.rows / 32, n_qb = (int)gridDim.z / nw;
+    const int h = blockIdx.x, b = blockIdx.y, qb = blockIdx.z / nw, w = blockIdx.z - qb * nw;
+    const RowOf row(a, qb, w, lane);
+    if (__builtin_amdgcn_ballot_w64(row.ok) == 0) return;        // (uniform over the work-group)
+    if (a.unrotate) load_parts<MERGE_WAVES>(a.rot + ((size_t)h * HEAD_PARTS + Q_PARTS_MAX) * PART, 2, wave, (uint32_t)lane * 16);
+    const size_t wg0 = ((size_t)(b * a.n_kv + h) * n_qb + qb) * a.n_splits;
+    float16v O[4];
+#pragma unroll
+    for (int db = 0; db < 4; db++) O[db] = (float16v){0};
+    float l_tot = 0.f, m = -INFINITY;
+    const float2* ml = (const float2*)a.part_ml + (wg0 * nw + w) * 32 + (lane & 31);
+    for (int c = 0; c < a.n_splits; c++) m = fmaxf(m, ml[(size_t)c * nw * 32].x);
+    for (int c = wave; c < a.n_splits; c += MERGE_WAVES) {
+        const float2 x = ml[(size_t)c * nw * 32];
+        const float f = x.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x.x - m);
+        l_tot += f * x.y;
+        const float* po = a.part_o + ((wg0 + c) * nw + w) * 64 * 64 + lane;
+#pragma unroll
+        for (int db = 0; db < 4; db++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) O[db][r] = fmaf(f, po[(16 * db + r) * 64], O[db][r]);
+    }
+    float* meet = (float*)(smem + 2 * PART);                     // [4][64 registers, denominator][lane]
+#pragma unroll
+    for (int half = MERGE_WAVES / 2; half >= 1; half >>= 1) {
+        float* at = meet + (wave & (half - 1)) * 65 * 64 + lane;
+        if (wave >= half && wave < 2 * half) {
+#pragma unroll
+            for (int r = 0; r < 64; r++) at[r * 64] = O[r >> 4][r & 15];
+            at[64 * 64] = l_tot;
+        }
+        __syncthreads();
+        if (wave < half) {
+#pragma unroll
+            for (int r = 0; r < 64; r++) O[r >> 4][r & 15] += at[r * 64];
+            l_tot += at[64 * 64];
+        }
+        __syncthreads();
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // this wave's share of the un-rotation
+    __syncthreads();
+    if (wave == 0) finish_rows(a, O, l_tot, row, b, h, lane);
+}
+
+// Rows of a work-group.  256 (one work-group a compute unit) fetch every tile for twice as many rows, which counts
+// where the chip is full and limited by power: 8k prompts 5 % faster.  128 (two a compute unit, no barrier between
+// their waves) fill the chip with half the rows and end with shorter tails: 1k to 2k prompts 5 to 20 % faster.
+int prompt_rows(int B, int n_kv, int gqa, int S) {
+    return gqa > MAX_GQA_ROWS || (int64_t)B * n_kv * gqa * S >= (int64_t)PROMPT_BIG * 256 ? 256 : 128;
+}
+// Tiles of one query block dealt to several work-groups where the blocks alone leave compute units idle, four
+// tiles or more each (below that set-up and merge cost more than the walk)
+int prompt_splits(int B, int n_kv, int gqa, int S, int T) {
+    const int rows = prompt_rows(B, n_kv, gqa, S), BQ = rows / gqa;
+    const int64_t wgs = (int64_t)B * n_kv * ((S + BQ - 1) / BQ), room = rows == 256 ? 256 : 512;
+    const int64_t want = std::max<int64_t>(1, room / std::max<int64_t>(wgs, 1));
+    const int64_t tiles = (T + MT - 1) / MT;
+    return (int)std::max<int64_t>(1, std::min(want, tiles / 4));
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t bgtq_prompt_workspace_bytes(int B, int n_kv, int gqa, int S, int T) {
+    if (B <= 0 || n_kv <= 0 || gqa <= 0 || gqa > 256 || S <= 0 || T <= 0) return 0;
+    const int ns = prompt_splits(B, n_kv, gqa, S, T), rows = prompt_rows(B, n_kv, gqa, S), BQ = rows / gqa;
+    const size_t wgs = (size_t)B * n_kv * ((S + BQ - 1) / BQ) * ns;
+    return (size_t)n_kv * HEAD_PARTS * PART + (size_t)B * n_kv * ((T + MT - 1) / MT) * TILE +
+           (ns > 1 ? wgs * (rows / 32) * (64 * 64 + 64) * sizeof(float) : 0);
+}
+
+int bgtq_prompt_attn(const bgtq_head_plan* plans,
+                     const void* q, int x_dtype, int rotate_q, int64_t q_sb, int64_t q_sh, int64_t q_ss,
+                     const void* k_packed, int64_t kp_sb, int64_t kp_sh, int64_t kp_st, int k_row_width,
+                     const void* k_norms, int64_t kn_sb, int64_t kn_sh, int64_t kn_st,
+                     const void* v_packed, int64_t vp_sb, int64_t vp_sh, int64_t vp_st, int v_row_width,
+                     const void* v_norms, int64_t vn_sb, int64_t vn_sh, int64_t vn_st,
+                     int B, int n_kv, int gqa, int S, int T, int q_pos_offset, int is_causal,
+                     int k_layout, int v_layout, float scale, int unrotate,
+                     void* workspace, size_t workspace_bytes,
+                     void* out, int64_t o_sb, int64_t o_sh, int64_t o_ss, void* stream) {
+    BGTQ_CHECK_ARG(plans && q && k_packed && k_norms && v_packed && v_norms && out);
+    BGTQ_CHECK_ARG(B >= 0 && n_kv > 0 && gqa > 0 && S >= 0 && T >= 0 && q_pos_offset >= 0);
+    BGTQ_CHECK_ARG(x_dtype == BGTQ_X_FP16 || (x_dtype == BGTQ_X_BF16 && rotate_q));
+    if (B == 0 || S == 0) return BGTQ_OK;            // no query rows: nothing to write
+    BGTQ_CHECK_ARG(k_layout == BGTQ_K_BITPACKED || k_layout == BGTQ_K_MIXED);
+    BGTQ_CHECK_ARG(v_layout == BGTQ_V_BITPACKED || v_layout == BGTQ_V_NIBBLE);
+    // layout requirements, those of bgtq_prefill_attn
+    if (!(scale > 0.f) || T == 0) return BGTQ_EUNSUPPORTED;
+    if (gqa > 256) return BGTQ_EUNSUPPORTED;
+    if ((kp_st & 3) || (kp_sb & 3) || (kp_sh & 3) || ((uintptr_t)k_packed & 3)) return BGTQ_EUNSUPPORTED;
+    if ((vp_st & 3) || (vp_sb & 3) || (vp_sh & 3) || ((uintptr_t)v_packed & 3)) return BGTQ_EUNSUPPORTED;
+    if (kp_st != k_row_width || k_row_width < 4 || k_row_width > 128) return BGTQ_EUNSUPPORTED;
+    if (vn_st != 1 || kn_st < 1 || kn_st > BGTQ_MAX_SEGMENTS) return BGTQ_EUNSUPPORTED;
+    if (v_row_width != 16 && v_row_width != 32 && v_row_width != 48 && v_row_width != 64) return BGTQ_EUNSUPPORTED;
+    if (vp_st < v_row_width || vp_st > v_row_width + 4) return BGTQ_EUNSUPPORTED;
+    if (v_layout == BGTQ_V_NIBBLE && v_row_width != 64) return BGTQ_EUNSUPPORTED;
+    if ((q_ss & 7) || (q_sh & 7) || (q_sb & 7) || ((uintptr_t)q & 15)) return BGTQ_EUNSUPPORTED;           // 16-byte query loads
+    if ((o_ss & 3) || (o_sh & 3) || (o_sb & 3) || ((uintptr_t)out & 7)) return BGTQ_EUNSUPPORTED;          // 8-byte output stores
+    BGTQ_CHECK_ARG(workspace && ((uintptr_t)workspace & 15) == 0);
+    if (workspace_bytes < bgtq_prompt_workspace_bytes(B, n_kv, gqa, S, T)) return BGTQ_EINVAL;
+    const int rows = prompt_rows(B, n_kv, gqa, S), BQ = rows / gqa, n_qb = (S + BQ - 1) / BQ, ns = prompt_splits(B, n_kv, gqa, S, T);
+    if ((int64_t)n_qb * std::max(ns, rows / 32) > 65535 || B > 65535) return BGTQ_EUNSUPPORTED;
+    static std::atomic<int> ready{0};
+    if (ready.load(std::memory_order_acquire) == 0) {
+        // offsets into the dynamic LDS block are used as LDS addresses: holds only without static LDS
+        int ok = 1;
+        for (const void* f : {(const void*)prompt_stage_kernel, (const void*)prompt_attn_kernel<false, 4>, (const void*)prompt_attn_kernel<true, 4>,
+                              (const void*)prompt_attn_kernel<false, 8>, (const void*)prompt_attn_kernel<true, 8>,
+                              (const void*)prompt_merge_kernel}) {
+            hipFuncAttributes fa;
+            hipError_t e = hipFuncGetAttributes(&fa, f);
+            if (e != hipSuccess) return (int)e;
+            e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            if (e != hipSuccess) return (int)e;
+            if (fa.sharedSizeBytes != 0) ok = -1;
+        }
+        ready.store(ok, std::memory_order_release);
+    }
+    if (ready.load(std::memory_order_acquire) < 0) return BGTQ_EUNSUPPORTED;
+    hipStream_t st = (hipStream_t)stream;
+
+    uint8_t* ws = (uint8_t*)workspace;
+    StageArgs g;
+    g.plans = plans;
+    g.kp = (const uint8_t*)k_packed; g.kp_sb = kp_sb; g.kp_sh = kp_sh;
+    g.kn = (const uint16_t*)k_norms; g.kn_sb = kn_sb; g.kn_sh = kn_sh; g.kn_st = (int)kn_st;
+    g.vp = (const uint8_t*)v_packed; g.vp_sb = vp_sb; g.vp_sh = vp_sh;
+    g.vn = (const uint16_t*)v_norms; g.vn_sb = vn_sb; g.vn_sh = vn_sh;
+    g.n_kv = n_kv; g.n_tiles = (T + MT - 1) / MT;
+    // causal rows see no record past the last query's position
+    g.T = is_causal ? (int)std::min<int64_t>(T, (int64_t)q_pos_offset + S) : T;
+    const int staged = (g.T + MT - 1) / MT;
+    g.k_layout = k_layout; g.v_layout = v_layout; g.k_row_width = k_row_width; g.v_stride = (int)vp_st;
+    const int raw = raw_bytes(k_row_width, (int)vp_st, (int)kn_st, g.kt, g.knr, g.vnr, g.vt);
+    // two work-groups fit a compute unit; tiles in equal shares over what that makes
+    g.per_wg = (int)std::max<int64_t>(1, ((int64_t)staged * B * n_kv + 511) / 512);
+    g.bf16 = x_dtype == BGTQ_X_BF16; g.rotate_q = rotate_q != 0;
+    g.rot = ws;
+    g.tiles = ws + (size_t)n_kv * HEAD_PARTS * PART;
+    PromptArgs a;
+    a.rot = g.rot; a.tiles = g.tiles;
+    a.q = (const uint16_t*)q; a.q_sb = q_sb; a.q_sh = q_sh; a.q_ss = q_ss;
+    a.n_kv = n_kv; a.gqa = gqa; a.S = S; a.T = T; a.n_tiles = g.n_tiles; a.q_pos_offset = q_pos_offset; a.causal = is_causal != 0;
+    a.n_splits = ns; a.rows = rows; a.scale = scale; a.rotate_q = rotate_q != 0; a.unrotate = unrotate != 0;
+    a.part_o = (float*)(g.tiles + (size_t)B * n_kv * g.n_tiles * TILE);
+    a.part_ml = a.part_o + (size_t)B * n_kv * n_qb * ns * (rows / 32) * 64 * 64;
+    a.out = (uint16_t*)out; a.o_sb = o_sb; a.o_sh = o_sh; a.o_ss = o_ss;
+    const int wgs_per = (staged + g.per_wg - 1) / g.per_wg;
+    g.tile_stride = g.n_tiles;
+    g.n_tiles = staged;
+    g.tile_wgs = wgs_per * B * n_kv;
+    hipLaunchKernelGGL(prompt_stage_kernel, dim3((unsigned)(g.tile_wgs + n_kv * ROT_WGS)), dim3(DQ_THR), (size_t)RAW_OFF + 2 * raw + DQ_TILE_BYTES, st, g);
+    const dim3 grid((unsigned)n_kv, (unsigned)B, (unsigned)(n_qb * ns));
+    auto attn = g.bf16 ? (rows == 256 ? prompt_attn_kernel<true, 8> : prompt_attn_kernel<true, 4>)
+                       : (rows == 256 ? prompt_attn_kernel<false, 8> : prompt_attn_kernel<false, 4>);
+    hipLaunchKernelGGL(attn, grid, dim3(2 * rows), PROMPT_LDS, st, a);
+    if (ns > 1)
+        hipLaunchKernelGGL(prompt_merge_kernel, dim3((unsigned)n_kv, (unsigned)B, (unsigned)(n_qb * (rows / 32))), dim3(64 * MERGE_WAVES), MERGE_LDS, st, a);
+    return bgtq_launch_status();
+}
+
+}  // extern "C"

@@ -269,47 +269,36 @@ def dequant_kv(plans: torch.Tensor, k_packed: torch.Tensor, k_norms: torch.Tenso
     return ko, vo
 
 
-UNSUPPORTED = -2          # BGTQ_EUNSUPPORTED: the fast kernel does not take this argument set
-
-
 @torch.no_grad()
 def prefill_attention_packed(plans: torch.Tensor, q_rot: torch.Tensor, k_packed: torch.Tensor,
                              k_norms: torch.Tensor, v_packed: torch.Tensor, v_norms: torch.Tensor,
                              T: int, *, k_layout: int = _plan.K_BITPACKED, v_layout: int = _plan.V_BITPACKED,
                              scale: Optional[float] = None, is_causal: bool = True, q_pos_offset: int = 0,
                              unrotate: bool = True, k_row_width: Optional[int] = None,
-                             v_row_width: Optional[int] = None) -> Optional[torch.Tensor]:
-    """Attention of many query tokens straight over the packed cache (``bgtq_prefill_attn``).
+                             v_row_width: Optional[int] = None, rotate_q: bool = False) -> Optional[torch.Tensor]:
+    """Attention of many query tokens over the packed cache (``bgtq_prompt_attn``).
 
-    q_rot (B, n_q, S, D) fp16 rotated queries; cache tensors as for ``decode_attention``.
+    q_rot (B, n_q, S, D) fp16 rotated queries - or, with ``rotate_q``, the model's own queries in fp16
+    or bf16, rotated inside the kernel; cache tensors as for ``decode_attention``.
     Query token s sees records ``t <= q_pos_offset + s`` when ``is_causal``.  Returns
     (B, n_q, S, D) fp16, or ``None`` when the kernel does not take this argument set
     (``prefill_attention_records`` copies records into rows the kernel can walk first)."""
     _capi.require_cuda(k_packed, "k_packed")
-    assert q_rot.dtype == torch.float16 and q_rot.dim() == 4 and q_rot.stride(-1) == 1
+    assert q_rot.dim() == 4 and q_rot.stride(-1) == 1
+    assert q_rot.dtype == torch.float16 or (rotate_q and q_rot.dtype == torch.bfloat16)
     assert k_packed.dtype == torch.uint8 and k_packed.stride(-1) == 1
     assert v_packed.dtype == torch.uint8 and v_packed.stride(-1) == 1
     assert k_norms.dtype == torch.float16 and v_norms.dtype == torch.float16
-    B, n_q, S, D = q_rot.shape
+    n_q, D = q_rot.shape[1], q_rot.shape[3]
     n_kv = k_packed.shape[1]
     assert D == _plan.HEAD_DIM and n_q % n_kv == 0 and k_packed.shape[2] >= T
     k_row_width = k_packed.shape[-1] if k_row_width is None else k_row_width
     v_row_width = v_packed.shape[-1] if v_row_width is None else v_row_width
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
-    out = torch.empty((B, n_q, S, D), dtype=torch.float16, device=q_rot.device)
-    code = _capi.lib().bgtq_prefill_attn(
-        _capi.ptr(plans), _capi.ptr(q_rot), q_rot.stride(0), q_rot.stride(1), q_rot.stride(2),
-        _capi.ptr(k_packed), k_packed.stride(0), k_packed.stride(1), k_packed.stride(2), k_row_width,
-        _capi.ptr(k_norms), k_norms.stride(0), k_norms.stride(1), k_norms.stride(2),
-        _capi.ptr(v_packed), v_packed.stride(0), v_packed.stride(1), v_packed.stride(2), v_row_width,
-        _capi.ptr(v_norms), v_norms.stride(0), v_norms.stride(1), v_norms.stride(2),
-        B, n_kv, n_q // n_kv, S, T, int(q_pos_offset), int(bool(is_causal)),
-        k_layout, v_layout, scale, int(bool(unrotate)),
-        _capi.ptr(out), out.stride(0), out.stride(1), out.stride(2), _capi.stream_ptr(q_rot.device))
-    if code == UNSUPPORTED:
-        return None
-    _capi.check(code, "bgtq_prefill_attn")
-    return out
+    from . import _host
+    return _host.module().prompt(plans, q_rot, int(rotate_q), k_packed, k_norms, v_packed, v_norms, int(T), k_row_width,
+                                 v_row_width, int(q_pos_offset), int(bool(is_causal)), k_layout, v_layout, scale,
+                                 int(bool(unrotate)))
 
 
 def _packed_rows(rec: torch.Tensor, T: int, width: int, v_rows: bool = False) -> torch.Tensor:
@@ -329,7 +318,7 @@ def _packed_rows(rec: torch.Tensor, T: int, width: int, v_rows: bool = False) ->
 @torch.no_grad()
 def prefill_attention_records(plans, q_rot, k_packed, k_norms, v_packed, v_norms, T, *, k_layout=_plan.K_BITPACKED,
                               v_layout=_plan.V_BITPACKED, scale=None, is_causal=True, q_pos_offset=0,
-                              unrotate=True, k_row_width=None, v_row_width=None) -> torch.Tensor:
+                              unrotate=True, k_row_width=None, v_row_width=None, rotate_q=False) -> torch.Tensor:
     """``prefill_attention_packed`` for any tensor layout: records whose rows the kernel cannot walk
     (token stride other than the row width, odd alignment) are first copied into rows it can, queries
     are made contiguous; an argument set the kernel still refuses raises."""
@@ -338,15 +327,19 @@ def prefill_attention_records(plans, q_rot, k_packed, k_norms, v_packed, v_norms
     B, n_q, S, D = q_rot.shape
     if T == 0 or B == 0:
         return torch.zeros((B, n_q, S, D), dtype=torch.float16, device=q_rot.device)
+    kw = dict(k_layout=k_layout, v_layout=v_layout, scale=scale, is_causal=is_causal, q_pos_offset=q_pos_offset,
+              unrotate=unrotate, v_row_width=v_row_width, rotate_q=rotate_q)
+    if q_rot.stride(-1) == 1 and k_norms.stride(-1) == 1:       # as they are, the usual case
+        out = prefill_attention_packed(plans, q_rot, k_packed, k_norms, v_packed, v_norms, T, k_row_width=k_row_width, **kw)
+        if out is not None:
+            return out
     kp = _packed_rows(k_packed, T, k_row_width)
     vp = _packed_rows(v_packed, T, v_row_width, v_rows=True)
     vn = v_norms if v_norms.stride(-1) == 1 else v_norms.contiguous()
     out = prefill_attention_packed(plans, q_rot.contiguous(), kp, k_norms.contiguous() if k_norms.stride(-1) != 1 else k_norms,
-                                   vp, vn, T, k_layout=k_layout, v_layout=v_layout, scale=scale, is_causal=is_causal,
-                                   q_pos_offset=q_pos_offset, unrotate=unrotate,
-                                   k_row_width=kp.stride(2), v_row_width=v_row_width)
+                                   vp, vn, T, k_row_width=kp.stride(2), **kw)
     if out is None:
-        raise RuntimeError("bgtq_prefill_attn does not take this argument set (more than 256 query heads per "
+        raise RuntimeError("bgtq_prompt_attn does not take this argument set (more than 256 query heads per "
                            "KV head, a V record that is not 16, 32, 48 or 64 bytes, or more than 8 norm columns)")
     return out
 

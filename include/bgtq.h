@@ -586,6 +586,29 @@ int bgtq_prefill_attn(const bgtq_head_plan* plans,
                       int k_layout, int v_layout, float scale, int unrotate,
                       void* out, int64_t o_sb, int64_t o_sh, int64_t o_ss, void* stream);
 
+/*
+ * The same attention with a workspace: every tile of records is dequantised once into it, in the
+ * order the matrix cores read their operands, instead of once per block of 256 query rows, and the
+ * queries may come as the model left them (rotate_q != 0: fp16 or bf16, permuted and rotated inside
+ * the kernel as by bgtq_rotate_q; rotate_q == 0: fp16, rotated already).  Where few query rows meet
+ * a long context, the tiles of a block are dealt to several work-groups and merged.  Same layout
+ * requirements and BGTQ_EUNSUPPORTED cases as bgtq_prefill_attn.
+ *   q          [B][n_kv*gqa][S][128] of x_dtype (BGTQ_X_*), strides in elements, rows 16-byte aligned
+ *   workspace  bgtq_prompt_workspace_bytes(B, n_kv, gqa, S, T) bytes of device memory on a 16-byte
+ *              boundary, free again when the launches are done
+ */
+size_t bgtq_prompt_workspace_bytes(int B, int n_kv, int gqa, int S, int T);
+int bgtq_prompt_attn(const bgtq_head_plan* plans,
+                     const void* q, int x_dtype, int rotate_q, int64_t q_sb, int64_t q_sh, int64_t q_ss,
+                     const void* k_packed, int64_t kp_sb, int64_t kp_sh, int64_t kp_st, int k_row_width,
+                     const void* k_norms, int64_t kn_sb, int64_t kn_sh, int64_t kn_st,
+                     const void* v_packed, int64_t vp_sb, int64_t vp_sh, int64_t vp_st, int v_row_width,
+                     const void* v_norms, int64_t vn_sb, int64_t vn_sh, int64_t vn_st,
+                     int B, int n_kv, int gqa, int S, int T, int q_pos_offset, int is_causal,
+                     int k_layout, int v_layout, float scale, int unrotate,
+                     void* workspace, size_t workspace_bytes,
+                     void* out, int64_t o_sb, int64_t o_sh, int64_t o_ss, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,72 @@
+"""GPU: prompt attention with a workspace (staged records, queries rotated inside, partitions merged)
+against the kernel that takes rotated queries and no workspace.
+
+Both dequantise to the same fp16 records and sum in fp32; they round probabilities, outputs and
+rotated queries to fp16 from sums in another order, i.e. each value is off by at most one rounding
+(2^-11 of it, 3e-4 on average) in three places: 2e-3 of the output's norm bounds them together."""
+import pytest
+import torch
+
+from blockgtq_amd import _capi, ops, plan as P, workloads as wl
+from blockgtq_amd.quantizer import build_batched_encode_args, encode_k_into, encode_v_into
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _cache(B, n_kv, T, kl, vl, bits):
+    k_bits, v_bits, lo, hi = bits
+    w = wl.Workload("t", 1, n_kv, n_kv, B, T, 1e6, k_bits=k_bits, v_bits=v_bits, min_bits=lo, max_bits=hi, seed=51)
+    qs, e = wl.calibrate_layer(w, 0, DEV)
+    args = build_batched_encode_args(qs, device=DEV)
+    k, v = wl.draw_kv(w, e, T, 3, DEV)
+    kw = P.cache_row_bytes(args['max_mixed_bytes'] if kl == P.K_MIXED else args['max_tpb'])
+    vw = 64 if vl == P.V_NIBBLE else args['v_packed_bytes']
+    kp = torch.zeros(B, n_kv, T, kw, dtype=torch.uint8, device=DEV)
+    kn = torch.zeros(B, n_kv, T, args['max_n_groups'], dtype=torch.float16, device=DEV)
+    vp = torch.zeros(B, n_kv, T, P.cache_row_bytes(vw), dtype=torch.uint8, device=DEV)[..., :vw]
+    vn = torch.zeros(B, n_kv, T, dtype=torch.float16, device=DEV)
+    encode_k_into(args['plans'], k, kp, kn, 0, kw, kn.shape[-1], kl)
+    encode_v_into(args['plans'], v, vp, vn, 0, vw, vl)
+    return args, qs, (kp, kn, vp, vn)
+
+
+def _no_workspace(args, q_rot, cache, T, off, causal, kl, vl, unrotate):
+    kp, kn, vp, vn = cache
+    B, n_q, S, _ = q_rot.shape
+    n_kv = kp.shape[1]
+    out = torch.empty_like(q_rot)
+    p = _capi.ptr
+    _capi.check(_capi.lib().bgtq_prefill_attn(
+        p(args['plans']), p(q_rot), *q_rot.stride()[:3], p(kp), *kp.stride()[:3], kp.shape[-1], p(kn), *kn.stride()[:3],
+        p(vp), *vp.stride()[:3], vp.shape[-1], p(vn), *vn.stride(), B, n_kv, n_q // n_kv, S, T, off, int(causal), kl, vl,
+        128 ** -0.5, int(unrotate), p(out), *out.stride()[:3], _capi.stream_ptr()), "bgtq_prefill_attn")
+    return out
+
+
+# (B, n_kv, query heads per KV head, queries, records, first position): one row, a long context for few rows
+# (partitions and merge), odd groups, groups wider than the small work-group, tile edges, rows that see nothing
+# of the last tile, many rows
+@pytest.mark.parametrize("B,n_kv,gqa,S,T,off", [
+    (1, 1, 1, 1, 1, 0), (1, 2, 1, 16, 3000, 2984), (2, 1, 7, 37, 137, 100), (1, 2, 40, 9, 640, 631), (1, 1, 130, 5, 129, 124),
+    (1, 1, 4, 64, 64, 0), (1, 1, 4, 65, 65, 0), (1, 2, 3, 300, 500, 50), (1, 8, 4, 1000, 1000, 0)])
+@pytest.mark.parametrize("kl,vl,bits,dtype", [(P.K_BITPACKED, P.V_BITPACKED, (3.0, 3, 1, 5), torch.bfloat16),
+                                              (P.K_MIXED, P.V_NIBBLE, (2.5, 2, 0, 8), torch.float16)])
+def test_prompt_attention_equals_the_kernel_without_workspace(B, n_kv, gqa, S, T, off, kl, vl, bits, dtype):
+    args, qs, cache = _cache(B, n_kv, T, kl, vl, bits)
+    gen = torch.Generator(device=DEV).manual_seed(S + T)
+    q = torch.randn(B, S, n_kv * gqa, 128, generator=gen, device=DEV).to(dtype).transpose(1, 2)
+    rot = []
+    for h, q8 in enumerate(qs):
+        m = torch.zeros(128, 128, dtype=torch.float64, device=DEV)
+        m[q8._head_perm] = q8._block_rot_T.double()
+        rot.append((q[:, h * gqa:(h + 1) * gqa].double() @ m).half())
+    q_rot = torch.cat(rot, 1).contiguous()
+    for causal, unrotate in ((True, True), (False, False)):
+        want = _no_workspace(args, q_rot, cache, T, off, causal, kl, vl, unrotate).float()
+        kw = dict(k_layout=kl, v_layout=vl, is_causal=causal, q_pos_offset=off, unrotate=unrotate)
+        got = {"rotated": ops.prefill_attention_packed(args['plans'], q_rot, *cache, T, **kw)}
+        got["raw"] = ops.prefill_attention_packed(args['plans'], q, *cache, T, rotate_q=True, **kw)
+        for name, g in got.items():
+            assert g.shape == want.shape and torch.isfinite(g).all()
+            assert (g.float() - want).norm() <= 2e-3 * want.norm(), name
