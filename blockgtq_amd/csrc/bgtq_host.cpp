@@ -8,11 +8,16 @@
 //
 // Every entry returns None for a call outside the shapes, types and strides it knows.  The Python caller
 // then goes its general way, which converts what can be converted and raises where it has to.
+//
+// What torch throws (out of memory, a tensor without storage, no device) becomes a Python exception at each
+// entry: an exception that leaves a C function would end the process.
 #include <Python.h>
 
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include "../../include/bgtq.h"
 
@@ -99,6 +104,7 @@ void layer_dealloc(PyObject* self) {
 // Layer(plans, k_packed, k_norms, v_packed, v_norms, k_row_width, norm_width, v_row_width, n_q,
 //       k_layout, v_layout, scale, baked, buf_k or None, buf_v or None)
 PyObject* layer_new(PyTypeObject* type, PyObject* args, PyObject*) {
+    HANDLE_TH_ERRORS
     PyObject *o[7];
     int kw, nw, vw, n_q, kl, vl, baked;
     float scale;
@@ -118,6 +124,7 @@ PyObject* layer_new(PyTypeObject* type, PyObject* args, PyObject*) {
     Layer* L = (Layer*)type->tp_alloc(type, 0);
     if (!L) return nullptr;
     at::Tensor** dst[7] = {&L->plans, &L->kp, &L->kn, &L->vp, &L->vn, &L->bk, &L->bv};
+    THPObjectPtr owner((PyObject*)L);                // (freed should one of the tensors have no storage)
     for (int i = 0; i < 7; i++) *dst[i] = t[i] ? new at::Tensor(*t[i]) : nullptr;
     bgtq_step& s = L->s;
     s = bgtq_step{};
@@ -140,7 +147,8 @@ PyObject* layer_new(PyTypeObject* type, PyObject* args, PyObject*) {
         s.w_sb = t[5]->stride(0); s.w_sh = t[5]->stride(1); s.w_st = t[5]->stride(2);
         s.win_W = (int)t[5]->size(2);
     }
-    return (PyObject*)L;
+    return owner.release();
+    END_HANDLE_TH_ERRORS
 }
 
 // k, v and (may be null) q of one step into s; false: not for this path
@@ -219,6 +227,7 @@ PyObject* finish_step(Layer* L, bgtq_step& s, int64_t T, int64_t n_splits, PyObj
 
 // step(q, k, v, t_pos, T, seq_lens or None, n_splits, quant_mode, workspace)
 PyObject* layer_step(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     Layer* L = (Layer*)self;
     int64_t T, n_splits, quant;
     if (n != 9 || !as_int(a[4], T) || !as_int(a[6], n_splits) || !as_int(a[7], quant)) Py_RETURN_NONE;
@@ -232,10 +241,12 @@ PyObject* layer_step(PyObject* self, PyObject* const* a, Py_ssize_t n) {
     }
     s.quant_mode = (int)quant;
     return finish_step(L, s, T, n_splits, a[8], false);
+    END_HANDLE_TH_ERRORS
 }
 
 // step_window(q, k, v, slot, t_flush, packed_len, buf_len, T, n_splits, quant_mode, workspace)
 PyObject* layer_step_window(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     Layer* L = (Layer*)self;
     int64_t T, n_splits, quant;
     if (n != 11 || !L->bk || !as_int(a[7], T) || !as_int(a[8], n_splits) || !as_int(a[9], quant)) Py_RETURN_NONE;
@@ -253,10 +264,12 @@ PyObject* layer_step_window(PyObject* self, PyObject* const* a, Py_ssize_t n) {
     s.win_lens = idx[3]->data_ptr<int32_t>();
     s.quant_mode = (int)quant;
     return finish_step(L, s, T, n_splits, a[10], true);
+    END_HANDLE_TH_ERRORS
 }
 
 // encode(k, v, t_pos, quant_mode) -> True
 PyObject* layer_encode(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     Layer* L = (Layer*)self;
     int64_t quant;
     if (n != 4 || !as_int(a[3], quant)) Py_RETURN_NONE;
@@ -270,6 +283,7 @@ PyObject* layer_encode(PyObject* self, PyObject* const* a, Py_ssize_t n) {
     Py_END_ALLOW_THREADS
     if (rc != BGTQ_OK) return fail("bgtq_encode_kv", rc);
     Py_RETURN_TRUE;
+    END_HANDLE_TH_ERRORS
 }
 
 PyMethodDef layer_methods[] = {
@@ -284,6 +298,7 @@ PyTypeObject LayerType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 // attend(plans, q_rot (B, n_q, 1, D) or (B, n_q, D), k_packed, k_norms, v_packed, v_norms, T, n_splits,
 //        k_layout, v_layout, scale, unrotate, workspace) -> fp16 of q's shape, or None
 PyObject* attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     int64_t T, n_splits, kl, vl, unrotate;
     if (n != 13 || !as_int(a[6], T) || !as_int(a[7], n_splits) || !as_int(a[8], kl) || !as_int(a[9], vl) ||
         !PyFloat_Check(a[10]) || !as_int(a[11], unrotate)) Py_RETURN_NONE;
@@ -331,12 +346,14 @@ PyObject* attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
         Py_DECREF(r);
     }
     return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
 }
 
 // ------------------------------------------------------------------------------------------ prompt phase
 // prompt(plans, q (B, n_q, S, D), rotate_q, k_packed, k_norms, v_packed, v_norms, T, k_row_width, v_row_width,
 //        q_pos_offset, is_causal, k_layout, v_layout, scale, unrotate) -> (B, n_q, S, D) fp16, or None
 PyObject* prompt(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     int64_t rotate, T, kw, vw, off, causal, kl, vl, unrotate;
     if (n != 16 || !as_int(a[2], rotate) || !as_int(a[7], T) || !as_int(a[8], kw) || !as_int(a[9], vw) || !as_int(a[10], off) ||
         !as_int(a[11], causal) || !as_int(a[12], kl) || !as_int(a[13], vl) || !PyFloat_Check(a[14]) || !as_int(a[15], unrotate)) Py_RETURN_NONE;
@@ -374,6 +391,7 @@ PyObject* prompt(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (rc == BGTQ_EUNSUPPORTED) Py_RETURN_NONE;
     if (rc != BGTQ_OK) return fail("bgtq_prompt_attn", rc);
     return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
 }
 
 PyObject* setup(PyObject*, PyObject* const* a, Py_ssize_t n) {
