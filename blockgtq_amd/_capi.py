@@ -46,6 +46,7 @@ _SIGNATURES = {
     "bgtq_set_decode_path": (c_i, [c_i]),
     "bgtq_workspace_bytes": (ctypes.c_size_t, [c_i, c_i, c_i]),
     "bgtq_default_splits": (c_i, [c_i, c_i, c_i]),
+    "bgtq_ragged_splits": (c_i, [c_i, c_i, c_i]),
     "bgtq_decode_attn": (c_i, [c_p, c_p, c_i64, c_i64,
                                c_p, c_i64, c_i64, c_i64, c_i,
                                c_p, c_i64, c_i64, c_i64,

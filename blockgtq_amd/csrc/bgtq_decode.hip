@@ -11,6 +11,8 @@
 // work-group, and thread (d, half) accumulates output dim d for one half of
 // the query heads over the tile's tokens.
 #include "bgtq_common.h"
+#include <algorithm>
+#include <cmath>
 #include <mutex>
 
 #include "bgtq_decode.h"
@@ -676,6 +678,34 @@ int scratch_of_current_device(void** out) {
     *out = g_scratch_ptr[dev];
     return BGTQ_OK;
 }
+// Partitions per (row, KV head).  A work-group keeps a compute unit busy, so what a launch takes is its rounds of 256
+// work-groups times (set-up and merge + tiles of a partition), in units of one tile at a work-group's full rate
+// (0.4 to 0.5 us); set-up and merge are worth 12 of them.  Only counts that just fill some number of rounds are
+// looked at, and a partition has at least 128 tokens.  One work-group too many costs a round:
+//   12 rows x 4 heads, 3001 tokens: 6 partitions (288 work-groups) 32.6 us a step, 5 (240) 26.0
+//   20 rows x 8 heads, 8k tokens:   2 (320) 105 us, 3 (480, two full rounds) 81
+// Rows of different lengths (the lengths are on the device): half of the longest on average, and where there are several
+// rounds the long partitions stick out behind the last one by some 0.65 of their length.
+//   8 rows x 2 heads, up to 32k tokens: 64 partitions (four rounds) 48.7 us a step, 16 33.0
+//   32 rows x 8 heads, up to 16k: 1 (one round) 144, 3 124, 4 121, 8 140; up to 4k: 1 50, 4 61
+int pick_splits(int B, int n_kv, int max_T, bool ragged) {
+    if (B <= 0 || n_kv <= 0 || max_T <= 0) return 1;
+    constexpr float FIXED = 12.f, MEAN = 0.53f, TAIL = 0.65f, MERGE = 1.f / 16.f;
+    const int64_t pairs = (int64_t)B * n_kv;
+    const int tiles = max_T / 64 + (max_T % 64 != 0);
+    const int most = std::min(max_T / 128 + (max_T % 128 != 0), (int)BGTQ_MAX_SPLITS);
+    int best = 1;
+    float best_cost = INFINITY;
+    for (int round = 1; round <= 8; round++) {
+        const int n = (int)std::max<int64_t>(1, std::min<int64_t>(most, 256 * round / pairs));
+        const int64_t rounds = (pairs * n + 255) / 256;
+        const float part = (float)((tiles + n - 1) / n);
+        const float cost = MERGE * n + (!ragged || rounds == 1 ? rounds * (FIXED + part) : rounds * (FIXED + MEAN * part) + TAIL * part);
+        if (cost < best_cost) { best = n; best_cost = cost; }
+    }
+    return best;
+}
+
 }  // namespace
 
 extern "C" {
@@ -693,18 +723,9 @@ size_t bgtq_workspace_bytes(int B, int n_q, int n_splits) {
     return (size_t)B * n_q * n_splits * (D + 1) * sizeof(float);
 }
 
-int bgtq_default_splits(int B, int n_kv, int max_T) {
-    // One work-group per partition and the fast kernel keeps a whole CU busy with
-    // one work-group, so aim for one partition per CU (256 of them), but never
-    // fewer than 128 tokens per partition.
-    if (B <= 0 || n_kv <= 0 || max_T <= 0) return 1;
-    int by_tokens = (max_T + 127) / 128;
-    int want = (256 + B * n_kv - 1) / (B * n_kv);
-    int s = want < by_tokens ? want : by_tokens;
-    if (s < 1) s = 1;
-    if (s > BGTQ_MAX_SPLITS) s = BGTQ_MAX_SPLITS;
-    return s;
-}
+int bgtq_default_splits(int B, int n_kv, int max_T) { return pick_splits(B, n_kv, max_T, false); }
+
+int bgtq_ragged_splits(int B, int n_kv, int max_T) { return pick_splits(B, n_kv, max_T, true); }
 
 int bgtq_decode_attn(const bgtq_head_plan* plans,
                      const void* q_rot, int64_t q_sb, int64_t q_sh,
@@ -790,7 +811,13 @@ int bgtq_decode_attend_static(const bgtq_head_plan* plans,
                               void* out, int64_t o_sb, int64_t o_sh, float* lse_out, void* stream) {
     BGTQ_CHECK_ARG(out);
     BGTQ_CHECK_ARG(B >= 0 && n_kv >= 0 && gqa >= 1 && gqa <= BGTQ_MAX_GQA);
-    if (n_splits <= 0) n_splits = bgtq_default_splits(B, n_kv, T > 0 ? T : 1);
+    if (n_splits <= 0) {
+        n_splits = bgtq_default_splits(B, n_kv, T > 0 ? T : 1);
+        // (no more than one round of them where more would not fit the array)
+        const int64_t pairs = (int64_t)B * n_kv;
+        if (n_splits > 1 && pairs > 0 && bgtq_workspace_bytes(B, n_kv * gqa, n_splits) > (size_t)BGTQ_STATIC_SCRATCH_BYTES)
+            n_splits = (int)std::min<int64_t>(n_splits, std::max<int64_t>(1, 256 / pairs));
+    }
     if (n_splits > BGTQ_MAX_SPLITS) return BGTQ_ELIMIT;
     if (B == 0 || n_kv == 0) return BGTQ_OK;
     const size_t rows = (size_t)B * n_kv * gqa * n_splits;         // (batch row, query head, partition)

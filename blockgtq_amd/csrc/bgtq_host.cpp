@@ -54,13 +54,7 @@ bool is_index(const at::Tensor& t, c10::DeviceIndex dev, int64_t n) {
 }
 
 int default_splits(int B, int n_kv, int64_t T, bool ragged) {
-    int n = bgtq_default_splits(B, n_kv, (int)(T > 1 ? T : 1));
-    if (ragged) {
-        // ragged rows: smaller partitions let the short rows' compute units pick up pieces of the long rows
-        const int64_t finer = std::min<int64_t>(4 * (int64_t)n, (T + 511) / 512);
-        n = (int)std::max<int64_t>(n, finer);
-    }
-    return n;
+    return (ragged ? bgtq_ragged_splits : bgtq_default_splits)(B, n_kv, (int)(T > 1 ? T : 1));
 }
 
 // At least `floats` fp32 values of the workspace object's buffer, grown as ops.Workspace grows it.

@@ -112,11 +112,8 @@ def decode_attention(plans: torch.Tensor, q_rot: torch.Tensor,
     v_row_width = v_packed.shape[-1] if v_row_width is None else v_row_width
     L = _capi.lib()
     if n_splits <= 0:
-        n_splits = L.bgtq_default_splits(B, n_kv, max(T, 1))
-        if seq_lens is not None:
-            # ragged rows: smaller partitions let the short rows' compute units pick up
-            # pieces of the long rows
-            n_splits = max(n_splits, min(4 * n_splits, (T + 511) // 512))
+        pick = L.bgtq_default_splits if seq_lens is None else L.bgtq_ragged_splits
+        n_splits = pick(B, n_kv, max(T, 1))
     ws = workspace or _default_ws
     part_out, part_lse = ws.get(B, n_q, n_splits, q_rot.device)
     st = _capi.stream_ptr(q_rot.device)

@@ -345,8 +345,11 @@ int bgtq_last_decode_path(void);
 /* Bytes of fp32 scratch bgtq_decode_attn needs for (B, n_q, n_splits). */
 size_t bgtq_workspace_bytes(int B, int n_q, int n_splits);
 
-/* Partition count bgtq_decode_attn would pick for n_splits <= 0. */
+/* Partition count for rows of max_T tokens (what bgtq_decode_attend_static picks for n_splits <= 0). */
 int bgtq_default_splits(int B, int n_kv, int max_T);
+
+/* The same for rows of different lengths, max_T tokens the longest. */
+int bgtq_ragged_splits(int B, int n_kv, int max_T);
 
 /*
  * Fused unpack + dequant + split-T decode attention over the packed cache,
@@ -411,6 +414,7 @@ int bgtq_lse_reduce(const bgtq_head_plan* plans,
  *
  *   arguments  as for bgtq_decode_attn (inputs) and bgtq_lse_reduce (unrotate, out,
  *              o_sb, o_sh, lse_out); n_splits <= 0 picks bgtq_default_splits
+ *              (or fewer, where that many partitions would not fit the array)
  *   limit      bgtq_workspace_bytes(B, n_kv * gqa, n_splits) must not exceed
  *              BGTQ_STATIC_SCRATCH_BYTES (8 MiB; BGTQ_ELIMIT otherwise) - e.g.
  *              B * n_q * n_splits <= 16256
