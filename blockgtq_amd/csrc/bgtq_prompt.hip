@@ -195,8 +195,8 @@ struct PromptArgs {
     int n_kv, gqa, S, T, n_tiles, q_pos_offset, causal, n_splits;
     float scale;
     int rotate_q, unrotate;
-    int rows;                                // query rows per work-group (32 a wave)
-    float *part_o, *part_ml;                 // n_splits > 1: sums [wg][wave][register][lane], (reference, denominator) [wg][wave][row]
+    int rows, n_qb;                          // query rows per work-group (32 a wave), blocks of them
+    float *part_o, *part_ml;                 // n_splits > 1: sums [wg][wave][register / 4][lane][4], (reference, denominator) [wg][wave][row]
     uint16_t* out; int64_t o_sb, o_sh, o_ss;
 };
 
@@ -348,7 +348,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
             if (live) add_part(voff);
             __syncthreads();
         }
-        if (tile0 < tile1) issue(tile0, K_PART);
+        if (tile0 < tile1) { issue(tile0, K_PART); issue(tile0, V_PART); }
 #pragma unroll
         for (int ob = 0; ob < 4; ob++)
 #pragma unroll
@@ -362,7 +362,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
             if (row.ok) { x0 = *(const uint2v*)(qrow + 16 * kk + 4 * lg); x1 = *(const uint2v*)(qrow + 16 * kk + 8 + 4 * lg); }
             Qb[kk] = __builtin_bit_cast(half8, (uint4v){x0.x, x0.y, x1.x, x1.y});
         }
-        if (tile0 < tile1) issue(tile0, K_PART);
+        if (tile0 < tile1) { issue(tile0, K_PART); issue(tile0, V_PART); }
     }
 
     const float c2 = a.scale * 1.44269504088896340736f;        // scores in log2 units
@@ -393,8 +393,10 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
                 if (32 * tb + 8 * (r >> 2) + (r & 3) >= rest) S[tb][r] = -INFINITY;
     };
     auto enter = [&](int tile) __attribute__((always_inline)) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // this wave's share of V of this tile and K of the next
-        __syncthreads();                                         // they are complete; everyone is done with the tile before
+        if (tile1 - tile0 > 1) {                                 // (a tile alone is complete already)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // this wave's share of V of this tile and K of the next
+            __syncthreads();                                     // they are complete; everyone is done with the tile before
+        }
         if (tile + 2 < tile1) issue(tile + 2, K_PART);
         if (tile + 1 < tile1) issue(tile + 1, V_PART);
         if (live && __builtin_amdgcn_ballot_w64(mx > m_ref)) {           // wave-uniform, rare after the first tiles
@@ -466,8 +468,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
     if (tile0 < tile1) {
         float16v Sa[2], Sb[2];
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();                                         // K of the first tile
-        issue(tile0, V_PART);
+        __syncthreads();                                         // the first tile
         if (tile0 + 1 < tile1) issue(tile0 + 1, K_PART);
         Sa[0] = Sa[1] = Sb[0] = Sb[1] = (float16v){0};
         if (live) {
@@ -507,58 +508,70 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
         }
         if (live) finish_rows(a, O, l_tot, row, b, h, lane);
     } else if (live) {
-        const size_t wg = ((size_t)(b * a.n_kv + h) * (gridDim.z / a.n_splits) + qb) * a.n_splits + c;
-        float* po = a.part_o + (wg * NW + wave) * 64 * 64 + lane;
+        const size_t wg = ((size_t)(b * a.n_kv + h) * a.n_qb + qb) * a.n_splits + c;
+        float4* po = (float4*)(a.part_o + (wg * NW + wave) * 64 * 64) + lane;
 #pragma unroll
-        for (int db = 0; db < 4; db++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) po[(16 * db + r) * 64] = O[db][r];
+        for (int i = 0; i < 16; i++) po[i * 64] = float4{O[i >> 2][4 * (i & 3)], O[i >> 2][4 * (i & 3) + 1], O[i >> 2][4 * (i & 3) + 2], O[i >> 2][4 * (i & 3) + 3]};
         if (lane < 32) *(float2*)(a.part_ml + ((wg * NW + wave) * 32 + lane) * 2) = float2{m_ref, l_tot};
     }
 }
 
 // ---- merge ------------------------------------------------------------------------------------------------
-// A work-group of 8 waves adds the partial sums of 32 rows (one wave of the attention): each wave takes every eighth
-// partition, then the eight meet in LDS.  (One wave walking all partitions took 43 us for 62 of them.)
-constexpr int MERGE_WAVES = 8;
-constexpr size_t MERGE_LDS = 2 * PART + 4 * (64 * 64 + 64) * sizeof(float);
-__global__ __launch_bounds__(64 * MERGE_WAVES) void prompt_merge_kernel(PromptArgs a) {
+// The partial sums of 32 rows (one wave of the attention) are added by PER waves.  Eight where few rows meet many
+// partitions: each wave takes every eighth of them, then the eight meet in LDS.  (One wave walking all of them took 43 us
+// for 62 partitions.)  One, and four groups of rows to a work-group, where the groups alone fill the chip and partitions
+// are few: 2 partitions of 1024 groups 28.9 us with eight waves a group (four rounds of work-groups that each fetch the
+// un-rotation and keep six waves waiting), 13.6 with one.
+constexpr int merge_waves(int per) { return per == 1 ? 4 : per; }
+constexpr size_t merge_lds(int per) { return 2 * PART + (per == 1 ? 0 : per / 2 * (64 * 64 + 64) * sizeof(float)); }
+template <int PER>
+__global__ __launch_bounds__(64 * merge_waves(PER)) void prompt_merge_kernel(PromptArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
+    constexpr int WAVES = merge_waves(PER);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nw = a.rows / 32, n_qb = (int)gridDim.z / nw;
-    const int h = blockIdx.x, b = blockIdx.y, qb = blockIdx.z / nw, w = blockIdx.z - qb * nw;
+    const int nw = a.rows / 32;
+    const int h = blockIdx.x, b = blockIdx.y;
+    const int group = min((int)blockIdx.z * (WAVES / PER) + wave / PER, a.n_qb * nw - 1);   // (a wave past the last group repeats it and stores nothing)
+    const bool mine = (int)blockIdx.z * (WAVES / PER) + wave / PER < a.n_qb * nw;
+    const int qb = group / nw, w = group - qb * nw, part = wave % PER;
     const RowOf row(a, qb, w, lane);
-    if (__builtin_amdgcn_ballot_w64(row.ok) == 0) return;        // (uniform over the work-group)
-    if (a.unrotate) load_parts<MERGE_WAVES>(a.rot + ((size_t)h * HEAD_PARTS + Q_PARTS_MAX) * PART, 2, wave, (uint32_t)lane * 16);
-    const size_t wg0 = ((size_t)(b * a.n_kv + h) * n_qb + qb) * a.n_splits;
+    if (PER == WAVES && __builtin_amdgcn_ballot_w64(row.ok) == 0) return;                    // (uniform over the work-group)
+    if (a.unrotate) load_parts<WAVES>(a.rot + ((size_t)h * HEAD_PARTS + Q_PARTS_MAX) * PART, 2, wave, (uint32_t)lane * 16);
+    const size_t wg0 = ((size_t)(b * a.n_kv + h) * a.n_qb + qb) * a.n_splits;
     float16v O[4];
 #pragma unroll
     for (int db = 0; db < 4; db++) O[db] = (float16v){0};
     float l_tot = 0.f, m = -INFINITY;
     const float2* ml = (const float2*)a.part_ml + (wg0 * nw + w) * 32 + (lane & 31);
     for (int c = 0; c < a.n_splits; c++) m = fmaxf(m, ml[(size_t)c * nw * 32].x);
-    for (int c = wave; c < a.n_splits; c += MERGE_WAVES) {
-        const float2 x = ml[(size_t)c * nw * 32];
-        const float f = x.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x.x - m);
-        l_tot += f * x.y;
-        const float* po = a.part_o + ((wg0 + c) * nw + w) * 64 * 64 + lane;
+    for (int c = part; c < a.n_splits; c += PER) {
+        const float4* po = (const float4*)(a.part_o + ((wg0 + c) * nw + w) * 64 * 64) + lane;
+        float4 x[16];
 #pragma unroll
-        for (int db = 0; db < 4; db++)
+        for (int i = 0; i < 16; i++) x[i] = po[i * 64];
+        const float2 y = ml[(size_t)c * nw * 32];
+        const float f = y.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(y.x - m);
+        l_tot += f * y.y;
 #pragma unroll
-            for (int r = 0; r < 16; r++) O[db][r] = fmaf(f, po[(16 * db + r) * 64], O[db][r]);
+        for (int i = 0; i < 16; i++) {
+            O[i >> 2][4 * (i & 3)] = fmaf(f, x[i].x, O[i >> 2][4 * (i & 3)]);
+            O[i >> 2][4 * (i & 3) + 1] = fmaf(f, x[i].y, O[i >> 2][4 * (i & 3) + 1]);
+            O[i >> 2][4 * (i & 3) + 2] = fmaf(f, x[i].z, O[i >> 2][4 * (i & 3) + 2]);
+            O[i >> 2][4 * (i & 3) + 3] = fmaf(f, x[i].w, O[i >> 2][4 * (i & 3) + 3]);
+        }
     }
-    float* meet = (float*)(smem + 2 * PART);                     // [4][64 registers, denominator][lane]
+    float* meet = (float*)(smem + 2 * PART);                     // [PER / 2][64 registers, denominator][lane]
 #pragma unroll
-    for (int half = MERGE_WAVES / 2; half >= 1; half >>= 1) {
-        float* at = meet + (wave & (half - 1)) * 65 * 64 + lane;
-        if (wave >= half && wave < 2 * half) {
+    for (int half = PER / 2; half >= 1; half >>= 1) {
+        float* at = meet + (part & (half - 1)) * 65 * 64 + lane;
+        if (part >= half && part < 2 * half) {
 #pragma unroll
             for (int r = 0; r < 64; r++) at[r * 64] = O[r >> 4][r & 15];
             at[64 * 64] = l_tot;
         }
         __syncthreads();
-        if (wave < half) {
+        if (part < half) {
 #pragma unroll
             for (int r = 0; r < 64; r++) O[r >> 4][r & 15] += at[r * 64];
             l_tot += at[64 * 64];
@@ -567,7 +580,7 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void prompt_merge_kernel(PromptAr
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // this wave's share of the un-rotation
     __syncthreads();
-    if (wave == 0) finish_rows(a, O, l_tot, row, b, h, lane);
+    if (part == 0 && mine) finish_rows(a, O, l_tot, row, b, h, lane);
 }
 
 // Rows of a work-group.  256 (one work-group a compute unit) fetch every tile for twice as many rows, which counts
@@ -636,7 +649,7 @@ int bgtq_prompt_attn(const bgtq_head_plan* plans,
         int ok = 1;
         for (const void* f : {(const void*)prompt_stage_kernel, (const void*)prompt_attn_kernel<false, 4>, (const void*)prompt_attn_kernel<true, 4>,
                               (const void*)prompt_attn_kernel<false, 8>, (const void*)prompt_attn_kernel<true, 8>,
-                              (const void*)prompt_merge_kernel}) {
+                              (const void*)prompt_merge_kernel<1>, (const void*)prompt_merge_kernel<8>}) {
             hipFuncAttributes fa;
             hipError_t e = hipFuncGetAttributes(&fa, f);
             if (e != hipSuccess) return (int)e;
@@ -671,7 +684,7 @@ int bgtq_prompt_attn(const bgtq_head_plan* plans,
     a.rot = g.rot; a.tiles = g.tiles;
     a.q = (const uint16_t*)q; a.q_sb = q_sb; a.q_sh = q_sh; a.q_ss = q_ss;
     a.n_kv = n_kv; a.gqa = gqa; a.S = S; a.T = T; a.n_tiles = g.n_tiles; a.q_pos_offset = q_pos_offset; a.causal = is_causal != 0;
-    a.n_splits = ns; a.rows = rows; a.scale = scale; a.rotate_q = rotate_q != 0; a.unrotate = unrotate != 0;
+    a.n_splits = ns; a.rows = rows; a.n_qb = n_qb; a.scale = scale; a.rotate_q = rotate_q != 0; a.unrotate = unrotate != 0;
     a.part_o = (float*)(g.tiles + (size_t)B * n_kv * g.n_tiles * TILE);
     a.part_ml = a.part_o + (size_t)B * n_kv * n_qb * ns * (rows / 32) * 64 * 64;
     a.out = (uint16_t*)out; a.o_sb = o_sb; a.o_sh = o_sh; a.o_ss = o_ss;
@@ -684,8 +697,13 @@ int bgtq_prompt_attn(const bgtq_head_plan* plans,
     auto attn = g.bf16 ? (rows == 256 ? prompt_attn_kernel<true, 8> : prompt_attn_kernel<true, 4>)
                        : (rows == 256 ? prompt_attn_kernel<false, 8> : prompt_attn_kernel<false, 4>);
     hipLaunchKernelGGL(attn, grid, dim3(2 * rows), PROMPT_LDS, st, a);
-    if (ns > 1)
-        hipLaunchKernelGGL(prompt_merge_kernel, dim3((unsigned)n_kv, (unsigned)B, (unsigned)(n_qb * (rows / 32))), dim3(64 * MERGE_WAVES), MERGE_LDS, st, a);
+    if (ns > 1) {
+        const int groups = n_qb * (rows / 32);
+        if ((int64_t)B * n_kv * groups > 256)
+            hipLaunchKernelGGL(prompt_merge_kernel<1>, dim3((unsigned)n_kv, (unsigned)B, (unsigned)((groups + 3) / 4)), dim3(64 * merge_waves(1)), merge_lds(1), st, a);
+        else
+            hipLaunchKernelGGL(prompt_merge_kernel<8>, dim3((unsigned)n_kv, (unsigned)B, (unsigned)groups), dim3(64 * merge_waves(8)), merge_lds(8), st, a);
+    }
     return bgtq_launch_status();
 }
 
