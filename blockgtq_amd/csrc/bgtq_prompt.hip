@@ -60,7 +60,6 @@ struct StageArgs {
     int k_layout, v_layout, k_row_width, v_stride;
     int kt, knr, vnr, vt;                    // raw tile areas in LDS
     int bf16, rotate_q;                      // parts of the query rotation: three bf16 / two fp16 / none
-    int tile_wgs;                            // work-groups that stage tiles; ROT_WGS per head follow
     uint8_t *rot, *tiles;
 };
 
@@ -71,7 +70,7 @@ __host__ __device__ inline int raw_bytes(int krow, int vstride, int kn_st, int& 
     vt = (MT * vstride + 32 + 15) & ~15;
     return kt + knr + vnr + vt;
 }
-constexpr int ROT_WGS = D * D / 8 / DQ_THR;   // work-groups per head that split its rotations
+constexpr int ROT_WGS = D * D / 8 / DQ_THR;   // work-groups per head that split its rotations, the first of the launch
 constexpr int RAW_OFF = BGTQ_VLUT_BYTES + BGTQ_LUT_IMAGE_BYTES;
 
 // One head's rotation parts.  A fragment (rows 32 ob .., step kk) holds, for lane (li, lg), row 32 ob + li and
@@ -120,20 +119,24 @@ __device__ __forceinline__ void stage_rotations(const StageArgs& a, int wg, int 
     }
 }
 
+// One set of raw records: two work-groups share a compute unit (at most 78 KB of LDS each) and one's loads run under the
+// other's lookups.  With two sets a work-group was alone there, and 292 of them (4100 records of 8 heads) took two rounds.
+// 4100 records of 8 heads: 19.9 -> 15.2 us, 4 x 8192 of 2 heads 26.9 -> 20.6.
 __global__ __launch_bounds__(DQ_THR) void prompt_stage_kernel(StageArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    if ((int)blockIdx.x >= a.tile_wgs) { stage_rotations(a, (int)blockIdx.x - a.tile_wgs, tid, smem); return; }
+    const int n_rot = ROT_WGS * a.n_kv;
+    if ((int)blockIdx.x < n_rot) { stage_rotations(a, (int)blockIdx.x, tid, smem); return; }
     const int wgs_per = (a.n_tiles + a.per_wg - 1) / a.per_wg;
-    const int pair = blockIdx.x / wgs_per, tile0 = ((int)blockIdx.x - pair * wgs_per) * a.per_wg;
+    const int pair = ((int)blockIdx.x - n_rot) / wgs_per, tile0 = ((int)blockIdx.x - n_rot - pair * wgs_per) * a.per_wg;
     const int tile1 = min(tile0 + a.per_wg, a.n_tiles);
     const int b = pair / a.n_kv, h = pair - b * a.n_kv;
     const bgtq_head_plan& P = a.plans[h];
     const bool vnib = a.v_layout == BGTQ_V_NIBBLE;
     const int krow = a.k_row_width, vrow = a.v_stride, kn_st = a.kn_st;
     const uint32_t voff = (uint32_t)lane * 16;
-    const uint32_t raw_set = (uint32_t)(a.kt + a.knr + a.vnr + a.vt), ktile = RAW_OFF + 2 * raw_set, vtile = ktile + MT * DQ_KROW;
+    const uint32_t kraw = RAW_OFF, knraw = kraw + a.kt, vnraw = knraw + a.knr, vraw = vnraw + a.vnr, ktile = vraw + a.vt, vtile = ktile + MT * DQ_KROW;
     const uint8_t* kp_base = a.kp + b * a.kp_sb + h * a.kp_sh;
     const uint8_t* vp_base = a.vp + b * a.vp_sb + h * a.vp_sh;
     const uint8_t* kn_base = (const uint8_t*)(a.kn + b * a.kn_sb + h * a.kn_sh);
@@ -143,7 +146,6 @@ __global__ __launch_bounds__(DQ_THR) void prompt_stage_kernel(StageArgs a) {
     // wave 0 fetches the K records, wave 1 the V records, wave 2 both norm arrays
     auto issue = [&](int tile) {
         const int t = tile * MT, nt = min(MT, a.T - t);
-        const uint32_t kraw = RAW_OFF + (uint32_t)(tile & 1) * raw_set, knraw = kraw + a.kt, vnraw = knraw + a.knr, vraw = vnraw + a.vnr;
         if (wave == 0) {
             dma_region<9>(kp_base - kph + (int64_t)t * krow, kraw, dma_shape((int)kph + nt * krow, voff), voff);
         } else if (wave == 1) {
@@ -168,11 +170,10 @@ __global__ __launch_bounds__(DQ_THR) void prompt_stage_kernel(StageArgs a) {
     for (int tile = tile0; tile < tile1; tile++) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();                     // raw tile (and tables) complete; the tile buffers have been read
-        const uint32_t raw0 = RAW_OFF + (uint32_t)(tile & 1) * raw_set, vn0 = raw0 + a.kt + a.knr;
-        if (tile + 1 < tile1) issue(tile + 1);
-        dq.run(raw0 + kph + (uint32_t)lane * krow, raw0 + a.kt + knph + (uint32_t)lane * kn_st * 2, vn0 + vnph, vn0 + a.vnr + vph, vrow,
+        dq.run(kraw + kph + (uint32_t)lane * krow, knraw + knph + (uint32_t)lane * kn_st * 2, vnraw + vnph, vraw + vph, vrow,
                min(MT, a.T - tile * MT), ktile, vtile);
         __syncthreads();
+        if (tile + 1 < tile1) issue(tile + 1);                   // (the raw tile has been read)
         uint8_t* o = out + (size_t)tile * TILE;
 #pragma unroll
         for (int c = 0; c < 2; c++) {        // K fragment (token block tb, step kk = wave); dims in the permuted order
@@ -691,8 +692,7 @@ int bgtq_prompt_attn(const bgtq_head_plan* plans,
     const int wgs_per = (staged + g.per_wg - 1) / g.per_wg;
     g.tile_stride = g.n_tiles;
     g.n_tiles = staged;
-    g.tile_wgs = wgs_per * B * n_kv;
-    hipLaunchKernelGGL(prompt_stage_kernel, dim3((unsigned)(g.tile_wgs + n_kv * ROT_WGS)), dim3(DQ_THR), (size_t)RAW_OFF + 2 * raw + DQ_TILE_BYTES, st, g);
+    hipLaunchKernelGGL(prompt_stage_kernel, dim3((unsigned)(n_kv * ROT_WGS + wgs_per * B * n_kv)), dim3(DQ_THR), (size_t)RAW_OFF + raw + DQ_TILE_BYTES, st, g);
     const dim3 grid((unsigned)n_kv, (unsigned)B, (unsigned)(n_qb * ns));
     auto attn = g.bf16 ? (rows == 256 ? prompt_attn_kernel<true, 8> : prompt_attn_kernel<true, 4>)
                        : (rows == 256 ? prompt_attn_kernel<false, 8> : prompt_attn_kernel<false, 4>);
