@@ -1168,10 +1168,8 @@ constexpr int PREP_ROWS = 1;       // rows of a work-group in the one-launch pre
 // ---- decode-step preparation: append-encode K and V and rotate the queries, one launch ----
 // Work-groups [0, nv) encode one V row each (the longest chain of the three goes out first),
 // [nv, nv + nk) one K row each, the rest rotate one or four query heads each.
-__global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq,
-                                                     int k_tiles, int v_tiles) {
-    __shared__ __align__(16) float rot_s[D * D];       // the work-group's rotation, whatever its role
-    int bid = blockIdx.x;
+__device__ __forceinline__ void prepare_part(const EncodeArgs& ak, const EncodeArgs& av, const RotQArgs& aq,
+                                             const int k_tiles, const int v_tiles, int bid, float* rot_s) {
     const int nk = k_tiles * ak.n_kv, nv = v_tiles * av.n_kv;
     if (bid < nv) {
         encode_rows<PREP_ROWS, true>(av, bid % v_tiles, bid / v_tiles, v_tiles, v_tiles, rot_s);
@@ -1181,6 +1179,23 @@ __global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs a
     } else {
         rotate_q_block(aq, bid - (nk + nv), rot_s);
     }
+}
+__global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq,
+                                                     int k_tiles, int v_tiles) {
+    __shared__ __align__(16) float rot_s[D * D];       // the work-group's rotation, whatever its role
+    prepare_part(ak, av, aq, k_tiles, v_tiles, blockIdx.x, rot_s);
+}
+// The same with the attention over the buffered tokens, which depends on none of it: the longer work-groups first, in
+// the LDS that is a rotation's otherwise; of the others two waves leave at once (a barrier counts the waves that are
+// left).  32 rows x 8 heads x 4 queries over 132 buffered tokens: 11.1 + 13.3 us as two launches,
+// 18.0 as one (1024 work-groups, two of them at a time on a compute unit).
+__global__ __launch_bounds__(WINDOW_THREADS, 2) void prepare_window_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, WindowArgs w,
+                                                                        int k_tiles, int v_tiles, int n_window) {
+    __shared__ __align__(16) float rot_s[D * D];
+    static_assert(window_lds_floats<4>(WINDOW_RIDE_W) <= D * D, "a window's scores fit the rotation's place");
+    const int bid = blockIdx.x, n_kv = ak.n_kv;
+    if (bid < n_window) window_attn_block<4>(w, bid % n_kv, bid / n_kv, rot_s);
+    else if (threadIdx.x < NT) prepare_part(ak, av, aq, k_tiles, v_tiles, bid - n_window, rot_s);
 }
 
 // argument checks + EncodeArgs assembly shared by the separate and the fused entry points
@@ -1242,10 +1257,10 @@ int launch_rotate_q(const bgtq_head_plan* plans, const void* q, int64_t q_sr, in
 
 // K and V appended and (q not null) the queries rotated: one launch for the few rows of a decode step
 int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, int64_t q_sr, int64_t q_sh, int q_bf16,
-                   void* q_rot, int64_t qr_sr, int64_t qr_sh, int gqa, hipStream_t st) {
+                   void* q_rot, int64_t qr_sr, int64_t qr_sh, int gqa, const WindowArgs* window, hipStream_t st) {
     const int B = ak.B, n_kv = ak.n_kv;
     const int64_t N = (int64_t)B * ak.S;
-    if (N > 64) {          // prefill-sized append: the three stages are big enough on their own
+    if (N > BGTQ_ONE_LAUNCH_ROWS) {          // prefill-sized append: the three stages are big enough on their own
         const int rc = launch_blocks(&ak, &av, st);
         if (rc != BGTQ_OK || !q) return rc;
         return launch_rotate_q(ak.plans, q, q_sr, q_sh, q_bf16, q_rot, qr_sr, qr_sh, B, n_kv, gqa, st);
@@ -1254,7 +1269,10 @@ int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, in
     RotQArgs aq{ak.plans, (const uint16_t*)q, q_sr, q_sh, (uint16_t*)q_rot, qr_sr, qr_sh, B, n_kv * gqa, gqa, group, q_bf16};
     const int tiles = (int)((N + PREP_ROWS - 1) / PREP_ROWS);
     const unsigned blocks = (unsigned)(2 * tiles * n_kv) + (q ? rotate_q_blocks(B, n_kv, gqa, group) : 0u);
-    hipLaunchKernelGGL(prepare_kernel, dim3(blocks), dim3(NT), 0, st, ak, av, aq, tiles, tiles);
+    if (window)
+        hipLaunchKernelGGL(prepare_window_kernel, dim3(blocks + (unsigned)(B * n_kv)), dim3(WINDOW_THREADS), 0, st, ak, av, aq, *window, tiles, tiles, B * n_kv);
+    else
+        hipLaunchKernelGGL(prepare_kernel, dim3(blocks), dim3(NT), 0, st, ak, av, aq, tiles, tiles);
     return bgtq_launch_status();
 }
 
@@ -1272,14 +1290,14 @@ int fill_step_args(const bgtq_step& s, EncodeArgs& ak, EncodeArgs& av) {
 
 }  // namespace
 
-int bgtq_step_prepare(const bgtq_step& s, bool kv_fp16, hipStream_t st) {
+int bgtq_step_prepare(const bgtq_step& s, bool kv_fp16, const WindowArgs* window, hipStream_t st) {
     EncodeArgs ak{}, av{};
     const int rc = fill_step_args(s, ak, av);
     if (rc != BGTQ_OK) return rc;
     const int q_bf16 = ak.bf16;
     if (kv_fp16) ak.bf16 = av.bf16 = 0;
     return launch_prepare(ak, av, s.q_rot ? s.q : nullptr, s.q_sb, s.q_sh, q_bf16, s.q_rot,
-                          (int64_t)s.n_kv * s.gqa * D, D, s.gqa, st);
+                          (int64_t)s.n_kv * s.gqa * D, D, s.gqa, window, st);
 }
 
 extern "C" {
@@ -1290,7 +1308,7 @@ int bgtq_encode_kv(const bgtq_step* step, void* stream) {
     EncodeArgs ak{}, av{};
     const int rc = fill_step_args(*step, ak, av);
     if (rc != BGTQ_OK) return rc;
-    return launch_prepare(ak, av, nullptr, 0, 0, 0, nullptr, 0, 0, 1, (hipStream_t)stream);
+    return launch_prepare(ak, av, nullptr, 0, 0, 0, nullptr, 0, 0, 1, nullptr, (hipStream_t)stream);
 }
 
 int bgtq_encode_k(const bgtq_head_plan* plans,
@@ -1383,7 +1401,7 @@ int bgtq_decode_prepare(const bgtq_head_plan* plans,
                      v_norms, vn_sb, vn_sh, vn_st, t_pos, t_pos_scalar, max_T, v_layout);
     if (rc != BGTQ_OK) return rc;
     BGTQ_CHECK_ARG((q == nullptr) == (q_rot == nullptr));     // both, or neither (queries rotated elsewhere)
-    return launch_prepare(ak, av, q, q_sr, q_sh, 0, q_rot, qr_sr, qr_sh, gqa, (hipStream_t)stream);
+    return launch_prepare(ak, av, q, q_sr, q_sh, 0, q_rot, qr_sr, qr_sh, gqa, nullptr, (hipStream_t)stream);
 }
 
 

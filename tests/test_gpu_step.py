@@ -64,3 +64,26 @@ def test_production_cache_step_and_append_equal_general_path(dtype, nibble, devi
     assert torch.equal(*outs) and outs[0].abs().max() > 0
     for name in ("k_packed", "k_norms", "v_packed", "v_norms"):
         assert torch.equal(getattr(caches[0], name), getattr(caches[1], name)), name
+
+
+# (rows, query heads, KV heads, window): the buffered tokens' partial rides with the preparation up to 64 rows, from two
+# query heads per KV head on and up to 3072 buffered tokens (4 of them sinks); beside each limit the launch of its own
+@pytest.mark.parametrize("batch,n_q,n_kv,window", [(64, 8, 2, 60), (65, 8, 2, 60), (3, 2, 2, 60), (3, 10, 2, 61), (1, 4, 1, 3068), (1, 4, 1, 3069)])
+def test_buffered_partial_with_and_without_the_preparation(batch, n_q, n_kv, window):
+    context = window + 70
+    lens = [max(context - 29 * b, window + 4) if b % 5 else context for b in range(batch)]      # (some rows fill just the buffer)
+    w = wl.Workload("t", 1, n_q, n_kv, batch, context, 1e6, seq_lens=lens, n_sink=4, window=window, seed=34)
+    mgrs = []
+    for _ in range(2):
+        mgr, energies = wl.build_manager(w, DEV)
+        wl.fill_cache(mgr, w, energies, DEV)
+        mgrs.append(mgr)
+    q, k, v = _inputs(w, energies, context, torch.bfloat16)
+    mgrs[1]._native = lambda li: mgrs[1]._ensure_storage()
+    for _ in range(2):                                                                  # (the ring moves on)
+        fast, slow = [m.append_and_attend(0, q, k, v) for m in mgrs]
+        assert fast.abs().max() > 0 and torch.equal(fast, slow)
+        for m in mgrs:
+            m.increment_seq_len()
+    for name in ("_k_packed", "_k_norms", "_v_packed", "_v_norms", "_buf_k", "_buf_v"):
+        assert torch.equal(getattr(mgrs[0], name)[0], getattr(mgrs[1], name)[0]), name
