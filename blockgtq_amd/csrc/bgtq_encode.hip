@@ -758,21 +758,18 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         }
         // ---- norms: the diagonal of X X^T; lane (li, lg) holds (row 4 lg + r, row li) in register r
         bool finite = true;
-        auto put_norm = [&](int g, const float4v& sum) {
-            const float ss = li & 2 ? (li & 1 ? sum[3] : sum[2]) : (li & 1 ? sum[1] : sum[0]);
-            const float n = __builtin_sqrtf(ss + 1e-30f);
-            const bool diag = (li >> 2) == lg;
-            finite = finite && (!diag || n < INFINITY);
-            if (diag) L.nrm[slot][g][li] = float2{n, 1.0f / n};
-        };
+        const bool diag = (li >> 2) == lg;
+        auto diagonal = [&](const float4v& sum) { return li & 2 ? (li & 1 ? sum[3] : sum[2]) : (li & 1 ? sum[1] : sum[0]); };
         if constexpr (IS_V) {
             float4v sum = {0, 0, 0, 0};
 #pragma unroll
             for (int kk = 0; kk < D / 4; kk++) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(A[kk], A[kk], sum, 0, 0, 0);
-            put_norm(0, sum);
+            const float n = __builtin_sqrtf(diagonal(sum) + 1e-30f);
+            if (diag) L.nrm[slot][0][li] = float2{n, 1.0f / n};
         } else {
-            // (CS 4: the groups are dealt to the waves)
-            for (int g = CS == 1 ? 0 : wave; g < n_seg; g += CS == 1 ? 1 : CS) {
+            constexpr int STEP = CS == 1 ? 1 : CS;            // (CS 4: the groups are dealt to the waves)
+            const int g_first = CS == 1 ? 0 : wave;
+            for (int g = g_first; g < n_seg; g += STEP) {
                 const int s = L.hdr[H_START + g], e = s + L.hdr[H_LEN + g];
                 float4v sum = {0, 0, 0, 0};
                 for (int q = s >> 4; q < (e + 15) >> 4; q++) {
@@ -784,7 +781,15 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
                         sum = __builtin_amdgcn_mfma_f32_16x16x4f32(x, x, sum, 0, 0, 0);
                     }
                 }
-                put_norm(g, sum);
+                if (diag) L.nrm[slot][g][li].x = diagonal(sum);
+            }
+            // roots and reciprocals of all groups together: four groups of 16 rows an instruction
+            asm volatile("" ::: "memory");                    // (a wave's LDS accesses keep their order)
+            for (int i = lane; g_first + STEP * (i >> 4) < n_seg; i += 64) {
+                float2* at = &L.nrm[slot][g_first + STEP * (i >> 4)][i & 15];
+                const float n = __builtin_sqrtf(at->x + 1e-30f);
+                finite = finite && n < INFINITY;
+                *at = float2{n, 1.0f / n};
             }
         }
         bool scalar_chain = !IS_V && __builtin_amdgcn_ballot_w64(!finite) != 0;           // (uniform)
@@ -816,18 +821,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         // codes of rows 4 lg .. + 3 from the values of column j
         auto quantise = [&](const float4v& y, int j, int g) -> uint32_t {
             uint32_t code[4] = {0, 0, 0, 0};
-            if constexpr (IS_V) {
-                auto count = [&](auto lo, auto hi) {           // (by halving: more instructions in the end, the choices cost as much)
-#pragma unroll
-                    for (int b = decltype(lo)::value; b < decltype(hi)::value; b++)
-#pragma unroll
-                        for (int r = 0; r < 4; r++) code[r] += y[r] > bd[b] ? 1u : 0u;
-                };
-                count(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
-                if (v_bits > 1) count(std::integral_constant<int, 1>{}, std::integral_constant<int, 3>{});      // (uniform)
-                if (v_bits > 2) count(std::integral_constant<int, 3>{}, std::integral_constant<int, 7>{});
-                if (v_bits > 3) count(std::integral_constant<int, 7>{}, std::integral_constant<int, 15>{});
-            } else if (a.quant_mode == BGTQ_QUANT_EXACT) {
+            if (a.quant_mode == BGTQ_QUANT_EXACT) {
                 const int nb = g >= 0 ? (1 << L.hdr[H_BW + g]) - 1 : 0;
 #pragma unroll 1
                 for (int b = 0; b < nb; b++)
@@ -872,37 +866,74 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         }
         // ---- rotate and quantise 16 columns at a time; codes of rows 4 lg .. + 3, column 16 cb + li
         uint32_t codes[D / 16 / CS];
+        // V: the cell search of 16 columns (the number of boundaries below a value) goes under the next 16 columns' products:
+        // behind its own, all waves of a SIMD would come to it together and leave the matrix core alone.  Operands are read
+        // eight steps ahead.
+        auto columns = [&](auto bits) {
+            constexpr int NB = (1 << decltype(bits)::value) - 1, EVERY = 32 / (NB + 1), NC = D / 16 / CS;
+            const float* rot = &L.rot[0][16 * (CS == 1 ? 0 : wave * NC) + li][lg];
+            float R[2][8];
+            auto fetch = [&](int at) {                        // eight steps: columns at / 4, steps 8 (at % 4) ..
 #pragma unroll
-        for (int c = 0; c < D / 16 / CS; c++) {
-            const int cb = CS == 1 ? c : wave * (D / 16 / CS) + c;
-            const int j = 16 * cb + li;
-            float4v y = {0, 0, 0, 0};
-            const float* rot = &L.rot[0][j][lg];              // + step * 4 D: two steps a read
-            int g = 0;
-            if constexpr (IS_V) {
+                for (int i = 0; i < 8; i++) R[at & 1][i] = rot[(at >> 2) * 64 + (8 * (at & 3) + i) * 4 * D];
+            };
+            fetch(0);
+            float4v y = {0, 0, 0, 0}, before = {0, 0, 0, 0};
+            uint32_t cell[4] = {0, 0, 0, 0};
 #pragma unroll
-                for (int q = 0; q < D / 16; q++) {
-#pragma unroll
-                    for (int i = 0; i < 4; i++) y = __builtin_amdgcn_mfma_f32_16x16x4f32(A[4 * q + i], rot[(4 * q + i) * 4 * D], y, 0, 0, 0);
+            for (int at = 0; at < 4 * NC; at++) {
+                if (at + 1 < 4 * NC) fetch(at + 1);
+                if ((at & 3) == 0) {
+                    before = y;
+                    y = (float4v){0, 0, 0, 0};
                 }
-            } else {
-                g = L.group[j];
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const int kk = 8 * (at & 3) + i;
+                    y = __builtin_amdgcn_mfma_f32_16x16x4f32(A[kk], R[at & 1][i], y, 0, 0, 0);
+                    if (at >= 4 && kk % EVERY == 0 && kk / EVERY < NB) {
+#pragma unroll
+                        for (int r = 0; r < 4; r++) cell[r] = (kk ? cell[r] : 0u) + (before[r] > bd[kk / EVERY] ? 1u : 0u);
+                    }
+                }
+                if (at >= 4 && (at & 3) == 3) codes[(at >> 2) - 1] = cell[0] | (cell[1] << 8) | (cell[2] << 16) | (cell[3] << 24);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                cell[r] = 0;
+#pragma unroll
+                for (int b = 0; b < NB; b++) cell[r] += y[r] > bd[b] ? 1u : 0u;
+            }
+            codes[NC - 1] = cell[0] | (cell[1] << 8) | (cell[2] << 16) | (cell[3] << 24);
+        };
+        if constexpr (IS_V) {
+            if (v_bits == 3) columns(std::integral_constant<int, 3>{});         // (uniform)
+            else if (v_bits == 4) columns(std::integral_constant<int, 4>{});
+            else if (v_bits == 2) columns(std::integral_constant<int, 2>{});
+            else columns(std::integral_constant<int, 1>{});
+        } else {
+#pragma unroll
+            for (int c = 0; c < D / 16 / CS; c++) {
+                const int cb = CS == 1 ? c : wave * (D / 16 / CS) + c;
+                const int j = 16 * cb + li;
+                float4v y = {0, 0, 0, 0};
+                const float* rot = &L.rot[0][j][lg];          // + step * 4 D: two steps a read
+                const int g = L.group[j];
                 if (scalar_chain) {
                     codes[c] = odd_codes[c];
                     continue;
                 }
-                {
-                    const int q_lo = __builtin_amdgcn_readfirstlane(L.span[cb].x), q_hi = __builtin_amdgcn_readfirstlane(L.span[cb].y);
+                const int q_lo = __builtin_amdgcn_readfirstlane(L.span[cb].x), q_hi = __builtin_amdgcn_readfirstlane(L.span[cb].y);
 #pragma unroll
-                    for (int q = 0; q < D / 16; q++)
-                        if (q >= q_lo && q < q_hi) {          // (uniform)
+                for (int q = 0; q < D / 16; q++)
+                    if (q >= q_lo && q < q_hi) {              // (uniform)
 #pragma unroll
-                            for (int i = 0; i < 4; i++) y = __builtin_amdgcn_mfma_f32_16x16x4f32(A[4 * q + i], rot[(4 * q + i) * 4 * D], y, 0, 0, 0);
-                        }
-                }
+                        for (int i = 0; i < 4; i++) y = __builtin_amdgcn_mfma_f32_16x16x4f32(A[4 * q + i], rot[(4 * q + i) * 4 * D], y, 0, 0, 0);
+                    }
+                codes[c] = quantise(y, j, g);
+                __builtin_amdgcn_sched_barrier(0);            // (operands of later columns would be read ahead and spill)
             }
-            codes[c] = quantise(y, j, g);
-            __builtin_amdgcn_sched_barrier(0);                // (operands of later columns would be read ahead and spill)
         }
         meet();                                               // (the raw rows are read)
 #pragma unroll
@@ -920,9 +951,25 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         };
         if (CS == 1 || wave == 0) {
             if (need_cent) {
-                for (int g = 0; g < n_seg; g++) {
-                    int s = 0, e = D, bw = 0;
-                    if constexpr (!IS_V) { s = L.hdr[H_START + g]; e = s + L.hdr[H_LEN + g]; bw = L.hdr[H_BW + g]; }
+                if constexpr (IS_V) {                         // the centroids of all codes in two bursts
+                    float4v sum = {0, 0, 0, 0};
+#pragma unroll
+                    for (int half = 0; half < 2; half++) {
+                        float cen[D / 8];
+#pragma unroll
+                        for (int q = 0; q < D / 32; q++) {
+                            const uint32_t* cw = (const uint32_t*)&raw[li * CROW + 64 * half + 16 * q];
+#pragma unroll
+                            for (int i = 0; i < 4; i++) cen[4 * q + i] = L.cent[(cw[i] >> (8 * lg)) & 15u];
+                        }
+#pragma unroll
+                        for (int i = 0; i < D / 8; i++) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(cen[i], cen[i], sum, 0, 0, 0);
+                    }
+                    const float cn = __builtin_sqrtf(diagonal(sum) + 1e-20f);
+                    if (diag) store_norm(0, li, L.nrm[slot][0][li].x / (cn > 1e-10f ? cn : 1.0f));
+                }
+                for (int g = 0; !IS_V && g < n_seg; g++) {
+                    const int s = L.hdr[H_START + g], e = s + L.hdr[H_LEN + g], bw = L.hdr[H_BW + g];
                     float4v sum = {0, 0, 0, 0};
 #pragma unroll 1
                     for (int q = s >> 4; q < (e + 15) >> 4; q++) {
@@ -932,28 +979,22 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
                         for (int i = 0; i < 4; i++) {
                             const int k = 16 * q + 4 * i + lg;
                             const uint32_t code = (cw[i] >> (8 * lg)) & 0xFFu;
-                            if constexpr (IS_V) c[i] = L.cent[code & 15u];
-                            else {
-                                c[i] = bw > 5 ? P.k_centroids[g][code] : L.cent[g * 32 + (code & 31u)];
-                                if (k < s || k >= e) c[i] = 0.f;
-                            }
+                            c[i] = bw > 5 ? P.k_centroids[g][code] : L.cent[g * 32 + (code & 31u)];
+                            if (k < s || k >= e) c[i] = 0.f;
                         }
 #pragma unroll
                         for (int i = 0; i < 4; i++) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(c[i], c[i], sum, 0, 0, 0);
                     }
-                    const float cs = li & 2 ? (li & 1 ? sum[3] : sum[2]) : (li & 1 ? sum[1] : sum[0]);
-                    if ((li >> 2) == lg) {
-                        const float n = L.nrm[slot][g][li].x;
-                        if constexpr (IS_V) {
-                            const float cn = __builtin_sqrtf(cs + 1e-20f);
-                            store_norm(0, li, n / (cn > 1e-10f ? cn : 1.0f));
-                        } else {
-                            store_norm(g, li, n / fmaxf(__builtin_sqrtf(cs), 1e-10f));
-                        }
+                    if (diag) L.nrm[slot][g][li].y = diagonal(sum);       // (the reciprocals have served)
+                }
+                if constexpr (!IS_V) {
+                    asm volatile("" ::: "memory");
+                    for (int i = lane; i < BGTQ_MAX_SEGMENTS * 16; i += 64) {
+                        const int g = i >> 4, row = i & 15;
+                        const float2 v = L.nrm[slot][g][row];
+                        store_norm(g, row, g < n_seg ? v.x / fmaxf(__builtin_sqrtf(v.y), 1e-10f) : 0.f);
                     }
                 }
-                if (!IS_V)
-                    for (int i = lane; i < (BGTQ_MAX_SEGMENTS - n_seg) * 16; i += 64) store_norm(n_seg + (i >> 4), i & 15, 0.f);
             } else {
                 for (int i = lane; i < BGTQ_MAX_SEGMENTS * 16; i += 64) {
                     const int g = i & 7, row = i >> 3;
@@ -969,6 +1010,9 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
             }
         } else if (4 * dw < a.row_width) {
             const int rows = 64 / lpr;
+            uint4 make[4];                                    // (the stores could alias the table for all the compiler knows: read once)
+#pragma unroll
+            for (int i = 0; i < 4; i++) make[i] = L.pack[4 * dw + i];
 #pragma unroll 2
             for (int r = lane / lpr + (CS == 1 ? 0 : wave * rows); r < 16; r += rows * CS) {
                 const int64_t dst = L.dst[slot][r];
@@ -976,7 +1020,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
                 uint32_t byte[4];
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const uint4 p = L.pack[4 * dw + i];
+                    const uint4 p = make[i];
                     const uint32_t* c = (const uint32_t*)&raw[r * CROW + (p.x & ~3u)];
                     const uint32_t c0 = c[0], c1 = c[1];
                     const uint32_t x = __builtin_amdgcn_alignbyte(c1, c0, p.x & 3u);
