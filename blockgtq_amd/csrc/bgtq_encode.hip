@@ -536,7 +536,7 @@ __global__ __launch_bounds__(NT) void encode_kernel(EncodeArgs a) {
 // rows): the 4 waves of a work-group split the columns of one block, which quarters its longest stage.
 // Bound by the matrix cores: 320 instructions of 32 clocks a V block.  65 536 records each of K and V (4 x 8192
 // tokens, 2 heads, K3V3): 135 us as two launches of 16-row tiles on the vector units (there the dense V rotation
-// alone is 55 us of FMA), 65 us here in one.
+// alone is 55 us of FMA), 61 us here in one (65 with the cell search behind its own columns' products).
 // ================================================================================================
 constexpr int RROW = D * 2 + 16;        // bytes from one raw row to the next: rows 4 banks apart
 constexpr int CROW = D + 8;             // bytes from one row of codes to the next (a byte's window of codes may reach 8 past the last)
@@ -1224,8 +1224,11 @@ __device__ __forceinline__ void prepare_part(const EncodeArgs& ak, const EncodeA
         rotate_q_block(aq, bid - (nk + nv), rot_s);
     }
 }
+// (BF16: some input is; asking at run time costs the chains of fp16 inputs 0.2 of 5.0 us)
+template <bool BF16>
 __global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq,
                                                      int k_tiles, int v_tiles) {
+    if (!BF16) ak.bf16 = av.bf16 = aq.bf16 = 0;
     __shared__ __align__(16) float rot_s[D * D];       // the work-group's rotation, whatever its role
     prepare_part(ak, av, aq, k_tiles, v_tiles, blockIdx.x, rot_s);
 }
@@ -1315,8 +1318,10 @@ int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, in
     const unsigned blocks = (unsigned)(2 * tiles * n_kv) + (q ? rotate_q_blocks(B, n_kv, gqa, group) : 0u);
     if (window)
         hipLaunchKernelGGL(prepare_window_kernel, dim3(blocks + (unsigned)(B * n_kv)), dim3(WINDOW_THREADS), 0, st, ak, av, aq, *window, tiles, tiles, B * n_kv);
+    else if (ak.bf16 || av.bf16 || (q && q_bf16))
+        hipLaunchKernelGGL(prepare_kernel<true>, dim3(blocks), dim3(NT), 0, st, ak, av, aq, tiles, tiles);
     else
-        hipLaunchKernelGGL(prepare_kernel, dim3(blocks), dim3(NT), 0, st, ak, av, aq, tiles, tiles);
+        hipLaunchKernelGGL(prepare_kernel<false>, dim3(blocks), dim3(NT), 0, st, ak, av, aq, tiles, tiles);
     return bgtq_launch_status();
 }
 
