@@ -234,8 +234,9 @@ def fill_decode_steps(p) -> None:
                     img[LUT_K5P // 4:LUT_K5P // 4 + 1024] = cb[e & 31].astype(np.uint32) | (cb[e >> 5].astype(np.uint32) << 16)
                 unit_bytes = 8
                 row = [0, 0, 0, 0, 0, VLUT_BYTES + table, 0]
-            if bw > 4 and len(units) % 2:
-                # the kernel takes pair-table units two at a time: an empty unit evens them out
+            if bw > 4 and n_pair == len(units) and n_pair % 2:
+                # pair-table units are an even number: an empty one ahead of the first raw-byte unit evens them out
+                # (between two raw-byte segments none may stand: it would count the first raw-byte unit as a pair-table one)
                 units.append(0)
                 progs.append([0] * 7)
                 offs.append(0)

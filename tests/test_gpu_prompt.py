@@ -19,16 +19,7 @@ def _cache(B, n_kv, T, kl, vl, bits):
     w = wl.Workload("t", 1, n_kv, n_kv, B, T, 1e6, k_bits=k_bits, v_bits=v_bits, min_bits=lo, max_bits=hi, seed=51)
     qs, e = wl.calibrate_layer(w, 0, DEV)
     args = build_batched_encode_args(qs, device=DEV)
-    k, v = wl.draw_kv(w, e, T, 3, DEV)
-    kw = P.cache_row_bytes(args['max_mixed_bytes'] if kl == P.K_MIXED else args['max_tpb'])
-    vw = 64 if vl == P.V_NIBBLE else args['v_packed_bytes']
-    kp = torch.zeros(B, n_kv, T, kw, dtype=torch.uint8, device=DEV)
-    kn = torch.zeros(B, n_kv, T, args['max_n_groups'], dtype=torch.float16, device=DEV)
-    vp = torch.zeros(B, n_kv, T, P.cache_row_bytes(vw), dtype=torch.uint8, device=DEV)[..., :vw]
-    vn = torch.zeros(B, n_kv, T, dtype=torch.float16, device=DEV)
-    encode_k_into(args['plans'], k, kp, kn, 0, kw, kn.shape[-1], kl)
-    encode_v_into(args['plans'], v, vp, vn, 0, vw, vl)
-    return args, qs, (kp, kn, vp, vn)
+    return args, qs, _encode(args, *wl.draw_kv(w, e, T, 3, DEV), kl, vl)
 
 
 def _no_workspace(args, q_rot, cache, T, off, causal, kl, vl, unrotate):
@@ -70,3 +61,41 @@ def test_prompt_attention_equals_the_kernel_without_workspace(B, n_kv, gqa, S, T
         for name, g in got.items():
             assert g.shape == want.shape and torch.isfinite(g).all()
             assert (g.float() - want).norm() <= 2e-3 * want.norm(), name
+
+
+def _plans_of(bits):
+    k_bits, v_bits, lo, hi = bits
+    w = wl.Workload("t", 1, 1, 1, 1, 64, 1e6, k_bits=k_bits, v_bits=v_bits, min_bits=lo, max_bits=hi, seed=52)
+    return build_batched_encode_args(wl.calibrate_layer(w, 0, DEV)[0], device=DEV)
+
+
+def _encode(args, k, v, kl, vl):
+    B, n_kv, T, _ = k.shape
+    kw = P.cache_row_bytes(args['max_mixed_bytes'] if kl == P.K_MIXED else args['max_tpb'])
+    vw = 64 if vl == P.V_NIBBLE else args['v_packed_bytes']
+    kp = torch.zeros(B, n_kv, T, kw, dtype=torch.uint8, device=DEV)
+    kn = torch.zeros(B, n_kv, T, args['max_n_groups'], dtype=torch.float16, device=DEV)
+    vp = torch.zeros(B, n_kv, T, P.cache_row_bytes(vw), dtype=torch.uint8, device=DEV)[..., :vw]
+    vn = torch.zeros(B, n_kv, T, dtype=torch.float16, device=DEV)
+    encode_k_into(args['plans'], k, kp, kn, 0, kw, kn.shape[-1], kl)
+    encode_v_into(args['plans'], v, vp, vn, 0, vw, vl)
+    return kp, kn, vp, vn
+
+
+@pytest.mark.parametrize("bits", [(4.0, 4, 1, 8), (5.0, 3, 3, 8)])
+@pytest.mark.parametrize("kl,vl", [(P.K_BITPACKED, P.V_BITPACKED), (P.K_MIXED, P.V_NIBBLE)])
+def test_records_with_several_raw_byte_segments(bits, kl, vl):
+    """5- and 6-bit codes and wider in one record, both kernels against fp64 attention over the records that another kernel
+    dequantises: probabilities and outputs are rounded to fp16 once each, 2^-11 of their size at most."""
+    T, S = 200, 64
+    args = _plans_of(bits)
+    assert (args['plans_np'][0]['seg_bw'] > 4).sum() > 1
+    gen = torch.Generator(device=DEV).manual_seed(6)
+    k, v = (torch.randn(1, 1, T, 128, generator=gen, device=DEV).half() for _ in range(2))
+    cache = _encode(args, k, v, kl, vl)
+    k_hat, v_hat = (t.double() for t in ops.dequant_kv(args['plans'], *cache, T, k_layout=kl, v_layout=vl))
+    q = torch.randn(1, 2, S, 128, generator=gen, device=DEV).half()
+    want = torch.softmax(q.double() @ k_hat.transpose(2, 3).contiguous() * 128 ** -0.5, 3) @ v_hat
+    got = ops.prefill_attention_packed(args['plans'], q, *cache, T, k_layout=kl, v_layout=vl, is_causal=False, unrotate=False)
+    for g in (got, _no_workspace(args, q, cache, T, 0, False, kl, vl, False)):
+        assert (g.double() - want).norm() <= 2 ** -10 * want.norm()

@@ -509,6 +509,29 @@ def test_step_tables_reproduce_the_checker_scores(oracle_lib, seed, min_bits, ma
             assert np.abs(got - ref).max() < 1e-9
 
 
+# blocks (of 2 dims) per code width: an odd number of units ahead of the second, third or fourth raw-byte segment
+@pytest.mark.parametrize("blocks", [{2: 11, 3: 13, 4: 10, 5: 25, 6: 5}, {1: 20, 6: 8, 8: 36}, {4: 12, 5: 4, 6: 4, 7: 8, 8: 36},
+                                    {5: 12, 7: 52}, {0: 10, 3: 9, 5: 5, 6: 5, 7: 5, 8: 30}])
+def test_step_tables_with_several_raw_byte_segments(oracle_lib, blocks):
+    alloc = [bw for bw, n in blocks.items() for _ in range(n)]
+    assert len(alloc) == 64
+    q, en = make_quantizer(seed=21, alloc=alloc)
+    k, _, qq = make_kv(en, 3, seed=21)
+    plan = q.plan()
+    p, ng = plan[0], int(plan[0]['n_seg'])
+    codes, raw, corr = oracle_lib.encode_k(plan, k)
+    qr = oracle_lib.rotate_q(plan, qq).astype(np.float32)
+    for mixed in (False, True):
+        pairs = sum((int(p['seg_len'][s]) + 7) // 8 for s in range(ng) if int(p['seg_bw'][s]) <= 4)
+        assert int(p['n_pair_units'][int(mixed)]) == pairs + pairs % 2
+        kp = oracle_lib.pack_k(plan, codes, int(mixed))
+        nr = (corr if mixed else raw)[:, :ng]
+        kn = oracle_lib.f2h(nr).view(np.float16).astype(np.float32)
+        for t in range(k.shape[0]):
+            ref = qr.astype(np.float64) @ oracle_lib.dequant_k(plan, codes[t:t + 1], oracle_lib.f2h(nr[t:t + 1]))[0].astype(np.float64)
+            assert np.abs(_emulate_steps(p, kp[t], kn[t], qr, int(mixed)) - ref).max() < 1e-9
+
+
 def test_cache_rows_avoid_strides_that_collide_in_lds():
     from blockgtq_amd.plan import cache_row_bytes
     for n in range(1, 129):
