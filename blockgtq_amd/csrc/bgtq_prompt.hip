@@ -428,11 +428,12 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
         }
         // ---- probabilities (raw scores stay in the registers; the scale goes into the exponent's multiply-add) under the
         // products of the next scores: a pair of exponentials, and the packing of the pair before, with every product
-        float p0 = 0.f, p1 = 0.f;
+        // (The denominator adds the exponentials as they are: below 2^-14 the rounded ones keep less than 11 bits, and a long
+        // tail of those can be a per cent of it.  Tile by tile, because one of them alone vanishes beside the whole sum.)
+        float p0 = 0.f, p1 = 0.f, l_tile = 0.f;
         auto pack = [&](int j) __attribute__((always_inline)) {
             Pw[j] = cvt_pk_f16(p0, p1);
-            // (the denominator adds the probabilities the values are weighted with: two a dot product)
-            l_part = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, Pw[j]), (half2v){(_Float16)1.f, (_Float16)1.f}, l_part, false);
+            l_tile += p0 + p1;
         };
 #pragma unroll
         for (int i = 0; i < 16; i++) {
@@ -447,6 +448,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
             if (next) __builtin_amdgcn_sched_barrier(0);
         }
         pack(15);
+        l_part += l_tile;
         // ---- O^T += V^T P^T: 16-token group 2 tb + hf; the maximum of the next scores underneath
         float m = -INFINITY;
 #pragma unroll

@@ -99,3 +99,26 @@ def test_records_with_several_raw_byte_segments(bits, kl, vl):
     got = ops.prefill_attention_packed(args['plans'], q, *cache, T, k_layout=kl, v_layout=vl, is_causal=False, unrotate=False)
     for g in (got, _no_workspace(args, q, cache, T, 0, False, kl, vl, False)):
         assert (g.double() - want).norm() <= 2 ** -10 * want.norm()
+
+
+def test_small_probabilities_count_in_the_denominator():
+    """Each query has one strong record among the first and 65 535 weak ones, e^-18 of it apiece and below the smallest fp16
+    number once the reference lies 4 octaves above the strong score; together they are 4e-3 of the denominator.
+    As fp16 values they lose most of that.  The numerator may drop them: over thousands of unrelated values
+    they come to some 1e-4 of the output; the rest of the bound is the output's own rounding (2^-11 at most)."""
+    T, gqa, n = 65536, 16, 32
+    args = _plans_of((4.0, 4, 1, 8))
+    gen = torch.Generator(device=DEV).manual_seed(5)
+    x = torch.randn(1, 1, T, 128, generator=gen, device=DEV)
+    cache = _encode(args, x.half(), torch.randn(1, 1, T, 128, generator=gen, device=DEV).half(), P.K_BITPACKED, P.V_BITPACKED)
+    k_hat, v_hat = (t[0, 0].double() for t in ops.dequant_kv(args['plans'], *cache, T))
+    own = k_hat[:n]
+    q = (own / own.square().sum(1, keepdim=True) * 18 * 128 ** 0.5).half()      # a score of 18 on the own record, 0 +- 1.6 elsewhere
+    p = torch.softmax(q.double() @ k_hat.T * 128 ** -0.5, 1)
+    assert (1 - p.max(1).values).min() > 2e-3
+    want = p @ v_hat
+    rows = q.repeat(4096 // n, 1).expand(1, gqa, 4096, 128)                     # (enough rows that the context is not split)
+    got = ops.prefill_attention_packed(args['plans'], rows, *cache, T, is_causal=False, unrotate=False)
+    got = got[0].reshape(-1, n, 128)
+    assert torch.equal(got, got[:1].expand_as(got))
+    assert (got[0].double() - want).norm() <= 6e-4 * want.norm()
