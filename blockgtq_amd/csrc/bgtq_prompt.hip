@@ -17,8 +17,10 @@
 //   merge   only where a few query rows meet a long context: the tiles of a query block are dealt to several
 //           work-groups, whose unnormalised sums this kernel adds and un-rotates.
 //
-// Arithmetic as in bgtq_prefill_attn: fp16(centroid * norm) records, fp16 rotated queries and probabilities, fp32
-// sums; rotations from parts that hold 22 (fp16) or 24 (bf16) bits of the fp32 matrices, summed in fp32.
+// Arithmetic: fp16(centroid * norm) records, fp16 rotated queries and probabilities, fp32 sums (the denominator from
+// the fp32 exponentials).  The query rotation counts with its fp32 values whole: three 16-bit parts of an entry add up to
+// it, their products with 16-bit queries are exact and summed in fp32.  The un-rotation takes two fp16 parts of either
+// factor, as bgtq_prefill_attn does: an error of 2^-22 of the largest terms, ahead of a rounding to fp16 (2^-11).
 //
 // Reference behaviour: blockgtq/prefill.py:66-101, blockgtq/kernels/fused_packed_attention.py:1876-2594.
 #include <algorithm>
@@ -40,8 +42,11 @@ constexpr int TILE = 2 * MT * D * 2;         // bytes of a staged tile: K fragme
 constexpr int PART = D * D * 2;              // bytes of one 16-bit part of a rotation
 constexpr float REFRESH = 4.0f;
 
-// rotation parts of a head: the query rotation (3 bf16 or 2 fp16 parts), then the un-rotation (2 fp16 parts)
-constexpr int Q_PARTS_MAX = 3, HEAD_PARTS = Q_PARTS_MAX + 2;
+// rotation parts of a head: the query rotation (3 parts in the type of the queries), then the un-rotation (2 fp16 parts)
+constexpr int Q_PARTS = 3, HEAD_PARTS = Q_PARTS + 2;
+// fp16 has no exponents for what a head leaves over (an entry of 0.01 and its remainders span 2^-7 to 2^-31): every
+// remainder is held 2^11 times as large as it is, which is about the size of the head
+constexpr float F16_STEP = 2048.f;
 
 __device__ __forceinline__ uint32_t cvt_pk_f16(float lo, float hi) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
@@ -59,7 +64,7 @@ struct StageArgs {
     int n_kv, T, n_tiles, per_wg, tile_stride;   // tiles of a (row, head), how many of them a work-group takes, the workspace's room
     int k_layout, v_layout, k_row_width, v_stride;
     int kt, knr, vnr, vt;                    // raw tile areas in LDS
-    int bf16, rotate_q;                      // parts of the query rotation: three bf16 / two fp16 / none
+    int bf16, rotate_q;                      // parts of the query rotation: bf16 / fp16, or none
     uint8_t *rot, *tiles;
 };
 
@@ -88,23 +93,25 @@ __device__ __forceinline__ void stage_rotations(const StageArgs& a, int wg, int 
         const int lane = i & 63, kk = (i >> 6) & 7, ob = i >> 9, li = lane & 31, lg = lane >> 5;
         const int row = 32 * ob + li;
         if (a.rotate_q) {
-            uint16_t part[3][8];
+            uint16_t part[Q_PARTS][8];
 #pragma unroll
             for (int e = 0; e < 8; e++) {
-                const float x = P.k_rot_T[inv[16 * kk + 8 * lg + e] * D + row];
-                if (a.bf16) {
-                    const __bf16 p0 = (__bf16)x, p1 = (__bf16)(x - (float)p0), p2 = (__bf16)(x - (float)p0 - (float)p1);
-                    part[0][e] = __builtin_bit_cast(uint16_t, p0);
-                    part[1][e] = __builtin_bit_cast(uint16_t, p1);
-                    part[2][e] = __builtin_bit_cast(uint16_t, p2);
-                } else {
-                    const _Float16 p0 = (_Float16)x, p1 = (_Float16)(x - (float)p0);
-                    part[0][e] = __builtin_bit_cast(uint16_t, p0);
-                    part[1][e] = __builtin_bit_cast(uint16_t, p1);
-                    part[2][e] = 0;
+                float x = P.k_rot_T[inv[16 * kk + 8 * lg + e] * D + row];
+#pragma unroll
+                for (int p = 0; p < Q_PARTS; p++) {              // (differences and powers of two: exact)
+                    if (a.bf16) {
+                        const __bf16 v = (__bf16)x;
+                        part[p][e] = __builtin_bit_cast(uint16_t, v);
+                        x -= (float)v;
+                    } else {
+                        const _Float16 v = (_Float16)x;
+                        part[p][e] = __builtin_bit_cast(uint16_t, v);
+                        x = (x - (float)v) * F16_STEP;
+                    }
                 }
             }
-            for (int p = 0; p < (a.bf16 ? 3 : 2); p++) *(uint4v*)(dst + p * PART + i * 16) = *(const uint4v*)part[p];
+#pragma unroll
+            for (int p = 0; p < Q_PARTS; p++) *(uint4v*)(dst + p * PART + i * 16) = *(const uint4v*)part[p];
         }
         uint16_t hi[8], lo[8];
 #pragma unroll
@@ -114,8 +121,8 @@ __device__ __forceinline__ void stage_rotations(const StageArgs& a, int wg, int 
             hi[e] = __builtin_bit_cast(uint16_t, p0);
             lo[e] = __builtin_bit_cast(uint16_t, p1);
         }
-        *(uint4v*)(dst + Q_PARTS_MAX * PART + i * 16) = *(const uint4v*)hi;
-        *(uint4v*)(dst + (Q_PARTS_MAX + 1) * PART + i * 16) = *(const uint4v*)lo;
+        *(uint4v*)(dst + Q_PARTS * PART + i * 16) = *(const uint4v*)hi;
+        *(uint4v*)(dst + (Q_PARTS + 1) * PART + i * 16) = *(const uint4v*)lo;
     }
 }
 
@@ -218,10 +225,10 @@ struct RowOf {
     }
 };
 
-// n consecutive rotation parts from the workspace to LDS address 0: each wave its share
+// n consecutive rotation parts from the workspace to LDS address dst: each wave its share
 template <int NW>
-__device__ __forceinline__ void load_parts(const uint8_t* src, int n, int wave, uint32_t voff) {
-    for (int c = wave; c < n * (PART / 4096); c += NW) dma_full<4>(voff, uniform_ptr(src + c * 4096), (uint32_t)c * 4096);
+__device__ __forceinline__ void load_parts(const uint8_t* src, int n, int wave, uint32_t voff, uint32_t dst = 0) {
+    for (int c = wave; c < n * (PART / 4096); c += NW) dma_full<4>(voff, uniform_ptr(src + c * 4096), dst + (uint32_t)c * 4096);
 }
 
 // Normalise, un-rotate (out^T = R^T O^T: both factors split into fp16 head and remainder, the product of the
@@ -285,7 +292,6 @@ __device__ __forceinline__ void finish_rows(const PromptArgs& a, float16v (&O)[4
 template <bool BF16, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
-    constexpr int Q_PARTS = BF16 ? 3 : 2;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.x, b = blockIdx.y;
@@ -315,8 +321,8 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
     half8 Qb[8];
     const uint16_t* qrow = a.q + b * a.q_sb + ((int64_t)h * a.gqa + (row.ok ? row.hq : 0)) * a.q_sh + (int64_t)(row.ok ? row.sq : 0) * a.q_ss;
     if (a.rotate_q) {
-        // the last two parts fit LDS at a time; three (bf16) come as the two small ones, then the head
-        load_parts<NW>(rot_h + (Q_PARTS - 2) * PART, 2, wave, voff);
+        // two parts fit LDS at a time: the remainders first; the head takes the last one's place under the products of the other
+        load_parts<NW>(rot_h + PART, 2, wave, voff);
         uint4v qv[8];                                            // lane: dims 16 kk + 8 lg .. + 7 of its query
 #pragma unroll
         for (int kk = 0; kk < 8; kk++) {
@@ -340,15 +346,22 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
         };
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        if (live) { add_part(PART + voff); add_part(voff); }     // (the small parts first)
+        auto step = [&]() {                                      // sums of a part in units of the next larger one
+            if constexpr (!BF16) {
+#pragma unroll
+                for (int ob = 0; ob < 4; ob++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) R[ob][r] *= 1.f / F16_STEP;
+            }
+        };
+        if (live) { add_part(PART + voff); step(); }
         __syncthreads();
-        if (BF16) {
-            load_parts<NW>(rot_h, 1, wave, voff);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
-            if (live) add_part(voff);
-            __syncthreads();
-        }
+        load_parts<NW>(rot_h, 1, wave, voff, PART);
+        if (live) { add_part(voff); step(); }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (live) add_part(PART + voff);
+        __syncthreads();
         if (tile0 < tile1) { issue(tile0, K_PART); issue(tile0, V_PART); }
 #pragma unroll
         for (int ob = 0; ob < 4; ob++)
@@ -505,7 +518,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
     if (a.n_splits == 1) {
         if (a.unrotate) {
             __syncthreads();                                     // every wave is done with the tiles
-            load_parts<NW>(rot_h + Q_PARTS_MAX * PART, 2, wave, voff);
+            load_parts<NW>(rot_h + Q_PARTS * PART, 2, wave, voff);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
         }
@@ -540,7 +553,7 @@ __global__ __launch_bounds__(64 * merge_waves(PER)) void prompt_merge_kernel(Pro
     const int qb = group / nw, w = group - qb * nw, part = wave % PER;
     const RowOf row(a, qb, w, lane);
     if (PER == WAVES && __builtin_amdgcn_ballot_w64(row.ok) == 0) return;                    // (uniform over the work-group)
-    if (a.unrotate) load_parts<WAVES>(a.rot + ((size_t)h * HEAD_PARTS + Q_PARTS_MAX) * PART, 2, wave, (uint32_t)lane * 16);
+    if (a.unrotate) load_parts<WAVES>(a.rot + ((size_t)h * HEAD_PARTS + Q_PARTS) * PART, 2, wave, (uint32_t)lane * 16);
     const size_t wg0 = ((size_t)(b * a.n_kv + h) * a.n_qb + qb) * a.n_splits;
     float16v O[4];
 #pragma unroll

@@ -4,6 +4,7 @@ against the kernel that takes rotated queries and no workspace.
 Both dequantise to the same fp16 records and sum in fp32; they round probabilities, outputs and
 rotated queries to fp16 from sums in another order, i.e. each value is off by at most one rounding
 (2^-11 of it, 3e-4 on average) in three places: 2e-3 of the output's norm bounds them together."""
+import numpy as np
 import pytest
 import torch
 
@@ -122,3 +123,27 @@ def test_small_probabilities_count_in_the_denominator():
     got = got[0].reshape(-1, n, 128)
     assert torch.equal(got, got[:1].expand_as(got))
     assert (got[0].double() - want).norm() <= 6e-4 * want.norm()
+
+
+@pytest.mark.parametrize("shift", [0, 14])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_rotation_keeps_the_bits_of_small_entries(shift, dtype):
+    """The rotation counts with all its fp32 bits, whatever the size of its entries: entries scaled by 2^-14 against queries
+    scaled by 2^14 give the same products.  An fp32 sum of 128 terms lands on the other side of an fp16 midpoint in about
+    2^-24 sqrt(128) / 2^-12 of the cases, 3e-3, so 70 % of the rows meet none and agree bit for bit; 0.4 is asked for."""
+    n_kv, S, T = 2, 256, 200
+    args, qs, cache = _cache(1, n_kv, T, P.K_BITPACKED, P.V_BITPACKED, (3.0, 3, 1, 5))
+    gen = torch.Generator(device=DEV).manual_seed(9)
+    q = torch.randn(1, n_kv, S, 128, generator=gen, device=DEV).mul(0.7).clamp(-3.9, 3.9).to(dtype)
+    rot = []
+    for h, q8 in enumerate(qs):
+        m = torch.zeros(128, 128, dtype=torch.float64, device=DEV)
+        m[q8._head_perm] = q8._block_rot_T.double()
+        rot.append((q[:, h:h + 1].double() @ m).half())
+    want = ops.prefill_attention_packed(args['plans'], torch.cat(rot, 1), *cache, T, scale=0.5, is_causal=False, unrotate=False)
+    small = args['plans_np'].copy()
+    small['k_rot_T'] *= np.float32(2.0 ** -shift)
+    got = ops.prefill_attention_packed(P.upload_plans(small, DEV), q * 2.0 ** shift, *cache, T, scale=0.5, is_causal=False,
+                                       unrotate=False, rotate_q=True)
+    same = (got == want).all(-1).float().mean().item()
+    assert same >= 0.4, same
