@@ -658,7 +658,9 @@ int bgtq_prompt_attn(const bgtq_head_plan* plans,
     BGTQ_CHECK_ARG(workspace && ((uintptr_t)workspace & 15) == 0);
     if (workspace_bytes < bgtq_prompt_workspace_bytes(B, n_kv, gqa, S, T)) return BGTQ_EINVAL;
     const int rows = prompt_rows(B, n_kv, gqa, S), BQ = rows / gqa, n_qb = (S + BQ - 1) / BQ, ns = prompt_splits(B, n_kv, gqa, S, T);
-    if ((int64_t)n_qb * std::max(ns, rows / 32) > 65535 || B > 65535) return BGTQ_EUNSUPPORTED;
+    // a grid dimension holds 65535 query blocks (the bound of bgtq_prefill_attn: blocks of fewer rows are only taken below
+    // 2^19 rows); with partitions there are at most 256 blocks, and as many groups of 32 rows as the merge's grid takes
+    if (n_qb > 65535 || B > 65535) return BGTQ_EUNSUPPORTED;
     static std::atomic<int> ready{0};
     if (ready.load(std::memory_order_acquire) == 0) {
         // offsets into the dynamic LDS block are used as LDS addresses: holds only without static LDS

@@ -337,6 +337,7 @@ def prefill_attention_records(plans, q_rot, k_packed, k_norms, v_packed, v_norms
                                    vp, vn, T, k_row_width=kp.stride(2), **kw)
     if out is None:
         raise RuntimeError("bgtq_prompt_attn does not take this argument set (more than 256 query heads per "
-                           "KV head, a V record that is not 16, 32, 48 or 64 bytes, or more than 8 norm columns)")
+                           "KV head, a V record that is not 16, 32, 48 or 64 bytes, more than 8 norm columns, or "
+                           "more than 65535 batch rows or blocks of 256 / gqa query tokens)")
     return out
 

@@ -572,6 +572,7 @@ int bgtq_dequant_kv(const bgtq_head_plan* plans,
  *   out        fp16 [B][n_kv*gqa][S][128], strides o_sb/o_sh/o_ss in halves
  * B == 0 or S == 0 returns BGTQ_OK with nothing written.  Returns BGTQ_EUNSUPPORTED,
  * with nothing launched, unless all of these hold: gqa <= 256, scale > 0, T > 0;
+ * B <= 65535 and at most 65535 blocks of 256 / gqa query tokens;
  * K rows follow each other (kp_st == k_row_width, 4..128, a multiple of 4; kp_sb, kp_sh
  * and the base multiples of 4); kn_st in 1..8; v_row_width one of 16, 32, 48, 64 (64 for
  * the nibble layout) with v_row_width <= vp_st <= v_row_width + 4 and vp_* and the base

@@ -147,3 +147,13 @@ def test_rotation_keeps_the_bits_of_small_entries(shift, dtype):
                                        unrotate=False, rotate_q=True)
     same = (got == want).all(-1).float().mean().item()
     assert same >= 0.4, same
+
+
+def test_many_query_rows_in_one_call():
+    """65 600 tokens of 32 query heads on one KV head, more groups of 32 rows than one grid dimension holds: as two halves."""
+    args, _, cache = _cache(1, 1, 70, P.K_BITPACKED, P.V_BITPACKED, (3.0, 3, 1, 5))
+    S = 65600
+    q = torch.randn(1, 32, S, 128, device=DEV, dtype=torch.float16)
+    got = ops.prefill_attention_records(args['plans'], q, *cache, 70, is_causal=False)
+    for part in (slice(0, S // 2), slice(S // 2, S)):
+        assert torch.equal(got[:, :, part], ops.prefill_attention_records(args['plans'], q[:, :, part], *cache, 70, is_causal=False))
