@@ -99,6 +99,9 @@ _SIGNATURES = {
 }
 
 
+UNSUPPORTED = -2                # BGTQ_EUNSUPPORTED: not for this kernel, nothing launched
+
+
 class BgtqError(RuntimeError):
     pass
 

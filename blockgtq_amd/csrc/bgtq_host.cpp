@@ -365,7 +365,8 @@ PyObject* prompt(PyObject*, PyObject* const* a, Py_ssize_t n) {
         kn.scalar_type() != at::kHalf || vn.scalar_type() != at::kHalf || kp.stride(3) != 1 || vp.stride(3) != 1 || kn.stride(3) != 1) Py_RETURN_NONE;
     const int64_t B = q.size(0), n_q = q.size(1), S = q.size(2), n_kv = kp.size(1);
     if (n_kv < 1 || n_q % n_kv || kp.size(2) < T || vp.size(2) < T || kn.size(2) < T || vn.size(2) < T || T < 0 || kp.size(0) < B) Py_RETURN_NONE;
-    const size_t bytes = bgtq_prompt_workspace_bytes((int)B, (int)n_kv, (int)(n_q / n_kv), (int)S, (int)T);
+    const int64_t seen = causal ? std::min(T, off + S) : T;      // records that some row sees
+    const size_t bytes = bgtq_prompt_workspace_bytes((int)B, (int)n_kv, (int)(n_q / n_kv), (int)S, (int)seen);
     // (the allocator hands the same block out again from call to call, and to nobody else before the launches are done)
     at::Tensor ws = at::empty({(int64_t)bytes}, q.options().dtype(at::kByte));
     at::Tensor out = at::empty({B, n_q, S, D}, q.options().dtype(at::kHalf));

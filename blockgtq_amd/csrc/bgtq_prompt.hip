@@ -61,7 +61,7 @@ struct StageArgs {
     const uint16_t* kn; int64_t kn_sb, kn_sh; int kn_st;
     const uint8_t* vp;  int64_t vp_sb, vp_sh;
     const uint16_t* vn; int64_t vn_sb, vn_sh;
-    int n_kv, T, n_tiles, per_wg, tile_stride;   // tiles of a (row, head), how many of them a work-group takes, the workspace's room
+    int n_kv, T, n_tiles, per_wg;            // tiles of a (row, head), how many of them a work-group takes
     int k_layout, v_layout, k_row_width, v_stride;
     int kt, knr, vnr, vt;                    // raw tile areas in LDS
     int bf16, rotate_q;                      // parts of the query rotation: bf16 / fp16, or none
@@ -173,7 +173,7 @@ __global__ __launch_bounds__(DQ_THR) void prompt_stage_kernel(StageArgs a) {
         lds_put<uint32_t>(ktile + (uint32_t)t * DQ_KROW + c * 4, 0u);
     }
     const int li = lane & 31, lg = lane >> 5;
-    uint8_t* out = a.tiles + (size_t)pair * a.tile_stride * TILE + voff;
+    uint8_t* out = a.tiles + (size_t)pair * a.n_tiles * TILE + voff;
     for (int tile = tile0; tile < tile1; tile++) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();                     // raw tile (and tables) complete; the tile buffers have been read
@@ -656,6 +656,7 @@ int bgtq_prompt_attn(const bgtq_head_plan* plans,
     if ((q_ss & 7) || (q_sh & 7) || (q_sb & 7) || ((uintptr_t)q & 15)) return BGTQ_EUNSUPPORTED;           // 16-byte query loads
     if ((o_ss & 3) || (o_sh & 3) || (o_sb & 3) || ((uintptr_t)out & 7)) return BGTQ_EUNSUPPORTED;          // 8-byte output stores
     BGTQ_CHECK_ARG(workspace && ((uintptr_t)workspace & 15) == 0);
+    if (is_causal) T = (int)std::min<int64_t>(T, (int64_t)q_pos_offset + S);                               // no row sees a record past the last query's position
     if (workspace_bytes < bgtq_prompt_workspace_bytes(B, n_kv, gqa, S, T)) return BGTQ_EINVAL;
     const int rows = prompt_rows(B, n_kv, gqa, S), BQ = rows / gqa, n_qb = (S + BQ - 1) / BQ, ns = prompt_splits(B, n_kv, gqa, S, T);
     // a grid dimension holds 65535 query blocks (the bound of bgtq_prefill_attn: blocks of fewer rows are only taken below
@@ -687,14 +688,11 @@ int bgtq_prompt_attn(const bgtq_head_plan* plans,
     g.kn = (const uint16_t*)k_norms; g.kn_sb = kn_sb; g.kn_sh = kn_sh; g.kn_st = (int)kn_st;
     g.vp = (const uint8_t*)v_packed; g.vp_sb = vp_sb; g.vp_sh = vp_sh;
     g.vn = (const uint16_t*)v_norms; g.vn_sb = vn_sb; g.vn_sh = vn_sh;
-    g.n_kv = n_kv; g.n_tiles = (T + MT - 1) / MT;
-    // causal rows see no record past the last query's position
-    g.T = is_causal ? (int)std::min<int64_t>(T, (int64_t)q_pos_offset + S) : T;
-    const int staged = (g.T + MT - 1) / MT;
+    g.n_kv = n_kv; g.T = T; g.n_tiles = (T + MT - 1) / MT;
     g.k_layout = k_layout; g.v_layout = v_layout; g.k_row_width = k_row_width; g.v_stride = (int)vp_st;
     const int raw = raw_bytes(k_row_width, (int)vp_st, (int)kn_st, g.kt, g.knr, g.vnr, g.vt);
     // two work-groups fit a compute unit; tiles in equal shares over what that makes
-    g.per_wg = (int)std::max<int64_t>(1, ((int64_t)staged * B * n_kv + 511) / 512);
+    g.per_wg = (int)std::max<int64_t>(1, ((int64_t)g.n_tiles * B * n_kv + 511) / 512);
     g.bf16 = x_dtype == BGTQ_X_BF16; g.rotate_q = rotate_q != 0;
     g.rot = ws;
     g.tiles = ws + (size_t)n_kv * HEAD_PARTS * PART;
@@ -706,9 +704,7 @@ int bgtq_prompt_attn(const bgtq_head_plan* plans,
     a.part_o = (float*)(g.tiles + (size_t)B * n_kv * g.n_tiles * TILE);
     a.part_ml = a.part_o + (size_t)B * n_kv * n_qb * ns * (rows / 32) * 64 * 64;
     a.out = (uint16_t*)out; a.o_sb = o_sb; a.o_sh = o_sh; a.o_ss = o_ss;
-    const int wgs_per = (staged + g.per_wg - 1) / g.per_wg;
-    g.tile_stride = g.n_tiles;
-    g.n_tiles = staged;
+    const int wgs_per = (g.n_tiles + g.per_wg - 1) / g.per_wg;
     hipLaunchKernelGGL(prompt_stage_kernel, dim3((unsigned)(n_kv * ROT_WGS + wgs_per * B * n_kv)), dim3(DQ_THR), (size_t)RAW_OFF + raw + DQ_TILE_BYTES, st, g);
     const dim3 grid((unsigned)n_kv, (unsigned)B, (unsigned)(n_qb * ns));
     auto attn = g.bf16 ? (rows == 256 ? prompt_attn_kernel<true, 8> : prompt_attn_kernel<true, 4>)

@@ -279,7 +279,11 @@ def prefill_attention_packed(plans: torch.Tensor, q_rot: torch.Tensor, k_packed:
     or bf16, rotated inside the kernel; cache tensors as for ``decode_attention``.
     Query token s sees records ``t <= q_pos_offset + s`` when ``is_causal``.  Returns
     (B, n_q, S, D) fp16, or ``None`` when the kernel does not take this argument set
-    (``prefill_attention_records`` copies records into rows the kernel can walk first)."""
+    (``prefill_attention_records`` copies records into rows the kernel can walk first).
+
+    The records that are seen are staged in a transient workspace, 512 bytes a record and KV head.  Where
+    the device has no room for it the kernel that dequantises tile by tile takes over (1.5 times as long
+    for 4 prompts of 8192 tokens)."""
     _capi.require_cuda(k_packed, "k_packed")
     assert q_rot.dim() == 4 and q_rot.stride(-1) == 1
     assert q_rot.dtype == torch.float16 or (rotate_q and q_rot.dtype == torch.bfloat16)
@@ -293,9 +297,48 @@ def prefill_attention_packed(plans: torch.Tensor, q_rot: torch.Tensor, k_packed:
     v_row_width = v_packed.shape[-1] if v_row_width is None else v_row_width
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
     from . import _host
-    return _host.module().prompt(plans, q_rot, int(rotate_q), k_packed, k_norms, v_packed, v_norms, int(T), k_row_width,
-                                 v_row_width, int(q_pos_offset), int(bool(is_causal)), k_layout, v_layout, scale,
-                                 int(bool(unrotate)))
+    try:
+        return _host.module().prompt(plans, q_rot, int(rotate_q), k_packed, k_norms, v_packed, v_norms, int(T), k_row_width,
+                                     v_row_width, int(q_pos_offset), int(bool(is_causal)), k_layout, v_layout, scale,
+                                     int(bool(unrotate)))
+    except torch.OutOfMemoryError:
+        pass                                                    # (outside: the exception holds on to nothing by then)
+    q = _rotate_prompt(plans, q_rot, n_kv) if rotate_q else q_rot
+    return _prefill_without_workspace(plans, q, k_packed, k_norms, v_packed, v_norms, int(T), k_row_width, v_row_width,
+                                      int(q_pos_offset), bool(is_causal), k_layout, v_layout, scale, bool(unrotate))
+
+
+def _rotate_prompt(plans: torch.Tensor, q: torch.Tensor, n_kv: int) -> torch.Tensor:
+    """q (B, n_q, S, D) of 16 bits -> permuted and rotated fp16 for a device that is short of memory: fp32 sums,
+    dim after dim (a library product would ask for a workspace of its own, 76 MB)."""
+    def field(name, dtype):
+        at, size = _plan.PLAN_DTYPE.fields[name][1], _plan.PLAN_DTYPE.fields[name][0].itemsize
+        return plans.reshape(n_kv, -1)[:, at:at + size].contiguous().view(dtype)
+    D = _plan.HEAD_DIM
+    rows = field('head_perm', torch.int32).long().unsqueeze(2).expand(n_kv, D, D)
+    rot = torch.zeros((n_kv, D, D), device=q.device).scatter_(1, rows, field('k_rot_T', torch.float32).view(n_kv, D, D))
+    x = q.unflatten(1, (n_kv, -1))
+    acc = torch.zeros(x.shape, device=q.device)
+    for d in range(D):
+        acc.addcmul_(x[..., d:d + 1].float(), rot[:, d].view(n_kv, 1, 1, D))
+    return acc.to(torch.float16).flatten(1, 2)
+
+
+def _prefill_without_workspace(plans, q_rot, k_packed, k_norms, v_packed, v_norms, T, k_row_width, v_row_width,
+                               q_pos_offset, is_causal, k_layout, v_layout, scale, unrotate) -> Optional[torch.Tensor]:
+    """``bgtq_prefill_attn`` on rotated fp16 queries, or ``None`` where it does not take the argument set."""
+    B, n_q, S, D = q_rot.shape
+    n_kv = k_packed.shape[1]
+    out = torch.empty((B, n_q, S, D), dtype=torch.float16, device=q_rot.device)
+    rc = _capi.lib().bgtq_prefill_attn(
+        _capi.ptr(plans), _capi.ptr(q_rot), *q_rot.stride()[:3], _capi.ptr(k_packed), *k_packed.stride()[:3], k_row_width,
+        _capi.ptr(k_norms), *k_norms.stride()[:3], _capi.ptr(v_packed), *v_packed.stride()[:3], v_row_width,
+        _capi.ptr(v_norms), *v_norms.stride(), B, n_kv, n_q // n_kv, S, T, q_pos_offset, int(is_causal), k_layout, v_layout,
+        scale, int(unrotate), _capi.ptr(out), *out.stride()[:3], _capi.stream_ptr(q_rot.device))
+    if rc == _capi.UNSUPPORTED:
+        return None
+    _capi.check(rc, "bgtq_prefill_attn")
+    return out
 
 
 def _packed_rows(rec: torch.Tensor, T: int, width: int, v_rows: bool = False) -> torch.Tensor:

@@ -3,7 +3,9 @@
 All prompt tokens go through one transformer layer at a time: QKV + RoPE for
 the whole prompt, one quantise-and-pack launch per K and V, causal attention
 over the records just written, MLP.  No fp16 KV cache of the full model is
-ever materialised.  Reference behaviour: blockgtq/prefill.py:24-111.
+ever materialised; while a layer attends, its visible records lie dequantised in
+a transient workspace (512 bytes a record and KV head).  Reference behaviour:
+blockgtq/prefill.py:24-111.
 
 As in the reference, attention inside the prompt sees the *quantised* keys and
 values (what later decode steps will see), not the layer's fp16 K/V:

@@ -599,8 +599,10 @@ int bgtq_prefill_attn(const bgtq_head_plan* plans,
  * a long context, the tiles of a block are dealt to several work-groups and merged.  Same layout
  * requirements and BGTQ_EUNSUPPORTED cases as bgtq_prefill_attn.
  *   q          [B][n_kv*gqa][S][128] of x_dtype (BGTQ_X_*), strides in elements, rows 16-byte aligned
- *   workspace  bgtq_prompt_workspace_bytes(B, n_kv, gqa, S, T) bytes of device memory on a 16-byte
- *              boundary, free again when the launches are done
+ *   workspace  bgtq_prompt_workspace_bytes(B, n_kv, gqa, S, seen) bytes of device memory on a 16-byte
+ *              boundary, free again when the launches are done; seen = T, or with is_causal the
+ *              records up to the last query, min(T, q_pos_offset + S).  512 bytes a record and KV head,
+ *              160 KB a KV head, and at most 34 MB for partitions
  */
 size_t bgtq_prompt_workspace_bytes(int B, int n_kv, int gqa, int S, int T);
 int bgtq_prompt_attn(const bgtq_head_plan* plans,

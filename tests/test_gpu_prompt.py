@@ -157,3 +157,38 @@ def test_many_query_rows_in_one_call():
     got = ops.prefill_attention_records(args['plans'], q, *cache, 70, is_causal=False)
     for part in (slice(0, S // 2), slice(S // 2, S)):
         assert torch.equal(got[:, :, part], ops.prefill_attention_records(args['plans'], q[:, :, part], *cache, 70, is_causal=False))
+
+
+def test_workspace_covers_the_records_that_are_seen():
+    """A causal call near the start of a long cache stages what its rows see: 100 records, not 40 000."""
+    T = 40000
+    args, _, cache = _cache(1, 1, T, P.K_BITPACKED, P.V_BITPACKED, (3.0, 3, 1, 5))
+    q = torch.randn(1, 4, 60, 128, device=DEV, dtype=torch.float16)
+    want = ops.prefill_attention_packed(args['plans'], q, *[t[:, :, :100] for t in cache], 100, q_pos_offset=40)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    got = ops.prefill_attention_packed(args['plans'], q, *cache, T, q_pos_offset=40)
+    torch.cuda.synchronize()
+    assert torch.cuda.max_memory_allocated() - before < 2 << 20
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("rotate", [False, True])
+def test_without_room_for_the_workspace(rotate):
+    """8 heads of 32 768 records stage into 134 MB.  Where the device has no room for that the kernel that takes none attends
+    (records of one tile at a time in LDS; the two agree as in the first test)."""
+    B, n_kv, T, S = 1, 8, 32768, 24
+    args, qs, cache = _cache(B, n_kv, T, P.K_BITPACKED, P.V_BITPACKED, (3.0, 3, 1, 5))
+    q = torch.randn(B, S, 4 * n_kv, 128, device=DEV).half().transpose(1, 2)
+    kw = dict(q_pos_offset=T - S, rotate_q=rotate)
+    want = ops.prefill_attention_records(args['plans'], q, *cache, T, **kw).float()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (64 << 20)) / total)
+    try:
+        got = ops.prefill_attention_records(args['plans'], q, *cache, T, **kw).float()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert (got - want).norm() <= 2e-3 * want.norm()
