@@ -25,11 +25,17 @@ def module():
     return _mod
 
 
-def layer(plans, k_packed, k_norms, v_packed, v_norms, k_row_width, norm_width, v_row_width, n_q,
+def layer(held, li, plans, k_packed, k_norms, v_packed, v_norms, k_row_width, norm_width, v_row_width, n_q,
           k_layout, v_layout, scale, baked, buf_k=None, buf_v=None):
-    """A native layer handle over one layer's plans and cache views, or None where they are not on the GPU
-    (the general path then says so)."""
+    """The native handle of layer ``li`` over its plans and cache: ``held`` if that is it, a new one otherwise, None where
+    the cache is not on the GPU (the general path then says so).  The cache tensors are one layer's, or all layers'
+    stacked."""
+    rest = (k_row_width, norm_width, v_row_width, n_q, k_layout, v_layout, scale, baked)
+    if held is not None and held.holds(li, plans, k_packed, k_norms, v_packed, v_norms, *rest, buf_k, buf_v):
+        return held
     if not (plans.is_cuda and k_packed.is_cuda):
         return None
-    return module().Layer(plans, k_packed, k_norms, v_packed, v_norms, k_row_width, norm_width, v_row_width, n_q,
-                          k_layout, v_layout, scale, baked, buf_k, buf_v)
+
+    def one(t, dims=4):
+        return t[li] if t is not None and t.dim() == dims + 1 else t
+    return module().Layer(plans, one(k_packed), one(k_norms), one(v_packed), one(v_norms, 3), *rest, one(buf_k), one(buf_v))

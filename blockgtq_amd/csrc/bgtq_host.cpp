@@ -2,8 +2,9 @@
 //
 // A decode step of one layer is 20 to 45 us of GPU work in three to five launches; issued from Python through
 // ctypes (some 45 arguments a call, three allocations, three dtype conversions) it took 60 us of host time
-// and the GPU waited.  Here a Layer keeps what does not change from step to step (plans, cache views,
-// widths, layouts) and one call per layer checks the three tensors that do, takes scratch from the owner's
+// and the GPU waited.  Here a Layer keeps what rarely changes from step to step (plans, cache views,
+// widths, layouts, scale); the owner asks it (holds) whether it still is what its attributes say and makes another one
+// if not.  One call per layer checks the three tensors that do change, takes scratch from the owner's
 // workspace, allocates the output and issues the launches.
 //
 // Every entry returns None for a call outside the shapes, types and strides it knows.  The Python caller
@@ -119,7 +120,8 @@ PyObject* layer_new(PyTypeObject* type, PyObject* args, PyObject*) {
     if (!L) return nullptr;
     at::Tensor** dst[7] = {&L->plans, &L->kp, &L->kn, &L->vp, &L->vn, &L->bk, &L->bv};
     THPObjectPtr owner((PyObject*)L);                // (freed should one of the tensors have no storage)
-    for (int i = 0; i < 7; i++) *dst[i] = t[i] ? new at::Tensor(*t[i]) : nullptr;
+    // (aliases: they keep the storage, and stay what they are if someone gives the tensor another one)
+    for (int i = 0; i < 7; i++) *dst[i] = t[i] ? new at::Tensor(t[i]->detach()) : nullptr;
     bgtq_step& s = L->s;
     s = bgtq_step{};
     s.plans = (const bgtq_head_plan*)t[0]->data_ptr();
@@ -142,6 +144,40 @@ PyObject* layer_new(PyTypeObject* type, PyObject* args, PyObject*) {
         s.win_W = (int)t[5]->size(2);
     }
     return owner.release();
+    END_HANDLE_TH_ERRORS
+}
+
+// Whether o is `have`, or holds it at index li of a leading dimension: the same memory, type, sizes and strides
+bool is_view(const at::Tensor* have, PyObject* o, int64_t li) {
+    const at::Tensor* t = tensor(o);
+    if (!t || !have) return o == Py_None && !have;
+    const int64_t more = t->dim() - have->dim();
+    if (more != 0 && more != 1) return false;
+    if (t->scalar_type() != have->scalar_type() || t->sizes().slice(more) != have->sizes() || t->strides().slice(more) != have->strides()) return false;
+    const char* at = (const char*)t->data_ptr() + (more ? li * t->stride(0) * (int64_t)t->element_size() : 0);
+    return at == (const char*)have->data_ptr() && (!more || (li >= 0 && li < t->size(0)));
+}
+
+// holds(li, the constructor's arguments, tensors of all layers in the place of one layer's where there are such):
+// whether this handle is what the constructor would make of them
+PyObject* layer_holds(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Layer* L = (Layer*)self;
+    const bgtq_step& s = L->s;
+    if (n != 16) { PyErr_SetString(PyExc_TypeError, "holds() takes a layer index and the arguments of Layer()"); return nullptr; }
+    int64_t li, v[6];
+    bool same = as_int(a[0], li);
+    for (int i = 0; i < 6; i++) same = same && as_int(a[6 + i], v[i]);
+    same = same && v[0] == s.k_row_width && v[1] == s.norm_width && v[2] == s.v_row_width && v[3] == (int64_t)s.n_kv * s.gqa &&
+           v[4] == s.k_layout && v[5] == s.v_layout;
+    const double scale = PyFloat_AsDouble(a[12]);
+    if (scale == -1.0 && PyErr_Occurred()) return nullptr;
+    const int baked = PyObject_IsTrue(a[13]);
+    if (baked < 0) return nullptr;
+    same = same && (float)scale == s.scale && baked == L->baked;
+    const at::Tensor* have[7] = {L->plans, L->kp, L->kn, L->vp, L->vn, L->bk, L->bv};
+    for (int i = 0; i < 7; i++) same = same && is_view(have[i], a[i < 5 ? 1 + i : 9 + i], li);
+    return PyBool_FromLong(same);
     END_HANDLE_TH_ERRORS
 }
 
@@ -281,6 +317,7 @@ PyObject* layer_encode(PyObject* self, PyObject* const* a, Py_ssize_t n) {
 }
 
 PyMethodDef layer_methods[] = {
+    {"holds", (PyCFunction)(void*)layer_holds, METH_FASTCALL, "whether this is the handle of these arguments"},
     {"step", (PyCFunction)(void*)layer_step, METH_FASTCALL, "one decode step of this layer, or None"},
     {"step_window", (PyCFunction)(void*)layer_step_window, METH_FASTCALL, "one decode step in with-buffer mode, or None"},
     {"encode", (PyCFunction)(void*)layer_encode, METH_FASTCALL, "append k and v, True or None"},

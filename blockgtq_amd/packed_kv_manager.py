@@ -69,7 +69,7 @@ class BlockGTQKVManager:
             raise ValueError("n_sink needs recent_window > 0")
         self._buf_k = self._buf_v = None
         self._step_src, self._step_idx = None, None     # per-step index tensors of the buffered append
-        self._layers = [None] * n_layers                # (native handle, rotation folded into q_proj) per layer
+        self._layers = [None] * n_layers                # native handle per layer
 
     # ------------------------------------------------------------ calibration
     def calibrate(self, layer_idx: int, q_data: torch.Tensor, k_data: torch.Tensor):
@@ -129,17 +129,13 @@ class BlockGTQKVManager:
             self._buf_v = torch.zeros(bshape, dtype=torch.float16, device=dev)
 
     def _native(self, li):
-        """The layer's native handle (None off the GPU)."""
-        baked = self.quantizers[li][0]._q_perm_baked
-        entry = self._layers[li]
-        if entry is None or entry[1] != baked:
-            self._ensure_storage()
-            entry = (_host.layer(self._batched_args[li]['plans'], self._k_packed[li], self._k_norms[li], self._v_packed[li],
-                                 self._v_norms[li], self._k_rows[li], self._k_norms.shape[-1], self._vpb, self.n_q,
-                                 _plan.K_BITPACKED, _plan.V_BITPACKED, self.scale, baked,
-                                 self._buf_k[li] if self.buffered else None, self._buf_v[li] if self.buffered else None), baked)
-            self._layers[li] = entry
-        return entry[0]
+        """The layer's native handle (None off the GPU), made anew when something it was made from has changed."""
+        self._ensure_storage()
+        h = self._layers[li] = _host.layer(
+            self._layers[li], li, self._batched_args[li]['plans'], self._k_packed[li], self._k_norms, self._v_packed,
+            self._v_norms, self._k_rows[li], self._k_norms.shape[-1], self._vpb, self.n_q, _plan.K_BITPACKED, _plan.V_BITPACKED,
+            self.scale, self.quantizers[li][0]._q_perm_baked, self._buf_k, self._buf_v)
+        return h
 
     def set_seq_lens(self, seq_lens):
         """Per-row visible lengths (ragged batch); ``None`` returns to one shared length."""

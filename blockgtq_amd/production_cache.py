@@ -60,20 +60,15 @@ class BlockGTQProductionCache:
         # K cell search: the reference's 256-bin table (blockgtq/quantizer.py:841-850);
         # plan.QUANT_EXACT gives the nearest centroid of the unpacked torch path
         self.quant_mode = _plan.QUANT_LUT256
-        self._layers = [None] * n_layers    # native handle per layer and what it was made from
+        self._layers = [None] * n_layers    # native handle per layer
 
     def _native(self, li):
-        """The layer's native handle (None off the GPU), made anew when the storage, the plans or the
-        folding of the query rotation have changed."""
-        plans, baked = self.batched_args[li]['plans'], self.quantizers[li][0]._q_perm_baked
-        e = self._layers[li]
-        if (e is None or e[1] is not plans or e[2] != baked or e[3] is not self.k_packed or e[4] is not self.k_norms
-                or e[5] is not self.v_packed or e[6] is not self.v_norms):
-            e = (_host.layer(plans, self.k_packed[li], self.k_norms[li], self.v_packed[li], self.v_norms[li],
-                             self.k_bytes_per_tok, self.max_ng, self.vpb, self.nq, self._k_layout, self._v_layout,
-                             self.scale, baked), plans, baked, self.k_packed, self.k_norms, self.v_packed, self.v_norms)
-            self._layers[li] = e
-        return e[0]
+        """The layer's native handle (None off the GPU), made anew when something it was made from has changed."""
+        h = self._layers[li] = _host.layer(
+            self._layers[li], li, self.batched_args[li]['plans'], self.k_packed, self.k_norms, self.v_packed, self.v_norms,
+            self.k_bytes_per_tok, self.max_ng, self.vpb, self.nq, self._k_layout, self._v_layout, self.scale,
+            self.quantizers[li][0]._q_perm_baked)
+        return h
 
     # ---------------------------------------------------------------- encode
     def _encode_batched(self, layer_idx, k, v, t_pos):

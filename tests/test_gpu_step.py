@@ -87,3 +87,88 @@ def test_buffered_partial_with_and_without_the_preparation(batch, n_q, n_kv, win
             m.increment_seq_len()
     for name in ("_k_packed", "_k_norms", "_v_packed", "_v_norms", "_buf_k", "_buf_v"):
         assert torch.equal(getattr(mgrs[0], name)[0], getattr(mgrs[1], name)[0]), name
+
+
+def _pair(nibble=True, baked=False):
+    """Two caches with the same 90 records, the second without native handles."""
+    w = wl.Workload("t", 1, 12, 4, 2, 90, 1e6, seed=35)
+    qs, e = wl.calibrate_layer(w, 0, DEV)
+    for q8 in qs:
+        q8._q_perm_baked = baked
+    k0, v0 = wl.draw_kv(w, e, 90, 5, DEV)
+    caches = []
+    for fast in (True, False):
+        c = BlockGTQProductionCache([qs], [build_batched_encode_args(qs, device=DEV)], [[q.build_kernel_args() for q in qs]],
+                                    1, 4, 12, 128, 120, k_nibble=nibble, v_nibble=nibble, device=DEV, batch_size=2)
+        if not fast:
+            c._native = lambda li: None
+        c._encode_batched(0, k0, v0, 0)
+        c.seq_len = 90
+        caches.append(c)
+    return w, e, caches
+
+
+def _step(caches, w, e, T, dtype=torch.float16):
+    q, k, v = _inputs(w, [e], T, dtype)
+    fast, slow = [c.encode_and_attend(0, q, k, v) for c in caches]
+    for c in caches:
+        c.increment_seq_len()
+    assert fast.abs().max() > 0 and torch.equal(fast, slow)
+    for name in ("k_packed", "k_norms", "v_packed", "v_norms"):
+        assert torch.equal(getattr(caches[0], name), getattr(caches[1], name)), name
+    return fast
+
+
+def test_production_cache_handle_follows_its_attributes():
+    """Scale, layout, row widths and storage may be set between steps; the next step goes by them."""
+    w, e, caches = _pair()
+    a = _step(caches, w, e, 90)
+    for c in caches:
+        c.scale *= 3
+    assert not torch.equal(a, _step(caches, w, e, 91))
+    for c in caches:                                                    # other storage behind the same tensor object
+        c.v_norms.data = c.v_norms * 2
+    _step(caches, w, e, 92)
+    for c in caches:                                                    # other tensors
+        c.k_packed, c.k_norms = c.k_packed.clone(), c.k_norms * 0.5
+    _step(caches, w, e, 93)
+    bit_packed = _pair(nibble=False)[2]
+    for c, b in zip(caches, bit_packed):                                # another layout, with the storage that goes with it
+        for name in ("_k_layout", "_v_layout", "k_bytes_per_tok", "vpb", "max_ng", "k_packed", "k_norms", "v_packed", "v_norms"):
+            setattr(c, name, getattr(b, name))
+        c.seq_len = 90
+    _step(caches, w, e, 90)
+
+
+@pytest.mark.parametrize("window", [0, 64])
+def test_manager_handle_follows_its_attributes(window):
+    w = wl.Workload("t", 1, 8, 2, 2, 150, 1e6, n_sink=4 if window else 0, window=window, seed=36)
+    mgrs = []
+    for _ in range(2):
+        mgr, energies = wl.build_manager(w, DEV)
+        wl.fill_cache(mgr, w, energies, DEV)
+        mgrs.append(mgr)
+    mgrs[1]._native = lambda li: mgrs[1]._ensure_storage()
+
+    def step():
+        q, k, v = _inputs(w, energies, 150, torch.float16)
+        outs = [m.append_and_attend(0, q, k, v) for m in mgrs]
+        assert outs[0].abs().max() > 0 and torch.equal(*outs)
+        for name in ("_k_packed", "_k_norms", "_v_packed", "_v_norms") + (("_buf_k", "_buf_v") if window else ()):
+            assert torch.equal(getattr(mgrs[0], name)[0], getattr(mgrs[1], name)[0]), name
+        return outs[0]
+
+    a = step()
+    for m in mgrs:
+        m.scale *= 3
+    assert not torch.equal(a, step())
+    for m in mgrs:
+        m._v_norms.data = m._v_norms * 2
+    step()
+    for m in mgrs:
+        m._k_norms, m._k_packed = m._k_norms * 0.5, [t.clone() for t in m._k_packed]
+    step()
+    if window:
+        for m in mgrs:
+            m._buf_k, m._buf_v = m._buf_k.clone(), m._buf_v * 2
+        step()
