@@ -8,7 +8,7 @@
 // y = xhat, when the group's rotation block is the identity).  This file is
 // compiled with floating-point contraction off so nothing else fuses.
 //
-// Two encoders keep it: a work-group of 128 threads for every row of a decode append (encode_rows: thread j
+// Two encoders keep it: a work-group of 128 threads for every row of a decode append (encode_row: thread j
 // owns packed dim j during normalise / rotate / quantise and output byte j while packing), and blocks of 16
 // rows on the matrix cores for anything larger (encode_blocks).
 #include <algorithm>
@@ -122,24 +122,19 @@ __device__ __forceinline__ float chain_sumsq_row(const float* x) {
     return ss;
 }
 
-template <int ROWS, bool IS_V>
-__device__ __forceinline__ void encode_rows(const EncodeArgs& a, const int bx, const int h,
-                                            const int64_t n_tiles, const int tile_stride,
-                                            float* rot_s) {
-    __shared__ __align__(16) float xs[ROWS + 1][D];     // (one more row of zeros: the compact rotation reads up to BGTQ_ROT_COL values past a segment's start)
-    __shared__ float nrm[ROWS][BGTQ_MAX_SEGMENTS];
-    __shared__ float nrm_out[ROWS][BGTQ_MAX_SEGMENTS];
-    __shared__ uint8_t cds[ROWS][D];
-    __shared__ uint16_t xraw[ROWS][D];
+template <bool IS_V>
+__device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, const int h, float* rot_s) {
+    __shared__ __align__(16) float xs[2 * D];     // (the row, then zeros: the compact rotation reads up to BGTQ_ROT_COL values past a segment's start)
+    __shared__ float nrm[BGTQ_MAX_SEGMENTS];
+    __shared__ float nrm_out[BGTQ_MAX_SEGMENTS];
+    __shared__ uint8_t cds[D];
+    __shared__ uint16_t xraw[D];
     __shared__ typename std::conditional<IS_V, StagedV, StagedK>::type sp;
 
     const int j = threadIdx.x;
     const bgtq_head_plan& P = a.plans[h];
-    const int64_t N = (int64_t)a.B * a.S;
-    const float* RT = IS_V ? P.v_rot_T : P.k_rot_T;
 
-    // ---- 0. one burst: plan tables, the first tile's raw rows, and (V) the rotation column ----
-    // A work-group stages the plan once and then walks tiles bx, bx + tile_stride, ...
+    // ---- 0. one burst: plan tables, the raw row and its position, the rotation column ----
     if constexpr (IS_V) {
         if (j == 0) sp.v_bits = P.v_bits;
         if (j < 16) { sp.centroids[j] = P.v_centroids[j]; sp.boundaries[j] = P.v_boundaries[j]; }
@@ -154,56 +149,42 @@ __device__ __forceinline__ void encode_rows(const EncodeArgs& a, const int bx, c
             sp.centroids[e] = P.k_centroids[e >> 5][e & 31];
         }
     }
-    xs[ROWS][j] = 0.f;
-    uint16_t xr[ROWS];                 // raw rows of the tile about to be processed
-    int tp[2];         // decode append: their cache positions, fetched with them
-    auto fetch_rows = [&](int64_t tile) {
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) {
-            int64_t n = tile * ROWS + r;
-            uint16_t v = 0;
-            int t = 0;
-            if (n < N) {
-                int b, s;
-                split_row(n, a.S, b, s);
-                v = a.x[b * a.x_sb + h * a.x_sh + s * a.x_ss + j];
-                if (ROWS <= 2) t = (a.t_pos ? a.t_pos[b] : a.t_pos_scalar) + s;
-            }
-            xr[r] = v;
-            if (ROWS <= 2) tp[r] = t;
-        }
-    };
-    fetch_rows(bx);
+    xs[D + j] = 0.f;
+    int b, s;
+    split_row(row, a.S, b, s);
+    const uint16_t xr = a.x[b * a.x_sb + h * a.x_sh + s * a.x_ss + j];
+    const int t = (a.t_pos ? a.t_pos[b] : a.t_pos_scalar) + s;
     int4 k_dim = {0, 0, 0, 0};
     uint2 k_byte = {0u, 0u};
-    float k_lut_off = 0.f, k_lut_scale = 0.f;
+    float lut_off = 0.f, lut_scale = 0.f;                    // K: this dim's cell-search parameters
     if constexpr (!IS_V) {
         k_dim = *(const int4*)P.enc_dim[j];
         k_byte = *(const uint2*)P.enc_byte[a.layout == BGTQ_K_MIXED ? 1 : 0][j];
-        k_lut_off = P.lut_offset[j];
-        k_lut_scale = P.lut_inv_scale[j];
+        lut_off = P.lut_offset[j];
+        lut_scale = P.lut_inv_scale[j];
     } else if (j < D / 2) {
         k_byte = *(const uint2*)P.enc_vbyte[a.layout == BGTQ_V_NIBBLE ? 1 : 0][j];
     }
-    // Decode append (tiles of one or two rows) is latency bound.  K: the whole rotation matrix is requested now,
-    // before anything else is known (which rows a thread needs is only known once the plan is in
-    // LDS), 16 bytes a lane and contiguous across the wave (32 loads a thread), and parked in LDS
-    // (rot_s) ahead of the rotation, which then reads its column from there.  16-row tiles fetch
-    // their column slices per tile instead.
-    // V's rotation is dense and is needed later than its rows: its column comes straight into
-    // registers, one 4-byte load per matrix row (the wide loads of the whole matrix land later).
-    constexpr bool STAGED = ROWS <= 2 && !IS_V;
-    constexpr int PF = (ROWS <= 2 && IS_V) ? D : 0;
-    rot_piece rst[STAGED ? D / 4 : 1];
-    float rpre[PF > 0 ? PF : 1];
-    // K, where no rotated segment is longer than BGTQ_ROT_COL dims: the plan also holds every dim's
-    // rotation column cut down to its segment, which goes straight into registers (12 wide loads
-    // instead of 32 and no trip through LDS)
-    constexpr int RC = STAGED ? BGTQ_ROT_COL : 4;
-    float rc[RC];
+    // Latency bound.  K: the whole rotation matrix is requested now, before anything else is known (which
+    // rows a thread needs is only known once the plan is in LDS), 16 bytes a lane and contiguous across
+    // the wave (32 loads a thread), and parked in LDS (rot_s) ahead of the rotation, which then reads its
+    // column from there.  Where no rotated segment is longer than BGTQ_ROT_COL dims, the plan also holds
+    // every dim's rotation column cut down to its segment, which goes straight into registers (12 wide
+    // loads instead of 32 and no trip through LDS).
+    // V's rotation is dense and is needed later than its row: its column comes straight into registers
+    // (the plan holds v_rot_T four rows interleaved: 16-byte loads, contiguous across the threads).
+    constexpr int RC = BGTQ_ROT_COL;
+    rot_piece rst[IS_V ? 1 : D / 4];
+    float rc[IS_V ? D : RC];
     bool compact = false;
-    if constexpr (STAGED) {
-        compact = P.rot_compact[0] != 0;                 // (uniform)
+    if constexpr (IS_V) {
+#pragma unroll
+        for (int i = 0; i < D / 4; i++) {
+            const float4 v = *(const float4*)P.v_rot_T4[i][j];
+            rc[4 * i] = v.x; rc[4 * i + 1] = v.y; rc[4 * i + 2] = v.z; rc[4 * i + 3] = v.w;
+        }
+    } else {
+        compact = P.rot_compact[0] != 0;                     // (uniform)
         if (compact) {
 #pragma unroll
             for (int i = 0; i < RC / 4; i++) {
@@ -211,25 +192,14 @@ __device__ __forceinline__ void encode_rows(const EncodeArgs& a, const int bx, c
                 rc[4 * i] = v.x; rc[4 * i + 1] = v.y; rc[4 * i + 2] = v.z; rc[4 * i + 3] = v.w;
             }
         } else {
-            fetch_rotation(RT, j, rst);
-        }
-    }
-    if constexpr (PF > 0) {
-        // (the plan holds v_rot_T four rows interleaved: 16-byte loads, contiguous across the threads)
-#pragma unroll
-        for (int i = 0; i < PF / 4; i++) {
-            const float4 v = *(const float4*)P.v_rot_T4[i][j];
-            rpre[4 * i] = v.x; rpre[4 * i + 1] = v.y; rpre[4 * i + 2] = v.z; rpre[4 * i + 3] = v.w;
+            fetch_rotation(P.k_rot_T, j, rst);
         }
     }
     if constexpr (!IS_V) __syncthreads();     // (K reads the staged header next; V's staged tables are first read three barriers on)
 
     // ---- per-thread static data, read ready-made from the plan (requested in the first burst) ----
     int n_seg = 1, g = 0, gs = 0, ge = D, ident = 0, src_dim = j;
-    float lut_off_j = 0.f, lut_scale_j = 0.f;          // K: this dim's cell-search parameters
     if constexpr (!IS_V) {
-        lut_off_j = k_lut_off;
-        lut_scale_j = k_lut_scale;
         n_seg = sp.hdr[H_NSEG];
         g = k_dim.x;
         gs = k_dim.y;
@@ -243,207 +213,154 @@ __device__ __forceinline__ void encode_rows(const EncodeArgs& a, const int bx, c
     const StreamSlot slot{0, (int)(k_byte.x >> 8), (int)((k_byte.x >> 6) & 3u)};
     const int c0 = (int)k_byte.y;                       // (the slot's first code is folded into the base)
 
-    for (int64_t tile = bx; tile < n_tiles; tile += tile_stride) {
-    const int64_t row0 = tile * ROWS;
-    int tcur[2] = {0, 0};              // this tile's positions (the prefetch below overwrites tp)
-    if (ROWS <= 2) { tcur[0] = tp[0]; tcur[1] = tp[ROWS == 2 ? 1 : 0]; }
-    // ---- 1. rows to LDS, next tile's rows on their way, gather by head_perm (K) -------------
+    // ---- 1. the row to LDS, gathered by head_perm (K) -------------
     if constexpr (IS_V) {              // (no gather: a thread converts its own value)
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) xs[r][j] = bgtq_h2f(bgtq_in16(xr[r], a.bf16));
-        if (tile + tile_stride < n_tiles) fetch_rows(tile + tile_stride);
+        xs[j] = bgtq_h2f(bgtq_in16(xr, a.bf16));
     } else {
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) xraw[r][j] = bgtq_in16(xr[r], a.bf16);
+        xraw[j] = bgtq_in16(xr, a.bf16);
         __syncthreads();
-        if (tile + tile_stride < n_tiles) fetch_rows(tile + tile_stride);
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) xs[r][j] = bgtq_h2f(xraw[r][src_dim]);
+        xs[j] = bgtq_h2f(xraw[src_dim]);
     }
     __syncthreads();
 
-    // ---- 2. group norms: thread (r, grp) runs one sequential chain ---------
-    if (j < ROWS * BGTQ_MAX_SEGMENTS) {
-        int r = j / BGTQ_MAX_SEGMENTS, gg = j % BGTQ_MAX_SEGMENTS;
+    // ---- 2. group norms: thread gg runs one sequential chain ---------
+    if (j < BGTQ_MAX_SEGMENTS) {
         float n = 0.f;
-        if (gg < n_seg) {
-            int s = 0, e = D;
-            if constexpr (!IS_V) { s = sp.hdr[H_START + gg]; e = s + sp.hdr[H_LEN + gg]; }
+        if (j < n_seg) {
             float ss = 0.f;
             if constexpr (IS_V) {
-                ss = chain_sumsq_row(xs[r]);
+                ss = chain_sumsq_row(xs);
             } else {                           // short ranges: the batches would mostly run masked
+                const int k0 = sp.hdr[H_START + j], k1 = k0 + sp.hdr[H_LEN + j];
 #pragma unroll 8
-                for (int k = s; k < e; k++) ss = __builtin_fmaf(xs[r][k], xs[r][k], ss);
+                for (int k = k0; k < k1; k++) ss = __builtin_fmaf(xs[k], xs[k], ss);
             }
             n = __builtin_sqrtf(ss + 1e-30f);
         }
-        nrm[r][gg] = n;
+        nrm[j] = n;
     }
     __syncthreads();
 
     // ---- 3. normalise -------------------------------------------------------
-    float xh[ROWS];
-#pragma unroll
-    for (int r = 0; r < ROWS; r++) {
-        float v = 0.f;
-        if (g >= 0) {
-            float n = nrm[r][g];
-            float safe = (n > (IS_V ? 1e-8f : 1e-10f)) ? n : 1.0f;
-            v = xs[r][j] / safe;
-        }
-        xh[r] = v;
-        xs[r][j] = v;     // only this thread ever touched xs[r][j] since the barrier
+    float xh = 0.f;
+    if (g >= 0) {
+        const float n = nrm[g];
+        const float safe = (n > (IS_V ? 1e-8f : 1e-10f)) ? n : 1.0f;
+        xh = xs[j] / safe;
     }
-    if constexpr (STAGED) { if (!compact) park_rotation(rot_s, j, rst); }   // (every tile of the walk: the registers stay as they are)
+    xs[j] = xh;               // only this thread ever touched xs[j] since the barrier
+    if constexpr (!IS_V) { if (!compact) park_rotation(rot_s, j, rst); }
     __syncthreads();
 
     // ---- 4. rotate ------------------------------------------------------------
-    // Same chain as written in the contract above; the matrix column is fetched in
-    // batches of RB independent loads so the chain never waits on one load at a time.
-    float y[ROWS];
+    // The chain of the contract above; the values of a batch are read from LDS ahead of the products
+    // that consume them.
+    float y = 0.f;
     if (ident || g < 0) {
+        y = xh;
+    } else if constexpr (IS_V) {
+        constexpr int CB = 32;
+        float4 xv[2][CB / 4];
+        auto load = [&](const int blk) {
 #pragma unroll
-        for (int r = 0; r < ROWS; r++) y[r] = xh[r];
-    } else {
+            for (int i = 0; i < CB / 4; i++) xv[blk & 1][i] = *(const float4*)&xs[blk * CB + 4 * i];
+        };
+        load(0);
 #pragma unroll
-        for (int r = 0; r < ROWS; r++) y[r] = 0.f;
-        if constexpr (STAGED) {
-            if (compact) {
-                // The column is in registers and is zero past the segment's end, so the chain runs over
-                // BGTQ_ROT_COL terms for every dim without a length test: a term x * 0 leaves the sum as it
-                // is (the row is followed by zeros, so every x read is finite).  The row values of a batch
-                // are read ahead of the chain.
-                constexpr int CB = 16;
+        for (int blk = 0; blk < D / CB; blk++) {
+            if (blk + 1 < D / CB) load(blk + 1);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int i0 = 0; i0 < RC; i0 += CB) {
-                    float xv[ROWS][CB];
-#pragma unroll
-                    for (int i = 0; i < CB; i++)
-#pragma unroll
-                        for (int r = 0; r < ROWS; r++) xv[r][i] = (&xs[r][0])[gs + i0 + i];
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int i = 0; i < CB; i++)
-#pragma unroll
-                        for (int r = 0; r < ROWS; r++) y[r] = __builtin_fmaf(xv[r][i], rc[i0 + i], y[r]);
-                }
-            } else
-            // column j of the parked rotation against the rows, the LDS reads a batch ahead of
-            // the chain that consumes them
-            {
-                constexpr int CB = 16;
-                for (int k0 = gs; k0 < ge; k0 += CB) {
-                    float rk[CB], xv[ROWS][CB];
-#pragma unroll
-                    for (int i = 0; i < CB; i++) {
-                        const int k = min(k0 + i, ge - 1);
-                        rk[i] = rot_s[k * D + j];
-#pragma unroll
-                        for (int r = 0; r < ROWS; r++) xv[r][i] = xs[r][k];
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int i = 0; i < CB; i++)
-                        if (k0 + i < ge) {
-#pragma unroll
-                            for (int r = 0; r < ROWS; r++) y[r] = __builtin_fmaf(xv[r][i], rk[i], y[r]);
-                        }
-                }
+            for (int i = 0; i < CB / 4; i++) {
+                const float4 x4 = xv[blk & 1][i];
+                const int k = blk * CB + 4 * i;
+                y = __builtin_fmaf(x4.x, rc[k], y);
+                y = __builtin_fmaf(x4.y, rc[k + 1], y);
+                y = __builtin_fmaf(x4.z, rc[k + 2], y);
+                y = __builtin_fmaf(x4.w, rc[k + 3], y);
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if constexpr (PF > 0) {                 // V: the column fetched at the top of the kernel
-            // row values come from LDS a batch of 32 dims ahead of the chain that consumes them
-            constexpr int CB = 32;
-            float4 xv[2][ROWS][CB / 4];
-            auto load = [&](const int b) {
+    } else if (compact) {
+        // The column is in registers and is zero past the segment's end, so the chain runs over
+        // BGTQ_ROT_COL terms for every dim without a length test: a term x * 0 leaves the sum as it
+        // is (the row is followed by zeros, so every x read is finite).
+        constexpr int CB = 16;
 #pragma unroll
-                for (int r = 0; r < ROWS; r++)
+        for (int i0 = 0; i0 < RC; i0 += CB) {
+            float xv[CB];
 #pragma unroll
-                    for (int i = 0; i < CB / 4; i++) xv[b & 1][r][i] = *(const float4*)&xs[r][b * CB + 4 * i];
-            };
-            load(0);
+            for (int i = 0; i < CB; i++) xv[i] = xs[gs + i0 + i];
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int b = 0; b < PF / CB; b++) {
-                if (b + 1 < PF / CB) load(b + 1);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < CB; i++) y = __builtin_fmaf(xv[i], rc[i0 + i], y);
+        }
+    } else {                                    // column j of the parked rotation
+        constexpr int CB = 16;
+        for (int k0 = gs; k0 < ge; k0 += CB) {
+            float rk[CB], xv[CB];
 #pragma unroll
-                for (int i = 0; i < CB / 4; i++)
-#pragma unroll
-                    for (int r = 0; r < ROWS; r++) {
-                        const float4 x4 = xv[b & 1][r][i];
-                        const int k = b * CB + 4 * i;
-                        y[r] = __builtin_fmaf(x4.x, rpre[k], y[r]);
-                        y[r] = __builtin_fmaf(x4.y, rpre[k + 1], y[r]);
-                        y[r] = __builtin_fmaf(x4.z, rpre[k + 2], y[r]);
-                        y[r] = __builtin_fmaf(x4.w, rpre[k + 3], y[r]);
-                    }
-                __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < CB; i++) {
+                const int k = min(k0 + i, ge - 1);
+                rk[i] = rot_s[k * D + j];
+                xv[i] = xs[k];
             }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < CB; i++)
+                if (k0 + i < ge) y = __builtin_fmaf(xv[i], rk[i], y);
         }
     }
 
     // ---- 5. scalar quantise ---------------------------------------------------
     const bool need_cent = IS_V || a.layout == BGTQ_K_MIXED || a.corrected;
+    int code = 0;
+    if constexpr (IS_V) {
+        // (all 15 slots are read at once; those past the codebook's last boundary are skipped)
+        const int nb = (1 << sp.v_bits) - 1;
+        float bd[15];
 #pragma unroll
-    for (int r = 0; r < ROWS; r++) {
-        int code = 0;
-        if (IS_V) {
-            if constexpr (IS_V) {
-                // (all 15 slots are read at once; those past the codebook's last boundary are skipped)
-                const int nb = (1 << sp.v_bits) - 1;
-                float bd[15];
+        for (int i = 0; i < 15; i++) bd[i] = sp.boundaries[i];
 #pragma unroll
-                for (int b = 0; b < 15; b++) bd[b] = sp.boundaries[b];
-#pragma unroll
-                for (int b = 0; b < 15; b++) code += (b < nb && y[r] > bd[b]) ? 1 : 0;
-            }
-        } else if (g >= 0) {
-            if constexpr (!IS_V) {
-                if (a.quant_mode == BGTQ_QUANT_EXACT) {
-                    int nb = (1 << sp.hdr[H_BW + g]) - 1;
-                    for (int b = 0; b < nb; b++) code += (P.k_boundaries[g][b] < y[r]) ? 1 : 0;
-                } else {
-                    float t = (y[r] - lut_off_j) * lut_scale_j;
-                    t = fminf(fmaxf(t, 0.0f), (float)(BGTQ_LUT_BINS - 1));
-                    code = sp.code_lut[g * BGTQ_LUT_BINS + (int)t];
-                }
-            }
+        for (int i = 0; i < 15; i++) code += (i < nb && y > bd[i]) ? 1 : 0;
+    } else if (g >= 0) {
+        if (a.quant_mode == BGTQ_QUANT_EXACT) {
+            const int nb = (1 << sp.hdr[H_BW + g]) - 1;
+            for (int i = 0; i < nb; i++) code += (P.k_boundaries[g][i] < y) ? 1 : 0;
+        } else {
+            float c = (y - lut_off) * lut_scale;
+            c = fminf(fmaxf(c, 0.0f), (float)(BGTQ_LUT_BINS - 1));
+            code = sp.code_lut[g * BGTQ_LUT_BINS + (int)c];
         }
-        cds[r][j] = (uint8_t)code;
-        // centroid of the chosen code for the norm correction below; it is parked in xs
-        // after the barrier (other threads may still be reading xs in their rotation)
-        if (need_cent) {
-            if constexpr (IS_V) y[r] = sp.centroids[code];
-            else y[r] = g < 0 ? 0.f : code < 32 ? sp.centroids[g * 32 + code] : P.k_centroids[g][code];
-        }
+    }
+    cds[j] = (uint8_t)code;
+    // centroid of the chosen code for the norm correction below; it is parked in xs
+    // after the barrier (other threads may still be reading xs in their rotation)
+    if (need_cent) {
+        if constexpr (IS_V) y = sp.centroids[code];
+        else y = g < 0 ? 0.f : code < 32 ? sp.centroids[g * 32 + code] : P.k_centroids[g][code];
     }
     __syncthreads();
-    if (need_cent) {
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) xs[r][j] = y[r];
-    }
+    if (need_cent) xs[j] = y;
     __syncthreads();
 
     // ---- 6. norms to store (raw or divided by ||centroids[codes]||) ---------
-    // Single-row tiles give this chain to the second wave: the first one packs the record meanwhile
-    // (neither needs anything of the other: the barrier between them is left out below).
-    const int jn = ROWS == 1 ? j - 64 : j;
-    if (jn >= 0 && jn < ROWS * BGTQ_MAX_SEGMENTS) {
-        int r = jn / BGTQ_MAX_SEGMENTS, gg = jn % BGTQ_MAX_SEGMENTS;
+    // The second wave's chain: the first one packs the record meanwhile (neither needs anything of the
+    // other).
+    const int gg = j - 64;
+    const bool has_norm = gg >= 0 && gg < BGTQ_MAX_SEGMENTS;
+    if (has_norm) {
         float out = 0.f;
         if (gg < n_seg) {
-            float n = nrm[r][gg];
-            if (IS_V) {
-                const float cs = chain_sumsq_row(xs[r]);
-                float cn = __builtin_sqrtf(cs + 1e-20f);
+            const float n = nrm[gg];
+            if constexpr (IS_V) {
+                const float cn = __builtin_sqrtf(chain_sumsq_row(xs) + 1e-20f);
                 out = n / (cn > 1e-10f ? cn : 1.0f);
             } else if (a.layout == BGTQ_K_MIXED || a.corrected) {
-                int s = 0, e = 0;
-                if constexpr (!IS_V) { s = sp.hdr[H_START + gg]; e = s + sp.hdr[H_LEN + gg]; }
+                const int k0 = sp.hdr[H_START + gg], k1 = k0 + sp.hdr[H_LEN + gg];
                 float cs = 0.f;
-                for (int k = s; k < e; k++) {
-                    float c = xs[r][k];
+                for (int k = k0; k < k1; k++) {
+                    const float c = xs[k];
                     cs = __builtin_fmaf(c, c, cs);
                 }
                 out = n / fmaxf(__builtin_sqrtf(cs), 1e-10f);
@@ -451,66 +368,39 @@ __device__ __forceinline__ void encode_rows(const EncodeArgs& a, const int bx, c
                 out = n;
             }
         }
-        nrm_out[r][gg] = out;
+        nrm_out[gg] = out;
     }
-    if (ROWS > 1 || a.codes_out) __syncthreads();       // (uniform; the cache norms below are stored by the thread that made them)
 
     // ---- 7a. unpacked outputs (codes path) ------------------------------------
-    if (a.codes_out) {
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) {
-            int64_t n = row0 + r;
-            if (n < N) a.codes_out[n * D + j] = cds[r][j];
-        }
+    if (a.codes_out) {                                  // (uniform)
+        __syncthreads();
+        a.codes_out[(int64_t)row * D + j] = cds[j];
         if (IS_V) {
-            if (j < ROWS && row0 + j < N && a.norms)
-                a.norms[row0 + j] = bgtq_f2h(nrm_out[j][0]);
-        } else if (a.norms_f32_out && j < ROWS * BGTQ_MAX_SEGMENTS) {
-            int r = j / BGTQ_MAX_SEGMENTS, gg = j % BGTQ_MAX_SEGMENTS;
-            if (row0 + r < N && gg < a.norm_width)
-                a.norms_f32_out[(row0 + r) * a.norm_width + gg] = nrm_out[r][gg];
+            if (j == 0 && a.norms) a.norms[row] = bgtq_f2h(nrm_out[0]);
+        } else if (a.norms_f32_out && j < BGTQ_MAX_SEGMENTS && j < a.norm_width) {
+            a.norms_f32_out[(int64_t)row * a.norm_width + j] = nrm_out[j];
         }
+        return;
     }
+    if (t < 0 || t >= a.max_T) return;                  // a position outside the cache: the record is dropped
 
-    // ---- 7b. cache norms --------------------------------------------------------
-    if (!a.codes_out && jn >= 0 && jn < ROWS * BGTQ_MAX_SEGMENTS) {
-        int r = jn / BGTQ_MAX_SEGMENTS, gg = jn % BGTQ_MAX_SEGMENTS;
-        int64_t n = row0 + r;
-        int width = IS_V ? 1 : a.norm_width;
-        if (n < N && gg < width) {
-            int b, s;
-            split_row(n, a.S, b, s);
-            int64_t t = ROWS <= 2 ? tcur[r & 1] : (a.t_pos ? a.t_pos[b] : a.t_pos_scalar) + s;
-            if (t >= 0 && t < a.max_T)
-                a.norms[b * a.n_sb + h * a.n_sh + t * a.n_st + gg] = bgtq_f2h(nrm_out[r][gg]);
-        }
-    }
+    // ---- 7b. cache norms, by the threads that made them ------------------------
+    if (has_norm && gg < (IS_V ? 1 : a.norm_width))
+        a.norms[b * a.n_sb + h * a.n_sh + (int64_t)t * a.n_st + gg] = bgtq_f2h(nrm_out[gg]);
 
-    // ---- 8. pack: thread j produces output byte j of every row ---------------
-    if (!a.codes_out && j < a.row_width) {
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) {
-            int64_t n = row0 + r;
-            if (n >= N) break;
-            int b, s;
-            split_row(n, a.S, b, s);
-            int64_t t = ROWS <= 2 ? tcur[r & 1] : (a.t_pos ? a.t_pos[b] : a.t_pos_scalar) + s;
-            if (t < 0 || t >= a.max_T) continue;
-            unsigned v = 0;
-            if (mode == 1)      v = stream_byte_batched(&cds[r][c0], slot, bw);
-            else if (mode == 2) v = cds[r][c0];
-            a.packed[b * a.p_sb + h * a.p_sh + t * a.p_st + j] = (uint8_t)v;
-        }
-    }
-    __syncthreads();            // the tile buffers are rewritten by the next tile
+    // ---- 8. pack: thread j produces output byte j ---------------
+    if (j < a.row_width) {
+        unsigned v = 0;
+        if (mode == 1)      v = stream_byte_batched(&cds[c0], slot, bw);
+        else if (mode == 2) v = cds[c0];
+        a.packed[b * a.p_sb + h * a.p_sh + (int64_t)t * a.p_st + j] = (uint8_t)v;
     }
 }
 
-template <int ROWS, bool IS_V>
+template <bool IS_V>
 __global__ __launch_bounds__(NT) void encode_kernel(EncodeArgs a) {
-    const int64_t N = (int64_t)a.B * a.S;
-    __shared__ __align__(16) float rot_s[(ROWS <= 2 && !IS_V) ? D * D : 4];
-    encode_rows<ROWS, IS_V>(a, blockIdx.x, blockIdx.y, (N + ROWS - 1) / ROWS, gridDim.x, rot_s);
+    __shared__ __align__(16) float rot_s[IS_V ? 4 : D * D];
+    encode_row<IS_V>(a, blockIdx.x, blockIdx.y, rot_s);
 }
 // ================================================================================================
 // Prompt-sized encoder: blocks of 16 rows, every chain of the contract on the fp32 matrix cores.
@@ -1084,7 +974,7 @@ int launch_encode(const EncodeArgs& a, hipStream_t st) {
     if (N == 0 || a.n_kv == 0) return BGTQ_OK;
     // few rows (a decode append): one row a work-group, the shortest chain of dependent stages
     if (N > 32) return IS_V ? launch_blocks(nullptr, &a, st) : launch_blocks(&a, nullptr, st);
-    hipLaunchKernelGGL((encode_kernel<1, IS_V>), dim3((unsigned)N, (unsigned)a.n_kv), dim3(NT), 0, st, a);
+    hipLaunchKernelGGL(encode_kernel<IS_V>, dim3((unsigned)N, (unsigned)a.n_kv), dim3(NT), 0, st, a);
     return bgtq_launch_status();
 }
 
@@ -1207,42 +1097,39 @@ __global__ __launch_bounds__(NT) void rotate_q_kernel(RotQArgs a) {
     rotate_q_block(a, blockIdx.x, rot_s);
 }
 
-constexpr int PREP_ROWS = 1;       // rows of a work-group in the one-launch preparation
-
 // ---- decode-step preparation: append-encode K and V and rotate the queries, one launch ----
-// Work-groups [0, nv) encode one V row each (the longest chain of the three goes out first),
-// [nv, nv + nk) one K row each, the rest rotate one or four query heads each.
+// Work-groups [0, n) encode one V row of one head each (the longest chain of the three goes out first),
+// [n, 2 n) one K row each, the rest rotate one or four query heads each.
 __device__ __forceinline__ void prepare_part(const EncodeArgs& ak, const EncodeArgs& av, const RotQArgs& aq,
-                                             const int k_tiles, const int v_tiles, int bid, float* rot_s) {
-    const int nk = k_tiles * ak.n_kv, nv = v_tiles * av.n_kv;
-    if (bid < nv) {
-        encode_rows<PREP_ROWS, true>(av, bid % v_tiles, bid / v_tiles, v_tiles, v_tiles, rot_s);
-    } else if (bid < nk + nv) {
-        bid -= nv;
-        encode_rows<PREP_ROWS, false>(ak, bid % k_tiles, bid / k_tiles, k_tiles, k_tiles, rot_s);
+                                             const int rows, int bid, float* rot_s) {
+    const int n = rows * ak.n_kv;
+    if (bid < n) {
+        encode_row<true>(av, bid % rows, bid / rows, rot_s);
+    } else if (bid < 2 * n) {
+        bid -= n;
+        encode_row<false>(ak, bid % rows, bid / rows, rot_s);
     } else {
-        rotate_q_block(aq, bid - (nk + nv), rot_s);
+        rotate_q_block(aq, bid - 2 * n, rot_s);
     }
 }
 // (BF16: some input is; asking at run time costs the chains of fp16 inputs 0.2 of 5.0 us)
 template <bool BF16>
-__global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq,
-                                                     int k_tiles, int v_tiles) {
+__global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, int rows) {
     if (!BF16) ak.bf16 = av.bf16 = aq.bf16 = 0;
     __shared__ __align__(16) float rot_s[D * D];       // the work-group's rotation, whatever its role
-    prepare_part(ak, av, aq, k_tiles, v_tiles, blockIdx.x, rot_s);
+    prepare_part(ak, av, aq, rows, blockIdx.x, rot_s);
 }
 // The same with the attention over the buffered tokens, which depends on none of it: the longer work-groups first, in
 // the LDS that is a rotation's otherwise; of the others two waves leave at once (a barrier counts the waves that are
 // left).  32 rows x 8 heads x 4 queries over 132 buffered tokens: 11.1 + 13.3 us as two launches,
 // 18.0 as one (1024 work-groups, two of them at a time on a compute unit).
 __global__ __launch_bounds__(WINDOW_THREADS, 2) void prepare_window_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, WindowArgs w,
-                                                                        int k_tiles, int v_tiles, int n_window) {
+                                                                        int rows, int n_window) {
     __shared__ __align__(16) float rot_s[D * D];
     static_assert(window_lds_floats<4>(WINDOW_RIDE_W) <= D * D, "a window's scores fit the rotation's place");
     const int bid = blockIdx.x, n_kv = ak.n_kv;
     if (bid < n_window) window_attn_block<4>(w, bid % n_kv, bid / n_kv, rot_s);
-    else if (threadIdx.x < NT) prepare_part(ak, av, aq, k_tiles, v_tiles, bid - n_window, rot_s);
+    else if (threadIdx.x < NT) prepare_part(ak, av, aq, rows, bid - n_window, rot_s);
 }
 
 // argument checks + EncodeArgs assembly shared by the separate and the fused entry points
@@ -1314,14 +1201,14 @@ int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, in
     }
     const int group = rotate_q_group_size(B, n_kv * gqa);
     RotQArgs aq{ak.plans, (const uint16_t*)q, q_sr, q_sh, (uint16_t*)q_rot, qr_sr, qr_sh, B, n_kv * gqa, gqa, group, q_bf16};
-    const int tiles = (int)((N + PREP_ROWS - 1) / PREP_ROWS);
-    const unsigned blocks = (unsigned)(2 * tiles * n_kv) + (q ? rotate_q_blocks(B, n_kv, gqa, group) : 0u);
+    const int rows = (int)N;
+    const unsigned blocks = (unsigned)(2 * rows * n_kv) + (q ? rotate_q_blocks(B, n_kv, gqa, group) : 0u);
     if (window)
-        hipLaunchKernelGGL(prepare_window_kernel, dim3(blocks + (unsigned)(B * n_kv)), dim3(WINDOW_THREADS), 0, st, ak, av, aq, *window, tiles, tiles, B * n_kv);
+        hipLaunchKernelGGL(prepare_window_kernel, dim3(blocks + (unsigned)(B * n_kv)), dim3(WINDOW_THREADS), 0, st, ak, av, aq, *window, rows, B * n_kv);
     else if (ak.bf16 || av.bf16 || (q && q_bf16))
-        hipLaunchKernelGGL(prepare_kernel<true>, dim3(blocks), dim3(NT), 0, st, ak, av, aq, tiles, tiles);
+        hipLaunchKernelGGL(prepare_kernel<true>, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows);
     else
-        hipLaunchKernelGGL(prepare_kernel<false>, dim3(blocks), dim3(NT), 0, st, ak, av, aq, tiles, tiles);
+        hipLaunchKernelGGL(prepare_kernel<false>, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows);
     return bgtq_launch_status();
 }
 
