@@ -102,6 +102,12 @@ def test_records_with_several_raw_byte_segments(bits, kl, vl):
         assert (g.double() - want).norm() <= 2 ** -10 * want.norm()
 
 
+# query heads wider than the small work-group over a split context: the merge with eight waves a group of rows, and with one
+@pytest.mark.parametrize("gqa,S,T,off", [(130, 3, 2000, 1997), (130, 40, 1100, 1060), (256, 2, 900, 890)])
+def test_wide_query_groups_over_a_split_context(gqa, S, T, off):
+    test_prompt_attention_equals_the_kernel_without_workspace(1, 1, gqa, S, T, off, P.K_MIXED, P.V_NIBBLE, (2.5, 2, 0, 8), torch.float16)
+
+
 def test_small_probabilities_count_in_the_denominator():
     """Each query has one strong record among the first and 65 535 weak ones, e^-18 of it apiece and below the smallest fp16
     number once the reference lies 4 octaves above the strong score; together they are 4e-3 of the denominator.

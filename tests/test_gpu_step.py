@@ -172,3 +172,17 @@ def test_manager_handle_follows_its_attributes(window):
         for m in mgrs:
             m._buf_k, m._buf_v = m._buf_k.clone(), m._buf_v * 2
         step()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_step_with_folded_rotation_and_strided_queries(dtype):
+    """With the rotation in the projection the fp16 queries go to the attention as they lie: heads behind a gap, in rows of a
+    wider projection.  (bf16 queries are converted on the general way.)"""
+    w, e, caches = _pair(baked=True)
+    q, k, v = _inputs(w, [e], 90, dtype)
+    wide = torch.randn(2, 1, 12, 3, 128, device=DEV).to(dtype)
+    wide[:, :, :, 1] = q.transpose(1, 2)
+    strided = wide[:, :, :, 1].transpose(1, 2)
+    assert strided.stride() != q.stride() and torch.equal(strided, q)
+    fast, slow, plain = caches[0].encode_and_attend(0, strided, k, v), caches[1].encode_and_attend(0, strided, k, v), caches[1].encode_and_attend(0, q, k, v)
+    assert fast.abs().max() > 0 and torch.equal(fast, slow) and torch.equal(fast, plain)
