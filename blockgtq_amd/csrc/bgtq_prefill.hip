@@ -20,9 +20,10 @@
 // exceeds it (to the maximum + 4 in log2 units), so the accumulators are rescaled rarely.  At the
 // end O is normalised and un-rotated against the plan's fp32 V rotation, again on the fp16 matrix
 // cores: both factors are split into an fp16 head and an fp16 remainder and three of the four
-// products are summed in fp32 (operands once more taken from the accumulator registers under a
-// permutation of the contraction index), then stored as fp16.  No fp16 K/V tensor of the layer
-// is written.
+// products are summed in fp32, to 2^-22 of the largest terms (operands once more taken from the
+// accumulator registers under a permutation of the contraction index), then stored as fp16.  No fp16
+// K/V tensor of the layer is written and no workspace is needed; callers that have room for one take
+// bgtq_prompt_attn, which does not dequantise a tile again for every block of query rows.
 //
 // Work-groups are numbered so that every (batch row, KV head) pair of the query block that sees
 // most tokens starts first and the short blocks fill the tail of the launch.
@@ -265,7 +266,8 @@ __global__ __launch_bounds__(NTHR, 8 / NWAVES) void prefill_mfma_kernel(PrefillA
     }
 
     // ---- normalise; un-rotate: out^T = R^T O^T on the fp16 matrix cores with both factors split into an
-    // fp16 head and an fp16 remainder (x = hi + lo up to 2^-22 |x|; the lo * lo product is dropped), fp32 sums
+    // fp16 head and an fp16 remainder (x = hi + lo up to 2^-22 |x|, or 2^-25 where lo is subnormal; the lo * lo
+    // product is dropped), fp32 sums
     const float l_tot = l_part + __shfl_xor(l_part, 32, 64);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
 #pragma unroll

@@ -158,9 +158,9 @@ def fused_blockgtq_prefill_attention(
 
     q (B, gqa, S_q, D) fp16 already permuted + rotated; cache slices as for the
     decode entry.  Query token s sees records ``t <= q_pos_offset + s`` when
-    ``is_causal``.  Returns (B, gqa, S_q, D) fp16.  ``bgtq_prefill_attn`` attends
-    straight over the records; record tensors whose rows it cannot walk are first
-    copied into rows it can.
+    ``is_causal``.  Returns (B, gqa, S_q, D) fp16.  ``bgtq_prompt_attn`` stages
+    the records' values once per call and attends; record tensors whose rows it cannot
+    walk are first copied into rows it can.
     ``block_q``, ``block_t`` and ``min_seg_for_dot`` tuned the reference kernel and
     are ignored."""
     assert q.dim() == 4

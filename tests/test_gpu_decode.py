@@ -613,7 +613,7 @@ def test_prompt_attention_rows_equal_decode_steps():
     (8, 1, 1, 150, 40, 0, 0, 3, 1, 5, False),      # no mask: every query sees all records
 ])
 def test_prompt_kernel_all_heads_in_one_launch(oracle_lib, decode_path, gqa, n_kv, B, T, S, kl, vl, vb, mn, mx, causal):
-    """``bgtq_prefill_attn`` (every KV head and batch row in one launch) against fp64 attention over the
+    """Prompt attention (every KV head and batch row in one call) against fp64 attention over the
     checker's dequantised records, row s seeing records t <= T - S + s."""
     if decode_path == "generic":
         pytest.skip("one kernel serves this entry point")
@@ -896,7 +896,7 @@ def test_mfma_kernel_refuses_strides_its_addressing_cannot_hold():
 
 
 def test_prompt_kernel_at_the_end_to_end_layer_shape(oracle_lib, decode_path):
-    """``bgtq_prefill_attn`` at the layer shape of the end-to-end workload (4 rows, 16 query / 2 KV heads,
+    """Prompt attention at the layer shape of the end-to-end workload (4 rows, 16 query / 2 KV heads,
     8192-token prompt, K3V3): sampled query rows (first, last, work-group and tile edges, random ones)
     against fp64 attention over the checker's dequantised records, then a chunk of 512 queries at
     position 7680 of the same cache."""
