@@ -40,10 +40,13 @@ def production_prefill(model, input_ids, cache, chunk_encode=64):
     out = model(input_ids, position_ids=position_ids, past_key_values=hf_cache, use_cache=True)
     for li in range(cache.n_layers):
         k, v = _layer_kv(hf_cache, li)
-        in_place = k.dtype == v.dtype and k.dtype in (torch.float16, torch.bfloat16) and k.stride(-1) == v.stride(-1) == 1
-        step = max(prompt_len, 1) if in_place else chunk_encode
-        for lo in range(0, prompt_len, step):
-            hi = min(lo + step, prompt_len)
+        if k.dtype == v.dtype and k.dtype in (torch.float16, torch.bfloat16) and k.stride(-1) == v.stride(-1) == 1:
+            if k.shape[2] > prompt_len:
+                k, v = k[:, :, :prompt_len], v[:, :, :prompt_len]
+            cache._encode_batched(li, k, v, 0)
+            continue
+        for lo in range(0, prompt_len, chunk_encode):
+            hi = min(lo + chunk_encode, prompt_len)
             cache._encode_batched(li, k[:, :, lo:hi], v[:, :, lo:hi], lo)
     cache.seq_len = prompt_len
     del hf_cache
