@@ -1122,7 +1122,7 @@ __global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs a
 // The same with the attention over the buffered tokens, which depends on none of it: the longer work-groups first, in
 // the LDS that is a rotation's otherwise; of the others two waves leave at once (a barrier counts the waves that are
 // left).  32 rows x 8 heads x 4 queries over 132 buffered tokens: 11.1 + 13.3 us as two launches,
-// 18.0 as one (1024 work-groups, two of them at a time on a compute unit).
+// 16.3 as one (1024 work-groups, two of them at a time on a compute unit).
 __global__ __launch_bounds__(WINDOW_THREADS, 2) void prepare_window_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, WindowArgs w,
                                                                         int rows, int n_window) {
     __shared__ __align__(16) float rot_s[D * D];

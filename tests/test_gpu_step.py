@@ -186,3 +186,47 @@ def test_step_with_folded_rotation_and_strided_queries(dtype):
     assert strided.stride() != q.stride() and torch.equal(strided, q)
     fast, slow, plain = caches[0].encode_and_attend(0, strided, k, v), caches[1].encode_and_attend(0, strided, k, v), caches[1].encode_and_attend(0, q, k, v)
     assert fast.abs().max() > 0 and torch.equal(fast, slow) and torch.equal(fast, plain)
+
+
+@pytest.mark.parametrize("owner", ["manager", "manager_window", "production_device_lengths"])
+def test_replayed_step_equals_eager_steps(owner):
+    """A captured step whose inputs are kept, replayed with eager work and synchronisations in between, against the same
+    number of eager steps of a twin.  (Nothing increments the length: every step writes its token at one place.)"""
+    T, dtype = 150, torch.bfloat16
+    w = wl.Workload("t", 1, 8, 2, 3, T, 1e6, seq_lens=[T, T - 7, T - 70], n_sink=4 if owner == "manager_window" else 0,
+                    window=64 if owner == "manager_window" else 0, seed=37)
+    twins = []
+    for _ in range(2):
+        if owner == "production_device_lengths":
+            qs, e = wl.calibrate_layer(w, 0, DEV)
+            c = BlockGTQProductionCache([qs], [build_batched_encode_args(qs, device=DEV)], [[q.build_kernel_args() for q in qs]],
+                                        1, 2, 8, 128, T + 8, device=DEV, batch_size=3)
+            c._encode_batched(0, *wl.draw_kv(w, e, T, 5, DEV), 0)
+            c.set_seq_lens(w.seq_lens)
+            c.use_device_lengths()
+            twins.append((c, c.encode_and_attend, ("k_packed", "k_norms", "v_packed", "v_norms")))
+            energies = [e]
+        else:
+            m, energies = wl.build_manager(w, DEV)
+            wl.fill_cache(m, w, energies, DEV)
+            twins.append((m, m.append_and_attend, ("_k_packed", "_k_norms", "_v_packed", "_v_norms") + (("_buf_k", "_buf_v") if w.window else ())))
+    q, k, v = _inputs(w, energies, T, dtype)
+    (a, step, names), (b, eager, _) = twins
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step(0, q, k, v)
+    torch.cuda.current_stream().wait_stream(side)
+    eager(0, q, k, v)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step(0, q, k, v)
+    for i in range(3):
+        for t in (q, k, v):                             # the same tensors with other values
+            t.copy_(torch.randn(t.shape, device=DEV))
+        graph.replay()
+        want = eager(0, q, k, v)
+        torch.cuda.synchronize()
+        assert torch.isfinite(want).all() and want.abs().max() > 0 and torch.equal(out, want), i
+        for name in names:
+            assert torch.equal(getattr(a, name)[0], getattr(b, name)[0]), (i, name)
