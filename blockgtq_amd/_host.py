@@ -25,17 +25,15 @@ def module():
     return _mod
 
 
-def layer(held, li, plans, k_packed, k_norms, v_packed, v_norms, k_row_width, norm_width, v_row_width, n_q,
-          k_layout, v_layout, scale, baked, buf_k=None, buf_v=None):
-    """The native handle of layer ``li`` over its plans and cache: ``held`` if that is it, a new one otherwise, None where
-    the cache is not on the GPU (the general path then says so).  The cache tensors are one layer's, or all layers'
-    stacked."""
-    rest = (k_row_width, norm_width, v_row_width, n_q, k_layout, v_layout, scale, baked)
-    if held is not None and held.holds(li, plans, k_packed, k_norms, v_packed, v_norms, *rest, buf_k, buf_v):
-        return held
+def layer(li, plans, k_packed, k_norms, v_packed, v_norms, k_row_width, norm_width, v_row_width, n_q,
+          k_layout, v_layout, scale, baked, buf_k, buf_v):
+    """A native handle of layer ``li`` over its plans and cache, or None where the cache is not on the GPU (the general
+    path then says so).  The cache tensors are one layer's, or all layers' stacked; the handle's ``holds`` takes the
+    same arguments and says whether it still is what this would make of them."""
     if not (plans.is_cuda and k_packed.is_cuda):
         return None
 
     def one(t, dims=4):
         return t[li] if t is not None and t.dim() == dims + 1 else t
-    return module().Layer(plans, one(k_packed), one(k_norms), one(v_packed), one(v_norms, 3), *rest, one(buf_k), one(buf_v))
+    return module().Layer(plans, one(k_packed), one(k_norms), one(v_packed), one(v_norms, 3), k_row_width, norm_width,
+                          v_row_width, n_q, k_layout, v_layout, scale, baked, one(buf_k), one(buf_v))

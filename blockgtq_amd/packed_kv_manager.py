@@ -131,10 +131,12 @@ class BlockGTQKVManager:
     def _native(self, li):
         """The layer's native handle (None off the GPU), made anew when something it was made from has changed."""
         self._ensure_storage()
-        h = self._layers[li] = _host.layer(
-            self._layers[li], li, self._batched_args[li]['plans'], self._k_packed[li], self._k_norms, self._v_packed,
-            self._v_norms, self._k_rows[li], self._k_norms.shape[-1], self._vpb, self.n_q, _plan.K_BITPACKED, _plan.V_BITPACKED,
-            self.scale, self.quantizers[li][0]._q_perm_baked, self._buf_k, self._buf_v)
+        h = self._layers[li]
+        args = (li, self._batched_args[li]['plans'], self._k_packed[li], self._k_norms, self._v_packed, self._v_norms,
+                self._k_rows[li], self._k_norms.size(-1), self._vpb, self.n_q, _plan.K_BITPACKED, _plan.V_BITPACKED,
+                self.scale, self.quantizers[li][0]._q_perm_baked, self._buf_k, self._buf_v)
+        if h is None or not h.holds(*args):
+            h = self._layers[li] = _host.layer(*args)
         return h
 
     def set_seq_lens(self, seq_lens):

@@ -64,10 +64,12 @@ class BlockGTQProductionCache:
 
     def _native(self, li):
         """The layer's native handle (None off the GPU), made anew when something it was made from has changed."""
-        h = self._layers[li] = _host.layer(
-            self._layers[li], li, self.batched_args[li]['plans'], self.k_packed, self.k_norms, self.v_packed, self.v_norms,
-            self.k_bytes_per_tok, self.max_ng, self.vpb, self.nq, self._k_layout, self._v_layout, self.scale,
-            self.quantizers[li][0]._q_perm_baked)
+        h = self._layers[li]
+        args = (li, self.batched_args[li]['plans'], self.k_packed, self.k_norms, self.v_packed, self.v_norms,
+                self.k_bytes_per_tok, self.max_ng, self.vpb, self.nq, self._k_layout, self._v_layout, self.scale,
+                self.quantizers[li][0]._q_perm_baked, None, None)
+        if h is None or not h.holds(*args):
+            h = self._layers[li] = _host.layer(*args)
         return h
 
     # ---------------------------------------------------------------- encode

@@ -7,6 +7,8 @@ import torch
 
 from .packed_kv_manager import run_decoder_stack
 
+_READ_IN_PLACE = (torch.float16, torch.bfloat16)      # what the encoders take as it lies
+
 
 @torch.no_grad()
 def production_decode_step(model, input_ids, position_ids, cache):
@@ -40,8 +42,8 @@ def production_prefill(model, input_ids, cache, chunk_encode=64):
     out = model(input_ids, position_ids=position_ids, past_key_values=hf_cache, use_cache=True)
     for li in range(cache.n_layers):
         k, v = _layer_kv(hf_cache, li)
-        if k.dtype == v.dtype and k.dtype in (torch.float16, torch.bfloat16) and k.stride(-1) == v.stride(-1) == 1:
-            if k.shape[2] > prompt_len:
+        if k.dtype in _READ_IN_PLACE and v.dtype == k.dtype and k.stride(-1) == 1 and v.stride(-1) == 1:
+            if k.size(2) > prompt_len:
                 k, v = k[:, :, :prompt_len], v[:, :, :prompt_len]
             cache._encode_batched(li, k, v, 0)
             continue
