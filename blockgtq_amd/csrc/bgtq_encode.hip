@@ -412,21 +412,27 @@ __global__ __launch_bounds__(NT) void encode_kernel(EncodeArgs a) {
 //
 // A block stays in one wave from the raw rows to the codes: lane (li, lg) of 16 x 4 holds dims k = 4 kk + lg
 // of row li in 32 registers, which is the A operand of step kk as it is.
-//   norms    X X^T: A and B are the same registers, the diagonal holds the 16 sums of squares (15 of 16 products
-//            are thrown away, but no lane waits for another's chain: lane = row chains left 48 lanes idle
-//            and took as long as the rotation)
+//   norms    V, and K where waves have blocks of their own: X X^T, A and B are the same registers, the diagonal holds
+//            the 16 sums of squares (15 of 16 products are thrown away, but no lane waits for another's chain: lane =
+//            row chains of V left 48 lanes idle and took as long as the rotation); K else: lane = (row, one of four groups)
 //   xhat     x / norm from the norm's rounded reciprocal, in registers (div_by below)
 //   rotate   16 columns at a time against the rotation in LDS, stored in operand order (one 16-byte read a lane
 //            feeds four steps, no bank conflicts); K takes only the steps its columns' segments reach
 //   codes    four rows of one column per lane, straight from the accumulator
-//   corrected norms  the centroids of the codes, once more X X^T
+//   corrected norms  the centroids of the codes: V once more X X^T, K lane = (row, group): its chains of 16 dims with
+//            a dependent code, centroid and product read each took 17 k of a block's 64 k clocks, these take 7 k
 //   packing  a lane makes four bytes of a record: a byte is a dot product of four code bytes with powers of two
 //
-// CS 1: 16 waves share a rotation, each walks blocks of its own and no barrier is met on the way.  CS 4 (few
-// rows): the 4 waves of a work-group split the columns of one block, which quarters its longest stage.
-// Bound by the matrix cores: 320 instructions of 32 clocks a V block.  65 536 records each of K and V (4 x 8192
-// tokens, 2 heads, K3V3): 135 us as two launches of 16-row tiles on the vector units (there the dense V rotation
-// alone is 55 us of FMA), 61 us here in one (65 with the cell search behind its own columns' products).
+// CS waves share a block and split its columns, groups, rows to load and rows to pack.  CS 1 (many blocks): 16 waves
+// share a rotation, each walks blocks of its own and no barrier is met on the way.  CS 2 (at most 8 blocks a
+// work-group): as many waves a compute unit again where CS 1 would leave half of it empty.  CS 4 (few rows): a
+// work-group of 4 waves a block, two of them a compute unit.
+// CS 1 is bound by the matrix cores and vector issue in turn: 320 instructions of 32 clocks a V block.  65 536 records
+// each of K and V (4 x 8192 tokens, 2 heads, K3V3): 135 us as two launches of 16-row tiles on the vector units (there the
+// dense V rotation alone is 55 us of FMA), 61 us here in one.  CS 2 and CS 4 are bound by one block's chain; 8 heads,
+// nibble records, against groups one after the other in K's norms and CS 1 from 513 blocks on: 128 tokens 18.3 -> 13.1 us,
+// 600 26.7 -> 18.8, 2001 30.4 -> 26.1, 9000 (CS 1) 89.6 -> 78.8; bit-packed records (no corrected K norms) 12.4 -> 11.4,
+// 20.6 -> 16.4, 23.9 -> 23.4, 70.1 -> 70.4.
 // ================================================================================================
 constexpr int RROW = D * 2 + 16;        // bytes from one raw row to the next: rows 4 banks apart
 constexpr int CROW = D + 8;             // bytes from one row of codes to the next (a byte's window of codes may reach 8 past the last)
@@ -435,7 +441,7 @@ struct TileArgs { EncodeArgs k, v; int k_groups, v_groups; };      // work-group
 
 template <int CS>
 struct EncodeLds {
-    static constexpr int NW = CS == 1 ? 16 : 4;               // waves at most
+    static constexpr int NW = CS == 4 ? 4 : 16;               // waves at most
     static constexpr int NB = NW / CS;                        // blocks at a time
     float rot[D / 4][D][4];             // the rotation, [step][column][k % 4]
     alignas(16) uint8_t raw[NB][16 * RROW];                   // raw rows [row][k % 4][k / 4] fp16, later the codes
@@ -444,7 +450,6 @@ struct EncodeLds {
     uint4 pack[D];                      // per record byte: first code, its bits (offset | width << 8), dot weights of the next ones
     float cent[BGTQ_MAX_SEGMENTS * 32];
     uint8_t lut[BGTQ_MAX_SEGMENTS * BGTQ_LUT_BINS];
-    int2 span[D / 16];                  // per 16 columns: first and last + 1 group of four steps
     int hdr[56];
     float2 bin[D];                      // K cell search of a packed dim
     int8_t group[D];                    // its group, -1: a 0-bit dim
@@ -462,7 +467,7 @@ __device__ __forceinline__ float div_by(float x, float2 dy) {
 
 template <int CS, bool IS_V>
 __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, const int first, const int stride, EncodeLds<CS>& L) {
-    const int NW = CS == 1 ? (int)blockDim.x >> 6 : 4, NTHR = NW * 64, NB = NW / CS;       // (at least 4 waves)
+    const int NW = CS == 4 ? 4 : (int)blockDim.x >> 6, NTHR = NW * 64, NB = NW / CS;       // (at least 4 waves)
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
@@ -472,7 +477,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
     const bool need_cent = IS_V || a.layout == BGTQ_K_MIXED || a.corrected;
 
     // ---- once per work-group: tables and the rotation (64 KB, straight from the plan into LDS).  Everything is
-    // requested in one burst; the dims' table is parked where the first raw rows go later
+    // requested in one burst
     {
         const uint32_t dst = (uint32_t)(uintptr_t)(lds_ptr_t)(uint8_t*)&L.rot[0][0][0];
         if constexpr (IS_V) {                                 // (the plan holds it in this order)
@@ -490,47 +495,29 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
     int n_seg = 1, v_bits = 0, n_zero = 0;
     float bd[15];                                             // V boundaries (+inf past the last)
     uint2 byte_of = {0u, 0u};
-    int4* dims = (int4*)&L.raw[0][0];
-    static_assert(sizeof(int4) * D <= sizeof(L.raw[0]), "the dims' table fits one block's rows");
+    uint32_t seg_of[4] = {0, 0, 0, 0};                        // group of dim 4 kk + lg, 4 bits each
     if constexpr (IS_V) {
         v_bits = P.v_bits;
 #pragma unroll
         for (int b = 0; b < 15; b++) bd[b] = P.v_boundaries[b];
         if (tid < 16) L.cent[tid] = P.v_centroids[tid];
         if (tid < D / 2) byte_of = *(const uint2*)P.enc_vbyte[a.layout == BGTQ_V_NIBBLE ? 1 : 0][tid];
+        if (tid < D) L.place[tid] = (uint16_t)(((tid & 3) * (D / 4) + (tid >> 2)) * 2);
     } else {
         n_seg = P.n_seg;
         n_zero = P.n_zero_dims;
+        const uint4 segs = ((const uint4*)((const uint8_t*)P.lut_image[BGTQ_K_BITPACKED] + BGTQ_LUT_KSEG))[lg];
+        seg_of[0] = segs.x; seg_of[1] = segs.y; seg_of[2] = segs.z; seg_of[3] = segs.w;
         if (tid < 56) L.hdr[tid] = ((const int*)&P)[tid];
         for (int i = tid; i < BGTQ_MAX_SEGMENTS * BGTQ_LUT_BINS / 4; i += NTHR) ((uint32_t*)L.lut)[i] = ((const uint32_t*)&P.code_lut[0][0])[i];
         if (tid < BGTQ_MAX_SEGMENTS * 32) L.cent[tid] = P.k_centroids[tid >> 5][tid & 31];
-        if (tid < D) {
-            dims[tid] = *(const int4*)P.enc_dim[tid];
+        if (tid < D) {                                        // packed dim k lies at [k % 4][k / 4] of a raw row
+            const int4 dim = *(const int4*)P.enc_dim[tid];
+            L.group[tid] = (int8_t)dim.x;
+            L.place[dim.w >> 8] = (uint16_t)(((tid & 3) * (D / 4) + (tid >> 2)) * 2);
             L.bin[tid] = float2{P.lut_offset[tid], P.lut_inv_scale[tid]};
             byte_of = *(const uint2*)P.enc_byte[a.layout == BGTQ_K_MIXED ? 1 : 0][tid];
         }
-    }
-    if constexpr (!IS_V) __syncthreads();
-    uint32_t seg_of[4] = {0, 0, 0, 0};                        // group of dim 4 kk + lg, 4 bits each
-    if constexpr (!IS_V) {
-#pragma unroll
-        for (int kk = 0; kk < D / 4; kk++) seg_of[kk >> 3] |= (uint32_t)max(dims[4 * kk + lg].x, 0) << (4 * (kk & 7));
-        if (tid < D / 16) {
-            int lo = D, hi = 0;
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int4 dim = dims[16 * tid + i];
-                lo = min(lo, dim.x >= 0 ? dim.y : D);
-                hi = max(hi, dim.x >= 0 ? dim.z : 0);
-            }
-            L.span[tid] = int2{lo >> 4, (hi + 15) >> 4};
-        }
-    }
-    if (tid < D) {
-        const int k = tid;                                    // packed dim k lies at [k % 4][k / 4] of a raw row
-        int src = k;
-        if constexpr (!IS_V) { src = dims[k].w >> 8; L.group[k] = (int8_t)dims[k].x; }
-        L.place[src] = (uint16_t)(((k & 3) * (D / 4) + (k >> 2)) * 2);
     }
     const int lpr = a.row_width > 64 ? 32 : 16;               // packing: lanes per row, lane = record dword dw
     const int dw = lane & (lpr - 1);
@@ -554,8 +541,8 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
     // (a stream of 1-bit codes; groups are in ascending width)
     const bool two_dots = IS_V ? v_bits == 1 && a.layout == BGTQ_V_BITPACKED : P.seg_bw[0] == 1 && a.layout == BGTQ_K_BITPACKED;
 
-    // ---- this wave's (CS 1) or this work-group's (CS 4) blocks
-    const int slot = CS == 1 ? wave : 0;
+    // ---- CS waves a block: the block's place in the work-group, this wave's part of it
+    const int slot = CS == 1 ? wave : wave / CS, part = CS == 1 ? 0 : wave % CS;
     uint8_t* raw = L.raw[slot];
     const bool wide = ((a.x_sb | a.x_sh | a.x_ss) & 7) == 0 && ((uintptr_t)a.x & 15) == 0;
     auto meet = [&]() {
@@ -564,8 +551,10 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         else __builtin_amdgcn_wave_barrier();                 // (a wave's LDS accesses keep their order)
         asm volatile("" ::: "memory");
     };
-    // (CS 1: neighbouring blocks to the waves of one work-group)
-    for (int blk = CS == 1 ? first * NW + wave : first; blk < n_blocks; blk += stride * NB) {
+    // (neighbouring blocks to the waves of one work-group; CS > 1: as many rounds for every wave of it, for the barriers'
+    // sake - rows past the last are zeros and stored nowhere)
+    for (int round = first * NB; CS == 1 ? round + slot < n_blocks : round < n_blocks; round += stride * NB) {
+        const int blk = round + slot;
         const unsigned n0 = (unsigned)blk * 16u;
         const int b0 = (int)(n0 / (unsigned)a.S), s0 = (int)(n0 - (unsigned)b0 * (unsigned)a.S);
         auto row_of = [&](int r, int& b, int& s) {            // (batch row, step) of the block's row r
@@ -580,7 +569,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
             uint4 x4[PASS];
 #pragma unroll
             for (int p = 0; p < PASS; p++) {
-                const int r = (CS == 1 ? 4 * p : 4 * wave) + (lane >> 4);
+                const int r = 4 * (part * PASS + p) + (lane >> 4);
                 x4[p] = uint4{0, 0, 0, 0};
                 if ((int64_t)n0 + r < N) {
                     int b, s;
@@ -597,7 +586,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
             }
             const uint4 at = *(const uint4*)&L.place[rc * 8];
             const uint32_t at2[4] = {at.x, at.y, at.z, at.w};
-            if (lane < 16 && (CS == 1 || wave == 0)) {        // where the rows go
+            if (lane < 16 && part == 0) {                     // where the rows go
                 int64_t dst = -1, nd = -1;
                 if ((int64_t)n0 + lane < N) {
                     int b, s;
@@ -614,7 +603,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
             }
 #pragma unroll
             for (int p = 0; p < PASS; p++) {
-                uint8_t* row = raw + ((CS == 1 ? 4 * p : 4 * wave) + (lane >> 4)) * RROW;
+                uint8_t* row = raw + (4 * (part * PASS + p) + (lane >> 4)) * RROW;
                 uint32_t w[4] = {x4[p].x, x4[p].y, x4[p].z, x4[p].w};
                 if (a.bf16) {
 #pragma unroll
@@ -651,15 +640,16 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         const bool diag = (li >> 2) == lg;
         auto diagonal = [&](const float4v& sum) { return li & 2 ? (li & 1 ? sum[3] : sum[2]) : (li & 1 ? sum[1] : sum[0]); };
         if constexpr (IS_V) {
-            float4v sum = {0, 0, 0, 0};
+            if (CS != 2 || part == 0) {                       // (CS 4: a barrier takes longer than the same products in every wave)
+                float4v sum = {0, 0, 0, 0};
 #pragma unroll
-            for (int kk = 0; kk < D / 4; kk++) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(A[kk], A[kk], sum, 0, 0, 0);
-            const float n = __builtin_sqrtf(diagonal(sum) + 1e-30f);
-            if (diag) L.nrm[slot][0][li] = float2{n, 1.0f / n};
-        } else {
-            constexpr int STEP = CS == 1 ? 1 : CS;            // (CS 4: the groups are dealt to the waves)
-            const int g_first = CS == 1 ? 0 : wave;
-            for (int g = g_first; g < n_seg; g += STEP) {
+                for (int kk = 0; kk < D / 4; kk++) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(A[kk], A[kk], sum, 0, 0, 0);
+                const float n = __builtin_sqrtf(diagonal(sum) + 1e-30f);
+                if (diag) L.nrm[slot][0][li] = float2{n, 1.0f / n};
+            }
+            if (CS == 2) __syncthreads();
+        } else if constexpr (CS == 1) {                       // (the matrix cores have room beside K's other work)
+            for (int g = 0; g < n_seg; g++) {
                 const int s = L.hdr[H_START + g], e = s + L.hdr[H_LEN + g];
                 float4v sum = {0, 0, 0, 0};
                 for (int q = s >> 4; q < (e + 15) >> 4; q++) {
@@ -675,11 +665,47 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
             }
             // roots and reciprocals of all groups together: four groups of 16 rows an instruction
             asm volatile("" ::: "memory");                    // (a wave's LDS accesses keep their order)
-            for (int i = lane; g_first + STEP * (i >> 4) < n_seg; i += 64) {
-                float2* at = &L.nrm[slot][g_first + STEP * (i >> 4)][i & 15];
+            for (int i = lane; (i >> 4) < n_seg; i += 64) {
+                float2* at = &L.nrm[slot][i >> 4][i & 15];
                 const float n = __builtin_sqrtf(at->x + 1e-30f);
                 finite = finite && n < INFINITY;
                 *at = float2{n, 1.0f / n};
+            }
+        } else {
+            // lane = (row li, group 4 p + lg): 64 chains side by side, over the blocks of 16 dims that the group touches
+            for (int p = part; 4 * p < n_seg; p += CS) {
+                const int g = 4 * p + lg, s = g < n_seg ? L.hdr[H_START + g] : 0, e = g < n_seg ? s + L.hdr[H_LEN + g] : 0;
+                const uint8_t* at = raw + li * RROW + (s >> 4) * 8;
+                int lo = s & 15, hi = e - (s & ~15);          // the group's dims, from this block's first one on
+                float sum = 0.f;
+                uint2 w[4];                                   // dims c, c + 4, c + 8, c + 12 of the block
+                auto fetch = [&]() {                          // (reads past the group stay inside the work-group's rows: masked below)
+#pragma unroll
+                    for (int c = 0; c < 4; c++) w[c] = *(const uint2*)(at + c * (D / 2));
+                };
+                fetch();
+                while (__builtin_amdgcn_ballot_w64(hi > 0) != 0) {
+                    uint2 v[4];
+#pragma unroll
+                    for (int c = 0; c < 4; c++) v[c] = w[c];
+                    at += 8;
+                    fetch();
+                    const uint32_t live = hi > 0 ? (0xFFFFu >> (16 - min(hi, 16))) & (0xFFFFu << lo) : 0u;
+#pragma unroll
+                    for (int i = 0; i < 16; i++) {
+                        const uint32_t d = i & 8 ? v[i & 3].y : v[i & 3].x;
+                        const uint32_t half = (d >> (i & 4 ? 16 : 0)) & (uint32_t)((int32_t)(live << (31 - i)) >> 31);
+                        const float x = bgtq_h2f((uint16_t)half);
+                        sum = __builtin_fmaf(x, x, sum);
+                    }
+                    lo = 0;
+                    hi -= 16;
+                }
+                if (g < n_seg) {
+                    const float n = __builtin_sqrtf(sum + 1e-30f);
+                    finite = finite && n < INFINITY;
+                    L.nrm[slot][g][li] = float2{n, 1.0f / n};
+                }
             }
         }
         bool scalar_chain = !IS_V && __builtin_amdgcn_ballot_w64(!finite) != 0;           // (uniform)
@@ -737,7 +763,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         if (!IS_V && scalar_chain) {
 #pragma unroll 1
             for (int c = 0; c < D / 16 / CS; c++) {
-                const int j = 16 * (CS == 1 ? c : wave * (D / 16 / CS) + c) + li;
+                const int j = 16 * (part * (D / 16 / CS) + c) + li;
                 const int4 dim = *(const int4*)P.enc_dim[j];
                 float4v y = {0, 0, 0, 0};
 #pragma unroll 1
@@ -761,7 +787,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         // eight steps ahead.
         auto columns = [&](auto bits) {
             constexpr int NB = (1 << decltype(bits)::value) - 1, EVERY = 32 / (NB + 1), NC = D / 16 / CS;
-            const float* rot = &L.rot[0][16 * (CS == 1 ? 0 : wave * NC) + li][lg];
+            const float* rot = &L.rot[0][16 * part * NC + li][lg];
             float R[2][8];
             auto fetch = [&](int at) {                        // eight steps: columns at / 4, steps 8 (at % 4) ..
 #pragma unroll
@@ -805,7 +831,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         } else {
 #pragma unroll
             for (int c = 0; c < D / 16 / CS; c++) {
-                const int cb = CS == 1 ? c : wave * (D / 16 / CS) + c;
+                const int cb = part * (D / 16 / CS) + c;
                 const int j = 16 * cb + li;
                 float4v y = {0, 0, 0, 0};
                 const float* rot = &L.rot[0][j][lg];          // + step * 4 D: two steps a read
@@ -814,7 +840,8 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
                     codes[c] = odd_codes[c];
                     continue;
                 }
-                const int q_lo = __builtin_amdgcn_readfirstlane(L.span[cb].x), q_hi = __builtin_amdgcn_readfirstlane(L.span[cb].y);
+                const uint32_t span = ((const uint32_t*)P.rot_span)[cb >> 2] >> ((cb & 3) * 8);
+                const int q_lo = (int)(span & 15u), q_hi = (int)((span >> 4) & 15u);
 #pragma unroll
                 for (int q = 0; q < D / 16; q++)
                     if (q >= q_lo && q < q_hi) {              // (uniform)
@@ -830,7 +857,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         for (int c = 0; c < D / 16 / CS; c++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
-                raw[(4 * lg + r) * CROW + 16 * (CS == 1 ? c : wave * (D / 16 / CS) + c) + li] = (uint8_t)(codes[c] >> (8 * r));
+                raw[(4 * lg + r) * CROW + 16 * (part * (D / 16 / CS) + c) + li] = (uint8_t)(codes[c] >> (8 * r));
         meet();
         // ---- norms to store
         auto store_norm = [&](int g, int row, float out) {
@@ -839,7 +866,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
             if (a.codes_out && !IS_V) { if (a.norms_f32_out && g < a.norm_width) a.norms_f32_out[nd * a.norm_width + g] = out; }
             else if (g < (IS_V ? 1 : a.norm_width) && a.norms) a.norms[nd + g] = bgtq_f2h(out);
         };
-        if (CS == 1 || wave == 0) {
+        if (part == 0 || (!IS_V && need_cent)) {
             if (need_cent) {
                 if constexpr (IS_V) {                         // the centroids of all codes in two bursts
                     float4v sum = {0, 0, 0, 0};
@@ -858,31 +885,42 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
                     const float cn = __builtin_sqrtf(diagonal(sum) + 1e-20f);
                     if (diag) store_norm(0, li, L.nrm[slot][0][li].x / (cn > 1e-10f ? cn : 1.0f));
                 }
-                for (int g = 0; !IS_V && g < n_seg; g++) {
-                    const int s = L.hdr[H_START + g], e = s + L.hdr[H_LEN + g], bw = L.hdr[H_BW + g];
-                    float4v sum = {0, 0, 0, 0};
+                if constexpr (!IS_V) {                        // the centroids' chains, lane = (row, group) as above
 #pragma unroll 1
-                    for (int q = s >> 4; q < (e + 15) >> 4; q++) {
-                        const uint32_t* cw = (const uint32_t*)&raw[li * CROW + 16 * q];
-                        float c[4];
+                    for (int p = part; p < 2; p += CS) {
+                        const int g = 4 * p + lg, s = g < n_seg ? L.hdr[H_START + g] : 0, len = g < n_seg ? L.hdr[H_LEN + g] : 0;
+                        const bool far = g < n_seg && L.hdr[H_BW + g] > 5;        // (its centroids are not in LDS)
+                        const bool any_far = __builtin_amdgcn_ballot_w64(far) != 0;
+                        const uint8_t* at = &raw[li * CROW + (s & ~3)];
+                        const float* cent = &L.cent[(g & 7) * 32];
+                        float sum = 0.f;
+                        uint32_t w[3];                        // codes s .. s + 7 from byte s & 3 on
+                        auto fetch = [&](int t) {
 #pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            const int k = 16 * q + 4 * i + lg;
-                            const uint32_t code = (cw[i] >> (8 * lg)) & 0xFFu;
-                            c[i] = bw > 5 ? P.k_centroids[g][code] : L.cent[g * 32 + (code & 31u)];
-                            if (k < s || k >= e) c[i] = 0.f;
+                            for (int i = 0; i < 3; i++) w[i] = *(const uint32_t*)(at + t + 4 * i);
+                        };
+                        fetch(0);
+                        for (int t = 0; __builtin_amdgcn_ballot_w64(t < len) != 0; t += 8) {
+                            const uint32_t lo = __builtin_amdgcn_alignbyte(w[1], w[0], s & 3), hi = __builtin_amdgcn_alignbyte(w[2], w[1], s & 3);
+                            float c[8];
+                            if (any_far) {                    // (uniform)
+#pragma unroll
+                                for (int i = 0; i < 8; i++) {
+                                    const uint32_t code = ((i < 4 ? lo : hi) >> (8 * (i & 3))) & 0xFFu;
+                                    c[i] = t + i >= len ? 0.f : far ? P.k_centroids[g][code] : cent[code & 31u];
+                                }
+                            } else {
+#pragma unroll
+                                for (int i = 0; i < 8; i++) c[i] = cent[((i < 4 ? lo : hi) >> (8 * (i & 3))) & 31u];
+                            }
+                            fetch(t + 8);
+#pragma unroll
+                            for (int i = 0; i < 8; i++) {
+                                const float m = t + i < len ? c[i] : 0.f;
+                                sum = __builtin_fmaf(m, m, sum);
+                            }
                         }
-#pragma unroll
-                        for (int i = 0; i < 4; i++) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(c[i], c[i], sum, 0, 0, 0);
-                    }
-                    if (diag) L.nrm[slot][g][li].y = diagonal(sum);       // (the reciprocals have served)
-                }
-                if constexpr (!IS_V) {
-                    asm volatile("" ::: "memory");
-                    for (int i = lane; i < BGTQ_MAX_SEGMENTS * 16; i += 64) {
-                        const int g = i >> 4, row = i & 15;
-                        const float2 v = L.nrm[slot][g][row];
-                        store_norm(g, row, g < n_seg ? v.x / fmaxf(__builtin_sqrtf(v.y), 1e-10f) : 0.f);
+                        store_norm(g, li, g < n_seg ? L.nrm[slot][g][li].x / fmaxf(__builtin_sqrtf(sum), 1e-10f) : 0.f);
                     }
                 }
             } else {
@@ -894,7 +932,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         }
         // ---- records
         if (a.codes_out) {
-            for (int i = CS == 1 ? lane : tid; i < 16 * (D / 4); i += 64 * CS) {
+            for (int i = part * 64 + lane; i < 16 * (D / 4); i += 64 * CS) {
                 const int64_t n = L.dst[slot][i >> 5];
                 if (n >= 0) *(uint32_t*)&a.codes_out[n * D + 4 * (i & 31)] = *(const uint32_t*)&raw[(i >> 5) * CROW + 4 * (i & 31)];
             }
@@ -904,7 +942,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
 #pragma unroll
             for (int i = 0; i < 4; i++) make[i] = L.pack[4 * dw + i];
 #pragma unroll 2
-            for (int r = lane / lpr + (CS == 1 ? 0 : wave * rows); r < 16; r += rows * CS) {
+            for (int r = lane / lpr + part * rows; r < 16; r += rows * CS) {
                 const int64_t dst = L.dst[slot][r];
                 if (dst < 0) continue;
                 uint32_t byte[4];
@@ -957,9 +995,17 @@ int launch_blocks(const EncodeArgs* k, const EncodeArgs* v, hipStream_t st) {
         return bgtq_launch_status();
     }
     // One work-group of up to 16 waves a compute unit, in equal shares over kinds and heads, each wave the same
-    // number of blocks; with fewer than 16 blocks a work-group, that many waves.
+    // number of blocks; with fewer than 16 blocks a work-group, that many waves; with at most 8, two waves a block (2600
+    // tokens of 2 heads, 6 blocks: 25.9 us with six waves, 18.0 with twelve).
     const int64_t most = std::max<int64_t>(1, 256 / (any.n_kv * kinds));
     const int64_t share = (blocks + most - 1) / most, rounds = (share + 15) / 16;
+    if (share <= 8) {
+        const int groups = (int)((blocks + share - 1) / share);
+        t.k_groups = k ? groups : 0;
+        t.v_groups = v ? groups : 0;
+        hipLaunchKernelGGL(encode_blocks_kernel<2>, dim3((unsigned)(groups * kinds * any.n_kv)), dim3((unsigned)std::max<int64_t>(4, 2 * share) * 64), 0, st, t);
+        return bgtq_launch_status();
+    }
     const int nw = (int)std::max<int64_t>(4, (share + rounds - 1) / rounds);
     const int groups = (int)((blocks + nw * rounds - 1) / (nw * rounds));
     t.k_groups = k ? groups : 0;

@@ -42,7 +42,7 @@ PLAN_DTYPE = np.dtype([
     ('v_rot_T', '<f4', (_D * _D,)), ('v_rot', '<f4', (_D * _D,)),
     ('v_rot_T4', '<f4', (_D // 4, _D, 4)), ('enc_vbyte', '<u4', (2, _D // 2, 2)),
     ('n_units', '<i4', (2,)), ('n_pair_units', '<i4', (2,)),
-    ('kend', '<u4', (2,)), ('kfirst', '<u4', (2, 2)), ('reserved1', '<u4', (2,)),
+    ('kend', '<u4', (2,)), ('kfirst', '<u4', (2, 2)), ('rot_span', 'u1', (_D // 16,)),
     ('kprog', '<u4', (2, MAX_UNITS, 8)), ('kunit', '<u4', (2, MAX_UNITS)),
     ('swalk', '<u4', (2, MAX_WALK, 4)), ('n_walk', '<u4', (4,)), ('sunit', '<u4', (2, MAX_UNITS)),
     ('lut_image', '<u4', (2, 20480 // 4)), ('vlut_image', '<u4', (2, 8192 // 4)),
@@ -52,6 +52,7 @@ PLAN_DTYPE = np.dtype([
 LUT_K = {3: 0, 2: 8192, 4: 10240, 1: 11264}    # each on a multiple of its size once VLUT_BYTES is added
 LUT_KRAW, LUT_K5P, LUT_IMAGE_BYTES = 11776, 13824, 20480
 LUT_KQ = {1: 17920, 2: 18432}                  # four codes per 8-byte entry (decode kernel, bit-packed image)
+LUT_KSEG = 18048                               # segments of the packed dims, 4 bits each (prompt-sized encoder, bit-packed image)
 LUTM_KRAW = 4096
 VLUT_BYTES = 8192          # the kernel's table area starts with the V table; the K image follows it
 
@@ -164,6 +165,13 @@ def fill_encoder_tables(p) -> None:
         ge = gs + int(p['seg_len'][g]) if g >= 0 else 0
         ident = int(p['seg_identity'][g]) if g >= 0 else 0
         p['enc_dim'][j] = [g, gs, ge, ident | (int(p['head_perm'][j]) << 8)]
+    for t in range(D // 16):
+        own = [d for d in p['enc_dim'][16 * t:16 * t + 16] if d[0] >= 0]
+        lo, hi = (min(int(d[1]) for d in own) // 16, (max(int(d[2]) for d in own) + 15) // 16) if own else (0, 0)
+        p['rot_span'][t] = lo | (hi << 4)
+    seg = np.maximum(p['group_of'], 0).astype(np.uint32).reshape(4, 8, 4)          # [q][i][c]
+    kseg = (seg << (4 * np.arange(8, dtype=np.uint32))[None, :, None]).sum(axis=1, dtype=np.uint32).T
+    p['lut_image'][K_BITPACKED, LUT_KSEG // 4:LUT_KSEG // 4 + 16] = kseg.reshape(-1)
     p['enc_byte'][...] = 0
     z, nps, npl = int(p['n_zero_dims']), int(p['nopack_start']), int(p['nopack_len'])
     for j in range(D):

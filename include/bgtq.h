@@ -55,6 +55,9 @@ extern "C" {
  * own) and 256 entries of 2-bit codes (on a multiple of its size in the kernel's table area) */
 #define BGTQ_LUT_K1Q     17920
 #define BGTQ_LUT_K2Q     18432
+/* bit-packed image, for the prompt-sized encoder: uint32[4][4], entry [c][q] holds the segments (0 for a 0-bit dim) of packed
+ * dims 32 q + 4 i + c, i = 0 .. 7, 4 bits each */
+#define BGTQ_LUT_KSEG    18048
 #define BGTQ_LUT_IMAGE_BYTES 20480               /* room for either K image */
 /* how a segment's units are unpacked */
 #define BGTQ_PATH_B1     1   /* bit-packed 1-bit codes: a unit is 1 byte, pair table of 4 entries x 32 replicas */
@@ -180,7 +183,8 @@ typedef struct bgtq_head_plan {
     int32_t  n_pair_units[2];
     uint32_t kend[2];
     uint32_t kfirst[2][2];
-    uint32_t reserved1[2];
+    /* rows of k_rot_T that columns 16 t .. 16 t + 15 reach, in groups of 16: first | one past the last << 4 */
+    uint8_t  rot_span[BGTQ_HEAD_DIM / 16];
     uint32_t kprog[2][BGTQ_MAX_UNITS][8];
     uint32_t kunit[2][BGTQ_MAX_UNITS];
     /*

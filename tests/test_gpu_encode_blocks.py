@@ -102,3 +102,32 @@ def test_blocks_drop_positions_outside_the_cache():
     want, wn = _encode(args, x, P.K_BITPACKED, P.V_BITPACKED, P.QUANT_LUT256, 43, 16)[:2]
     assert torch.equal(kp[0, 0, 30:], want[0, 0, 3:33]) and torch.equal(kp[1, 0, :30], want[1, 0, 13:])
     assert (kp[0, 0, :30] == 0xA5).all() and (kp[1, 0, 30:] == 0xA5).all() and (kn[1, 0, 30:] == 7.0).all()
+
+
+# 8 heads of K or V: 64 blocks are still a work-group each, from 65 on two waves share a block (3 of them a work-group, the
+# last work-group not full; exactly 8), from 257 on every wave has its own (9 a work-group, in one round; 17, in two)
+@pytest.mark.parametrize("S", [1024, 1025, 2010, 4096, 4097, 8200])
+@pytest.mark.parametrize("bits,kl,vl", [((3.0, 3, 1, 8), P.K_MIXED, P.V_NIBBLE), ((4.0, 4, 0, 8), P.K_BITPACKED, P.V_BITPACKED)])
+def test_blocks_by_waves_per_block(S, bits, kl, vl):
+    args = _plans(8, bits, seed=47)
+    gen = torch.Generator(device=DEV).manual_seed(S)
+    x = (torch.randn(1, 8, S, 128, generator=gen, device=DEV) * torch.rand(1, 8, S, 1, generator=gen, device=DEV) * 30).half()
+    x[0, 0, 5] = 0
+    x[0, 3, S - 1, 77] = float("inf")                          # (the other rows of its block take another way)
+    got, want = _encode(args, x, kl, vl, P.QUANT_LUT256, S + 9), _encode(args, x, kl, vl, P.QUANT_LUT256, S + 9, 32)
+    for o in got + want:
+        o[0, 3, 3 + S - 1] = 0
+    _same(got, want)
+
+
+def test_segment_tables_of_the_block_encoder():
+    """`rot_span` covers the rows that 16 columns' segments reach, the segment nibbles repeat `group_of`."""
+    for bits in ((3.0, 3, 1, 8), (2.0, 2, 0, 4), (1.0, 1, 0, 3)):
+        for p in _plans(2, bits)['plans_np']:
+            seg = p['lut_image'][P.K_BITPACKED][P.LUT_KSEG // 4:][:16].reshape(4, 4)
+            rot = p['k_rot_T'].reshape(128, 128)
+            for k in range(128):
+                assert (int(seg[k % 4, k // 32]) >> (4 * ((k // 4) % 8))) & 15 == max(int(p['group_of'][k]), 0)
+                lo, hi = int(p['rot_span'][k // 16]) & 15, int(p['rot_span'][k // 16]) >> 4
+                rows = [r for r in range(128) if rot[r, k] and p['group_of'][k] >= 0]
+                assert all(16 * lo <= r < 16 * hi for r in rows)
