@@ -688,7 +688,7 @@ int bgtq_window_attn(const void* q, int64_t q_sb, int64_t q_sh,
     if (W > 8192) return BGTQ_ELIMIT;
     if (B == 0 || n_kv == 0) return BGTQ_OK;
     const WindowArgs a{(const uint16_t*)q, q_sb, q_sh, 0, (const uint16_t*)kbuf, (const uint16_t*)vbuf, w_sb, w_sh, w_st,
-                       lens, W, n_kv * gqa, gqa, scale, part_out, part_lse};
+                       lens, W, n_kv * gqa, gqa, scale, part_out, part_lse, {}};
     return launch_window_attn(a, B, n_kv, (hipStream_t)stream);
 }
 
@@ -717,14 +717,21 @@ int bgtq_decode_step(const bgtq_step* step, void* stream) {
         BGTQ_CHECK_ARG(s.k && s.v && s.win_W >= 1);
         if (s.win_W > 8192) return BGTQ_ELIMIT;
         window = WindowArgs{(const uint16_t*)s.q, s.q_sb, s.q_sh, s.x_dtype == BGTQ_X_BF16, (const uint16_t*)s.win_k, (const uint16_t*)s.win_v,
-                            s.w_sb, s.w_sh, s.w_st, s.win_lens, s.win_W, n_q, s.gqa, s.scale, s.win_out, s.win_lse};
+                            s.w_sb, s.w_sh, s.w_st, s.win_lens, s.win_W, n_q, s.gqa, s.scale, s.win_out, s.win_lse, {}};
+        // small batches: the buffer's partial in the preparation's launch, and the swap as well where the new tokens can be
+        // read in the place of their slot
+        const WindowSwap swap{s.win_slot, (const uint16_t*)s.k, (const uint16_t*)s.v, s.k_sb, s.k_sh, s.v_sb, s.v_sh};
+        const bool rides = s.B <= BGTQ_ONE_LAUNCH_ROWS && window_rides(window);
         uint16_t *old_k = (uint16_t*)s.win_old, *old_v = old_k + (size_t)s.B * s.n_kv * D;
-        int rc = launch_window_swap(s.win_k, s.win_v, s.w_sb, s.w_sh, s.w_st, s.k, s.v, s.k_sb, s.k_sh, s.v_sb, s.v_sh,
-                                    s.x_dtype == BGTQ_X_BF16, s.win_slot, s.win_W, s.B, s.n_kv, old_k, old_v, st);
-        if (rc != BGTQ_OK) return rc;
-        // small batches: with the preparation's launch
-        if (s.B > BGTQ_ONE_LAUNCH_ROWS || !window_rides(window)) {
-            rc = launch_window_attn(window, s.B, s.n_kv, st);
+        if (rides && window_swaps(swap)) {
+            window.swap = swap;
+        } else {
+            const int rc = launch_window_swap(s.win_k, s.win_v, s.w_sb, s.w_sh, s.w_st, s.k, s.v, s.k_sb, s.k_sh, s.v_sb, s.v_sh,
+                                              s.x_dtype == BGTQ_X_BF16, s.win_slot, s.win_W, s.B, s.n_kv, old_k, old_v, st);
+            if (rc != BGTQ_OK) return rc;
+        }
+        if (!rides) {
+            const int rc = launch_window_attn(window, s.B, s.n_kv, st);
             if (rc != BGTQ_OK) return rc;
             window.q = nullptr;
         }

@@ -122,8 +122,16 @@ __device__ __forceinline__ float chain_sumsq_row(const float* x) {
     return ss;
 }
 
-template <bool IS_V>
-__device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, const int h, float* rot_s) {
+// Thread j = 0 .. 127 of its row.  PAIRED: the V row and the K row of one token by the two halves of a work-group, which
+// meet the same barriers (V's chains have fewer stages, K's barriers are met all the same).  ring: the row is the token that leaves slot
+// ring->slot[b] of the fp16 buffer, and the new one takes its place.
+struct RingArgs {
+    const int32_t* slot;
+    uint16_t* buf; int64_t b_sb, b_sh, b_st; int W;
+    const uint16_t* in; int64_t in_sb, in_sh; int bf16;
+};
+template <bool IS_V, bool PAIRED = false>
+__device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, const int h, const int j, float* rot_s, const RingArgs* ring = nullptr) {
     __shared__ __align__(16) float xs[2 * D];     // (the row, then zeros: the compact rotation reads up to BGTQ_ROT_COL values past a segment's start)
     __shared__ float nrm[BGTQ_MAX_SEGMENTS];
     __shared__ float nrm_out[BGTQ_MAX_SEGMENTS];
@@ -131,7 +139,6 @@ __device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, c
     __shared__ uint16_t xraw[D];
     __shared__ typename std::conditional<IS_V, StagedV, StagedK>::type sp;
 
-    const int j = threadIdx.x;
     const bgtq_head_plan& P = a.plans[h];
 
     // ---- 0. one burst: plan tables, the raw row and its position, the rotation column ----
@@ -152,7 +159,18 @@ __device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, c
     xs[D + j] = 0.f;
     int b, s;
     split_row(row, a.S, b, s);
-    const uint16_t xr = a.x[b * a.x_sb + h * a.x_sh + s * a.x_ss + j];
+    uint16_t xr = 0;
+    if (!ring) {
+        xr = a.x[b * a.x_sb + h * a.x_sh + s * a.x_ss + j];
+    } else {
+        const int slot = ring->slot[b];
+        if (slot >= 0 && slot < ring->W) {
+            uint16_t* at = ring->buf + b * ring->b_sb + h * ring->b_sh + (int64_t)slot * ring->b_st + j;
+            const uint16_t fresh = ring->in[b * ring->in_sb + h * ring->in_sh + j];
+            xr = *at;
+            *at = bgtq_in16(fresh, ring->bf16);
+        }
+    }
     const int t = (a.t_pos ? a.t_pos[b] : a.t_pos_scalar) + s;
     int4 k_dim = {0, 0, 0, 0};
     uint2 k_byte = {0u, 0u};
@@ -195,7 +213,7 @@ __device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, c
             fetch_rotation(P.k_rot_T, j, rst);
         }
     }
-    if constexpr (!IS_V) __syncthreads();     // (K reads the staged header next; V's staged tables are first read three barriers on)
+    if constexpr (!IS_V || PAIRED) __syncthreads();     // (K reads the staged header next; V's staged tables are first read three barriers on)
 
     // ---- per-thread static data, read ready-made from the plan (requested in the first burst) ----
     int n_seg = 1, g = 0, gs = 0, ge = D, ident = 0, src_dim = j;
@@ -216,6 +234,7 @@ __device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, c
     // ---- 1. the row to LDS, gathered by head_perm (K) -------------
     if constexpr (IS_V) {              // (no gather: a thread converts its own value)
         xs[j] = bgtq_h2f(bgtq_in16(xr, a.bf16));
+        if constexpr (PAIRED) __syncthreads();
     } else {
         xraw[j] = bgtq_in16(xr, a.bf16);
         __syncthreads();
@@ -400,7 +419,7 @@ __device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, c
 template <bool IS_V>
 __global__ __launch_bounds__(NT) void encode_kernel(EncodeArgs a) {
     __shared__ __align__(16) float rot_s[IS_V ? 4 : D * D];
-    encode_row<IS_V>(a, blockIdx.x, blockIdx.y, rot_s);
+    encode_row<IS_V>(a, blockIdx.x, blockIdx.y, threadIdx.x, rot_s);
 }
 // ================================================================================================
 // Prompt-sized encoder: blocks of 16 rows, every chain of the contract on the fp32 matrix cores.
@@ -1150,10 +1169,10 @@ __device__ __forceinline__ void prepare_part(const EncodeArgs& ak, const EncodeA
                                              const int rows, int bid, float* rot_s) {
     const int n = rows * ak.n_kv;
     if (bid < n) {
-        encode_row<true>(av, bid % rows, bid / rows, rot_s);
+        encode_row<true>(av, bid % rows, bid / rows, threadIdx.x, rot_s);
     } else if (bid < 2 * n) {
         bid -= n;
-        encode_row<false>(ak, bid % rows, bid / rows, rot_s);
+        encode_row<false>(ak, bid % rows, bid / rows, threadIdx.x, rot_s);
     } else {
         rotate_q_block(aq, bid - 2 * n, rot_s);
     }
@@ -1166,16 +1185,31 @@ __global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs a
     prepare_part(ak, av, aq, rows, blockIdx.x, rot_s);
 }
 // The same with the attention over the buffered tokens, which depends on none of it: the longer work-groups first, in
-// the LDS that is a rotation's otherwise; of the others two waves leave at once (a barrier counts the waves that are
-// left).  32 rows x 8 heads x 4 queries over 132 buffered tokens: 11.1 + 13.3 us as two launches,
-// 16.3 as one (1024 work-groups, two of them at a time on a compute unit).
+// the LDS that is a rotation's otherwise; then the token that leaves the buffer, K and V by the two halves of a
+// work-group, then the queries by two waves (a barrier counts the waves that are left).  SWAP: the step's token enters the
+// buffer here, put there by those who read the one that leaves.
+// 32 rows x 8 heads x 4 queries over 132 buffered tokens: 4.9 (swap) + 11.1 + 13.3 us as launches of their own, 4.9 + 16.3
+// with K and V a work-group each and the swap ahead of them (1024 work-groups, two of them at a time on a compute unit).
+template <bool SWAP>
 __global__ __launch_bounds__(WINDOW_THREADS, 2) void prepare_window_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, WindowArgs w,
-                                                                        int rows, int n_window) {
+                                                                        RingArgs rk, RingArgs rv, int rows, int n_window) {
     __shared__ __align__(16) float rot_s[D * D];
     static_assert(window_lds_floats<4>(WINDOW_RIDE_W) <= D * D, "a window's scores fit the rotation's place");
-    const int bid = blockIdx.x, n_kv = ak.n_kv;
-    if (bid < n_window) window_attn_block<4>(w, bid % n_kv, bid / n_kv, rot_s);
-    else if (threadIdx.x < NT) prepare_part(ak, av, aq, rows, bid - n_window, rot_s);
+    static_assert(WINDOW_THREADS == 2 * NT, "");
+    int bid = blockIdx.x;
+    const int n_kv = ak.n_kv, tid = threadIdx.x;
+    if (bid < n_window) {
+        window_attn_block<4, SWAP>(w, bid % n_kv, bid / n_kv, rot_s);
+        return;
+    }
+    bid -= n_window;
+    if (bid < rows * n_kv) {
+        const int row = bid % rows, h = bid / rows;
+        if (tid < NT) encode_row<true, true>(av, row, h, tid, rot_s, SWAP ? &rv : nullptr);
+        else encode_row<false, true>(ak, row, h, tid - NT, rot_s, SWAP ? &rk : nullptr);
+    } else if (tid < NT) {
+        rotate_q_block(aq, bid - rows * n_kv, rot_s);
+    }
 }
 
 // argument checks + EncodeArgs assembly shared by the separate and the fused entry points
@@ -1249,9 +1283,14 @@ int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, in
     RotQArgs aq{ak.plans, (const uint16_t*)q, q_sr, q_sh, (uint16_t*)q_rot, qr_sr, qr_sh, B, n_kv * gqa, gqa, group, q_bf16};
     const int rows = (int)N;
     const unsigned blocks = (unsigned)(2 * rows * n_kv) + (q ? rotate_q_blocks(B, n_kv, gqa, group) : 0u);
-    if (window)
-        hipLaunchKernelGGL(prepare_window_kernel, dim3(blocks + (unsigned)(B * n_kv)), dim3(WINDOW_THREADS), 0, st, ak, av, aq, *window, rows, B * n_kv);
-    else if (ak.bf16 || av.bf16 || (q && q_bf16))
+    if (window) {
+        const WindowArgs& w = *window;
+        const dim3 grid(blocks - (unsigned)(rows * n_kv) + (unsigned)(B * n_kv));
+        const RingArgs rk{w.swap.slot, (uint16_t*)w.kbuf, w.w_sb, w.w_sh, w.w_st, w.W, w.swap.k, w.swap.k_sb, w.swap.k_sh, w.bf16};
+        const RingArgs rv{w.swap.slot, (uint16_t*)w.vbuf, w.w_sb, w.w_sh, w.w_st, w.W, w.swap.v, w.swap.v_sb, w.swap.v_sh, w.bf16};
+        if (w.swap.slot) hipLaunchKernelGGL(prepare_window_kernel<true>, grid, dim3(WINDOW_THREADS), 0, st, ak, av, aq, w, rk, rv, rows, B * n_kv);
+        else hipLaunchKernelGGL(prepare_window_kernel<false>, grid, dim3(WINDOW_THREADS), 0, st, ak, av, aq, w, rk, rv, rows, B * n_kv);
+    } else if (ak.bf16 || av.bf16 || (q && q_bf16))
         hipLaunchKernelGGL(prepare_kernel<true>, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows);
     else
         hipLaunchKernelGGL(prepare_kernel<false>, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows);

@@ -230,3 +230,29 @@ def test_replayed_step_equals_eager_steps(owner):
         assert torch.isfinite(want).all() and want.abs().max() > 0 and torch.equal(out, want), i
         for name in names:
             assert torch.equal(getattr(a, name)[0], getattr(b, name)[0]), (i, name)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("offset", [0, 1])                      # new tokens on 16-byte boundaries, and off them (swapped by a launch of their own)
+def test_buffered_step_slots(dtype, offset):
+    """Slots at both ends of the buffer, behind the visible tokens and outside it (nothing enters, a row of zeros is packed)."""
+    n_q, n_kv, W, B, context = 8, 2, 20, 7, 60
+    w = wl.Workload("t", 1, n_q, n_kv, B, context, 1e6, seq_lens=[context] * B, n_sink=4, window=W - 4, seed=38)
+    mgrs = []
+    for _ in range(2):
+        mgr, energies = wl.build_manager(w, DEV)
+        wl.fill_cache(mgr, w, energies, DEV)
+        mgrs.append(mgr)
+    q, k, v = _inputs(w, energies, context, dtype)
+    if offset:
+        k, v = (torch.cat([torch.zeros_like(t[..., :1]), t], -1).contiguous()[..., 1:] for t in (k, v))
+    i32 = dict(dtype=torch.int32, device=DEV)
+    idx = (torch.arange(B, device=DEV), torch.tensor([0, W - 1, 5, -1, W, 11, 3], **i32), torch.arange(30, 30 + B, **i32),
+           torch.tensor([41, 40, 1, 7, 41, 30, 0], **i32), torch.tensor([W, W, 6, W, W, 9, 1], **i32))
+    mgrs[1]._native = lambda li: mgrs[1]._ensure_storage()
+    for m in mgrs:
+        m._buffered_step_indices = lambda: idx
+    fast, slow = [m.append_and_attend(0, q, k, v) for m in mgrs]
+    assert torch.isfinite(slow).all() and slow.abs().max() > 0 and torch.equal(fast, slow)
+    for name in ("_k_packed", "_k_norms", "_v_packed", "_v_norms", "_buf_k", "_buf_v"):
+        assert torch.equal(getattr(mgrs[0], name)[0], getattr(mgrs[1], name)[0]), name
