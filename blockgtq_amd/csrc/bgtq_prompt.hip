@@ -208,7 +208,7 @@ struct PromptArgs {
     uint16_t* out; int64_t o_sb, o_sh, o_ss;
 };
 
-// LDS of the attention: two staged tiles; two parts of a rotation take their place before and after the walk
+// LDS of four waves' attention: two staged tiles; two parts of a rotation take their place before and after the walk
 constexpr size_t PROMPT_LDS = 2 * TILE;
 static_assert(2 * PART <= PROMPT_LDS, "");
 
@@ -226,7 +226,7 @@ struct RowOf {
 };
 
 // n consecutive rotation parts from the workspace to LDS address dst: each wave its share
-template <int NW>
+template <int NW>                                               // (waves that take part, `wave` counts through them)
 __device__ __forceinline__ void load_parts(const uint8_t* src, int n, int wave, uint32_t voff, uint32_t dst = 0) {
     for (int c = wave; c < n * (PART / 4096); c += NW) dma_full<4>(voff, uniform_ptr(src + c * 4096), dst + (uint32_t)c * 4096);
 }
@@ -289,11 +289,22 @@ __device__ __forceinline__ void finish_rows(const PromptArgs& a, float16v (&O)[4
     }
 }
 
-template <bool BF16, int NW>
-__global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
+// TEAMS 2: two teams of NW waves hold the same rows and walk one half of the partition's tiles each, in LDS of their own;
+// their sums meet in LDS.  That takes the place of two work-groups on a compute unit with a partition each, and of a launch
+// that reads their sums back (33 MB and 14 us for 1000 queries over 4100 records of 8 heads; the attention itself takes longer,
+// since its first and last part wait for the slower team: the call 97.5 -> 96.4 us).
+// Turns: with one barrier a tile the two waves of a SIMD fell into step, both at their exponentials and then both at the value
+// products.  A second barrier after the exponentials, and one team (one half of eight waves) half a tile behind: the same
+// 1000 queries 96.4 -> 94.2 us, 28 heads of 1000 queries 39.1 -> 37.8 (43.2 with partitions and a merge), 4 x 8k prompts
+// 1113 -> 1100 (the clock is down to 1.75 GHz there: the matrix cores are busy 60 % of the cycles).
+constexpr int prompt_ring(int nw) { return nw == 8 ? 4 : 2; }    // tiles in LDS, for each team
+constexpr size_t prompt_lds(int nw, int teams) { return teams * prompt_ring(nw) * TILE + (teams > 1 ? nw * 64 * 8 : 0); }
+template <bool BF16, int NW, int TEAMS>
+__global__ __launch_bounds__(64 * NW * TEAMS, 2) void prompt_attn_kernel(PromptArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), team = TEAMS == 1 ? 0 : wave_all / NW, wave = wave_all - team * NW;
+    const uint32_t lds0 = (uint32_t)team * (uint32_t)PROMPT_LDS;
     const int h = blockIdx.x, b = blockIdx.y;
     // the query block that sees most tokens first, so that the short blocks fill the tail of the launch
     const int nz = (int)gridDim.z - 1 - (int)blockIdx.z, qb = nz / a.n_splits, c = nz - qb * a.n_splits;
@@ -302,18 +313,24 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
     const int s_last = min(row.s0 + a.rows / a.gqa, a.S) - 1;
     const int t_end = a.causal ? min(a.T, a.q_pos_offset + s_last + 1) : a.T;
     const int n_all = (t_end + MT - 1) / MT;
-    const int tile0 = (int)((int64_t)n_all * c / a.n_splits), tile1 = (int)((int64_t)n_all * (c + 1) / a.n_splits);
+    const int parts = a.n_splits * TEAMS, mine = c * TEAMS + team;
+    const int tile0 = (int)((int64_t)n_all * mine / parts), tile1 = (int)((int64_t)n_all * (mine + 1) / parts);
     const int n_full = min(tile1, (a.causal ? min(a.T, a.q_pos_offset + row.s0 + 1) : a.T) / MT);   // tiles before this one are seen whole by every row
     const int lim = !row.ok ? a.T : a.causal ? min(a.T, a.q_pos_offset + row.sq + 1) : a.T;    // tokens t < lim are visible to this row
     const bool live = __builtin_amdgcn_ballot_w64(row.ok) != 0;                              // (a wave without rows only moves data)
+    // the two waves of a SIMD take turns: while one computes scores and exponentials, the other, `late` by half a tile, adds up values.
+    // The half of eight waves that is not late moves the tiles, into the third and fourth place while the late ones read two.
+    constexpr bool TURNS = TEAMS > 1 || NW == 8;
+    constexpr int RING = prompt_ring(NW), MOVERS = TEAMS == 1 && NW == 8 ? NW / 2 : NW;
+    const bool late = TURNS && (TEAMS > 1 ? team == 1 : wave >= NW / 2), mover = MOVERS == NW || !late;
 
     const uint32_t voff = (uint32_t)lane * 16;
     const uint8_t* rot_h = a.rot + (size_t)h * HEAD_PARTS * PART;
-    const uint8_t* tiles = a.tiles + (size_t)(b * a.n_kv + h) * a.n_tiles * TILE + wave * (TILE / 2 / NW);
-    // this wave's share of a tile's K or V fragments; tile t lies in half t & 1 of the LDS
+    const uint8_t* tiles = a.tiles + (size_t)(b * a.n_kv + h) * a.n_tiles * TILE + wave * (TILE / 2 / MOVERS);
+    // this wave's share of a tile's K or V fragments; tile t lies in place t % RING of the LDS
     auto issue = [&](int tile, int part) {
-        constexpr int N = TILE / 2 / NW / 1024;
-        dma_full<N>(voff, uniform_ptr(tiles + (size_t)tile * TILE + part), (uint32_t)(tile & 1) * TILE + part + wave * (TILE / 2 / NW));
+        constexpr int N = TILE / 2 / MOVERS / 1024;
+        if (mover && tile < tile1) dma_full<N>(voff, uniform_ptr(tiles + (size_t)tile * TILE + part), lds0 + (uint32_t)(tile & (RING - 1)) * TILE + part + wave * (TILE / 2 / MOVERS));
     };
     constexpr int K_PART = 0, V_PART = TILE / 2;
 
@@ -323,7 +340,8 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
     if (a.rotate_q) {
         // two parts fit LDS at a time: the remainders first; the head takes the last one's place under the products of the other
         // (1000 fp16 queries over 4100 records of 8 heads: this kernel 74 us with two parts and a denominator from fp16 values, 78 now)
-        load_parts<NW>(rot_h + PART, 2, wave, voff);
+        if (TEAMS == 1) load_parts<NW>(rot_h + PART, 2, wave, voff);
+        else load_parts<NW * TEAMS>(rot_h, 3, wave_all, voff);   // (two teams' room holds all three)
         uint4v qv[8];                                            // lane: dims 16 kk + 8 lg .. + 7 of its query
 #pragma unroll
         for (int kk = 0; kk < 8; kk++) {
@@ -355,15 +373,23 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
                     for (int r = 0; r < 16; r++) R[ob][r] *= 1.f / F16_STEP;
             }
         };
-        if (live) { add_part(PART + voff); step(); }
+        if constexpr (TEAMS == 1) {
+            if (live) { add_part(PART + voff); step(); }
+            __syncthreads();
+            load_parts<NW>(rot_h, 1, wave, voff, PART);
+            if (live) { add_part(voff); step(); }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (live) add_part(PART + voff);
+        } else if (live) {
+            add_part(2 * PART + voff);
+            step();
+            add_part(PART + voff);
+            step();
+            add_part(voff);
+        }
         __syncthreads();
-        load_parts<NW>(rot_h, 1, wave, voff, PART);
-        if (live) { add_part(voff); step(); }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (live) add_part(PART + voff);
-        __syncthreads();
-        if (tile0 < tile1) { issue(tile0, K_PART); issue(tile0, V_PART); }
+        issue(tile0, K_PART); issue(tile0, V_PART);
 #pragma unroll
         for (int ob = 0; ob < 4; ob++)
 #pragma unroll
@@ -377,7 +403,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
             if (row.ok) { x0 = *(const uint2v*)(qrow + 16 * kk + 4 * lg); x1 = *(const uint2v*)(qrow + 16 * kk + 8 + 4 * lg); }
             Qb[kk] = __builtin_bit_cast(half8, (uint4v){x0.x, x0.y, x1.x, x1.y});
         }
-        if (tile0 < tile1) { issue(tile0, K_PART); issue(tile0, V_PART); }
+        issue(tile0, K_PART); issue(tile0, V_PART);
     }
 
     const float c2 = a.scale * 1.44269504088896340736f;        // scores in log2 units
@@ -392,7 +418,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
     // cores are busy 53 % of the time, at 1.9 GHz, and the clock gives way to more.  970 TFLOP/s here, 1290 for the
     // library's bf16 product of 8192 x 8192 matrices on the same card.)
     auto frags = [&](int tile) __attribute__((always_inline)) {
-        uint32_t at = (uint32_t)(tile & 1) * TILE + voff;
+        uint32_t at = lds0 + (uint32_t)(tile & (RING - 1)) * TILE + voff;
         asm("" : "+v"(at));                                      // (fragments at immediate offsets: left alone, every address gets an instruction)
         return at;
     };
@@ -408,12 +434,12 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
                 if (32 * tb + 8 * (r >> 2) + (r & 3) >= rest) S[tb][r] = -INFINITY;
     };
     auto enter = [&](int tile) __attribute__((always_inline)) {
-        if (tile1 - tile0 > 1) {                                 // (a tile alone is complete already)
+        if (TURNS || tile1 - tile0 > 1) {                        // (a tile alone is complete already)
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // this wave's share of V of this tile and K of the next
             __syncthreads();                                     // they are complete; everyone is done with the tile before
         }
-        if (tile + 2 < tile1) issue(tile + 2, K_PART);
-        if (tile + 1 < tile1) issue(tile + 1, V_PART);
+        issue(tile + 2, K_PART);
+        issue(tile + 1, V_PART);
         if (live && __builtin_amdgcn_ballot_w64(mx > m_ref)) {           // wave-uniform, rare after the first tiles
             const float top = fmaxf(mx, __shfl_xor(mx, 32, 64));
             const float m_new = top > m_ref ? top + REFRESH : m_ref;
@@ -424,6 +450,13 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) O[db][r] *= alpha;
             m_ref = m_new;
+        }
+    };
+    auto change_phase = [&]() __attribute__((always_inline)) {
+        if constexpr (TURNS) {
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
     // One straight line of code.  S: scores of this tile, N: those of the next (NEXT: there is one; CUT: it needs the mask)
@@ -463,6 +496,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
         }
         pack(15);
         l_part += l_tile;
+        change_phase();
         // ---- O^T += V^T P^T: 16-token group 2 tb + hf; the maximum of the next scores underneath
         float m = -INFINITY;
 #pragma unroll
@@ -486,7 +520,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
         float16v Sa[2], Sb[2];
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();                                         // the first tile
-        if (tile0 + 1 < tile1) issue(tile0 + 1, K_PART);
+        issue(tile0 + 1, K_PART);
         Sa[0] = Sa[1] = Sb[0] = Sb[1] = (float16v){0};
         if (live) {
             const uint32_t kf = frags(tile0);
@@ -497,27 +531,61 @@ __global__ __launch_bounds__(64 * NW, 2) void prompt_attn_kernel(PromptArgs a) {
             for (int r = 0; r < 16; r++) mx = fmaxf(fmaxf(mx, Sa[0][r]), Sa[1][r]);
             mx *= c2;
         }
+        if (late) change_phase();
         int tile = tile0;
-        while (tile + 2 < n_full) {                              // two tiles a round: the two sets of scores change places
+        if (TURNS && !live) {
+            for (; tile + 1 < tile1; tile++) { enter(tile); change_phase(); }
+        }
+        while ((!TURNS || live) && tile + 2 < n_full) {          // two tiles a round: the two sets of scores change places
             enter(tile);
-            if (live) products(std::true_type{}, std::false_type{}, Sa, Sb, tile);
+            if (TURNS || live) products(std::true_type{}, std::false_type{}, Sa, Sb, tile);
             enter(++tile);
-            if (live) products(std::true_type{}, std::false_type{}, Sb, Sa, tile);
+            if (TURNS || live) products(std::true_type{}, std::false_type{}, Sb, Sa, tile);
             ++tile;
         }
-        for (; tile + 1 < tile1; tile++) {
+        for (; tile + 1 < tile1; tile++) {                       // (a wave without rows is past them)
             enter(tile);
-            if (live) products(std::true_type{}, std::true_type{}, Sa, Sb, tile);
+            if (TURNS || live) products(std::true_type{}, std::true_type{}, Sa, Sb, tile);
             Sa[0] = Sb[0];
             Sa[1] = Sb[1];
         }
         enter(tile);
         if (live) products(std::false_type{}, std::false_type{}, Sa, Sb, tile);
+        else change_phase();
+        if (TURNS && !late) change_phase();
     }
 
-    const float l_tot = l_part + __shfl_xor(l_part, 32, 64);
+    float l_tot = l_part + __shfl_xor(l_part, 32, 64);
+    if constexpr (TEAMS > 1) {
+        static_assert(TEAMS == 2 && NW * 64 * 64 * 4 <= PROMPT_LDS, "a team's sums fit its tiles");
+        // both teams meet as many barriers as the longer walk has (two a tile, and two)
+        const int n = tile1 - tile0, longest = (n_all + parts - 1) / parts;
+        for (int i = n > 0 ? 2 * n + 2 : 0; i < 2 * longest + 2; i++) __syncthreads();
+        __syncthreads();                                         // every wave is done with the tiles
+        // the second team's sums in the place of its tiles, [wave][register][lane], (reference, denominator) behind both teams'
+        float* sums = (float*)(smem + PROMPT_LDS) + wave * 64 * 64 + lane;
+        float2* ml = (float2*)(smem + 2 * PROMPT_LDS) + wave * 64 + lane;
+        if (team == 1) {
+#pragma unroll
+            for (int r = 0; r < 64; r++) sums[r * 64] = O[r >> 4][r & 15];
+            *ml = float2{m_ref, l_tot};
+        }
+        if (a.n_splits == 1 && a.unrotate) {                     // ... the un-rotation in the place of the first team's
+            load_parts<NW * TEAMS>(rot_h + Q_PARTS * PART, 2, wave_all, voff);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        __syncthreads();
+        if (team == 1) return;
+        const float2 y = *ml;
+        const float m = fmaxf(m_ref, y.x);
+        const float f0 = m_ref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_ref - m), f1 = y.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(y.x - m);
+        l_tot = fmaf(f1, y.y, f0 * l_tot);
+#pragma unroll
+        for (int r = 0; r < 64; r++) O[r >> 4][r & 15] = fmaf(f1, sums[r * 64], f0 * O[r >> 4][r & 15]);
+        m_ref = m;
+    }
     if (a.n_splits == 1) {
-        if (a.unrotate) {
+        if (TEAMS == 1 && a.unrotate) {
             __syncthreads();                                     // every wave is done with the tiles
             load_parts<NW>(rot_h + Q_PARTS * PART, 2, wave, voff);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -601,11 +669,14 @@ __global__ __launch_bounds__(64 * merge_waves(PER)) void prompt_merge_kernel(Pro
 }
 
 // Rows of a work-group.  256 (one work-group a compute unit) fetch every tile for twice as many rows, which counts
-// where the chip is full and limited by power: 8k prompts 5 % faster.  128 (two a compute unit, no barrier between
-// their waves) fill the chip with half the rows and end with shorter tails: 1k to 2k prompts 5 to 20 % faster.
+// where the chip is full and limited by power: 8k prompts 5 % faster.  128 (two a compute unit) fill the chip with half the rows and end with shorter tails: 1k to 2k prompts 5 to 20 % faster.
 int prompt_rows(int B, int n_kv, int gqa, int S) {
     return gqa > MAX_GQA_ROWS || (int64_t)B * n_kv * gqa * S >= (int64_t)PROMPT_BIG * 256 ? 256 : 128;
 }
+// Two teams to a work-group where that deals the tiles into as many parts as work-groups of one team would: 128 rows, and
+// twice the partitions that fill the compute units once.  (With an odd number, say 3 partitions of 160 blocks, teams would
+// leave compute units idle that the partitions use; where a short context makes fewer, each partition has one to itself.)
+int prompt_teams(int64_t wgs, int rows, int ns) { return rows == 128 && ns >= 2 && ns == 2 * (256 / wgs) ? 2 : 1; }
 // Tiles of one query block dealt to several work-groups where the blocks alone leave compute units idle, four
 // tiles or more each (below that set-up and merge cost more than the walk)
 int prompt_splits(int B, int n_kv, int gqa, int S, int T) {
@@ -623,9 +694,9 @@ extern "C" {
 size_t bgtq_prompt_workspace_bytes(int B, int n_kv, int gqa, int S, int T) {
     if (B <= 0 || n_kv <= 0 || gqa <= 0 || gqa > 256 || S <= 0 || T <= 0) return 0;
     const int ns = prompt_splits(B, n_kv, gqa, S, T), rows = prompt_rows(B, n_kv, gqa, S), BQ = rows / gqa;
-    const size_t wgs = (size_t)B * n_kv * ((S + BQ - 1) / BQ) * ns;
+    const size_t blocks = (size_t)B * n_kv * ((S + BQ - 1) / BQ), ng = ns / prompt_teams((int64_t)blocks, rows, ns);
     return (size_t)n_kv * HEAD_PARTS * PART + (size_t)B * n_kv * ((T + MT - 1) / MT) * TILE +
-           (ns > 1 ? wgs * (rows / 32) * (64 * 64 + 64) * sizeof(float) : 0);
+           (ng > 1 ? blocks * ns * (rows / 32) * (64 * 64 + 64) * sizeof(float) : 0);   // (ns: never less than fewer records need)
 }
 
 int bgtq_prompt_attn(const bgtq_head_plan* plans,
@@ -659,7 +730,8 @@ int bgtq_prompt_attn(const bgtq_head_plan* plans,
     BGTQ_CHECK_ARG(workspace && ((uintptr_t)workspace & 15) == 0);
     if (is_causal) T = (int)std::min<int64_t>(T, (int64_t)q_pos_offset + S);                               // no row sees a record past the last query's position
     if (workspace_bytes < bgtq_prompt_workspace_bytes(B, n_kv, gqa, S, T)) return BGTQ_EINVAL;
-    const int rows = prompt_rows(B, n_kv, gqa, S), BQ = rows / gqa, n_qb = (S + BQ - 1) / BQ, ns = prompt_splits(B, n_kv, gqa, S, T);
+    const int rows = prompt_rows(B, n_kv, gqa, S), BQ = rows / gqa, n_qb = (S + BQ - 1) / BQ, all_parts = prompt_splits(B, n_kv, gqa, S, T);
+    const int teams = prompt_teams((int64_t)B * n_kv * n_qb, rows, all_parts), ns = all_parts / teams;
     // a grid dimension holds 65535 query blocks (the bound of bgtq_prefill_attn: blocks of fewer rows are only taken below
     // 2^19 rows); with partitions there are at most 256 blocks, and as many groups of 32 rows as the merge's grid takes
     if (n_qb > 65535 || B > 65535) return BGTQ_EUNSUPPORTED;
@@ -667,8 +739,9 @@ int bgtq_prompt_attn(const bgtq_head_plan* plans,
     if (ready.load(std::memory_order_acquire) == 0) {
         // offsets into the dynamic LDS block are used as LDS addresses: holds only without static LDS
         int ok = 1;
-        for (const void* f : {(const void*)prompt_stage_kernel, (const void*)prompt_attn_kernel<false, 4>, (const void*)prompt_attn_kernel<true, 4>,
-                              (const void*)prompt_attn_kernel<false, 8>, (const void*)prompt_attn_kernel<true, 8>,
+        for (const void* f : {(const void*)prompt_stage_kernel, (const void*)prompt_attn_kernel<false, 4, 1>, (const void*)prompt_attn_kernel<true, 4, 1>,
+                              (const void*)prompt_attn_kernel<false, 4, 2>, (const void*)prompt_attn_kernel<true, 4, 2>,
+                              (const void*)prompt_attn_kernel<false, 8, 1>, (const void*)prompt_attn_kernel<true, 8, 1>,
                               (const void*)prompt_merge_kernel<1>, (const void*)prompt_merge_kernel<8>}) {
             hipFuncAttributes fa;
             hipError_t e = hipFuncGetAttributes(&fa, f);
@@ -708,9 +781,9 @@ int bgtq_prompt_attn(const bgtq_head_plan* plans,
     const int wgs_per = (g.n_tiles + g.per_wg - 1) / g.per_wg;
     hipLaunchKernelGGL(prompt_stage_kernel, dim3((unsigned)(n_kv * ROT_WGS + wgs_per * B * n_kv)), dim3(DQ_THR), (size_t)RAW_OFF + raw + DQ_TILE_BYTES, st, g);
     const dim3 grid((unsigned)n_kv, (unsigned)B, (unsigned)(n_qb * ns));
-    auto attn = g.bf16 ? (rows == 256 ? prompt_attn_kernel<true, 8> : prompt_attn_kernel<true, 4>)
-                       : (rows == 256 ? prompt_attn_kernel<false, 8> : prompt_attn_kernel<false, 4>);
-    hipLaunchKernelGGL(attn, grid, dim3(2 * rows), PROMPT_LDS, st, a);
+    auto attn = g.bf16 ? (rows == 256 ? prompt_attn_kernel<true, 8, 1> : teams == 2 ? prompt_attn_kernel<true, 4, 2> : prompt_attn_kernel<true, 4, 1>)
+                       : (rows == 256 ? prompt_attn_kernel<false, 8, 1> : teams == 2 ? prompt_attn_kernel<false, 4, 2> : prompt_attn_kernel<false, 4, 1>);
+    hipLaunchKernelGGL(attn, grid, dim3(2 * rows * teams), prompt_lds(rows / 32, teams), st, a);
     if (ns > 1) {
         const int groups = n_qb * (rows / 32);
         if ((int64_t)B * n_kv * groups > 256)

@@ -108,6 +108,13 @@ def test_wide_query_groups_over_a_split_context(gqa, S, T, off):
     test_prompt_attention_equals_the_kernel_without_workspace(1, 1, gqa, S, T, off, P.K_MIXED, P.V_NIBBLE, (2.5, 2, 0, 8), torch.float16)
 
 
+# work-groups of two teams: an early block whose first team has no tile, a ragged end, teams that still leave partitions to merge
+@pytest.mark.parametrize("n_kv,gqa,S,T,off", [(8, 4, 800, 800, 0), (8, 3, 1000, 1801, 777), (4, 4, 1000, 1027, 27)])
+def test_two_teams_over_one_block_of_rows(n_kv, gqa, S, T, off):
+    test_prompt_attention_equals_the_kernel_without_workspace(1, n_kv, gqa, S, T, off, P.K_MIXED, P.V_NIBBLE, (2.5, 2, 0, 8), torch.float16)
+    test_prompt_attention_equals_the_kernel_without_workspace(1, n_kv, gqa, S, T, off, P.K_BITPACKED, P.V_BITPACKED, (3.0, 3, 1, 5), torch.bfloat16)
+
+
 def test_small_probabilities_count_in_the_denominator():
     """Each query has one strong record among the first and 65 535 weak ones, e^-18 of it apiece and below the smallest fp16
     number once the reference lies 4 octaves above the strong score; together they are 4e-3 of the denominator.
