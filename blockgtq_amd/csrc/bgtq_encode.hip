@@ -431,14 +431,13 @@ __global__ __launch_bounds__(NT) void encode_kernel(EncodeArgs a) {
 //
 // A block stays in one wave from the raw rows to the codes: lane (li, lg) of 16 x 4 holds dims k = 4 kk + lg
 // of row li in 32 registers, which is the A operand of step kk as it is.
-//   norms    V, and K where waves have blocks of their own: X X^T, A and B are the same registers, the diagonal holds
-//            the 16 sums of squares (15 of 16 products are thrown away, but no lane waits for another's chain: lane =
-//            row chains of V left 48 lanes idle and took as long as the rotation); K else: lane = (row, one of four groups)
+//   norms    lane = row for V, (row, one of four groups) for K: chains of mixed multiply-adds on the raw fp16 values,
+//            one instruction a dim (V in the diagonal of X X^T: 32 matrix instructions, 1024 clocks, here 128 of 2.5)
 //   xhat     x / norm from the norm's rounded reciprocal, in registers (div_by below)
 //   rotate   16 columns at a time against the rotation in LDS, stored in operand order (one 16-byte read a lane
 //            feeds four steps, no bank conflicts); K takes only the steps its columns' segments reach
 //   codes    four rows of one column per lane, straight from the accumulator
-//   corrected norms  the centroids of the codes: V once more X X^T, K lane = (row, group): its chains of 16 dims with
+//   corrected norms  the centroids of the codes: V the diagonal of X X^T, K lane = (row, group): its chains of 16 dims with
 //            a dependent code, centroid and product read each took 17 k of a block's 64 k clocks, these take 7 k
 //   packing  a lane makes four bytes of a record: a byte is a dot product of four code bytes with powers of two
 //
@@ -446,12 +445,14 @@ __global__ __launch_bounds__(NT) void encode_kernel(EncodeArgs a) {
 // share a rotation, each walks blocks of its own and no barrier is met on the way.  CS 2 (at most 8 blocks a
 // work-group): as many waves a compute unit again where CS 1 would leave half of it empty.  CS 4 (few rows): a
 // work-group of 4 waves a block, two of them a compute unit.
-// CS 1 is bound by the matrix cores and vector issue in turn: 320 instructions of 32 clocks a V block.  65 536 records
-// each of K and V (4 x 8192 tokens, 2 heads, K3V3): 135 us as two launches of 16-row tiles on the vector units (there the
-// dense V rotation alone is 55 us of FMA), 61 us here in one.  CS 2 and CS 4 are bound by one block's chain; 8 heads,
+// CS 1 is bound by the matrix cores and vector issue in turn: an fp32 matrix instruction keeps its SIMD's vector unit busy
+// for its whole 32 clocks (two waves, one of either kind: the sum of both times), and a V block has 288 of them.  65 536
+// records each of K and V (4 x 8192 tokens, 2 heads, K3V3): 135 us as two launches of 16-row tiles on the vector units (there
+// the dense V rotation alone is 55 us of FMA), 61 us in one with norms as diagonals, a compare and an add for every
+// boundary of a V cell and quotients of two residual steps, 56 with what is here, 53 with the priorities below.  CS 2 and CS 4 are bound by one block's chain; 8 heads,
 // nibble records, against groups one after the other in K's norms and CS 1 from 513 blocks on: 128 tokens 18.3 -> 13.1 us,
-// 600 26.7 -> 18.8, 2001 30.4 -> 26.1, 9000 (CS 1) 89.6 -> 78.8; bit-packed records (no corrected K norms) 12.4 -> 11.4,
-// 20.6 -> 16.4, 23.9 -> 23.4, 70.1 -> 70.4.
+// 600 26.7 -> 18.2, 2001 30.4 -> 24.2, 9000 (CS 1) 89.6 -> 68.9; bit-packed records (no corrected K norms) 12.4 -> 11.4,
+// 20.6 -> 15.8, 23.9 -> 21.8, 70.1 -> 61.3.
 // ================================================================================================
 constexpr int RROW = D * 2 + 16;        // bytes from one raw row to the next: rows 4 banks apart
 constexpr int CROW = D + 8;             // bytes from one row of codes to the next (a byte's window of codes may reach 8 past the last)
@@ -475,12 +476,11 @@ struct EncodeLds {
     alignas(16) uint16_t place[D];      // source dim -> byte offset in a raw row
 };
 
-// x / d correctly rounded from y = RN(1 / d) (Markstein: a quotient within one unit in the last place and a
-// correctly rounded reciprocal give the rounded quotient after one residual step; the first step brings x * y
-// within that unit).  For finite x, and d and y normal.
+// x / d correctly rounded from y = RN(1 / d), for x a finite fp16 value, and d and y normal (Markstein: a quotient within one
+// unit in the last place and a correctly rounded reciprocal give the rounded quotient after one residual step.  x * y can be
+// 1.5 units off, but no quotient of an 11-bit x lies near enough to a midpoint: all 2^10 x 2^23 mantissas were compared.)
 __device__ __forceinline__ float div_by(float x, float2 dy) {
-    float q = x * dy.y;
-    q = __builtin_fmaf(__builtin_fmaf(-dy.x, q, x), dy.y, q);
+    const float q = x * dy.y;
     return __builtin_fmaf(__builtin_fmaf(-dy.x, q, x), dy.y, q);
 }
 
@@ -574,6 +574,10 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
     // sake - rows past the last are zeros and stored nowhere)
     for (int round = first * NB; CS == 1 ? round + slot < n_blocks : round < n_blocks; round += stride * NB) {
         const int blk = round + slot;
+        // The oldest wave of a SIMD would run ahead, and the youngest end alone with a matrix core that it fills by half
+        // (56 -> 53 us at 65 536 records): waves that are behind go first, by blocks left and by halves of a block.
+        const bool more = round + stride * NB + slot < n_blocks;
+        if (CS == 1) { if (more) __builtin_amdgcn_s_setprio(3); else __builtin_amdgcn_s_setprio(1); }
         const unsigned n0 = (unsigned)blk * 16u;
         const int b0 = (int)(n0 / (unsigned)a.S), s0 = (int)(n0 - (unsigned)b0 * (unsigned)a.S);
         auto row_of = [&](int r, int& b, int& s) {            // (batch row, step) of the block's row r
@@ -650,46 +654,26 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
 #pragma unroll
             for (int i = 0; i < 8; i++) A[8 * q + i] = (float)v[i];
         };
-        if constexpr (IS_V) {
-#pragma unroll
-            for (int q = 0; q < D / 32; q++) load_a(q);
-        }
-        // ---- norms: the diagonal of X X^T; lane (li, lg) holds (row 4 lg + r, row li) in register r
+        // ---- norms
         bool finite = true;
-        const bool diag = (li >> 2) == lg;
+        const bool diag = (li >> 2) == lg;                    // lane (li, lg) holds (row 4 lg + r, row li) of X X^T in register r
         auto diagonal = [&](const float4v& sum) { return li & 2 ? (li & 1 ? sum[3] : sum[2]) : (li & 1 ? sum[1] : sum[0]); };
+        float2 v_nrm = {0.f, 0.f};                            // V: of row li
         if constexpr (IS_V) {
-            if (CS != 2 || part == 0) {                       // (CS 4: a barrier takes longer than the same products in every wave)
-                float4v sum = {0, 0, 0, 0};
+            float sum = 0.f;
 #pragma unroll
-                for (int kk = 0; kk < D / 4; kk++) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(A[kk], A[kk], sum, 0, 0, 0);
-                const float n = __builtin_sqrtf(diagonal(sum) + 1e-30f);
-                if (diag) L.nrm[slot][0][li] = float2{n, 1.0f / n};
-            }
-            if (CS == 2) __syncthreads();
-        } else if constexpr (CS == 1) {                       // (the matrix cores have room beside K's other work)
-            for (int g = 0; g < n_seg; g++) {
-                const int s = L.hdr[H_START + g], e = s + L.hdr[H_LEN + g];
-                float4v sum = {0, 0, 0, 0};
-                for (int q = s >> 4; q < (e + 15) >> 4; q++) {
-                    const uint2 w = *(const uint2*)(arow + 8 * q);
+            for (int q = 0; q < D / 32; q++) {
+                half8 v[4];
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int k = 16 * q + 4 * i + lg;
-                        const float x = k >= s && k < e ? bgtq_h2f((uint16_t)((i < 2 ? w.x : w.y) >> (16 * (i & 1)))) : 0.f;
-                        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(x, x, sum, 0, 0, 0);
-                    }
-                }
-                if (diag) L.nrm[slot][g][li].x = diagonal(sum);
+                for (int c = 0; c < 4; c++) v[c] = *(const half8*)(raw + li * RROW + c * (D / 2) + 16 * q);
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+#pragma unroll
+                    for (int c = 0; c < 4; c++) sum = __builtin_fmaf((float)v[c][i], (float)v[c][i], sum);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            // roots and reciprocals of all groups together: four groups of 16 rows an instruction
-            asm volatile("" ::: "memory");                    // (a wave's LDS accesses keep their order)
-            for (int i = lane; (i >> 4) < n_seg; i += 64) {
-                float2* at = &L.nrm[slot][i >> 4][i & 15];
-                const float n = __builtin_sqrtf(at->x + 1e-30f);
-                finite = finite && n < INFINITY;
-                *at = float2{n, 1.0f / n};
-            }
+            const float n = __builtin_sqrtf(sum + 1e-30f);
+            v_nrm = float2{n, 1.0f / n};
         } else {
             // lane = (row li, group 4 p + lg): 64 chains side by side, over the blocks of 16 dims that the group touches
             for (int p = part; 4 * p < n_seg; p += CS) {
@@ -710,11 +694,19 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
                     at += 8;
                     fetch();
                     const uint32_t live = hi > 0 ? (0xFFFFu >> (16 - min(hi, 16))) & (0xFFFFu << lo) : 0u;
+                    // (dims of other groups become zeros, two at a time)
+                    auto dim_bits = [&](int i) { return (uint32_t)((int32_t)(live << (31 - i)) >> 31); };
+                    if (__builtin_amdgcn_ballot_w64(live != 0xFFFFu) != 0) {          // (uniform)
+#pragma unroll
+                        for (int c = 0; c < 4; c++) {
+                            v[c].x &= __builtin_amdgcn_perm(dim_bits(c + 4), dim_bits(c), 0x05040100u);
+                            v[c].y &= __builtin_amdgcn_perm(dim_bits(c + 12), dim_bits(c + 8), 0x05040100u);
+                        }
+                    }
 #pragma unroll
                     for (int i = 0; i < 16; i++) {
-                        const uint32_t d = i & 8 ? v[i & 3].y : v[i & 3].x;
-                        const uint32_t half = (d >> (i & 4 ? 16 : 0)) & (uint32_t)((int32_t)(live << (31 - i)) >> 31);
-                        const float x = bgtq_h2f((uint16_t)half);
+                        const half2v d = __builtin_bit_cast(half2v, i & 8 ? v[i & 3].y : v[i & 3].x);
+                        const float x = (float)d[(i >> 2) & 1];
                         sum = __builtin_fmaf(x, x, sum);
                     }
                     lo = 0;
@@ -728,15 +720,18 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
             }
         }
         bool scalar_chain = !IS_V && __builtin_amdgcn_ballot_w64(!finite) != 0;           // (uniform)
-        if (CS == 1 || IS_V) asm volatile("" ::: "memory");   // (V: every wave of a work-group has written the same norms)
+        if (CS == 1 || IS_V) asm volatile("" ::: "memory");
         else scalar_chain = __syncthreads_or(scalar_chain) != 0;
         // ---- xhat.  (The contract divides by 1 where the norm is at most 1e-10, for V 1e-8: a non-zero fp16 value alone
         // makes it 6e-8, so those norms belong to rows of zeros, which stay zeros whatever they are divided by.  An
         // infinite or NaN norm of V makes every value of its row NaN, as the dense rotation would.)
         if constexpr (IS_V) {
-            const float2 dy = L.nrm[slot][0][li];
 #pragma unroll
-            for (int kk = 0; kk < D / 4; kk++) A[kk] = div_by(A[kk], dy);
+            for (int q = 0; q < D / 32; q++) {
+                load_a(q);
+#pragma unroll
+                for (int i = 0; i < 8; i++) A[8 * q + i] = div_by(A[8 * q + i], v_nrm);
+            }
         } else {
 #pragma unroll
             for (int q = 0; q < D / 32; q++) {
@@ -802,10 +797,10 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         // ---- rotate and quantise 16 columns at a time; codes of rows 4 lg .. + 3, column 16 cb + li
         uint32_t codes[D / 16 / CS];
         // V: the cell search of 16 columns (the number of boundaries below a value) goes under the next 16 columns' products:
-        // behind its own, all waves of a SIMD would come to it together and leave the matrix core alone.  Operands are read
-        // eight steps ahead.
+        // behind its own, all waves of a SIMD would come to it together and leave the matrix core alone.  3 compares, 4 selects
+        // and 3 additions with carry for a value of 3 bits (7 and 7 before).  Operands are read eight steps ahead.
         auto columns = [&](auto bits) {
-            constexpr int NB = (1 << decltype(bits)::value) - 1, EVERY = 32 / (NB + 1), NC = D / 16 / CS;
+            constexpr int BITS = decltype(bits)::value, NC = D / 16 / CS;
             const float* rot = &L.rot[0][16 * part * NC + li][lg];
             float R[2][8];
             auto fetch = [&](int at) {                        // eight steps: columns at / 4, steps 8 (at % 4) ..
@@ -813,8 +808,23 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
                 for (int i = 0; i < 8; i++) R[at & 1][i] = rot[(at >> 2) * 64 + (8 * (at & 3) + i) * 4 * D];
             };
             fetch(0);
+            // number of boundaries below x, its bits from the highest down, under the bits of `below`
+            auto search = [&](float x, uint32_t below) {
+                float cand[(1 << BITS) - 1];                  // in-order: the boundaries still in question
+#pragma unroll
+                for (int b = 0; b < (1 << BITS) - 1; b++) cand[b] = bd[b];
+#pragma unroll
+                for (int n = (1 << BITS) - 1; n >= 1; n >>= 1) {
+                    const bool up = x > cand[n >> 1];
+                    const uint64_t carry = __builtin_amdgcn_ballot_w64(up);
+                    asm("v_addc_co_u32 %0, vcc, %1, %1, %2" : "=v"(below) : "v"(below), "s"(carry) : "vcc");
+#pragma unroll
+                    for (int b = 0; b < n >> 1; b++) cand[b] = up ? cand[b + (n >> 1) + 1] : cand[b];
+                }
+                return below;
+            };
             float4v y = {0, 0, 0, 0}, before = {0, 0, 0, 0};
-            uint32_t cell[4] = {0, 0, 0, 0};
+            uint32_t cell = 0;
 #pragma unroll
             for (int at = 0; at < 4 * NC; at++) {
                 if (at + 1 < 4 * NC) fetch(at + 1);
@@ -826,21 +836,14 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
                 for (int i = 0; i < 8; i++) {
                     const int kk = 8 * (at & 3) + i;
                     y = __builtin_amdgcn_mfma_f32_16x16x4f32(A[kk], R[at & 1][i], y, 0, 0, 0);
-                    if (at >= 4 && kk % EVERY == 0 && kk / EVERY < NB) {
-#pragma unroll
-                        for (int r = 0; r < 4; r++) cell[r] = (kk ? cell[r] : 0u) + (before[r] > bd[kk / EVERY] ? 1u : 0u);
-                    }
+                    if (at >= 4 && i == 0) cell = search(before[3 - (at & 3)], cell << (8 - BITS));
                 }
-                if (at >= 4 && (at & 3) == 3) codes[(at >> 2) - 1] = cell[0] | (cell[1] << 8) | (cell[2] << 16) | (cell[3] << 24);
+                if (at >= 4 && (at & 3) == 3) codes[(at >> 2) - 1] = cell;
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                cell[r] = 0;
-#pragma unroll
-                for (int b = 0; b < NB; b++) cell[r] += y[r] > bd[b] ? 1u : 0u;
-            }
-            codes[NC - 1] = cell[0] | (cell[1] << 8) | (cell[2] << 16) | (cell[3] << 24);
+            for (int r = 3; r >= 0; r--) cell = search(y[r], cell << (8 - BITS));
+            codes[NC - 1] = cell;
         };
         if constexpr (IS_V) {
             if (v_bits == 3) columns(std::integral_constant<int, 3>{});         // (uniform)
@@ -878,6 +881,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
             for (int r = 0; r < 4; r++)
                 raw[(4 * lg + r) * CROW + 16 * (part * (D / 16 / CS) + c) + li] = (uint8_t)(codes[c] >> (8 * r));
         meet();
+        if (CS == 1) { if (more) __builtin_amdgcn_s_setprio(2); else __builtin_amdgcn_s_setprio(0); }
         // ---- norms to store
         auto store_norm = [&](int g, int row, float out) {
             const int64_t nd = L.ndst[slot][row];
@@ -902,7 +906,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
                         for (int i = 0; i < D / 8; i++) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(cen[i], cen[i], sum, 0, 0, 0);
                     }
                     const float cn = __builtin_sqrtf(diagonal(sum) + 1e-20f);
-                    if (diag) store_norm(0, li, L.nrm[slot][0][li].x / (cn > 1e-10f ? cn : 1.0f));
+                    if (diag) store_norm(0, li, v_nrm.x / (cn > 1e-10f ? cn : 1.0f));
                 }
                 if constexpr (!IS_V) {                        // the centroids' chains, lane = (row, group) as above
 #pragma unroll 1

@@ -120,6 +120,20 @@ def test_blocks_by_waves_per_block(S, bits, kl, vl):
     _same(got, want)
 
 
+@pytest.mark.parametrize("S", [100, 1100, 4100])
+def test_blocks_over_the_whole_fp16_range(S):
+    """Rows of any finite fp16 values, of few of the largest, of subnormals only and of zeros, as blocks and one by one."""
+    args = _plans(8, (3.0, 3, 0, 8), seed=48)
+    gen = torch.Generator(device=DEV).manual_seed(S)
+    x = torch.randint(0, 0x7C00, (1, 8, S, 128), generator=gen, device=DEV, dtype=torch.int16)
+    x[:, :, 1::5] &= 0x3FF                                     # subnormals
+    x[:, :, 2::5] *= (torch.rand(1, 8, len(range(2, S, 5)), 128, generator=gen, device=DEV) < 0.05)
+    x[:, :, 3::5] = 0
+    x[:, :, 4::5] = x[:, :, 4::5] // 8 + 0x3000                # of one size
+    x = torch.where(torch.rand(x.shape, generator=gen, device=DEV) < 0.5, x, x | -0x8000).view(torch.float16)
+    _same(_encode(args, x, P.K_MIXED, P.V_NIBBLE, P.QUANT_LUT256, S + 9), _encode(args, x, P.K_MIXED, P.V_NIBBLE, P.QUANT_LUT256, S + 9, 32))
+
+
 def test_segment_tables_of_the_block_encoder():
     """`rot_span` covers the rows that 16 columns' segments reach, the segment nibbles repeat `group_of`."""
     for bits in ((3.0, 3, 1, 8), (2.0, 2, 0, 4), (1.0, 1, 0, 3)):
