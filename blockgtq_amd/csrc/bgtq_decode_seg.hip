@@ -395,10 +395,12 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a
         const int nt = min(MT, t1 - tile);
         int n_loads;
         if (nt == MT) {
-            dma_chunks(voff_k, k_al, kbuf, full_k.nfull);
-            if (full_kn.nfull) dma_chunks(voff_kn, kn_al, knbuf, full_kn.nfull);
+            int nk = full_k.nfull, nn = full_kn.nfull;
+            asm volatile("" : "+s"(nk), "+s"(nn));           // (the branches on them would be worked out ahead of the loop, and kept in lanes)
+            dma_chunks(voff_k, k_al, kbuf, nk);
+            if (nn) dma_chunks(voff_kn, kn_al, knbuf, nn);
             dma_tails(voff_k, tail_k, voff_kn, tail_kn, voff_vn, tail_vn);
-            n_loads = full_k.nfull + full_kn.nfull + 3;
+            n_loads = nk + nn + 3;
         } else {
             const DmaShape sk = dma_shape_uniform((int)kph + nt * krow), sn = dma_shape_uniform((int)knph + nt * kn_st * 2);
             const DmaShape sv = dma_shape_uniform((int)vnph + nt * 2);
@@ -416,9 +418,11 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a
         const int nt = min(MT, t1 - tile);
         int n_loads;
         if (nt == MT) {
-            dma_chunks(voff_v, v_al, vbuf, full_v.nfull);
+            int nv = full_v.nfull;
+            asm volatile("" : "+s"(nv));
+            dma_chunks(voff_v, v_al, vbuf, nv);
             dma_tail(voff_v, tail_v);
-            n_loads = full_v.nfull + 1;
+            n_loads = nv + 1;
         } else {
             const DmaShape sv = dma_shape_uniform((int)vph + nt * vrow);
             dma_chunks(voff_v, v_al, vbuf, sv.nfull);
@@ -474,6 +478,45 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a
     if (tile < t1) k_loads = issue_k(tile);
     bool fresh = true;                                     // (the wave has no sums yet)
 
+    // ---- what the walk needs of a lane, worked out here, while the loads are on their way (the compiler would do all of it
+    // behind the barrier: 150 instructions of a lone wave, 1.1k clocks of each work-group; 45 are left.  32 ragged rows of 8
+    // heads with a window 220.8 -> 214.9 us, 12 ragged rows of 7-head groups 91.1 -> 89.6, one row of 4k 68.1 -> 67.2)
+    float c2 = a.scale * 1.44269504088896340736f;      // scores are kept in log2 units
+    uint32_t rep = ((uint32_t)lane & 31u) * 4u;          // this lane's replica of the 32-fold tables
+    // QK^T operands: this lane's record and norm row, its A rows (a head's struct or the zero struct)
+    uint32_t krow_l = kbuf + kph + (uint32_t)lane * krow;
+    uint32_t knrow_l = kbuf + tl.kt + knph + (uint32_t)lane * kn_st * 2;
+    uint32_t vn_l = kbuf + tl.kt + tl.knr + vnph + (uint32_t)lane * 2;
+    const int q_head = ScoreAcc<HEADS>::head_of_lane(lane);
+    uint32_t qs_l = QS_OFF + (q_head >= 0 ? q_head : HEADS) * QSTRUCT;
+    // PV operands: V table replica (the table sits at LDS address 0, so field bits OR-ed in never meet the
+    // base; the 256-entry tables are not replicated), raw codes, P rows
+    // V table replica (the table sits at LDS address 0, so field bits OR-ed in never meet the base; the
+    // 256-entry tables are not replicated)
+    constexpr bool V_UNREP = VBW == 4;                        // also every nibble record (VBW 4 by construction)
+    constexpr int VWIN = V_UNREP ? 0 : 8;                     // replicated tables: codes fetched with the byte in front of them
+    uint32_t vbank = V_UNREP ? 0u : rep;
+    constexpr int vshift = V_UNREP ? 2 : 7;
+    const int vc = (int)vph + li * VBW - (V_UNREP ? 0 : 1);
+    uint32_t vbase = vbuf + (uint32_t)(vc & ~3) + (uint32_t)lg * 4 * vrow, v_sh = (uint32_t)vc & 3u;
+    uint32_t p_wr = pbuf + (uint32_t)lane * 4;                                   // + head pair * PROW
+    uint32_t p_rd = pbuf + (uint32_t)((li & 7) >> 1) * PROW + (uint32_t)lg * 16;   // + block * 64
+    // A row (head h = li & 7, dim parity e = li >> 3) takes its head's half of the P dword into the half of
+    // parity e and zero into the other: a byte permute per dword
+    uint32_t p_sel = (li & 8) ? ((li & 1) ? 0x03020C0Cu : 0x01000C0Cu) : ((li & 1) ? 0x0C0C0302u : 0x0C0C0100u);
+
+    float m_ref[8], l_part[8];      // per head: reference in log2 units (never below a score seen), this lane's share of the denominator
+#pragma unroll
+    for (int hh = 0; hh < 8; hh++) { m_ref[hh] = -INFINITY; l_part[hh] = 0.f; }
+    float4v acc[4];                 // acc[jb][r] = out[head 4(lg & 1) + r][dim 8 li + 2 jb + (lg >> 1)]
+#pragma unroll
+    for (int e = 0; e < 4; e++) acc[e] = (float4v){0, 0, 0, 0};
+    asm volatile("" : "+v"(rep), "+v"(krow_l), "+v"(knrow_l), "+v"(vn_l), "+v"(qs_l), "+v"(vbase), "+v"(v_sh), "+v"(p_wr), "+v"(p_rd), "+v"(p_sel), "+v"(c2));
+#pragma unroll
+    for (int hh = 0; hh < 8; hh++) asm volatile("" : "+v"(m_ref[hh]), "+v"(l_part[hh]));
+#pragma unroll
+    for (int e = 0; e < 4; e++) asm volatile("" : "+v"(acc[e]));
+
     // ---- the set-up slots.  The wait covers the walk words, the wave's table chunks and query words
     wait_loads(k_loads);
     asm volatile("" : "+v"(seg_w) :: "memory");
@@ -498,37 +541,6 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a
         }
     __syncthreads();
 
-    const float c2 = a.scale * 1.44269504088896340736f;      // scores are kept in log2 units
-    const uint32_t rep = ((uint32_t)lane & 31u) * 4u;          // this lane's replica of the 32-fold tables
-    // QK^T operands: this lane's record and norm row, its A rows (a head's struct or the zero struct)
-    const uint32_t krow_l = kbuf + kph + (uint32_t)lane * krow;
-    const uint32_t knrow_l = kbuf + tl.kt + knph + (uint32_t)lane * kn_st * 2;
-    const uint32_t vn_l = kbuf + tl.kt + tl.knr + vnph + (uint32_t)lane * 2;
-    const int q_head = ScoreAcc<HEADS>::head_of_lane(lane);
-    const uint32_t qs_l = QS_OFF + (q_head >= 0 ? q_head : HEADS) * QSTRUCT;
-    // PV operands: V table replica (the table sits at LDS address 0, so field bits OR-ed in never meet the
-    // base; the 256-entry tables are not replicated), raw codes, P rows
-    // V table replica (the table sits at LDS address 0, so field bits OR-ed in never meet the base; the
-    // 256-entry tables are not replicated)
-    constexpr bool V_UNREP = VBW == 4;                        // also every nibble record (VBW 4 by construction)
-    constexpr int VWIN = V_UNREP ? 0 : 8;                     // replicated tables: codes fetched with the byte in front of them
-    const uint32_t vbank = V_UNREP ? 0u : rep;
-    constexpr int vshift = V_UNREP ? 2 : 7;
-    const int vc = (int)vph + li * VBW - (V_UNREP ? 0 : 1);
-    const uint32_t vbase = vbuf + (uint32_t)(vc & ~3) + (uint32_t)lg * 4 * vrow, v_sh = (uint32_t)vc & 3u;
-    const uint32_t p_wr = pbuf + (uint32_t)lane * 4;                                   // + head pair * PROW
-    const uint32_t p_rd = pbuf + (uint32_t)((li & 7) >> 1) * PROW + (uint32_t)lg * 16;   // + block * 64
-    // A row (head h = li & 7, dim parity e = li >> 3) takes its head's half of the P dword into the half of
-    // parity e and zero into the other: a byte permute per dword
-    const uint32_t p_sel = (li & 8) ? ((li & 1) ? 0x03020C0Cu : 0x01000C0Cu) : ((li & 1) ? 0x0C0C0302u : 0x0C0C0100u);
-
-    float m_ref[8], l_part[8];      // per head: reference in log2 units (never below a score seen), this lane's share of the denominator
-#pragma unroll
-    for (int hh = 0; hh < 8; hh++) { m_ref[hh] = -INFINITY; l_part[hh] = 0.f; }
-    float4v acc[4];                 // acc[jb][r] = out[head 4(lg & 1) + r][dim 8 li + 2 jb + (lg >> 1)]
-#pragma unroll
-    for (int e = 0; e < 4; e++) acc[e] = (float4v){0, 0, 0, 0};
-
     for (; tile < t1; tile += step_tiles) {
         const int nt = min(MT, t1 - tile);
         const bool more = tile + step_tiles < t1;
@@ -537,7 +549,8 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a
         // last, of these the ones at the scores (lowered before the softmax: ±1 % against lowered behind it).  8 rows x 2 heads
         // of 32k nibble records 164.1 -> 156.5 us (4 layers), 1 x 8 heads of 128k K2V2 83.9 -> 79.3 (2), 12 ragged rows, 7 heads
         // a group, K4V4 93.3 -> 91.0 (4), 32 ragged rows of 8 heads 228.8 -> 220.2 (2); 32k bit-packed K3V3 +-0.5 %.
-        if (more) __builtin_amdgcn_s_setprio(3); else __builtin_amdgcn_s_setprio(1);
+        __builtin_amdgcn_s_setprio(1);
+        if (more) __builtin_amdgcn_s_setprio(3);
         // Streaming order behind the first tile: the V tile is requested when the K tile has arrived and
         // the K tile of the wave's next tile when the V tile has, so every wait is for all loads in flight.
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // K records and norms of this tile are in LDS
@@ -576,7 +589,8 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a
         asm volatile("" ::: "memory");
         __builtin_amdgcn_wave_barrier();
 
-        if (more) __builtin_amdgcn_s_setprio(2); else __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_s_setprio(0);
+        if (more) __builtin_amdgcn_s_setprio(2);
         // ---- online softmax: lane = token ----------------------------------------------------
         // FULL: every lane holds a token (all tiles but a row's last); FRESH: the wave's first tile (no
         // sums to rescale yet).  Both are wave-uniform and known before the tile: four copies of the code.
