@@ -1193,7 +1193,7 @@ __global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs a
 // work-group, then the queries by two waves (a barrier counts the waves that are left).  SWAP: the step's token enters the
 // buffer here, put there by those who read the one that leaves.
 // 32 rows x 8 heads x 4 queries over 132 buffered tokens: 4.9 (swap) + 11.1 + 13.3 us as launches of their own, 4.9 + 16.3
-// with K and V a work-group each and the swap ahead of them (1024 work-groups, two of them at a time on a compute unit).
+// with K and V a work-group each and the swap ahead of them (1024 work-groups, two of them at a time on a compute unit), 14 here.
 template <bool SWAP>
 __global__ __launch_bounds__(WINDOW_THREADS, 2) void prepare_window_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, WindowArgs w,
                                                                         RingArgs rk, RingArgs rv, int rows, int n_window) {
