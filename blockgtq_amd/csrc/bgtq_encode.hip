@@ -101,23 +101,33 @@ __device__ __forceinline__ void park_rotation(float* rot_s, const int j, const r
 }
 
 // Sum of x[k]^2 over a whole row of D values in LDS (V) as ONE fmaf chain in increasing k.  The reads
-// of a batch are all issued before its first fmaf (left to itself the compiler waits for every few
-// reads in turn); the chain itself runs at the 8 clocks of a dependent instruction.
+// of a batch are all issued before its first fmaf (left to itself the compiler waits for every few reads in
+// turn), AHEAD: under the chain of the batch before (3 trips to LDS less; 50 registers more, which the launch with the
+// window does not have); the chain itself runs at the 8 clocks of a dependent instruction.
+template <bool AHEAD>
 __device__ __forceinline__ float chain_sumsq_row(const float* x) {
+    constexpr int CB = 32;
     float ss = 0.f;
+    float4 v[AHEAD ? 2 : 1][CB / 4];
+    auto load = [&](const int blk) {
 #pragma unroll
-    for (int k0 = 0; k0 < D; k0 += 32) {
-        float4 v[8];
+        for (int i = 0; i < CB / 4; i++) v[AHEAD ? blk & 1 : 0][i] = *(const float4*)&x[CB * blk + 4 * i];
+    };
+    if (AHEAD) load(0);
 #pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = *(const float4*)&x[k0 + 4 * i];
+    for (int blk = 0; blk < D / CB; blk++) {
+        if (!AHEAD) load(blk);
+        else if (blk + 1 < D / CB) load(blk + 1);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            ss = __builtin_fmaf(v[i].x, v[i].x, ss);
-            ss = __builtin_fmaf(v[i].y, v[i].y, ss);
-            ss = __builtin_fmaf(v[i].z, v[i].z, ss);
-            ss = __builtin_fmaf(v[i].w, v[i].w, ss);
+        for (int i = 0; i < CB / 4; i++) {
+            const float4 x4 = v[AHEAD ? blk & 1 : 0][i];
+            ss = __builtin_fmaf(x4.x, x4.x, ss);
+            ss = __builtin_fmaf(x4.y, x4.y, ss);
+            ss = __builtin_fmaf(x4.z, x4.z, ss);
+            ss = __builtin_fmaf(x4.w, x4.w, ss);
         }
+        if (AHEAD) __builtin_amdgcn_sched_barrier(0);
     }
     return ss;
 }
@@ -132,6 +142,7 @@ struct RingArgs {
 };
 template <bool IS_V, bool PAIRED = false>
 __device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, const int h, const int j, float* rot_s, const RingArgs* ring = nullptr) {
+    __shared__ __align__(16) float xh_s[IS_V ? D : 4];       // V: the normalised row, beside the raw one (a barrier less)
     __shared__ __align__(16) float xs[2 * D];     // (the row, then zeros: the compact rotation reads up to BGTQ_ROT_COL values past a segment's start)
     __shared__ float nrm[BGTQ_MAX_SEGMENTS];
     __shared__ float nrm_out[BGTQ_MAX_SEGMENTS];
@@ -213,7 +224,7 @@ __device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, c
             fetch_rotation(P.k_rot_T, j, rst);
         }
     }
-    if constexpr (!IS_V || PAIRED) __syncthreads();     // (K reads the staged header next; V's staged tables are first read three barriers on)
+    if constexpr (!IS_V || PAIRED) __syncthreads();     // (K reads the staged header next; V's staged tables are first read two barriers on)
 
     // ---- per-thread static data, read ready-made from the plan (requested in the first burst) ----
     int n_seg = 1, g = 0, gs = 0, ge = D, ident = 0, src_dim = j;
@@ -242,13 +253,18 @@ __device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, c
     }
     __syncthreads();
 
-    // ---- 2. group norms: thread gg runs one sequential chain ---------
-    if (j < BGTQ_MAX_SEGMENTS) {
+    // ---- 2. group norms: thread gg runs one sequential chain; V alone: every thread the same one, so that none waits for it.
+    // (With the reads ahead, two barriers and a trip through LDS less, 4 rows x 2 heads of 8k tokens take 155.3 -> 153.3 us a
+    // pass of eight layers, one row x 8 heads of 4k 67.3 -> 66.6 of four.)
+    float v_norm = 0.f;
+    if constexpr (IS_V && !PAIRED) {
+        v_norm = __builtin_sqrtf(chain_sumsq_row<true>(xs) + 1e-30f);
+    } else if (j < BGTQ_MAX_SEGMENTS) {
         float n = 0.f;
         if (j < n_seg) {
             float ss = 0.f;
             if constexpr (IS_V) {
-                ss = chain_sumsq_row(xs);
+                ss = chain_sumsq_row<false>(xs);
             } else {                           // short ranges: the batches would mostly run masked
                 const int k0 = sp.hdr[H_START + j], k1 = k0 + sp.hdr[H_LEN + j];
 #pragma unroll 8
@@ -258,16 +274,17 @@ __device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, c
         }
         nrm[j] = n;
     }
-    __syncthreads();
+    if constexpr (!IS_V || PAIRED) __syncthreads();       // (V alone goes on with its own sum)
 
     // ---- 3. normalise -------------------------------------------------------
     float xh = 0.f;
     if (g >= 0) {
-        const float n = nrm[g];
+        const float n = IS_V && !PAIRED ? v_norm : nrm[g];
         const float safe = (n > (IS_V ? 1e-8f : 1e-10f)) ? n : 1.0f;
         xh = xs[j] / safe;
     }
-    xs[j] = xh;               // only this thread ever touched xs[j] since the barrier
+    if constexpr (IS_V) xh_s[j] = xh;
+    else xs[j] = xh;          // only this thread ever touched xs[j] since the barrier
     if constexpr (!IS_V) { if (!compact) park_rotation(rot_s, j, rst); }
     __syncthreads();
 
@@ -282,7 +299,7 @@ __device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, c
         float4 xv[2][CB / 4];
         auto load = [&](const int blk) {
 #pragma unroll
-            for (int i = 0; i < CB / 4; i++) xv[blk & 1][i] = *(const float4*)&xs[blk * CB + 4 * i];
+            for (int i = 0; i < CB / 4; i++) xv[blk & 1][i] = *(const float4*)&xh_s[blk * CB + 4 * i];
         };
         load(0);
 #pragma unroll
@@ -305,14 +322,19 @@ __device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, c
         // BGTQ_ROT_COL terms for every dim without a length test: a term x * 0 leaves the sum as it
         // is (the row is followed by zeros, so every x read is finite).
         constexpr int CB = 16;
+        float xv[2][CB];
+        auto load = [&](const int blk) {
 #pragma unroll
-        for (int i0 = 0; i0 < RC; i0 += CB) {
-            float xv[CB];
+            for (int i = 0; i < CB; i++) xv[blk & 1][i] = xs[gs + blk * CB + i];
+        };
+        load(0);
 #pragma unroll
-            for (int i = 0; i < CB; i++) xv[i] = xs[gs + i0 + i];
+        for (int blk = 0; blk < RC / CB; blk++) {
+            if (blk + 1 < RC / CB) load(blk + 1);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < CB; i++) y = __builtin_fmaf(xv[i], rc[i0 + i], y);
+            for (int i = 0; i < CB; i++) y = __builtin_fmaf(xv[blk & 1][i], rc[blk * CB + i], y);
+            __builtin_amdgcn_sched_barrier(0);
         }
     } else {                                    // column j of the parked rotation
         constexpr int CB = 16;
@@ -354,12 +376,13 @@ __device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, c
     }
     cds[j] = (uint8_t)code;
     // centroid of the chosen code for the norm correction below; it is parked in xs
-    // after the barrier (other threads may still be reading xs in their rotation)
+    // after the barrier (K: other threads may still be reading xs in their rotation)
     if (need_cent) {
         if constexpr (IS_V) y = sp.centroids[code];
         else y = g < 0 ? 0.f : code < 32 ? sp.centroids[g * 32 + code] : P.k_centroids[g][code];
     }
-    __syncthreads();
+    // (V's last reads of xs were the norm's, ahead of the barrier before the rotation)
+    if constexpr (!IS_V || PAIRED) __syncthreads();
     if (need_cent) xs[j] = y;
     __syncthreads();
 
@@ -371,9 +394,9 @@ __device__ __forceinline__ void encode_row(const EncodeArgs& a, const int row, c
     if (has_norm) {
         float out = 0.f;
         if (gg < n_seg) {
-            const float n = nrm[gg];
+            const float n = IS_V && !PAIRED ? v_norm : nrm[gg];
             if constexpr (IS_V) {
-                const float cn = __builtin_sqrtf(chain_sumsq_row(xs) + 1e-20f);
+                const float cn = __builtin_sqrtf(chain_sumsq_row<!PAIRED>(xs) + 1e-20f);
                 out = n / (cn > 1e-10f ? cn : 1.0f);
             } else if (a.layout == BGTQ_K_MIXED || a.corrected) {
                 const int k0 = sp.hdr[H_START + gg], k1 = k0 + sp.hdr[H_LEN + gg];
