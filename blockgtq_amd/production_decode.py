@@ -27,46 +27,83 @@ def production_decode_step(model, input_ids, position_ids, cache):
 def production_prefill(model, input_ids, cache, chunk_encode=64):
     """Prefill with the model's own attention, then pack its fp16 K/V.
 
-    Runs the HF forward with a ``DynamicCache`` (``_prompt_cache``), reads the post-RoPE K/V of
-    every layer back and encodes the prompt's tokens into ``cache`` (positions a
-    model adds behind them stay out).  ``chunk_encode`` bounded the reference
+    Runs the HF forward with a ``DynamicCache`` (``_prompt_cache``) and encodes the post-RoPE K/V of the
+    prompt's tokens of every layer into ``cache`` (positions a model adds behind them stay out): a
+    layer that the model hands over whole as it arrives, so that the model may write the same tensors again
+    for its next layer, others behind the forward pass.  (A model that does so and then appends to the first layer
+    within one pass runs once more, with a cache that copies.)  ``chunk_encode`` bounded the reference
     encoder's temporaries by slicing the prompt; fp16 and bf16 rows are encoded
     where they lie, independently and without temporaries, so they go in one launch
     per layer whatever it is (a 2001-token prompt of 8 KV heads: 374 us in slices
-    of 64, host bound, 28 us whole), and it bounds the fp16 copies that rows of
-    other types or strides are converted to.  Returns the prompt logits.
+    of 64, host bound, 26 us whole), and it bounds the fp16 copies that rows of
+    other types or strides are converted to.  A forward pass that fails behind its first packed
+    layer leaves ``cache`` empty.  Returns the prompt logits.
     """
     prompt_len = input_ids.shape[1]
     position_ids = torch.arange(prompt_len, device=input_ids.device).unsqueeze(0)
-    hf_cache = _prompt_cache()
-    out = model(input_ids, position_ids=position_ids, past_key_values=hf_cache, use_cache=True)
-    for li in range(cache.n_layers):
-        k, v = _layer_kv(hf_cache, li)
+    home = _stream(input_ids)
+    packed = {}
+
+    def pack(li, k, v):
         if k.dtype in _READ_IN_PLACE and v.dtype == k.dtype and k.stride(-1) == 1 and v.stride(-1) == 1:
             if k.size(2) > prompt_len:
                 k, v = k[:, :, :prompt_len], v[:, :, :prompt_len]
             cache._encode_batched(li, k, v, 0)
-            continue
+            return
         for lo in range(0, prompt_len, chunk_encode):
             hi = min(lo + chunk_encode, prompt_len)
             cache._encode_batched(li, k[:, :, lo:hi], v[:, :, lo:hi], lo)
+
+    def arrived(li, k, v):
+        # (on another stream the cache's records may still be read by what was launched before: packed at the end)
+        if li >= cache.n_layers or k.size(2) < prompt_len or _stream(k) != home:
+            return False
+        packed[li] = k, v
+        cache.seq_len = 0          # (until the forward pass is over: whatever was there, this layer's records are gone)
+        pack(li, k, v)
+        return True
+
+    for copies in (False, True):
+        hf_cache = _prompt_cache(None if copies else arrived, copies)
+        try:
+            out = model(input_ids, position_ids=position_ids, past_key_values=hf_cache, use_cache=True)
+            break
+        except _Refilled:
+            packed.clear()
+    for li in range(cache.n_layers):
+        k, v = _layer_kv(hf_cache, li)
+        if li not in packed or packed[li][0] is not k or packed[li][1] is not v:     # (appended to, cut or replaced since)
+            pack(li, k, v)
     cache.seq_len = prompt_len
     del hf_cache
     return out.logits
 
 
+class _Refilled(RuntimeError):
+    """Tokens were to be appended to kept ones that are gone."""
+
+
+def _stream(t):
+    return torch.cuda.current_stream(t.device) if t.is_cuda else None
+
+
+def _address(t):
+    return t.untyped_storage().data_ptr()
+
+
 def _whole(t):
     """Whether a tensor is all that its storage holds."""
-    return t.untyped_storage().nbytes() <= t.numel() * t.element_size()
+    return type(t) is torch.Tensor and 0 < t.untyped_storage().nbytes() <= t.numel() * t.element_size()
 
 
 @functools.lru_cache(maxsize=None)
-def _kept_layer():
-    """The layer class of ``_prompt_cache`` and the one it stands for (None: a generation without layer objects)."""
+def _kept_classes():
+    """The cache and layer classes of ``_prompt_cache`` and the layer class they stand for (None, None, None: a
+    generation without layer objects)."""
     try:
-        from transformers.cache_utils import DynamicLayer
+        from transformers.cache_utils import DynamicCache, DynamicLayer
     except ImportError:
-        return None, None
+        return None, None, None
 
     class KeptLayer(DynamicLayer):
         def update(self, key_states, value_states, *args, **kwargs):
@@ -77,21 +114,48 @@ def _kept_layer():
             self.keys, self.values = key_states, value_states
             return key_states, value_states
 
-    return KeptLayer, DynamicLayer
+    class KeptCache(DynamicCache):
+        def update(self, key_states, value_states, layer_idx, *args, **kwargs):
+            if torch.compiler.is_compiling():
+                return super().update(key_states, value_states, layer_idx, *args, **kwargs)
+            if self.kept:
+                for t in (key_states, value_states):
+                    if type(t) is torch.Tensor and _address(t) in self.kept:
+                        self.refilled.add(self.kept[_address(t)])
+                if layer_idx in self.refilled:
+                    raise _Refilled(f"the K and V kept of layer {layer_idx} were written again, and more tokens follow")
+            keys, values = super().update(key_states, value_states, layer_idx, *args, **kwargs)
+            if keys is key_states and values is value_states:
+                if self.arrived is None or self.arrived(layer_idx, keys, values):
+                    self.kept[_address(keys)] = self.kept[_address(values)] = layer_idx
+                else:
+                    keys, values = keys.clone(), values.clone()
+                    self.layers[layer_idx].keys, self.layers[layer_idx].values = keys, values
+            return keys, values
+
+    return KeptCache, KeptLayer, DynamicLayer
 
 
-def _prompt_cache():
+def _prompt_cache(arrived=None, copies=False):
     """A ``DynamicCache`` that keeps the first K and V of a layer as the model hands them over.
 
     ``DynamicCache`` appends them to an empty tensor: two copies of the layer's K and V (20 of 47 us for a 2001-token
     prompt of 8 KV heads) of which nothing is left once the prompt is packed.  What is a part of a larger tensor (a
     projection of queries, keys and values in one) is still copied, so that the rest can be freed; what comes later is
-    appended as ever."""
+    appended as ever.
+
+    Nothing says that the model leaves a kept layer's tensors alone for the rest of its pass.  ``arrived(layer, k, v)``
+    therefore reads them then and there; where it returns False they are copied after all.  Memory that comes back with
+    another layer, or with more tokens of the same one, was filled again: appending to the layer that was there raises
+    ``_Refilled``, and the pass has to be made again with ``copies``, a plain ``DynamicCache``."""
     from transformers import DynamicCache
-    cache = DynamicCache()
-    kept, plain = _kept_layer()
-    if kept is not None and getattr(cache, 'layer_class_to_replicate', None) is plain:
-        cache.layer_class_to_replicate = kept
+    kept_cache, kept_layer, plain_layer = _kept_classes()
+    if copies or kept_cache is None:
+        return DynamicCache()
+    cache = kept_cache()
+    if getattr(cache, 'layer_class_to_replicate', None) is plain_layer:
+        cache.layer_class_to_replicate = kept_layer
+    cache.arrived, cache.kept, cache.refilled = arrived, {}, set()      # kept: address -> layer that has its tokens there
     return cache
 
 

@@ -71,3 +71,116 @@ def test_prompt_cache_keeps_whole_tensors_and_appends_to_them():
     for li in range(2):
         for a, b in zip(_layer_kv(ours, li), _layer_kv(plain, li)):
             assert torch.equal(a, b)
+
+
+class _Reads(_Cache):
+    """Reads what it is given when it is given it, as an encoder does."""
+
+    def _encode_batched(self, li, k, v, t_pos):
+        super()._encode_batched(li, k.clone(), v.clone(), t_pos)
+
+
+class _Scratch:
+    """Hands every layer's K and V over in the same two tensors, ``piece`` tokens at a time."""
+
+    def __init__(self, k, v, piece, fails_at=None):
+        self.k, self.v, self.piece, self.fails_at, self.logits, self.passes = k, v, piece, fails_at, "logits", 0
+
+    def __call__(self, input_ids, position_ids=None, past_key_values=None, use_cache=True):
+        self.passes += 1
+        n = self.k.shape[-2]
+        for lo in range(0, n, self.piece):
+            buf_k, buf_v = torch.empty_like(self.k[0, :, :, lo:lo + self.piece]), torch.empty_like(self.v[0, :, :, lo:lo + self.piece])
+            for li in range(self.k.shape[0]):
+                if li == self.fails_at:
+                    raise MemoryError("out of memory")
+                buf_k.copy_(self.k[li, :, :, lo:lo + self.piece])
+                buf_v.copy_(self.v[li, :, :, lo:lo + self.piece])
+                got = past_key_values.update(buf_k, buf_v, li)
+                assert torch.equal(got[0], self.k[li, :, :, :lo + self.piece])
+                assert torch.equal(got[1], self.v[li, :, :, :lo + self.piece])
+        return self
+
+
+def _layers(tokens, dtype, n=3):
+    gen = torch.Generator().manual_seed(tokens)
+    return [torch.randn(n, 1, 2, tokens, 8, generator=gen).to(dtype) for _ in range(2)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("piece", [7, 50, 57])
+def test_a_model_that_fills_the_same_tensors_for_every_layer(dtype, piece):
+    k, v = _layers(57, dtype, 2)
+    for tokens in (50, 57):                              # (the prompt ends inside what the model hands over, or with it)
+        cache = _Reads()
+        model = _Scratch(k, v, piece)
+        production_prefill(model, torch.zeros(1, tokens, dtype=torch.long), cache)
+        # the prompt at once, then more tokens: the first ones are gone by then, so the pass is made again
+        assert model.passes == (2 if piece == tokens == 50 else 1)
+        for li in range(2):
+            assert sorted(cache.k[li]) == list(range(tokens))
+            for s in range(tokens):
+                assert torch.equal(cache.k[li][s], k[li][:, :, s]) and torch.equal(cache.v[li][s], v[li][:, :, s])
+
+
+def test_tokens_behind_a_whole_prompt_and_a_changed_layer():
+    k, v = _layers(30, torch.float16, 2)
+
+    class Model:
+        logits = "logits"
+
+        def __call__(self, input_ids, past_key_values=None, **kwargs):
+            for lo, hi in ((0, 20), (20, 30)):           # tensors of their own for every layer
+                for li in range(2):
+                    got = past_key_values.update(k[li, :, :, lo:hi].clone(), v[li, :, :, lo:hi].clone(), li)
+                    assert torch.equal(got[0], k[li, :, :, :hi]) and torch.equal(got[1], v[li, :, :, :hi])
+            past_key_values.layers[1].keys = past_key_values.layers[1].keys + 1
+            return self
+
+    cache = _Reads()
+    production_prefill(Model(), torch.zeros(1, 20, dtype=torch.long), cache)
+    for s in range(20):
+        assert torch.equal(cache.k[0][s], k[0][:, :, s]) and torch.equal(cache.k[1][s], (k[1] + 1)[:, :, s])
+        assert torch.equal(cache.v[0][s], v[0][:, :, s]) and torch.equal(cache.v[1][s], v[1][:, :, s])
+
+
+@pytest.mark.parametrize("fails_at,left", [(0, 9), (1, 0)])
+def test_a_forward_pass_that_fails(fails_at, left):
+    k, v = _layers(12, torch.float16, 2)
+    cache = _Reads()
+    cache.seq_len = 9                                    # of an earlier prompt: gone once a layer is packed over it
+    with pytest.raises(MemoryError):
+        production_prefill(_Scratch(k, v, 12, fails_at=fails_at), torch.zeros(1, 12, dtype=torch.long), cache)
+    assert cache.seq_len == left
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("aside", [False, True])           # the model's layers on another stream: copied, packed at the end
+def test_records_of_a_model_that_fills_the_same_tensors(aside):
+    from blockgtq_amd import workloads as wl
+    from blockgtq_amd.production_cache import BlockGTQProductionCache
+    from blockgtq_amd.quantizer import build_batched_encode_args
+    dev, n, T = "cuda:0", 3, 130
+    w = wl.Workload("t", n, 4, 2, 1, T, 1e6, seed=51)
+    drawn = [wl.calibrate_layer(w, li, dev) for li in range(n)]
+    qs = [q for q, _ in drawn]
+    ours, want = [BlockGTQProductionCache(qs, [build_batched_encode_args(q, device=dev) for q in qs],
+                                          [[q8.build_kernel_args() for q8 in q] for q in qs], n, 2, 4, 128, T + 8, device=dev)
+                  for _ in range(2)]
+    k, v = (torch.stack(t) for t in zip(*[wl.draw_kv(w, drawn[li][1], T, li, dev) for li in range(n)]))
+    for li in range(n):
+        want._encode_batched(li, k[li], v[li], 0)
+    side, scratch = torch.cuda.Stream(), _Scratch(k, v, T)
+
+    def model(*args, **kwargs):
+        if not aside:
+            return scratch(*args, **kwargs)
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            out = scratch(*args, **kwargs)
+        torch.cuda.current_stream().wait_stream(side)
+        return out
+
+    production_prefill(model, torch.zeros(1, T, dtype=torch.long, device=dev), ours)
+    for name in ("k_packed", "k_norms", "v_packed", "v_norms"):
+        assert torch.equal(getattr(ours, name)[:, :, :, :T], getattr(want, name)[:, :, :, :T]), name
