@@ -99,7 +99,7 @@ def _whole(t):
 @functools.lru_cache(maxsize=None)
 def _kept_classes():
     """The cache and layer classes of ``_prompt_cache`` and the layer class they stand for (None, None, None: a
-    generation without layer objects)."""
+    generation without layer objects, or with ones that start, hold or grow otherwise than ``KeptLayer`` has it)."""
     try:
         from transformers.cache_utils import DynamicCache, DynamicLayer
     except ImportError:
@@ -133,7 +133,13 @@ def _kept_classes():
                     self.layers[layer_idx].keys, self.layers[layer_idx].values = keys, values
             return keys, values
 
-    return KeptCache, KeptLayer, DynamicLayer
+    try:                                    # one token, then one more: kept as it is, then appended to
+        layer, one = KeptLayer(), torch.empty(1, 1, 1, 1, device="cpu")
+        fits = (layer.update(one, one)[0] is one and layer.keys is one and layer.values is one and
+                layer.update(one, one)[0].shape == layer.keys.shape == layer.values.shape == (1, 1, 2, 1))
+    except (AttributeError, TypeError):
+        fits = False
+    return (KeptCache, KeptLayer, DynamicLayer) if fits else (None, None, None)
 
 
 def _prompt_cache(arrived=None, copies=False):

@@ -154,6 +154,51 @@ def test_a_forward_pass_that_fails(fails_at, left):
     assert cache.seq_len == left
 
 
+@pytest.mark.parametrize("change", ["arguments", "no such method"])
+def test_another_generation_of_the_cache_library(monkeypatch, change):
+    """Layers that are set up otherwise than the installed library's: the prompt's K and V are copied, as the library has it."""
+    from transformers import cache_utils
+    from blockgtq_amd import production_decode
+    Plain, Cache = cache_utils.DynamicLayer, cache_utils.DynamicCache
+
+    class OtherLayer(Plain):
+        if change == "arguments":
+            def lazy_initialization(self, key_states):
+                self.is_initialized = True
+        else:
+            @property
+            def lazy_initialization(self):
+                raise AttributeError("lazy_initialization")
+
+        def __init__(self):
+            self.held, self.is_initialized = Plain(), False
+
+        def update(self, key_states, value_states, *args, **kwargs):
+            self.keys, self.values = self.held.update(key_states, value_states, *args, **kwargs)
+            self.is_initialized = True
+            return self.keys, self.values
+
+    class OtherCache(Cache):
+        def __init__(self, *args, **kwargs):
+            super().__init__(*args, **kwargs)
+            self.layer_class_to_replicate = OtherLayer
+
+    monkeypatch.setattr(cache_utils, "DynamicLayer", OtherLayer)
+    monkeypatch.setattr(cache_utils, "DynamicCache", OtherCache)
+    monkeypatch.setattr("transformers.DynamicCache", OtherCache)
+    production_decode._kept_classes.cache_clear()
+    try:
+        k, v = _layers(11, torch.float16, 2)
+        cache = _Reads()
+        production_prefill(_Scratch(k, v, 11), torch.zeros(1, 11, dtype=torch.long), cache)
+    finally:
+        production_decode._kept_classes.cache_clear()
+    for li in range(2):
+        assert sorted(cache.k[li]) == list(range(11))
+        for s in range(11):
+            assert torch.equal(cache.k[li][s], k[li][:, :, s]) and torch.equal(cache.v[li][s], v[li][:, :, s])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("aside", [False, True])           # the model's layers on another stream: copied, packed at the end
 def test_records_of_a_model_that_fills_the_same_tensors(aside):
