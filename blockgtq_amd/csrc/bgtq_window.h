@@ -201,7 +201,8 @@ __device__ __forceinline__ void window_attn_block(const WindowArgs& a, const int
 #pragma unroll
         for (int g = 0; g < HG; g++) o0[g] = o1[g] = 0.f;
         auto values = [&](uint32_t (&vc)[PB], const int t0) {
-            if (SWAP && slot >= t0 && slot < t0 + PSTEP && (slot - t0) % NW == 0) {  // (uniform)
+            // (uniform; a row behind the visible ones stays zeros: what is masked below is a product with it)
+            if (SWAP && slot >= t0 && slot < min(t0 + PSTEP, n) && (slot - t0) % NW == 0) {
 #pragma unroll
                 for (int u = 0; u < PB; u++) vc[u] = t0 + u * NW == slot ? own_v : vc[u];
             }

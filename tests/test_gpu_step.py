@@ -256,3 +256,28 @@ def test_buffered_step_slots(dtype, offset):
     assert torch.isfinite(slow).all() and slow.abs().max() > 0 and torch.equal(fast, slow)
     for name in ("_k_packed", "_k_norms", "_v_packed", "_v_norms", "_buf_k", "_buf_v"):
         assert torch.equal(getattr(mgrs[0], name)[0], getattr(mgrs[1], name)[0]), name
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("n_q", [8, 14])                        # heads of a group all served at once, and a last one of three
+def test_buffered_step_with_a_new_token_that_nobody_sees(bad, n_q):
+    """A new token that is not finite, in a slot behind the visible ones: no output depends on it."""
+    n_kv, W, B, context = 2, 20, 6, 60
+    w = wl.Workload("t", 1, n_q, n_kv, B, context, 1e6, seq_lens=[context] * B, n_sink=4, window=W - 4, seed=39)
+    mgrs = []
+    for _ in range(2):
+        mgr, energies = wl.build_manager(w, DEV)
+        wl.fill_cache(mgr, w, energies, DEV)
+        mgrs.append(mgr)
+    q, k, v = _inputs(w, energies, context, torch.float16)
+    k[:, :, :, 5], v[:, :, :, 7] = bad, bad
+    i32 = dict(dtype=torch.int32, device=DEV)
+    slots, seen = [11, 3, W - 1, 9, 13, W], [9, 1, 17, 9, 2, W]
+    idx = (torch.arange(B, device=DEV), torch.tensor(slots, **i32), torch.arange(30, 30 + B, **i32),
+           torch.tensor([41, 40, 1, 7, 0, 30], **i32), torch.tensor(seen, **i32))
+    assert all(s >= n for s, n in zip(slots, seen))
+    mgrs[1]._native = lambda li: mgrs[1]._ensure_storage()
+    for m in mgrs:
+        m._buffered_step_indices = lambda: idx
+    fast, slow = [m.append_and_attend(0, q, k, v) for m in mgrs]
+    assert torch.isfinite(slow).all() and slow.abs().max() > 0 and torch.equal(fast, slow)
