@@ -426,6 +426,15 @@ PyObject* prompt(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// stream(t): the current stream of t's device, as something to compare
+PyObject* stream(PyObject*, PyObject* o) {
+    HANDLE_TH_ERRORS
+    const at::Tensor* t = tensor(o);
+    if (!t || !t->is_cuda()) { PyErr_SetString(PyExc_TypeError, "stream(tensor on the GPU)"); return nullptr; }
+    return Py_BuildValue("iK", (int)t->get_device(), (unsigned long long)(uintptr_t)stream_of(*t));
+    END_HANDLE_TH_ERRORS
+}
+
 PyObject* setup(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 2) { PyErr_SetString(PyExc_TypeError, "setup(error class, path hook)"); return nullptr; }
     Py_INCREF(a[0]);
@@ -440,6 +449,7 @@ PyObject* setup(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef module_methods[] = {
     {"attend", (PyCFunction)(void*)attend, METH_FASTCALL, "decode attention over packed records, or None"},
     {"prompt", (PyCFunction)(void*)prompt, METH_FASTCALL, "prompt-phase attention over packed records, or None"},
+    {"stream", (PyCFunction)stream, METH_O, "(device, current stream) of a tensor"},
     {"setup", (PyCFunction)(void*)setup, METH_FASTCALL, "hand over the error class and the hook that notes which kernel ran"},
     {nullptr, nullptr, 0, nullptr}};
 

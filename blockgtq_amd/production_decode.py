@@ -7,6 +7,7 @@ import functools
 
 import torch
 
+from . import _host
 from .packed_kv_manager import run_decoder_stack
 
 _READ_IN_PLACE = (torch.float16, torch.bfloat16)      # what the encoders take as it lies
@@ -42,7 +43,6 @@ def production_prefill(model, input_ids, cache, chunk_encode=64):
     prompt_len = input_ids.shape[1]
     position_ids = torch.arange(prompt_len, device=input_ids.device).unsqueeze(0)
     home = _stream(input_ids)
-    packed = {}
 
     def pack(li, k, v):
         if k.dtype in _READ_IN_PLACE and v.dtype == k.dtype and k.stride(-1) == 1 and v.stride(-1) == 1:
@@ -58,21 +58,22 @@ def production_prefill(model, input_ids, cache, chunk_encode=64):
         # (on another stream the cache's records may still be read by what was launched before: packed at the end)
         if li >= cache.n_layers or k.size(2) < prompt_len or _stream(k) != home:
             return False
-        packed[li] = k, v
         cache.seq_len = 0          # (until the forward pass is over: whatever was there, this layer's records are gone)
         pack(li, k, v)
         return True
 
     for copies in (False, True):
-        hf_cache = _prompt_cache(None if copies else arrived, copies)
+        hf_cache = _prompt_cache(arrived, copies)
         try:
             out = model(input_ids, position_ids=position_ids, past_key_values=hf_cache, use_cache=True)
             break
         except _Refilled:
-            packed.clear()
+            pass
+    packed = getattr(hf_cache, 'kept', {})
     for li in range(cache.n_layers):
         k, v = _layer_kv(hf_cache, li)
-        if li not in packed or packed[li][0] is not k or packed[li][1] is not v:     # (appended to, cut or replaced since)
+        was = packed.get(li)
+        if was is None or was[0] is not k or was[1] is not v:       # (or appended to, cut, replaced since)
             pack(li, k, v)
     cache.seq_len = prompt_len
     del hf_cache
@@ -84,11 +85,7 @@ class _Refilled(RuntimeError):
 
 
 def _stream(t):
-    return torch.cuda.current_stream(t.device) if t.is_cuda else None
-
-
-def _address(t):
-    return t.untyped_storage().data_ptr()
+    return _host.module().stream(t) if t.is_cuda else None
 
 
 def _whole(t):
@@ -96,50 +93,77 @@ def _whole(t):
     return type(t) is torch.Tensor and 0 < t.untyped_storage().nbytes() <= t.numel() * t.element_size()
 
 
-@functools.lru_cache(maxsize=None)
-def _kept_classes():
-    """The cache and layer classes of ``_prompt_cache`` and the layer class they stand for (None, None, None: a
-    generation without layer objects, or with ones that start, hold or grow otherwise than ``KeptLayer`` has it)."""
-    try:
-        from transformers.cache_utils import DynamicCache, DynamicLayer
-    except ImportError:
-        return None, None, None
+def _kept_layer(Layer):
+    """``Layer`` that takes its first K and V as they are."""
 
-    class KeptLayer(DynamicLayer):
+    class KeptLayer(Layer):
         def update(self, key_states, value_states, *args, **kwargs):
-            if (torch.compiler.is_compiling() or getattr(self, 'is_initialized', True) or
-                    not (_whole(key_states) and _whole(value_states))):
+            if self.is_initialized or torch.compiler.is_compiling() or not (_whole(key_states) and _whole(value_states)):
                 return super().update(key_states, value_states, *args, **kwargs)
-            self.lazy_initialization(key_states, value_states)
+            self.dtype, self.device, self.is_initialized = key_states.dtype, key_states.device, True
             self.keys, self.values = key_states, value_states
             return key_states, value_states
 
-    class KeptCache(DynamicCache):
+    return KeptLayer
+
+
+def _stands_for(kept, plain):
+    """Whether a layer with its first token kept has what one that copied it has, and grows by the next one alike."""
+    one, kept, plain = torch.empty(1, 1, 1, 1, device="cpu"), kept(), plain()
+    if kept.update(one, one)[0] is not one or kept.is_initialized is not True:
+        return False
+    plain.update(one, one)
+    mine, theirs = vars(kept), vars(plain)
+    return (mine.keys() == theirs.keys() and mine['keys'] is one and mine['values'] is one and
+            all(torch.is_tensor(x) or x == mine[name] for name, x in theirs.items()) and
+            kept.update(one, one)[0].shape == kept.keys.shape == kept.values.shape == (1, 1, 2, 1))
+
+
+def _kept_cache(Cache):
+    """``Cache`` with what ``_prompt_cache`` says of kept layers."""
+
+    class KeptCache(Cache):
         def update(self, key_states, value_states, layer_idx, *args, **kwargs):
             if torch.compiler.is_compiling():
                 return super().update(key_states, value_states, layer_idx, *args, **kwargs)
             if self.kept:
-                for t in (key_states, value_states):
-                    if type(t) is torch.Tensor and _address(t) in self.kept:
-                        self.refilled.add(self.kept[_address(t)])
-                if layer_idx in self.refilled:
-                    raise _Refilled(f"the K and V kept of layer {layer_idx} were written again, and more tokens follow")
+                self.look_for(key_states, value_states, layer_idx)
             keys, values = super().update(key_states, value_states, layer_idx, *args, **kwargs)
             if keys is key_states and values is value_states:
                 if self.arrived is None or self.arrived(layer_idx, keys, values):
-                    self.kept[_address(keys)] = self.kept[_address(values)] = layer_idx
+                    self.kept[layer_idx] = keys, values
                 else:
                     keys, values = keys.clone(), values.clone()
                     self.layers[layer_idx].keys, self.layers[layer_idx].values = keys, values
             return keys, values
 
-    try:                                    # one token, then one more: kept as it is, then appended to
-        layer, one = KeptLayer(), torch.empty(1, 1, 1, 1, device="cpu")
-        fits = (layer.update(one, one)[0] is one and layer.keys is one and layer.values is one and
-                layer.update(one, one)[0].shape == layer.keys.shape == layer.values.shape == (1, 1, 2, 1))
-    except (AttributeError, TypeError):
-        fits = False
-    return (KeptCache, KeptLayer, DynamicLayer) if fits else (None, None, None)
+        def look_for(self, key_states, value_states, layer_idx):
+            for li in list(self.kept)[self.listed:]:
+                for t in self.kept[li]:
+                    self.where[t.untyped_storage().data_ptr()] = li
+            self.listed = len(self.kept)
+            for t in (key_states, value_states):
+                if type(t) is torch.Tensor:
+                    self.refilled.add(self.where.get(t.untyped_storage().data_ptr()))
+            if layer_idx in self.refilled:
+                raise _Refilled(f"the K and V kept of layer {layer_idx} were written again, and more tokens follow")
+
+    return KeptCache
+
+
+@functools.lru_cache(maxsize=None)
+def _prompt_classes():
+    """The cache class of ``_prompt_cache``, and its layer class with the one that stands for (None, None: a generation
+    without layer objects, or with ones that start, hold or grow otherwise than a kept layer does)."""
+    from transformers import DynamicCache
+    try:
+        from transformers.cache_utils import DynamicLayer
+        kept = _kept_layer(DynamicLayer)
+        if _stands_for(kept, DynamicLayer) and getattr(DynamicCache(), 'layer_class_to_replicate', None) is DynamicLayer:
+            return DynamicCache, _kept_cache(DynamicCache), kept
+    except (ImportError, AttributeError, KeyError, TypeError):
+        pass
+    return DynamicCache, None, None
 
 
 def _prompt_cache(arrived=None, copies=False):
@@ -154,14 +178,13 @@ def _prompt_cache(arrived=None, copies=False):
     therefore reads them then and there; where it returns False they are copied after all.  Memory that comes back with
     another layer, or with more tokens of the same one, was filled again: appending to the layer that was there raises
     ``_Refilled``, and the pass has to be made again with ``copies``, a plain ``DynamicCache``."""
-    from transformers import DynamicCache
-    kept_cache, kept_layer, plain_layer = _kept_classes()
+    plain, kept_cache, kept_layer = _prompt_classes()
     if copies or kept_cache is None:
-        return DynamicCache()
+        return plain()
     cache = kept_cache()
-    if getattr(cache, 'layer_class_to_replicate', None) is plain_layer:
-        cache.layer_class_to_replicate = kept_layer
-    cache.arrived, cache.kept, cache.refilled = arrived, {}, set()      # kept: address -> layer that has its tokens there
+    cache.layer_class_to_replicate = kept_layer
+    # kept: layer -> K, V; where: address -> layer, of the first `listed` ones; refilled: layers whose memory came again
+    cache.arrived, cache.kept, cache.where, cache.listed, cache.refilled = arrived, {}, {}, 0, set()
     return cache
 
 

@@ -186,13 +186,13 @@ def test_another_generation_of_the_cache_library(monkeypatch, change):
     monkeypatch.setattr(cache_utils, "DynamicLayer", OtherLayer)
     monkeypatch.setattr(cache_utils, "DynamicCache", OtherCache)
     monkeypatch.setattr("transformers.DynamicCache", OtherCache)
-    production_decode._kept_classes.cache_clear()
+    production_decode._prompt_classes.cache_clear()
     try:
         k, v = _layers(11, torch.float16, 2)
         cache = _Reads()
         production_prefill(_Scratch(k, v, 11), torch.zeros(1, 11, dtype=torch.long), cache)
     finally:
-        production_decode._kept_classes.cache_clear()
+        production_decode._prompt_classes.cache_clear()
     for li in range(2):
         assert sorted(cache.k[li]) == list(range(11))
         for s in range(11):
