@@ -61,7 +61,7 @@ struct StageArgs {
     const uint16_t* kn; int64_t kn_sb, kn_sh; int kn_st;
     const uint8_t* vp;  int64_t vp_sb, vp_sh;
     const uint16_t* vn; int64_t vn_sb, vn_sh;
-    int n_kv, T, n_tiles, per_wg;            // tiles of a (row, head), how many of them a work-group takes
+    int n_kv, pairs, T, n_tiles, per_wg;     // (row, head) pairs, tiles of one, how many of them a work-group takes
     int k_layout, v_layout, k_row_width, v_stride;
     int kt, knr, vnr, vt;                    // raw tile areas in LDS
     int bf16, rotate_q;                      // parts of the query rotation: bf16 / fp16, or none
@@ -128,16 +128,19 @@ __device__ __forceinline__ void stage_rotations(const StageArgs& a, int wg, int 
 
 // One set of raw records: two work-groups share a compute unit (at most 78 KB of LDS each) and one's loads run under the
 // other's lookups.  With two sets a work-group was alone there, and 292 of them (4100 records of 8 heads) took two rounds.
-// 4100 records of 8 heads: 19.9 -> 12.2 us, 4 x 8192 of 2 heads 26.9 -> 18.2.
+// 4100 records of 8 heads: 19.9 -> 12.2 us, 4 x 8192 of 2 heads 26.9 -> 18.2 (a large copy or merge in front of each).
+// Bound by the loads and lookups of a tile, one behind the other.  Work-groups are numbered as the attention's are, (row, head)
+// fastest: with 8 pairs an XCD then writes the tiles it will read, and that it read in the call before.  Tiles that lie in
+// the L2 of another XCD, from a call just ended in the same workspace, made it 16.0 us (12.6 with 66 MB copied in between, which
+// drives them out); 11.1 now, 11.4 behind the copy.
 __global__ __launch_bounds__(DQ_THR) void prompt_stage_kernel(StageArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n_rot = ROT_WGS * a.n_kv;
     if ((int)blockIdx.x < n_rot) { stage_rotations(a, (int)blockIdx.x, tid, smem); return; }
-    const int wgs_per = (a.n_tiles + a.per_wg - 1) / a.per_wg;
-    const int pair = ((int)blockIdx.x - n_rot) / wgs_per, tile0 = ((int)blockIdx.x - n_rot - pair * wgs_per) * a.per_wg;
-    const int tile1 = min(tile0 + a.per_wg, a.n_tiles);
+    const int part = ((int)blockIdx.x - n_rot) / a.pairs, pair = (int)blockIdx.x - n_rot - part * a.pairs;
+    const int tile0 = part * a.per_wg, tile1 = min(tile0 + a.per_wg, a.n_tiles);
     const int b = pair / a.n_kv, h = pair - b * a.n_kv;
     const bgtq_head_plan& P = a.plans[h];
     const bool vnib = a.v_layout == BGTQ_V_NIBBLE;
@@ -762,7 +765,7 @@ int bgtq_prompt_attn(const bgtq_head_plan* plans,
     g.kn = (const uint16_t*)k_norms; g.kn_sb = kn_sb; g.kn_sh = kn_sh; g.kn_st = (int)kn_st;
     g.vp = (const uint8_t*)v_packed; g.vp_sb = vp_sb; g.vp_sh = vp_sh;
     g.vn = (const uint16_t*)v_norms; g.vn_sb = vn_sb; g.vn_sh = vn_sh;
-    g.n_kv = n_kv; g.T = T; g.n_tiles = (T + MT - 1) / MT;
+    g.n_kv = n_kv; g.pairs = B * n_kv; g.T = T; g.n_tiles = (T + MT - 1) / MT;
     g.k_layout = k_layout; g.v_layout = v_layout; g.k_row_width = k_row_width; g.v_stride = (int)vp_st;
     const int raw = raw_bytes(k_row_width, (int)vp_st, (int)kn_st, g.kt, g.knr, g.vnr, g.vt);
     // two work-groups fit a compute unit; tiles in equal shares over what that makes

@@ -115,6 +115,13 @@ def test_two_teams_over_one_block_of_rows(n_kv, gqa, S, T, off):
     test_prompt_attention_equals_the_kernel_without_workspace(1, n_kv, gqa, S, T, off, P.K_BITPACKED, P.V_BITPACKED, (3.0, 3, 1, 5), torch.bfloat16)
 
 
+# staging in shares of two tiles, the last of one; fewer (row, head) pairs than XCDs, and more
+@pytest.mark.parametrize("B,n_kv,T", [(2, 3, 5800), (3, 4, 2817)])
+def test_several_tiles_to_a_staging_work_group(B, n_kv, T):
+    assert 512 < -(-T // 64) * B * n_kv <= 1024 and -(-T // 64) % 2 == 1
+    test_prompt_attention_equals_the_kernel_without_workspace(B, n_kv, 2, 20, T, T - 20, P.K_MIXED, P.V_NIBBLE, (2.5, 2, 0, 8), torch.float16)
+
+
 def test_small_probabilities_count_in_the_denominator():
     """Each query has one strong record among the first and 65 535 weak ones, e^-18 of it apiece and below the smallest fp16
     number once the reference lies 4 octaves above the strong score; together they are 4e-3 of the denominator.
