@@ -520,7 +520,8 @@ struct EncodeLds {
 
 // x / d correctly rounded from y = RN(1 / d), for x a finite fp16 value, and d and y normal (Markstein: a quotient within one
 // unit in the last place and a correctly rounded reciprocal give the rounded quotient after one residual step.  x * y can be
-// 1.5 units off, but no quotient of an 11-bit x lies near enough to a midpoint: all 2^10 x 2^23 mantissas were compared.)
+// 1.5 units off, but no quotient of an 11-bit x lies near enough to a midpoint: tests/test_quotient.py compares all 2^10 x 2^23
+// mantissas.)
 __device__ __forceinline__ float div_by(float x, float2 dy) {
     const float q = x * dy.y;
     return __builtin_fmaf(__builtin_fmaf(-dy.x, q, x), dy.y, q);
