@@ -491,8 +491,6 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a
     uint32_t qs_l = QS_OFF + (q_head >= 0 ? q_head : HEADS) * QSTRUCT;
     // PV operands: V table replica (the table sits at LDS address 0, so field bits OR-ed in never meet the
     // base; the 256-entry tables are not replicated), raw codes, P rows
-    // V table replica (the table sits at LDS address 0, so field bits OR-ed in never meet the base; the
-    // 256-entry tables are not replicated)
     constexpr bool V_UNREP = VBW == 4;                        // also every nibble record (VBW 4 by construction)
     constexpr int VWIN = V_UNREP ? 0 : 8;                     // replicated tables: codes fetched with the byte in front of them
     uint32_t vbank = V_UNREP ? 0u : rep;

@@ -464,7 +464,7 @@ __global__ __launch_bounds__(NT) void encode_kernel(EncodeArgs a) {
     encode_row<IS_V>(a, blockIdx.x, blockIdx.y, threadIdx.x, rot_s);
 }
 // ================================================================================================
-// Prompt-sized encoder: blocks of 16 rows, every chain of the contract on the fp32 matrix cores.
+// Prompt-sized encoder: blocks of 16 rows, rotations and V's corrected norms on the fp32 matrix cores, norms as chains of a lane.
 //
 // v_mfma_f32_16x16x4_f32 adds its four products to the accumulator one after the other, each as one fused
 // multiply-add rounded to nearest with subnormals kept: such instructions over ascending k are the contract's

@@ -417,9 +417,10 @@ __global__ __launch_bounds__(64 * NW * TEAMS, 2) void prompt_attn_kernel(PromptA
 
     // The walk is one tile deep: while a tile's scores become probabilities on the vector unit, the matrix core
     // works on the scores of the next one, and the maximum of those is taken under the value product.  (4 x 8k prompts
-    // 1186 -> 1167 us, 1000 queries over 4100 records 122 -> 119, against the same parts one after the other: the matrix
-    // cores are busy 53 % of the time, at 1.9 GHz, and the clock gives way to more.  970 TFLOP/s here, 1290 for the
-    // library's bf16 product of 8192 x 8192 matrices on the same card.)
+    // 1186 -> 1167 us, 1000 queries over 4100 records 122 -> 119, against the same parts one after the other; that was before
+    // the two waves of a SIMD took turns, with the matrix cores busy 53 % of the cycles at 1.9 GHz.  The clock gives way to
+    // more: 60 % at 1.75 GHz with turns, 980 TFLOP/s, where the library's bf16 product of 8192 x 8192 matrices reaches 1290
+    // on the same card.)
     auto frags = [&](int tile) __attribute__((always_inline)) {
         uint32_t at = lds0 + (uint32_t)(tile & (RING - 1)) * TILE + voff;
         asm("" : "+v"(at));                                      // (fragments at immediate offsets: left alone, every address gets an instruction)
