@@ -154,6 +154,23 @@ def test_a_forward_pass_that_fails(fails_at, left):
     assert cache.seq_len == left
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_library_model_is_served_as_with_its_own_cache(dtype):
+    from transformers import DynamicCache, Qwen2Config, Qwen2ForCausalLM
+    from blockgtq_amd.production_decode import _layer_kv
+    torch.manual_seed(5)
+    model = Qwen2ForCausalLM(Qwen2Config(vocab_size=64, hidden_size=32, intermediate_size=48, num_hidden_layers=2,
+                                         num_attention_heads=4, num_key_value_heads=2)).to(dtype).eval()
+    ids, plain, cache = torch.randint(0, 64, (1, 19)), DynamicCache(), _Reads()
+    logits = production_prefill(model, ids, cache, chunk_encode=8)
+    with torch.no_grad():
+        want = model(ids, past_key_values=plain, use_cache=True).logits
+    assert torch.equal(logits, want) and cache.seq_len == 19
+    for li in range(2):
+        k, v = _layer_kv(plain, li)
+        assert all(torch.equal(cache.k[li][s], k[:, :, s]) and torch.equal(cache.v[li][s], v[:, :, s]) for s in range(19))
+
+
 @pytest.mark.parametrize("change", ["arguments", "no such method"])
 def test_another_generation_of_the_cache_library(monkeypatch, change):
     """Layers that are set up otherwise than the installed library's: the prompt's K and V are copied, as the library has it."""
