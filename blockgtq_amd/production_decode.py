@@ -31,8 +31,9 @@ def production_prefill(model, input_ids, cache, chunk_encode=64):
     Runs the HF forward with a ``DynamicCache`` (``_prompt_cache``) and encodes the post-RoPE K/V of the
     prompt's tokens of every layer into ``cache`` (positions a model adds behind them stay out): a
     layer that the model hands over whole as it arrives, so that the model may write the same tensors again
-    for its next layer, others behind the forward pass.  (A model that does so and then appends to the first layer
-    within one pass runs once more, with a cache that copies.)  ``chunk_encode`` bounded the reference
+    for its next layer, others behind the forward pass.  (A model that does so and then appends to or changes an
+    earlier layer of the cache within one pass runs once more, with a cache that copies; what it reads there is what it
+    has written since.)  ``chunk_encode`` bounded the reference
     encoder's temporaries by slicing the prompt; fp16 and bf16 rows are encoded
     where they lie, independently and without temporaries, so they go in one launch
     per layer whatever it is (a 2001-token prompt of 8 KV heads: 374 us in slices
@@ -66,21 +67,25 @@ def production_prefill(model, input_ids, cache, chunk_encode=64):
         hf_cache = _prompt_cache(arrived, copies)
         try:
             out = model(input_ids, position_ids=position_ids, past_key_values=hf_cache, use_cache=True)
-            break
         except _Refilled:
-            pass
-    packed = getattr(hf_cache, 'kept', {})
-    for li in range(cache.n_layers):
-        k, v = _layer_kv(hf_cache, li)
-        was = packed.get(li)
-        if was is None or was[0] is not k or was[1] is not v:       # (or appended to, cut, replaced since)
-            pack(li, k, v)
+            continue
+        packed = getattr(hf_cache, 'kept', {})
+        rest = []
+        for li in range(cache.n_layers):
+            k, v = _layer_kv(hf_cache, li)
+            was = packed.get(li)
+            if was is None or was[0] is not k or was[1] is not v:   # (or appended to, cut, replaced since)
+                rest.append((li, k, v))
+        if not packed or hf_cache.refilled.isdisjoint(li for li, _, _ in rest):
+            break
+    for li, k, v in rest:
+        pack(li, k, v)
     cache.seq_len = prompt_len
     del hf_cache
     return out.logits
 
 
-class _Refilled(RuntimeError):
+class _Refilled(Exception):
     """Tokens were to be appended to kept ones that are gone."""
 
 
@@ -130,7 +135,7 @@ def _kept_cache(Cache):
                 self.look_for(key_states, value_states, layer_idx)
             keys, values = super().update(key_states, value_states, layer_idx, *args, **kwargs)
             if keys is key_states and values is value_states:
-                if self.arrived is None or self.arrived(layer_idx, keys, values):
+                if self.arrived is None or self.me == id(self) and self.arrived(layer_idx, keys, values):
                     self.kept[layer_idx] = keys, values
                 else:
                     keys, values = keys.clone(), values.clone()
@@ -176,15 +181,15 @@ def _prompt_cache(arrived=None, copies=False):
 
     Nothing says that the model leaves a kept layer's tensors alone for the rest of its pass.  ``arrived(layer, k, v)``
     therefore reads them then and there; where it returns False they are copied after all.  Memory that comes back with
-    another layer, or with more tokens of the same one, was filled again: appending to the layer that was there raises
-    ``_Refilled``, and the pass has to be made again with ``copies``, a plain ``DynamicCache``."""
+    another layer, or with more tokens of the same one, was filled again: the layer that was there is in ``refilled``,
+    appending to it raises ``_Refilled``, and the pass has to be made again with ``copies``, a plain ``DynamicCache``."""
     plain, kept_cache, kept_layer = _prompt_classes()
     if copies or kept_cache is None:
         return plain()
     cache = kept_cache()
     cache.layer_class_to_replicate = kept_layer
-    # kept: layer -> K, V; where: address -> layer, of the first `listed` ones; refilled: layers whose memory came again
-    cache.arrived, cache.kept, cache.where, cache.listed, cache.refilled = arrived, {}, {}, 0, set()
+    # me: not a copy of it that the model made; kept: layer -> K, V; where: address -> layer, of the first `listed` ones; refilled: layers whose memory came again
+    cache.arrived, cache.me, cache.kept, cache.where, cache.listed, cache.refilled = arrived, id(cache), {}, {}, 0, set()
     return cache
 
 

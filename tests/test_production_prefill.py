@@ -144,6 +144,28 @@ def test_tokens_behind_a_whole_prompt_and_a_changed_layer():
         assert torch.equal(cache.v[0][s], v[0][:, :, s]) and torch.equal(cache.v[1][s], v[1][:, :, s])
 
 
+def test_a_cache_that_is_copied_or_cut_in_the_pass():
+    import copy
+    k, v = _layers(20, torch.float16, 3)
+
+    class Model(_Scratch):
+        def __call__(self, input_ids, past_key_values=None, **kwargs):
+            other = copy.deepcopy(past_key_values)
+            super().__call__(input_ids, past_key_values=past_key_values)
+            for li in range(3):                          # a second pass with a cache of its own
+                other.update(self.k[li] + 1, self.v[li] + 1, li)
+            past_key_values.layers[0].keys = past_key_values.layers[0].keys[:, :, 3:]
+            past_key_values.layers[0].values = past_key_values.layers[0].values[:, :, 3:]
+            return self
+
+    model, cache = Model(k, v, 20), _Reads()
+    production_prefill(model, torch.zeros(1, 17, dtype=torch.long), cache)
+    assert model.passes == 2
+    for s in range(17):
+        assert torch.equal(cache.k[0][s], k[0][:, :, s + 3]) and torch.equal(cache.v[0][s], v[0][:, :, s + 3])
+        assert torch.equal(cache.k[1][s], k[1][:, :, s]) and torch.equal(cache.v[1][s], v[1][:, :, s])
+
+
 @pytest.mark.parametrize("fails_at,left", [(0, 9), (1, 0)])
 def test_a_forward_pass_that_fails(fails_at, left):
     k, v = _layers(12, torch.float16, 2)
