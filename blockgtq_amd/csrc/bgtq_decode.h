@@ -35,6 +35,7 @@ struct DecodeArgs {
     int nfull[4];
     uint64_t last[4];
     int per_tiles, rem_tiles;   // MFMA kernel, equal row lengths: tiles per partition, partitions with one more
+    const int32_t* row_order;   // MFMA kernel: batch row of a grid row, or null: rows as they come
 };
 
 // Fast path: MFMA kernel for packed K and V records (bgtq_decode_seg.hip).
@@ -47,4 +48,5 @@ constexpr int BGTQ_ONE_LAUNCH_ROWS = 64;
 
 // The preparation part of bgtq_decode_step (bgtq_encode.hip).  kv_fp16: k and v are fp16 whatever x_dtype says.
 // window: the buffered tokens' partial, computed in the same launch (window_rides, at most BGTQ_ONE_LAUNCH_ROWS rows), or null.
-int bgtq_step_prepare(const bgtq_step& s, bool kv_fp16, const WindowArgs* window, hipStream_t st);
+// order: null, or where the batch rows go by falling s.seq_lens (s.B * s.S at most BGTQ_ONE_LAUNCH_ROWS).
+int bgtq_step_prepare(const bgtq_step& s, bool kv_fp16, const WindowArgs* window, int32_t* order, hipStream_t st);

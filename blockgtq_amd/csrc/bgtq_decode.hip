@@ -547,6 +547,75 @@ int pick_splits(int B, int n_kv, int max_T, bool ragged) {
     return best;
 }
 
+// Whether a step sends rows of different lengths out by falling length (ranked in the launch that prepares the step): where
+// there is more than one round of work-groups, the long partitions first and the short ones into the places that come free.
+// The same partitions, the same results.  us a step, rows as they come and in order:
+//   20 rows x 8 heads, up to 8k:  48.3, 40.8 (3 partitions)    16 x 8, 16k: 64.4, 56.3 (6)
+//   24 rows x 4 heads, up to 16k: 55.6, 52.7 (8)               32 x 8, 16k: 96.2, 94.5 (4)
+// and with all rows equal after all 54.7, 54.8; 73.1, 73.5; 62.6, 63.3; 142.1, 141.4.  (Fewer partitions would do now, 90.2 us with
+// two for the last; other partitions mean other roundings.)
+bool orders_rows(int B, int n_kv, int S, int n_splits, bool ragged) {
+    return ragged && B > 1 && (int64_t)B * S <= BGTQ_ONE_LAUNCH_ROWS && (int64_t)B * n_kv * n_splits > 256;
+}
+
+// The order lies at the start of the step's output, which nothing else writes before the partitions are merged: not where
+// an input lies there too, or where it would not be aligned
+bool order_fits(const bgtq_step& s) {
+    const uintptr_t lo = (uintptr_t)s.out, hi = lo + (size_t)s.B * sizeof(int32_t);
+    auto apart = [&](const void* p, int64_t sb, int64_t n, int64_t sh, int64_t m, int64_t ss) {
+        if (sb < 0 || sh < 0 || ss < 0) return false;
+        const uintptr_t at = (uintptr_t)p;
+        return at >= hi || at + (size_t)((s.B - 1) * sb + (n - 1) * sh + (m - 1) * ss + D) * 2 <= lo;
+    };
+    return (lo & 3) == 0 && apart(s.q, s.q_sb, (int64_t)s.n_kv * s.gqa, s.q_sh, 1, 0) && apart(s.k, s.k_sb, s.n_kv, s.k_sh, s.S, s.k_ss) &&
+           apart(s.v, s.v_sb, s.n_kv, s.v_sh, s.S, s.v_ss);
+}
+
+int decode_attn(const bgtq_head_plan* plans,
+                const void* q_rot, int64_t q_sb, int64_t q_sh,
+                const void* k_packed, int64_t kp_sb, int64_t kp_sh, int64_t kp_st, int k_row_width,
+                const void* k_norms, int64_t kn_sb, int64_t kn_sh, int64_t kn_st,
+                const void* v_packed, int64_t vp_sb, int64_t vp_sh, int64_t vp_st, int v_row_width,
+                const void* v_norms, int64_t vn_sb, int64_t vn_sh, int64_t vn_st,
+                const int32_t* seq_lens, int T,
+                int B, int n_kv, int gqa, int n_splits,
+                float* partial_out, float* partial_lse,
+                int k_layout, int v_layout, float scale, const int32_t* row_order, void* stream) {
+    BGTQ_CHECK_ARG(plans && q_rot && k_packed && k_norms && v_packed && v_norms);
+    BGTQ_CHECK_ARG(partial_out && partial_lse);
+    BGTQ_CHECK_ARG(B >= 0 && n_kv >= 0 && T >= 0);
+    BGTQ_CHECK_ARG(gqa >= 1 && gqa <= BGTQ_MAX_GQA);
+    BGTQ_CHECK_ARG(k_layout == BGTQ_K_BITPACKED || k_layout == BGTQ_K_MIXED);
+    BGTQ_CHECK_ARG(v_layout == BGTQ_V_BITPACKED || v_layout == BGTQ_V_NIBBLE);
+    if (n_splits > BGTQ_MAX_SPLITS) return BGTQ_ELIMIT;
+    BGTQ_CHECK_ARG(n_splits >= 1);
+    if (B == 0 || n_kv == 0) return BGTQ_OK;
+    DecodeArgs a{};
+    a.plans = plans;
+    a.q = (const uint16_t*)q_rot; a.q_sb = q_sb; a.q_sh = q_sh;
+    a.kp = (const uint8_t*)k_packed; a.kp_sb = kp_sb; a.kp_sh = kp_sh; a.kp_st = kp_st;
+    a.kn = (const uint16_t*)k_norms; a.kn_sb = kn_sb; a.kn_sh = kn_sh; a.kn_st = kn_st;
+    a.vp = (const uint8_t*)v_packed; a.vp_sb = vp_sb; a.vp_sh = vp_sh; a.vp_st = vp_st;
+    a.vn = (const uint16_t*)v_norms; a.vn_sb = vn_sb; a.vn_sh = vn_sh; a.vn_st = vn_st;
+    a.seq_lens = seq_lens; a.T = T; a.row_order = row_order;
+    a.B = B; a.n_kv = n_kv; a.gqa = gqa; a.n_splits = n_splits;
+    a.part_out = partial_out; a.part_lse = partial_lse;
+    a.k_layout = k_layout; a.v_layout = v_layout; a.scale = scale;
+    BGTQ_CHECK_ARG(k_row_width >= 1 && k_row_width <= BGTQ_D);
+    BGTQ_CHECK_ARG(v_row_width >= 1 && v_row_width <= BGTQ_D / 2);
+    a.k_row_width = k_row_width; a.v_row_width = v_row_width;
+    hipStream_t st = (hipStream_t)stream;
+    if (g_decode_path != 1) {
+        int rc = bgtq_launch_decode_seg(a, st);
+        if (rc != BGTQ_EUNSUPPORTED) { g_last_path = 2; return rc; }
+        if (g_decode_path == 2) return rc;        // forced fast path: report why it refused
+    }
+    g_last_path = 1;
+    if (gqa <= 4) return launch_generic<4>(a, st);
+    if (gqa <= 8) return launch_generic<8>(a, st);
+    return launch_generic<16>(a, st);
+}
+
 }  // namespace
 
 extern "C" {
@@ -578,39 +647,9 @@ int bgtq_decode_attn(const bgtq_head_plan* plans,
                      int B, int n_kv, int gqa, int n_splits,
                      float* partial_out, float* partial_lse,
                      int k_layout, int v_layout, float scale, void* stream) {
-    BGTQ_CHECK_ARG(plans && q_rot && k_packed && k_norms && v_packed && v_norms);
-    BGTQ_CHECK_ARG(partial_out && partial_lse);
-    BGTQ_CHECK_ARG(B >= 0 && n_kv >= 0 && T >= 0);
-    BGTQ_CHECK_ARG(gqa >= 1 && gqa <= BGTQ_MAX_GQA);
-    BGTQ_CHECK_ARG(k_layout == BGTQ_K_BITPACKED || k_layout == BGTQ_K_MIXED);
-    BGTQ_CHECK_ARG(v_layout == BGTQ_V_BITPACKED || v_layout == BGTQ_V_NIBBLE);
-    if (n_splits > BGTQ_MAX_SPLITS) return BGTQ_ELIMIT;
-    BGTQ_CHECK_ARG(n_splits >= 1);
-    if (B == 0 || n_kv == 0) return BGTQ_OK;
-    DecodeArgs a{};
-    a.plans = plans;
-    a.q = (const uint16_t*)q_rot; a.q_sb = q_sb; a.q_sh = q_sh;
-    a.kp = (const uint8_t*)k_packed; a.kp_sb = kp_sb; a.kp_sh = kp_sh; a.kp_st = kp_st;
-    a.kn = (const uint16_t*)k_norms; a.kn_sb = kn_sb; a.kn_sh = kn_sh; a.kn_st = kn_st;
-    a.vp = (const uint8_t*)v_packed; a.vp_sb = vp_sb; a.vp_sh = vp_sh; a.vp_st = vp_st;
-    a.vn = (const uint16_t*)v_norms; a.vn_sb = vn_sb; a.vn_sh = vn_sh; a.vn_st = vn_st;
-    a.seq_lens = seq_lens; a.T = T;
-    a.B = B; a.n_kv = n_kv; a.gqa = gqa; a.n_splits = n_splits;
-    a.part_out = partial_out; a.part_lse = partial_lse;
-    a.k_layout = k_layout; a.v_layout = v_layout; a.scale = scale;
-    BGTQ_CHECK_ARG(k_row_width >= 1 && k_row_width <= BGTQ_D);
-    BGTQ_CHECK_ARG(v_row_width >= 1 && v_row_width <= BGTQ_D / 2);
-    a.k_row_width = k_row_width; a.v_row_width = v_row_width;
-    hipStream_t st = (hipStream_t)stream;
-    if (g_decode_path != 1) {
-        int rc = bgtq_launch_decode_seg(a, st);
-        if (rc != BGTQ_EUNSUPPORTED) { g_last_path = 2; return rc; }
-        if (g_decode_path == 2) return rc;        // forced fast path: report why it refused
-    }
-    g_last_path = 1;
-    if (gqa <= 4) return launch_generic<4>(a, st);
-    if (gqa <= 8) return launch_generic<8>(a, st);
-    return launch_generic<16>(a, st);
+    return decode_attn(plans, q_rot, q_sb, q_sh, k_packed, kp_sb, kp_sh, kp_st, k_row_width, k_norms, kn_sb, kn_sh, kn_st,
+                       v_packed, vp_sb, vp_sh, vp_st, v_row_width, v_norms, vn_sb, vn_sh, vn_st, seq_lens, T, B, n_kv, gqa,
+                       n_splits, partial_out, partial_lse, k_layout, v_layout, scale, nullptr, stream);
 }
 
 int bgtq_lse_reduce(const bgtq_head_plan* plans,
@@ -738,14 +777,15 @@ int bgtq_decode_step(const bgtq_step* step, void* stream) {
         s.k = old_k; s.v = old_v;
         s.k_sb = s.v_sb = (int64_t)s.n_kv * D; s.k_sh = s.v_sh = D; s.k_ss = s.v_ss = D;
     }
-    int rc = bgtq_step_prepare(s, windowed && s.x_dtype == BGTQ_X_BF16, window.q ? &window : nullptr, st);
+    int32_t* order = orders_rows(s.B, s.n_kv, s.S, s.n_splits, s.seq_lens != nullptr) && order_fits(*step) ? (int32_t*)s.out : nullptr;
+    int rc = bgtq_step_prepare(s, windowed && s.x_dtype == BGTQ_X_BF16, window.q ? &window : nullptr, order, st);
     if (rc != BGTQ_OK) return rc;
     const void* q = s.q_rot ? s.q_rot : s.q;
-    rc = bgtq_decode_attn(s.plans, q, s.q_rot ? (int64_t)n_q * D : s.q_sb, s.q_rot ? D : s.q_sh,
+    rc = decode_attn(s.plans, q, s.q_rot ? (int64_t)n_q * D : s.q_sb, s.q_rot ? D : s.q_sh,
                           s.k_packed, s.kp_sb, s.kp_sh, s.kp_st, s.k_row_width, s.k_norms, s.kn_sb, s.kn_sh, s.kn_st,
                           s.v_packed, s.vp_sb, s.vp_sh, s.vp_st, s.v_row_width, s.v_norms, s.vn_sb, s.vn_sh, s.vn_st,
                           s.seq_lens, s.T, s.B, s.n_kv, s.gqa, s.n_splits, s.partial_out, s.partial_lse,
-                          s.k_layout, s.v_layout, s.scale, stream);
+                          s.k_layout, s.v_layout, s.scale, order, stream);
     if (rc != BGTQ_OK) return rc;
     return bgtq_lse_reduce(s.plans, s.partial_out, s.partial_lse, s.n_splits, windowed ? s.win_out : nullptr,
                            windowed ? s.win_lse : nullptr, windowed ? 1 : 0, s.B, s.n_kv, s.gqa, 1,
@@ -754,7 +794,7 @@ int bgtq_decode_step(const bgtq_step* step, void* stream) {
 
 size_t bgtq_plan_sizeof(void) { return sizeof(bgtq_head_plan); }
 int bgtq_abi_version(void) { return 8; }
-int bgtq_decode_kernel_revision(void) { return 8; }
+int bgtq_decode_kernel_revision(void) { return 9; }
 
 const char* bgtq_strerror(int code) {
     switch (code) {

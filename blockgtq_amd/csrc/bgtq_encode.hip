@@ -1209,6 +1209,19 @@ __global__ __launch_bounds__(NT) void rotate_q_kernel(RotQArgs a) {
     rotate_q_block(a, blockIdx.x, rot_s);
 }
 
+// ---- batch rows by falling length, for the attention launch that follows: lengths on the device, one work-group ----
+struct RankArgs { const int32_t* lens; int32_t* order; int B; };      // order null: not asked for
+
+__device__ __forceinline__ void rank_rows(const RankArgs& r, const int tid, int* lens_s) {
+    const int len = tid < r.B ? r.lens[tid] : 0;
+    if (tid < r.B) lens_s[tid] = len;
+    __syncthreads();
+    if (tid >= r.B) return;
+    int rank = 0;                                             // (equal rows stay in order)
+    for (int i = 0; i < r.B; i++) rank += lens_s[i] > len || (lens_s[i] == len && i < tid) ? 1 : 0;
+    r.order[rank] = tid;
+}
+
 // ---- decode-step preparation: append-encode K and V and rotate the queries, one launch ----
 // Work-groups [0, n) encode one V row of one head each (the longest chain of the three goes out first),
 // [n, 2 n) one K row each, the rest rotate one or four query heads each.
@@ -1225,10 +1238,14 @@ __device__ __forceinline__ void prepare_part(const EncodeArgs& ak, const EncodeA
     }
 }
 // (BF16: some input is; asking at run time costs the chains of fp16 inputs 0.2 of 5.0 us)
-template <bool BF16>
-__global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, int rows) {
+template <bool BF16, bool RANK>
+__global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, int rows, RankArgs rank) {
     if (!BF16) ak.bf16 = av.bf16 = aq.bf16 = 0;
     __shared__ __align__(16) float rot_s[D * D];       // the work-group's rotation, whatever its role
+    if (RANK && blockIdx.x == gridDim.x - 1) {         // (uniform)
+        rank_rows(rank, threadIdx.x, (int*)rot_s);
+        return;
+    }
     prepare_part(ak, av, aq, rows, blockIdx.x, rot_s);
 }
 // The same with the attention over the buffered tokens, which depends on none of it: the longer work-groups first, in
@@ -1237,14 +1254,18 @@ __global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs a
 // buffer here, put there by those who read the one that leaves.
 // 32 rows x 8 heads x 4 queries over 132 buffered tokens: 4.9 (swap) + 11.1 + 13.3 us as launches of their own, 4.9 + 16.3
 // with K and V a work-group each and the swap ahead of them (1024 work-groups, two of them at a time on a compute unit), 14 here.
-template <bool SWAP>
+template <bool SWAP, bool RANK>
 __global__ __launch_bounds__(WINDOW_THREADS, 2) void prepare_window_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, WindowArgs w,
-                                                                        RingArgs rk, RingArgs rv, int rows, int n_window) {
+                                                                        RingArgs rk, RingArgs rv, int rows, int n_window, RankArgs rank) {
     __shared__ __align__(16) float rot_s[D * D];
     static_assert(window_lds_floats<4>(WINDOW_RIDE_W) <= D * D, "a window's scores fit the rotation's place");
     static_assert(WINDOW_THREADS == 2 * NT, "");
     int bid = blockIdx.x;
     const int n_kv = ak.n_kv, tid = threadIdx.x;
+    if (RANK && bid == (int)gridDim.x - 1) {
+        rank_rows(rank, tid, (int*)rot_s);
+        return;
+    }
     if (bid < n_window) {
         window_attn_block<4, SWAP>(w, bid % n_kv, bid / n_kv, rot_s);
         return;
@@ -1318,7 +1339,7 @@ int launch_rotate_q(const bgtq_head_plan* plans, const void* q, int64_t q_sr, in
 
 // K and V appended and (q not null) the queries rotated: one launch for the few rows of a decode step
 int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, int64_t q_sr, int64_t q_sh, int q_bf16,
-                   void* q_rot, int64_t qr_sr, int64_t qr_sh, int gqa, const WindowArgs* window, hipStream_t st) {
+                   void* q_rot, int64_t qr_sr, int64_t qr_sh, int gqa, const WindowArgs* window, const RankArgs& rank, hipStream_t st) {
     const int B = ak.B, n_kv = ak.n_kv;
     const int64_t N = (int64_t)B * ak.S;
     if (N > BGTQ_ONE_LAUNCH_ROWS) {          // prefill-sized append: the three stages are big enough on their own
@@ -1329,18 +1350,21 @@ int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, in
     const int group = rotate_q_group_size(B, n_kv * gqa);
     RotQArgs aq{ak.plans, (const uint16_t*)q, q_sr, q_sh, (uint16_t*)q_rot, qr_sr, qr_sh, B, n_kv * gqa, gqa, group, q_bf16};
     const int rows = (int)N;
-    const unsigned blocks = (unsigned)(2 * rows * n_kv) + (q ? rotate_q_blocks(B, n_kv, gqa, group) : 0u);
+    const unsigned blocks = (unsigned)(2 * rows * n_kv) + (q ? rotate_q_blocks(B, n_kv, gqa, group) : 0u) + (rank.order ? 1u : 0u);
     if (window) {
         const WindowArgs& w = *window;
         const dim3 grid(blocks - (unsigned)(rows * n_kv) + (unsigned)(B * n_kv));
         const RingArgs rk{w.swap.slot, (uint16_t*)w.kbuf, w.w_sb, w.w_sh, w.w_st, w.W, w.swap.k, w.swap.k_sb, w.swap.k_sh, w.bf16};
         const RingArgs rv{w.swap.slot, (uint16_t*)w.vbuf, w.w_sb, w.w_sh, w.w_st, w.W, w.swap.v, w.swap.v_sb, w.swap.v_sh, w.bf16};
-        if (w.swap.slot) hipLaunchKernelGGL(prepare_window_kernel<true>, grid, dim3(WINDOW_THREADS), 0, st, ak, av, aq, w, rk, rv, rows, B * n_kv);
-        else hipLaunchKernelGGL(prepare_window_kernel<false>, grid, dim3(WINDOW_THREADS), 0, st, ak, av, aq, w, rk, rv, rows, B * n_kv);
-    } else if (ak.bf16 || av.bf16 || (q && q_bf16))
-        hipLaunchKernelGGL(prepare_kernel<true>, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows);
-    else
-        hipLaunchKernelGGL(prepare_kernel<false>, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows);
+        auto kern = w.swap.slot ? (rank.order ? prepare_window_kernel<true, true> : prepare_window_kernel<true, false>)
+                                : (rank.order ? prepare_window_kernel<false, true> : prepare_window_kernel<false, false>);
+        hipLaunchKernelGGL(kern, grid, dim3(WINDOW_THREADS), 0, st, ak, av, aq, w, rk, rv, rows, B * n_kv, rank);
+    } else {
+        const bool bf16 = ak.bf16 || av.bf16 || (q && q_bf16);
+        auto kern = rank.order ? (bf16 ? prepare_kernel<true, true> : prepare_kernel<false, true>)
+                               : (bf16 ? prepare_kernel<true, false> : prepare_kernel<false, false>);
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows, rank);
+    }
     return bgtq_launch_status();
 }
 
@@ -1358,14 +1382,14 @@ int fill_step_args(const bgtq_step& s, EncodeArgs& ak, EncodeArgs& av) {
 
 }  // namespace
 
-int bgtq_step_prepare(const bgtq_step& s, bool kv_fp16, const WindowArgs* window, hipStream_t st) {
+int bgtq_step_prepare(const bgtq_step& s, bool kv_fp16, const WindowArgs* window, int32_t* order, hipStream_t st) {
     EncodeArgs ak{}, av{};
     const int rc = fill_step_args(s, ak, av);
     if (rc != BGTQ_OK) return rc;
     const int q_bf16 = ak.bf16;
     if (kv_fp16) ak.bf16 = av.bf16 = 0;
     return launch_prepare(ak, av, s.q_rot ? s.q : nullptr, s.q_sb, s.q_sh, q_bf16, s.q_rot,
-                          (int64_t)s.n_kv * s.gqa * D, D, s.gqa, window, st);
+                          (int64_t)s.n_kv * s.gqa * D, D, s.gqa, window, RankArgs{s.seq_lens, order, s.B}, st);
 }
 
 extern "C" {
@@ -1376,7 +1400,7 @@ int bgtq_encode_kv(const bgtq_step* step, void* stream) {
     EncodeArgs ak{}, av{};
     const int rc = fill_step_args(*step, ak, av);
     if (rc != BGTQ_OK) return rc;
-    return launch_prepare(ak, av, nullptr, 0, 0, 0, nullptr, 0, 0, 1, nullptr, (hipStream_t)stream);
+    return launch_prepare(ak, av, nullptr, 0, 0, 0, nullptr, 0, 0, 1, nullptr, RankArgs{}, (hipStream_t)stream);
 }
 
 int bgtq_encode_k(const bgtq_head_plan* plans,
@@ -1469,7 +1493,7 @@ int bgtq_decode_prepare(const bgtq_head_plan* plans,
                      v_norms, vn_sb, vn_sh, vn_st, t_pos, t_pos_scalar, max_T, v_layout);
     if (rc != BGTQ_OK) return rc;
     BGTQ_CHECK_ARG((q == nullptr) == (q_rot == nullptr));     // both, or neither (queries rotated elsewhere)
-    return launch_prepare(ak, av, q, q_sr, q_sh, 0, q_rot, qr_sr, qr_sh, gqa, nullptr, (hipStream_t)stream);
+    return launch_prepare(ak, av, q, q_sr, q_sh, 0, q_rot, qr_sr, qr_sh, gqa, nullptr, RankArgs{}, (hipStream_t)stream);
 }
 
 

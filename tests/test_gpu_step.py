@@ -281,3 +281,26 @@ def test_buffered_step_with_a_new_token_that_nobody_sees(bad, n_q):
         m._buffered_step_indices = lambda: idx
     fast, slow = [m.append_and_attend(0, q, k, v) for m in mgrs]
     assert torch.isfinite(slow).all() and slow.abs().max() > 0 and torch.equal(fast, slow)
+
+
+# more than one round of work-groups: rows go out by falling length.  Ties, equal rows, empty rows, all 64 rows a step ranks
+@pytest.mark.parametrize("batch,n_kv,splits,window,kind", [(33, 8, 1, 0, "mixed"), (64, 1, 5, 0, "mixed"), (64, 8, 2, 0, "equal"), (9, 2, 16, 0, "mixed"),
+                                                           (33, 4, 2, 64, "mixed"), (65, 4, 1, 0, "mixed")])
+def test_rows_by_falling_length_change_nothing(batch, n_kv, splits, window, kind):
+    context = 700
+    gen = torch.Generator().manual_seed(batch)
+    lens = [context] * batch if kind == "equal" else torch.randint(window + 5 if window else 0, context + 1, (batch,), generator=gen).tolist()
+    lens[0] = context
+    lens[batch // 2] = lens[batch // 3]
+    w = wl.Workload("t", 1, 2 * n_kv, n_kv, batch, context, 1e6, seq_lens=lens, n_sink=4 if window else 0, window=window, seed=37)
+    mgrs = []
+    for _ in range(2):
+        mgr, energies = wl.build_manager(w, DEV)
+        wl.fill_cache(mgr, w, energies, DEV)
+        mgr.n_splits = splits
+        mgrs.append(mgr)
+    q, k, v = _inputs(w, energies, context, torch.float16)
+    general = mgrs[1]
+    general._native = lambda li: general._ensure_storage()          # (rows as they come)
+    for _ in range(2):
+        assert torch.equal(mgrs[0].append_and_attend(0, q, k, v), general.append_and_attend(0, q, k, v))
