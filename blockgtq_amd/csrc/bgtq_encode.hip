@@ -539,46 +539,125 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
     const bool need_cent = IS_V || a.layout == BGTQ_K_MIXED || a.corrected;
 
     // ---- once per work-group: tables and the rotation (64 KB, straight from the plan into LDS).  Everything is
-    // requested in one burst
-    {
+    // requested in one burst: every thread loads, the ones past a table's end its last words, and stores behind all loads (a
+    // load inside `if (tid < ..)` is waited for there, and K's tables were six round trips one after the other: 19.3 -> 18.6 us for
+    // 8 heads of 2001 tokens)
+    constexpr int RT = CS == 4 ? 4 : 1;                       // K: 4 x 4 pieces of the rotation in flight a thread
+    float4 rot4[RT][4];
+    auto fetch_rot = [&](int at) {                            // (k_rot_T is zero outside a column's own segment)
+#pragma unroll
+        for (int n = 0; n < RT; n++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int piece = min(at + n * NTHR, D * D / 16 - 1);        // rows 4 (piece / 32) .., columns 4 (piece % 32) ..
+                rot4[n][r] = *(const float4*)&P.k_rot_T[((piece >> 5) * 4 + r) * D + (piece & 31) * 4];
+            }
+    };
+    if constexpr (IS_V) {                                     // (the plan holds it in this order)
         const uint32_t dst = (uint32_t)(uintptr_t)(lds_ptr_t)(uint8_t*)&L.rot[0][0][0];
-        if constexpr (IS_V) {                                 // (the plan holds it in this order)
-            const uint8_t* src = (const uint8_t*)&P.v_rot_T4[0][0][0];
-            for (int c = wave * 4; c < 64; c += NW * 4) dma_full<4>((uint32_t)lane * 16, uniform_ptr(src + c * 1024), dst + c * 1024);
-        } else {                                              // four rows interleaved on the way: lane = (column, row) of 16 x 4
-            const uint32_t off = (uint32_t)((lane & 3) * D + (lane >> 2)) * 4;
-            for (int c = wave; c < 256; c += NW) {            // (k_rot_T is zero outside a column's own segment)
-                const uint8_t* src = uniform_ptr((const uint8_t*)P.k_rot_T + (c >> 3) * (4 * D * 4) + (c & 7) * 64);
-                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1\n"
-                             :: "v"(off), "s"(src), "s"(dst + c * 256) : "memory", "m0");
+        const uint8_t* src = (const uint8_t*)&P.v_rot_T4[0][0][0];
+        for (int c = wave * 4; c < 64; c += NW * 4) dma_full<4>((uint32_t)lane * 16, uniform_ptr(src + c * 1024), dst + c * 1024);
+    } else {
+        fetch_rot(tid);
+    }
+    // ---- CS waves a block: the block's place in the work-group, this wave's part of it
+    const int slot = CS == 1 ? wave : wave / CS, part = CS == 1 ? 0 : wave % CS;
+    const bool wide = ((a.x_sb | a.x_sh | a.x_ss) & 7) == 0 && ((uintptr_t)a.x & 15) == 0;
+    // (batch row, step) of row r of the block whose first row is step s0 of batch row b0
+    auto row_of = [&](int b0, int s0, int r, int& b, int& s) {
+        b = b0;
+        s = s0 + r;
+        if (s >= a.S) { const unsigned q = (unsigned)s / (unsigned)a.S; b += (int)q; s -= (int)q * a.S; }
+    };
+    // Raw rows, 16 lanes a row, 8 values each.  AHEAD: the first block's with the tables, the next one's before a block's
+    // records go out (8 heads of 128 tokens 14.0 -> 11.5 us, of 2001 17.5 -> 16.4; with a wave a block V's waves came to the
+    // matrix core together and the registers spilled: 31.4 -> 35.3)
+    constexpr int PASS = 4 / CS;
+    constexpr bool AHEAD = CS > 1;
+    uint4 x4[PASS];
+    auto fetch_rows = [&](int blk) {
+        const unsigned n0 = (unsigned)blk * 16u;
+        const int b0 = (int)(n0 / (unsigned)a.S), s0 = (int)(n0 - (unsigned)b0 * (unsigned)a.S);
+#pragma unroll
+        for (int p = 0; p < PASS; p++) {
+            const int r = 4 * (part * PASS + p) + (lane >> 4);
+            x4[p] = uint4{0, 0, 0, 0};
+            if ((int64_t)n0 + r < N) {
+                int b, s;
+                row_of(b0, s0, r, b, s);
+                const uint16_t* src = a.x + b * a.x_sb + h * a.x_sh + s * a.x_ss + (lane & 15) * 8;
+                if (wide) x4[p] = *(const uint4*)src;
+                else {
+                    uint32_t w[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) w[i] = (uint32_t)src[2 * i] | ((uint32_t)src[2 * i + 1] << 16);
+                    x4[p] = uint4{w[0], w[1], w[2], w[3]};
+                }
             }
         }
-    }
+    };
+    if (AHEAD) fetch_rows(first * NB + slot);
     int n_seg = 1, v_bits = 0, n_zero = 0;
     float bd[15];                                             // V boundaries (+inf past the last)
     uint2 byte_of = {0u, 0u};
     uint32_t seg_of[4] = {0, 0, 0, 0};                        // group of dim 4 kk + lg, 4 bits each
+    const int td = tid & (D - 1);
     if constexpr (IS_V) {
         v_bits = P.v_bits;
 #pragma unroll
         for (int b = 0; b < 15; b++) bd[b] = P.v_boundaries[b];
-        if (tid < 16) L.cent[tid] = P.v_centroids[tid];
-        if (tid < D / 2) byte_of = *(const uint2*)P.enc_vbyte[a.layout == BGTQ_V_NIBBLE ? 1 : 0][tid];
+        const float cent = P.v_centroids[tid & 15];
+        byte_of = *(const uint2*)P.enc_vbyte[a.layout == BGTQ_V_NIBBLE ? 1 : 0][tid & (D / 2 - 1)];
+        if (tid < 16) L.cent[tid] = cent;
+        if (tid >= D / 2) byte_of = uint2{0u, 0u};
         if (tid < D) L.place[tid] = (uint16_t)(((tid & 3) * (D / 4) + (tid >> 2)) * 2);
     } else {
         n_seg = P.n_seg;
         n_zero = P.n_zero_dims;
+        constexpr int LUT_WORDS = BGTQ_MAX_SEGMENTS * BGTQ_LUT_BINS / 4, N_CENT = BGTQ_MAX_SEGMENTS * 32;
+        static_assert(N_CENT <= 256 && LUT_WORDS <= 512, "at least 256 threads, two words of the cell tables each");
         const uint4 segs = ((const uint4*)((const uint8_t*)P.lut_image[BGTQ_K_BITPACKED] + BGTQ_LUT_KSEG))[lg];
+        const int hdr = ((const int*)&P)[min(tid, 55)];
+        const uint32_t* cells = (const uint32_t*)&P.code_lut[0][0];
+        const uint32_t cell0 = cells[min(tid, LUT_WORDS - 1)], cell1 = cells[min(tid + NTHR, LUT_WORDS - 1)];
+        const float cent = (&P.k_centroids[0][0])[(min(tid, N_CENT - 1) >> 5) * (int)(sizeof(P.k_centroids[0]) / sizeof(float)) + (tid & 31)];
+        const int4 dim = *(const int4*)P.enc_dim[td];
+        const float2 bin = {P.lut_offset[td], P.lut_inv_scale[td]};
+        byte_of = *(const uint2*)P.enc_byte[a.layout == BGTQ_K_MIXED ? 1 : 0][td];
         seg_of[0] = segs.x; seg_of[1] = segs.y; seg_of[2] = segs.z; seg_of[3] = segs.w;
-        if (tid < 56) L.hdr[tid] = ((const int*)&P)[tid];
-        for (int i = tid; i < BGTQ_MAX_SEGMENTS * BGTQ_LUT_BINS / 4; i += NTHR) ((uint32_t*)L.lut)[i] = ((const uint32_t*)&P.code_lut[0][0])[i];
-        if (tid < BGTQ_MAX_SEGMENTS * 32) L.cent[tid] = P.k_centroids[tid >> 5][tid & 31];
+        if (tid < 56) L.hdr[tid] = hdr;
+        if (tid < LUT_WORDS) ((uint32_t*)L.lut)[tid] = cell0;
+        if (tid + NTHR < LUT_WORDS) ((uint32_t*)L.lut)[tid + NTHR] = cell1;
+        if (tid < N_CENT) L.cent[tid] = cent;
         if (tid < D) {                                        // packed dim k lies at [k % 4][k / 4] of a raw row
-            const int4 dim = *(const int4*)P.enc_dim[tid];
             L.group[tid] = (int8_t)dim.x;
             L.place[dim.w >> 8] = (uint16_t)(((tid & 3) * (D / 4) + (tid >> 2)) * 2);
-            L.bin[tid] = float2{P.lut_offset[tid], P.lut_inv_scale[tid]};
-            byte_of = *(const uint2*)P.enc_byte[a.layout == BGTQ_K_MIXED ? 1 : 0][tid];
+            L.bin[tid] = bin;
+        }
+        // The rotation, four rows interleaved on the way (as 256 loads of 16 columns of a row into LDS 0.4 us more).  A thread's columns leave in an order of its own, from column
+        // (tid / 4) % 4 of the four on: 16 lanes then write 256 bytes of 64 banks.
+        for (int at = tid;;) {
+#pragma unroll
+            for (int n = 0; n < RT; n++) {
+                const int piece = at + n * NTHR, turn = (piece >> 2) & 3;
+                if (piece >= D * D / 16) continue;
+                float x[4][4];                                // [row][columns from `turn` on]
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float c[4] = {rot4[n][r].x, rot4[n][r].y, rot4[n][r].z, rot4[n][r].w};
+                    float half[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) half[i] = turn & 2 ? c[(i + 2) & 3] : c[i];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) x[r][i] = turn & 1 ? half[(i + 1) & 3] : half[i];
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    *(float4v*)L.rot[piece >> 5][(piece & 31) * 4 + ((i + turn) & 3)] = (float4v){x[0][i], x[1][i], x[2][i], x[3][i]};
+            }
+            at += RT * NTHR;
+            if (at - tid >= D * D / 16) break;                // (uniform)
+            fetch_rot(at);
         }
     }
     const int lpr = a.row_width > 64 ? 32 : 16;               // packing: lanes per row, lane = record dword dw
@@ -590,23 +669,20 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         const int mode = (int)(e.x & 3u), bw = (int)((e.x >> 2) & 15u), skip = (int)((e.x >> 6) & 3u), n = (int)(e.x >> 8);
         uint4 p = {e.y, 0u, 0u, 0u};
         if (mode == 2 || (mode == 1 && n > 0)) p.y = (uint32_t)skip | ((8u - skip) << 8);
-        if (mode == 1)
-            for (int c = 1; c < n; c++) {
-                const uint32_t w = 1u << (c * bw - skip);
-                if (c < 4) p.z |= w << (8 * c);
-                else p.w |= (w >> 4) << (8 * (c - 4));        // (1-bit codes only: the second four make a nibble of their own)
-            }
+#pragma unroll
+        for (int c = 1; c < 8; c++) {
+            const uint32_t w = mode == 1 && c < n ? 1u << ((c * bw - skip) & 31) : 0u;
+            if (c < 4) p.z |= w << (8 * c);
+            else p.w |= (w >> 4) << (8 * (c - 4));            // (1-bit codes only: the second four make a nibble of their own)
+        }
         L.pack[tid] = p;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // this wave's share of the rotation
     __syncthreads();
     // (a stream of 1-bit codes; groups are in ascending width)
-    const bool two_dots = IS_V ? v_bits == 1 && a.layout == BGTQ_V_BITPACKED : P.seg_bw[0] == 1 && a.layout == BGTQ_K_BITPACKED;
+    const bool two_dots = IS_V ? v_bits == 1 && a.layout == BGTQ_V_BITPACKED : L.hdr[H_BW] == 1 && a.layout == BGTQ_K_BITPACKED;
 
-    // ---- CS waves a block: the block's place in the work-group, this wave's part of it
-    const int slot = CS == 1 ? wave : wave / CS, part = CS == 1 ? 0 : wave % CS;
     uint8_t* raw = L.raw[slot];
-    const bool wide = ((a.x_sb | a.x_sh | a.x_ss) & 7) == 0 && ((uintptr_t)a.x & 15) == 0;
     auto meet = [&]() {
         asm volatile("" ::: "memory");
         if (CS > 1) __syncthreads();
@@ -623,40 +699,17 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         if (CS == 1) { if (more) __builtin_amdgcn_s_setprio(3); else __builtin_amdgcn_s_setprio(1); }
         const unsigned n0 = (unsigned)blk * 16u;
         const int b0 = (int)(n0 / (unsigned)a.S), s0 = (int)(n0 - (unsigned)b0 * (unsigned)a.S);
-        auto row_of = [&](int r, int& b, int& s) {            // (batch row, step) of the block's row r
-            b = b0;
-            s = s0 + r;
-            if (s >= a.S) { const unsigned q = (unsigned)s / (unsigned)a.S; b += (int)q; s -= (int)q * a.S; }
-        };
-        // ---- raw rows to LDS: 16 lanes a row, 8 values each
+        // ---- raw rows to LDS
+        if (!AHEAD) fetch_rows(blk);
         {
-            constexpr int PASS = 4 / CS;
             const int rc = lane & 15;
-            uint4 x4[PASS];
-#pragma unroll
-            for (int p = 0; p < PASS; p++) {
-                const int r = 4 * (part * PASS + p) + (lane >> 4);
-                x4[p] = uint4{0, 0, 0, 0};
-                if ((int64_t)n0 + r < N) {
-                    int b, s;
-                    row_of(r, b, s);
-                    const uint16_t* src = a.x + b * a.x_sb + h * a.x_sh + s * a.x_ss + rc * 8;
-                    if (wide) x4[p] = *(const uint4*)src;
-                    else {
-                        uint32_t w[4];
-#pragma unroll
-                        for (int i = 0; i < 4; i++) w[i] = (uint32_t)src[2 * i] | ((uint32_t)src[2 * i + 1] << 16);
-                        x4[p] = uint4{w[0], w[1], w[2], w[3]};
-                    }
-                }
-            }
             const uint4 at = *(const uint4*)&L.place[rc * 8];
             const uint32_t at2[4] = {at.x, at.y, at.z, at.w};
             if (lane < 16 && part == 0) {                     // where the rows go
                 int64_t dst = -1, nd = -1;
                 if ((int64_t)n0 + lane < N) {
                     int b, s;
-                    row_of(lane, b, s);
+                    row_of(b0, s0, lane, b, s);
                     const int64_t t = (int64_t)(a.t_pos ? a.t_pos[b] : a.t_pos_scalar) + s;
                     if (a.codes_out) dst = nd = (int64_t)n0 + lane;
                     else if (t >= 0 && t < a.max_T) {
@@ -779,16 +832,22 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
 #pragma unroll
             for (int q = 0; q < D / 32; q++) {
                 load_a(q);
+                // (addresses and masks that are the same for every block would be worked out ahead of the loop: 560 instructions
+                // a wave there, half of them moves of masks to lanes and back; 18.4 -> 17.5 us for K of 8 heads of 2001 tokens)
+                uint32_t segs = seg_of[q];
+                asm volatile("" : "+v"(segs));
 #pragma unroll
                 for (int i = 0; i < 8; i++) {
                     const int kk = 8 * q + i;
-                    A[kk] = div_by(A[kk], L.nrm[slot][(seg_of[q] >> (4 * i)) & 15u][li]);
+                    A[kk] = div_by(A[kk], L.nrm[slot][(segs >> (4 * i)) & 15u][li]);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (n_zero) {                                     // (uniform) 0-bit dims come first
+                int zeros = n_zero - lg;
+                asm volatile("" : "+v"(zeros));
 #pragma unroll
-                for (int kk = 0; kk < D / 4; kk++) A[kk] = 4 * kk + lg < n_zero ? 0.f : A[kk];
+                for (int kk = 0; kk < D / 4; kk++) A[kk] = 4 * kk < zeros ? 0.f : A[kk];
             }
         }
         // codes of rows 4 lg .. + 3 from the values of column j
@@ -996,6 +1055,7 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
                 }
             }
         }
+        if (AHEAD && round + stride * NB < n_blocks) fetch_rows(round + stride * NB + slot);
         // ---- records
         if (a.codes_out) {
             for (int i = part * 64 + lane; i < 16 * (D / 4); i += 64 * CS) {
