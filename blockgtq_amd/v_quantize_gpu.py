@@ -26,10 +26,13 @@ class PolarQuantGPU:
         rot = haar_rotation(d, seed, zero_sign_fix=False)
         self.rotation = torch.from_numpy(rot.astype(np.float32)).to(self.device)
         cents = mc_lloyd_centroids(bit_width, d)
-        self.centroids = torch.from_numpy(cents.astype(np.float32)).to(self.device)
+        # centroids and, behind them in the same allocation, their fp16 table
+        c32 = cents.astype(np.float32)
+        both = torch.from_numpy(np.concatenate([c32.view(np.uint8), c32.astype(np.float16).view(np.uint8)])).to(self.device)
+        self.centroids = both[:c32.nbytes].view(torch.float32)
         self.boundaries = torch.from_numpy(
             ((cents[:-1] + cents[1:]) / 2.0).astype(np.float32)).to(self.device)
-        self._lut = self._laid_out()
+        self._lut = self._laid_out(both[c32.nbytes:].view(torch.float16))
 
     @torch.no_grad()
     def quantize(self, v: torch.Tensor):
@@ -70,9 +73,9 @@ class PolarQuantGPU:
             have = self._lut = self._laid_out()
         return self.centroids.to(torch.float16) if have is None else have[3]
 
-    def _laid_out(self):
+    def _laid_out(self, lut=None):
         """(centroids, their version, the table's version, the table); None for tensors that count no versions."""
         if self.centroids.is_inference() or torch.is_inference_mode_enabled():
             return None
-        lut = self.centroids.to(torch.float16, copy=True)
+        lut = self.centroids.to(torch.float16, copy=True) if lut is None else lut
         return self.centroids, self.centroids._version, lut._version, lut
