@@ -1298,14 +1298,16 @@ __device__ __forceinline__ void prepare_part(const EncodeArgs& ak, const EncodeA
     }
 }
 // (BF16: some input is; asking at run time costs the chains of fp16 inputs 0.2 of 5.0 us)
-template <bool BF16, bool RANK>
-__global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, int rows, RankArgs rank) {
+// Rank: RankArgs of a last work-group that ranks the rows, or nothing
+template <bool BF16, class... Rank>
+__global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, int rows, Rank... rank) {
     if (!BF16) ak.bf16 = av.bf16 = aq.bf16 = 0;
     __shared__ __align__(16) float rot_s[D * D];       // the work-group's rotation, whatever its role
-    if (RANK && blockIdx.x == gridDim.x - 1) {         // (uniform)
-        rank_rows(rank, threadIdx.x, (int*)rot_s);
-        return;
-    }
+    if constexpr (sizeof...(Rank) != 0)
+        if (blockIdx.x == gridDim.x - 1) {             // (uniform)
+            rank_rows(rank..., threadIdx.x, (int*)rot_s);
+            return;
+        }
     prepare_part(ak, av, aq, rows, blockIdx.x, rot_s);
 }
 // The same with the attention over the buffered tokens, which depends on none of it: the longer work-groups first, in
@@ -1421,9 +1423,13 @@ int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, in
         hipLaunchKernelGGL(kern, grid, dim3(WINDOW_THREADS), 0, st, ak, av, aq, w, rk, rv, rows, B * n_kv, rank);
     } else {
         const bool bf16 = ak.bf16 || av.bf16 || (q && q_bf16);
-        auto kern = rank.order ? (bf16 ? prepare_kernel<true, true> : prepare_kernel<false, true>)
-                               : (bf16 ? prepare_kernel<true, false> : prepare_kernel<false, false>);
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows, rank);
+        if (rank.order) {
+            auto kern = bf16 ? prepare_kernel<true, RankArgs> : prepare_kernel<false, RankArgs>;
+            hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows, rank);
+        } else {
+            auto kern = bf16 ? prepare_kernel<true> : prepare_kernel<false>;
+            hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows);
+        }
     }
     return bgtq_launch_status();
 }
