@@ -35,13 +35,13 @@ struct DecodeArgs {
     int nfull[4];
     uint64_t last[4];
     int per_tiles, rem_tiles;   // MFMA kernel, equal row lengths: tiles per partition, partitions with one more
-    const int32_t* row_order;   // MFMA kernel: batch row of a grid row, or null: rows as they come
 };
 
 // Fast path: MFMA kernel for packed K and V records (bgtq_decode_seg.hip).
 // Returns BGTQ_EUNSUPPORTED when the arguments do not meet its layout
 // requirements, in which case the caller takes the layout-agnostic kernel.
-int bgtq_launch_decode_seg(const DecodeArgs& a, hipStream_t stream);
+// row_order: batch row of each grid row, or null: rows as they come.
+int bgtq_launch_decode_seg(const DecodeArgs& a, const int32_t* row_order, hipStream_t stream);
 
 // Rows (batch x new tokens) up to which a step's append and query rotation are one launch
 constexpr int BGTQ_ONE_LAUNCH_ROWS = 64;

@@ -597,7 +597,7 @@ int decode_attn(const bgtq_head_plan* plans,
     a.kn = (const uint16_t*)k_norms; a.kn_sb = kn_sb; a.kn_sh = kn_sh; a.kn_st = kn_st;
     a.vp = (const uint8_t*)v_packed; a.vp_sb = vp_sb; a.vp_sh = vp_sh; a.vp_st = vp_st;
     a.vn = (const uint16_t*)v_norms; a.vn_sb = vn_sb; a.vn_sh = vn_sh; a.vn_st = vn_st;
-    a.seq_lens = seq_lens; a.T = T; a.row_order = row_order;
+    a.seq_lens = seq_lens; a.T = T;
     a.B = B; a.n_kv = n_kv; a.gqa = gqa; a.n_splits = n_splits;
     a.part_out = partial_out; a.part_lse = partial_lse;
     a.k_layout = k_layout; a.v_layout = v_layout; a.scale = scale;
@@ -606,7 +606,7 @@ int decode_attn(const bgtq_head_plan* plans,
     a.k_row_width = k_row_width; a.v_row_width = v_row_width;
     hipStream_t st = (hipStream_t)stream;
     if (g_decode_path != 1) {
-        int rc = bgtq_launch_decode_seg(a, st);
+        int rc = bgtq_launch_decode_seg(a, row_order, st);
         if (rc != BGTQ_EUNSUPPORTED) { g_last_path = 2; return rc; }
         if (g_decode_path == 2) return rc;        // forced fast path: report why it refused
     }

@@ -287,19 +287,23 @@ __device__ __forceinline__ void step_raw(float (&S)[8], float n, uint32_t xp, in
     for (int e = 0; e < HEADS; e++) S[e] = fmaf(n, acc.get(e), S[e]);
 }
 
+// batch row of the work-group
+__device__ __forceinline__ int grid_row() { return blockIdx.z; }
+__device__ __forceinline__ int grid_row(const int32_t* order) { return order[blockIdx.z]; }
+
 // HEADS: query heads per KV head the MFMA layout serves (4 or 8)
 // VBW: bits per V code; VST: bytes from one V record to the next (the record itself is
 // 16 * VBW bytes; a padded stride keeps the rows of a tile on different LDS banks)
-// ORDERED: the grid's rows are the batch rows of a.row_order.  (Asked at run time, here and in the preparation, it cost steps without
-// an order 0.6 us a layer, 2 to 3 %.)
-template <int HEADS, int VBW, int VST, bool ORDERED>
-__global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a) {
+// Order: the batch row of each grid row, or nothing.  (Asked at run time, here and in the preparation, it cost steps without an
+// order 0.6 us a layer, 2 to 3 %; as a member of DecodeArgs 0.5 %.)
+template <int HEADS, int VBW, int VST, class... Order>
+__global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a, Order... order) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nw = a.nw, nthr = nw * 64;                 // waves launched; the first nwt of them own tiles and tile buffers,
     const int nwt = a.nw_tiles;                          // the others help with the set-up and the merge of short partitions
-    const int c = blockIdx.x, h = blockIdx.y, b = ORDERED ? a.row_order[blockIdx.z] : (int)blockIdx.z;
+    const int c = blockIdx.x, h = blockIdx.y, b = grid_row(order...);
     const bgtq_head_plan& P = a.plans[h];
     const int gqa = a.gqa;
     const int li = lane & 15, lg = lane >> 4;           // MFMA row/col index, lane group (value product)
@@ -814,7 +818,7 @@ size_t seg_smem_bytes(const TileLayout& tl, int nw, bool p_over_k) {
 }
 
 template <int HEADS, int VBW, int VST>
-int launch_kernel(DecodeArgs a, hipStream_t st) {
+int launch_kernel(DecodeArgs a, const int32_t* order, hipStream_t st) {
     a.tl = tile_layout(a.k_row_width, VST, (int)a.kn_st);
     // no more waves than the longest partition has tiles
     const int tiles = (a.T + MT - 1) / MT;
@@ -846,7 +850,8 @@ int launch_kernel(DecodeArgs a, hipStream_t st) {
     }
     a.per_tiles = tiles / a.n_splits;
     a.rem_tiles = tiles - a.per_tiles * a.n_splits;
-    auto kern = a.row_order ? decode_seg_kernel<HEADS, VBW, VST, true> : decode_seg_kernel<HEADS, VBW, VST, false>;
+    auto kern = decode_seg_kernel<HEADS, VBW, VST>;
+    auto ordered = decode_seg_kernel<HEADS, VBW, VST, const int32_t*>;
     // 1: usable, -1: not usable.  Two threads racing through the first call both run the idempotent
     // set-up below and store the same value.
     static std::atomic<int> ready{0};
@@ -854,11 +859,11 @@ int launch_kernel(DecodeArgs a, hipStream_t st) {
         // the kernel uses offsets into its dynamic LDS block as LDS addresses: that holds only
         // while it has no static LDS in front of the dynamic block
         int usable = 1;
-        for (auto each : {decode_seg_kernel<HEADS, VBW, VST, true>, decode_seg_kernel<HEADS, VBW, VST, false>}) {
+        for (const void* each : {(const void*)kern, (const void*)ordered}) {
             hipFuncAttributes fa;
-            hipError_t e = hipFuncGetAttributes(&fa, (const void*)each);
+            hipError_t e = hipFuncGetAttributes(&fa, each);
             if (e != hipSuccess) return (int)e;
-            e = hipFuncSetAttribute((const void*)each, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_LIMIT);
+            e = hipFuncSetAttribute(each, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_LIMIT);
             if (e != hipSuccess) return (int)e;
             if (fa.sharedSizeBytes != 0) usable = -1;
         }
@@ -866,21 +871,22 @@ int launch_kernel(DecodeArgs a, hipStream_t st) {
     }
     if (ready.load(std::memory_order_acquire) < 0) return BGTQ_EUNSUPPORTED;
     dim3 grid((unsigned)a.n_splits, (unsigned)a.n_kv, (unsigned)a.B);
-    hipLaunchKernelGGL(kern, grid, dim3(a.nw * 64), smem, st, a);
+    if (order) hipLaunchKernelGGL(ordered, grid, dim3(a.nw * 64), smem, st, a, order);
+    else hipLaunchKernelGGL(kern, grid, dim3(a.nw * 64), smem, st, a);
     return bgtq_launch_status();
 }
 
 template <int VBW, int VST>
-int launch(const DecodeArgs& a, hipStream_t st) {
-    return a.gqa > 4 ? launch_kernel<8, VBW, VST>(a, st) : launch_kernel<4, VBW, VST>(a, st);
+int launch(const DecodeArgs& a, const int32_t* order, hipStream_t st) {
+    return a.gqa > 4 ? launch_kernel<8, VBW, VST>(a, order, st) : launch_kernel<4, VBW, VST>(a, order, st);
 }
 
 }  // namespace
 
 
-static int launch_group(const DecodeArgs& a, hipStream_t stream);
+static int launch_group(const DecodeArgs& a, const int32_t* row_order, hipStream_t stream);
 
-int bgtq_launch_decode_seg(const DecodeArgs& all, hipStream_t stream) {
+int bgtq_launch_decode_seg(const DecodeArgs& all, const int32_t* row_order, hipStream_t stream) {
     // one launch takes up to 8 query heads per KV head; 9..16 go as two launches over halves of the
     // heads (the records are streamed twice, which still beats the generic kernel several times over)
     if (all.gqa > 16) return BGTQ_EUNSUPPORTED;
@@ -890,13 +896,13 @@ int bgtq_launch_decode_seg(const DecodeArgs& all, hipStream_t stream) {
         a.gqa_all = all.gqa;
         a.head0 = g * first;
         a.gqa = g == 0 ? first : all.gqa - first;
-        const int rc = launch_group(a, stream);
+        const int rc = launch_group(a, row_order, stream);
         if (rc != BGTQ_OK) return rc;            // a refusal comes from the first group, before any launch
     }
     return BGTQ_OK;
 }
 
-static int launch_group(const DecodeArgs& a, hipStream_t stream) {
+static int launch_group(const DecodeArgs& a, const int32_t* row_order, hipStream_t stream) {
     // layout requirements of the fast path; anything else takes the generic kernel
     if (a.gqa > 8 || !(a.scale > 0.f)) return BGTQ_EUNSUPPORTED;
     // the kernel forms its addresses from 32-bit factors: batch and head strides, and the bytes of one
@@ -920,10 +926,10 @@ static int launch_group(const DecodeArgs& a, hipStream_t stream) {
     // (32 or 64 bytes) would put the rows of a tile on the same LDS banks
     const int64_t pad = a.vp_st - a.v_row_width;
     switch (a.v_row_width) {
-    case 16: return pad == 0 ? launch<1, 16>(a, stream) : BGTQ_EUNSUPPORTED;
-    case 32: return pad == 0 ? launch<2, 32>(a, stream) : pad == 4 ? launch<2, 36>(a, stream) : BGTQ_EUNSUPPORTED;
-    case 48: return pad == 0 ? launch<3, 48>(a, stream) : BGTQ_EUNSUPPORTED;
-    case 64: return pad == 0 ? launch<4, 64>(a, stream) : pad == 4 ? launch<4, 68>(a, stream) : BGTQ_EUNSUPPORTED;
+    case 16: return pad == 0 ? launch<1, 16>(a, row_order, stream) : BGTQ_EUNSUPPORTED;
+    case 32: return pad == 0 ? launch<2, 32>(a, row_order, stream) : pad == 4 ? launch<2, 36>(a, row_order, stream) : BGTQ_EUNSUPPORTED;
+    case 48: return pad == 0 ? launch<3, 48>(a, row_order, stream) : BGTQ_EUNSUPPORTED;
+    case 64: return pad == 0 ? launch<4, 64>(a, row_order, stream) : pad == 4 ? launch<4, 68>(a, row_order, stream) : BGTQ_EUNSUPPORTED;
     default: return BGTQ_EUNSUPPORTED;
     }
 }
