@@ -26,13 +26,9 @@ class PolarQuantGPU:
         rot = haar_rotation(d, seed, zero_sign_fix=False)
         self.rotation = torch.from_numpy(rot.astype(np.float32)).to(self.device)
         cents = mc_lloyd_centroids(bit_width, d)
-        # centroids and, behind them in the same allocation, their fp16 table
-        c32 = cents.astype(np.float32)
-        both = torch.from_numpy(np.concatenate([c32.view(np.uint8), c32.astype(np.float16).view(np.uint8)])).to(self.device)
-        self.centroids = both[:c32.nbytes].view(torch.float32)
+        self.centroids = torch.from_numpy(cents.astype(np.float32)).to(self.device)
         self.boundaries = torch.from_numpy(
             ((cents[:-1] + cents[1:]) / 2.0).astype(np.float32)).to(self.device)
-        self._lut = self._laid_out(both[c32.nbytes:].view(torch.float16))
 
     @torch.no_grad()
     def quantize(self, v: torch.Tensor):
@@ -65,17 +61,5 @@ class PolarQuantGPU:
 
     @property
     def v_lut(self) -> torch.Tensor:
-        """Centroids as fp16, the table the attention kernel dequantises with.  Laid out with the quantizer: a launch
-        a call of the entry that takes one KV head's slice at a time, 14.2 -> 10.8 us at 1k tokens.  Centroids or a table that
-        were changed since are laid out again."""
-        have = getattr(self, '_lut', None)
-        if have is None or have[0] is not self.centroids or have[1:3] != (have[0]._version, have[3]._version):
-            have = self._lut = self._laid_out()
-        return self.centroids.to(torch.float16) if have is None else have[3]
-
-    def _laid_out(self, lut=None):
-        """(centroids, their version, the table's version, the table); None for tensors that count no versions."""
-        if self.centroids.is_inference() or torch.is_inference_mode_enabled():
-            return None
-        lut = self.centroids.to(torch.float16, copy=True) if lut is None else lut
-        return self.centroids, self.centroids._version, lut._version, lut
+        """Centroids as fp16, the table the attention kernel dequantises with."""
+        return self.centroids.to(torch.float16)

@@ -1,4 +1,4 @@
-"""The fp16 table of V centroids that is laid out once follows the centroids (no GPU)."""
+"""The fp16 table of V centroids is what the centroids are when it is read, and its reader's own."""
 import copy
 import pickle
 
@@ -13,30 +13,53 @@ def _follows(q):
 
 
 @pytest.mark.parametrize("bits", [1, 3, 4])
-def test_table_follows_the_centroids(bits):
+def test_table_follows_the_centroids_however_they_are_changed(bits):
     q = PolarQuantGPU(128, bits)
     _follows(q)
-    assert q.v_lut is q.v_lut
     q.centroids.mul_(2)
     _follows(q)
-    q.v_lut.zero_()                                   # (the table is the caller's to change as before)
+    q.centroids.data.mul_(2)                          # (counted by no version)
+    _follows(q)
+    q.centroids.numpy()[:] *= 2
+    _follows(q)
+    q.centroids.data = q.centroids.data + 1
     _follows(q)
     q.centroids = q.centroids + 1
     _follows(q)
-    for other in (copy.deepcopy(q), pickle.loads(pickle.dumps(q))):
-        other.centroids.add_(1)
-        _follows(other)
-    del q.__dict__['_lut']                            # (an object that was saved without the table)
-    _follows(q)
-
-
-def test_tensors_without_versions():
-    q = PolarQuantGPU(128, 3)
     with torch.inference_mode():
+        q.centroids.add_(1)
         _follows(q)
-        made = PolarQuantGPU(128, 3)
-        _follows(made)
-    _follows(made)
-    with torch.inference_mode():
-        made.centroids.mul_(2)
-    _follows(made)
+    for other in (copy.deepcopy(q), pickle.loads(pickle.dumps(q))):
+        other.centroids.data.add_(1)
+        _follows(other)
+
+
+def test_each_reader_has_a_table_of_its_own():
+    q = PolarQuantGPU(128, 3)
+    mine, theirs = q.v_lut, q.v_lut
+    theirs.zero_()
+    assert torch.equal(mine, q.centroids.half())
+    assert q.centroids.untyped_storage().nbytes() == q.centroids.nbytes       # (and the centroids share theirs with none)
+
+
+@pytest.mark.gpu
+def test_table_read_under_capture():
+    """Replays read the centroids as they are then, and what was only recorded is nobody else's table."""
+    q = PolarQuantGPU(128, 3, device="cuda:0")
+    _follows(q)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        q.centroids = q.centroids * 2
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            table = q.v_lut
+    _follows(q)                                       # before any replay
+    for _ in range(3):
+        q.centroids.data.mul_(1.5)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(table, q.centroids.half())
+        _follows(q)
