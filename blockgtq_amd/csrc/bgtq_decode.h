@@ -1,6 +1,7 @@
 // Argument block shared by the decode attention kernels (internal).
 #pragma once
 #include "bgtq_common.h"
+#include "bgtq_row_order.h"
 #include "bgtq_window.h"
 
 // LDS bytes of one wave's tile buffers in the MFMA kernel (filled in by its launcher)
@@ -42,9 +43,6 @@ struct DecodeArgs {
 // requirements, in which case the caller takes the layout-agnostic kernel.
 // row_order: batch row of each grid row, or null: rows as they come.
 int bgtq_launch_decode_seg(const DecodeArgs& a, const int32_t* row_order, hipStream_t stream);
-
-// Rows (batch x new tokens) up to which a step's append and query rotation are one launch
-constexpr int BGTQ_ONE_LAUNCH_ROWS = 64;
 
 // The preparation part of bgtq_decode_step (bgtq_encode.hip).  kv_fp16: k and v are fp16 whatever x_dtype says.
 // window: the buffered tokens' partial, computed in the same launch (window_rides, at most BGTQ_ONE_LAUNCH_ROWS rows), or null.

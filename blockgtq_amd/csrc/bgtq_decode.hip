@@ -547,30 +547,6 @@ int pick_splits(int B, int n_kv, int max_T, bool ragged) {
     return best;
 }
 
-// Whether a step sends rows of different lengths out by falling length (ranked in the launch that prepares the step): where
-// there is more than one round of work-groups, the long partitions first and the short ones into the places that come free.
-// The same partitions, the same results.  us a step, rows as they come and in order:
-//   20 rows x 8 heads, up to 8k:  48.3, 40.8 (3 partitions)    16 x 8, 16k: 64.4, 56.3 (6)
-//   24 rows x 4 heads, up to 16k: 55.6, 52.7 (8)               32 x 8, 16k: 96.2, 94.5 (4)
-// and with all rows equal after all 54.7, 54.8; 73.1, 73.5; 62.6, 63.3; 142.1, 141.4.  (Fewer partitions would do now, 90.2 us with
-// two for the last; other partitions mean other roundings.)
-bool orders_rows(int B, int n_kv, int S, int n_splits, bool ragged) {
-    return ragged && B > 1 && (int64_t)B * S <= BGTQ_ONE_LAUNCH_ROWS && (int64_t)B * n_kv * n_splits > 256;
-}
-
-// The order lies at the start of the step's output, which nothing else writes before the partitions are merged: not where
-// an input lies there too, or where it would not be aligned
-bool order_fits(const bgtq_step& s) {
-    const uintptr_t lo = (uintptr_t)s.out, hi = lo + (size_t)s.B * sizeof(int32_t);
-    auto apart = [&](const void* p, int64_t sb, int64_t n, int64_t sh, int64_t m, int64_t ss) {
-        if (sb < 0 || sh < 0 || ss < 0) return false;
-        const uintptr_t at = (uintptr_t)p;
-        return at >= hi || at + (size_t)((s.B - 1) * sb + (n - 1) * sh + (m - 1) * ss + D) * 2 <= lo;
-    };
-    return (lo & 3) == 0 && apart(s.q, s.q_sb, (int64_t)s.n_kv * s.gqa, s.q_sh, 1, 0) && apart(s.k, s.k_sb, s.n_kv, s.k_sh, s.S, s.k_ss) &&
-           apart(s.v, s.v_sb, s.n_kv, s.v_sh, s.S, s.v_ss);
-}
-
 int decode_attn(const bgtq_head_plan* plans,
                 const void* q_rot, int64_t q_sb, int64_t q_sh,
                 const void* k_packed, int64_t kp_sb, int64_t kp_sh, int64_t kp_st, int k_row_width,
@@ -777,7 +753,7 @@ int bgtq_decode_step(const bgtq_step* step, void* stream) {
         s.k = old_k; s.v = old_v;
         s.k_sb = s.v_sb = (int64_t)s.n_kv * D; s.k_sh = s.v_sh = D; s.k_ss = s.v_ss = D;
     }
-    int32_t* order = orders_rows(s.B, s.n_kv, s.S, s.n_splits, s.seq_lens != nullptr) && order_fits(*step) ? (int32_t*)s.out : nullptr;
+    int32_t* order = bgtq_orders_rows(s.B, s.n_kv, s.S, s.n_splits, s.seq_lens != nullptr) && bgtq_order_fits(*step) ? (int32_t*)s.out : nullptr;
     int rc = bgtq_step_prepare(s, windowed && s.x_dtype == BGTQ_X_BF16, window.q ? &window : nullptr, order, st);
     if (rc != BGTQ_OK) return rc;
     const void* q = s.q_rot ? s.q_rot : s.q;

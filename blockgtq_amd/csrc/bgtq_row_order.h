@@ -1,0 +1,49 @@
+// Rows of a decode step by falling length: when a step sends them out so, where the order lies meanwhile.
+// No device types: it compiles for the CPU alone as well.
+#pragma once
+#include <stddef.h>
+#include <stdint.h>
+
+#include "../../include/bgtq.h"
+
+// Rows (batch x new tokens) up to which a step's append and query rotation are one launch
+constexpr int BGTQ_ONE_LAUNCH_ROWS = 64;
+
+// Whether a step sends rows of different lengths out by falling length (ranked in the launch that prepares the step): where
+// there is more than one round of work-groups, the long partitions first and the short ones into the places that come free.
+// The same partitions, the same results.  us a step, rows as they come and in order:
+//   20 rows x 8 heads, up to 8k:  48.3, 40.8 (3 partitions)    16 x 8, 16k: 64.4, 56.3 (6)
+//   24 rows x 4 heads, up to 16k: 55.6, 52.7 (8)               32 x 8, 16k: 96.2, 94.5 (4)
+// and with all rows equal after all 54.7, 54.8; 73.1, 73.5; 62.6, 63.3; 142.1, 141.4.  (Fewer partitions would do now, 90.2 us with
+// two for the last; other partitions mean other roundings.)
+inline bool bgtq_orders_rows(int B, int n_kv, int S, int n_splits, bool ragged) {
+    return ragged && B > 1 && (int64_t)B * S <= BGTQ_ONE_LAUNCH_ROWS && (int64_t)B * n_kv * n_splits > 256;
+}
+
+// The order lies at the start of the step's output, which nothing else writes before the partitions are merged.  It is written
+// while the step's inputs and scratch are in use, and the attention takes what it finds there for batch rows: not where any other
+// buffer of the step has a byte there (`out` over the queries or over scratch is allowed, the merge is the last to use them), nor
+// where that is not plain (strides that run backwards), nor where the order would not be aligned.
+inline bool bgtq_order_fits(const bgtq_step& s) {
+    const int64_t B = s.B, n_kv = s.n_kv, n_q = n_kv * s.gqa, D = BGTQ_HEAD_DIM;
+    const uintptr_t lo = (uintptr_t)s.out, hi = lo + (size_t)B * sizeof(int32_t);
+    auto apart = [&](const void* p, int64_t bytes) { return !p || bytes <= 0 || (uintptr_t)p >= hi || (uintptr_t)p + (size_t)bytes <= lo; };
+    // B x n x m rows of `last` elements
+    auto rows_apart = [&](const void* p, int64_t size, int64_t sb, int64_t n, int64_t sh, int64_t m, int64_t ss, int64_t last) {
+        return sb >= 0 && sh >= 0 && ss >= 0 && apart(p, m < 1 ? 0 : ((B - 1) * sb + (n - 1) * sh + (m - 1) * ss + last) * size);
+    };
+    const int64_t rows = s.T > s.max_T ? s.T : s.max_T;
+    if ((lo & 3) != 0 || !apart(s.plans, n_kv * (int64_t)sizeof(bgtq_head_plan))) return false;
+    if (!rows_apart(s.q, 2, s.q_sb, n_q, s.q_sh, 1, 0, D) || !rows_apart(s.k, 2, s.k_sb, n_kv, s.k_sh, s.S, s.k_ss, D) ||
+        !rows_apart(s.v, 2, s.v_sb, n_kv, s.v_sh, s.S, s.v_ss, D) || !apart(s.q_rot, B * n_q * D * 2)) return false;
+    if (!rows_apart(s.k_packed, 1, s.kp_sb, n_kv, s.kp_sh, rows, s.kp_st, s.k_row_width) ||
+        !rows_apart(s.k_norms, 2, s.kn_sb, n_kv, s.kn_sh, rows, s.kn_st, s.norm_width) ||
+        !rows_apart(s.v_packed, 1, s.vp_sb, n_kv, s.vp_sh, rows, s.vp_st, s.v_row_width) ||
+        !rows_apart(s.v_norms, 2, s.vn_sb, n_kv, s.vn_sh, rows, s.vn_st, 1)) return false;
+    if (!apart(s.t_pos, B * 4) || !apart(s.seq_lens, B * 4) || !apart(s.partial_out, B * n_q * s.n_splits * D * 4) ||
+        !apart(s.partial_lse, B * n_q * s.n_splits * 4)) return false;
+    if (!s.win_k) return true;                                // (the other fields of the buffer are not read then)
+    return rows_apart(s.win_k, 2, s.w_sb, n_kv, s.w_sh, s.win_W, s.w_st, D) && rows_apart(s.win_v, 2, s.w_sb, n_kv, s.w_sh, s.win_W, s.w_st, D) &&
+           apart(s.win_slot, B * 4) && apart(s.win_lens, B * 4) && apart(s.win_old, 2 * B * n_kv * D * 2) &&
+           apart(s.win_out, B * n_q * D * 4) && apart(s.win_lse, B * n_q * 4);
+}

@@ -460,7 +460,9 @@ int bgtq_decode_attend_static(const bgtq_head_plan* plans,
  *              win_old (fp16 [2][B][n_kv][128]), win_out (fp32 [B][n_q][128]) and win_lse (fp32 [B][n_q])
  *              are scratch
  *   partial_out, partial_lse  as for bgtq_decode_attn
- *   out        fp16 [B][n_kv*gqa][128] contiguous
+ *   out        fp16 [B][n_kv*gqa][128] contiguous.  Written last: it may share memory with q, k, v, q_rot or
+ *              win_old.  Where it shares memory with no other buffer of the step, its first 4 B bytes may be used
+ *              as scratch from the step's start on (also by a step that returns an error)
  */
 #define BGTQ_X_FP16 0
 #define BGTQ_X_BF16 1
