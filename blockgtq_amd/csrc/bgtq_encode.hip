@@ -1271,6 +1271,7 @@ __global__ __launch_bounds__(NT) void rotate_q_kernel(RotQArgs a) {
 
 // ---- batch rows by falling length, for the attention launch that follows: lengths on the device, one work-group ----
 struct RankArgs { const int32_t* lens; int32_t* order; int B; };      // order null: not asked for
+static_assert(BGTQ_ONE_LAUNCH_ROWS <= NT, "a thread a row");
 
 __device__ __forceinline__ void rank_rows(const RankArgs& r, const int tid, int* lens_s) {
     const int len = tid < r.B ? r.lens[tid] : 0;

@@ -17,7 +17,8 @@ constexpr int BGTQ_ONE_LAUNCH_ROWS = 64;
 // and with all rows equal after all 54.7, 54.8; 73.1, 73.5; 62.6, 63.3; 142.1, 141.4.  (Fewer partitions would do now, 90.2 us with
 // two for the last; other partitions mean other roundings.)
 inline bool bgtq_orders_rows(int B, int n_kv, int S, int n_splits, bool ragged) {
-    return ragged && B > 1 && (int64_t)B * S <= BGTQ_ONE_LAUNCH_ROWS && (int64_t)B * n_kv * n_splits > 256;
+    // (a step without new tokens is a launch of any number of rows)
+    return ragged && B > 1 && S >= 1 && (int64_t)B * S <= BGTQ_ONE_LAUNCH_ROWS && (int64_t)B * n_kv * n_splits > 256;
 }
 
 // The order lies at the start of the step's output, which nothing else writes before the partitions are merged.  It is written

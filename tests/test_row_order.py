@@ -7,7 +7,7 @@ import subprocess
 import pytest
 import torch
 
-from blockgtq_amd import _capi, workloads as wl
+from blockgtq_amd import _capi, ops, workloads as wl
 from blockgtq_amd.build import CSRC
 
 DEV = "cuda:0"
@@ -52,6 +52,7 @@ extern "C" int fits_without(void) {
     s.win_k = s.win_v = s.win_old = nullptr; s.win_slot = s.win_lens = nullptr; s.win_out = s.win_lse = nullptr;
     return bgtq_order_fits(s);
 }
+extern "C" int orders(int B, int n_kv, int S, int splits, int ragged) { return bgtq_orders_rows(B, n_kv, S, splits, ragged); }
 extern "C" int64_t plan_bytes(void) { return sizeof(bgtq_head_plan); }
 """
 
@@ -96,6 +97,14 @@ def test_strides_that_run_backwards_and_unaligned_outputs_keep_rows_as_they_come
         assert not rule.fits_backwards(stride.encode()), stride
     assert rule.fits_backwards(b"") and rule.fits_without()
     assert [rule.fits_out_off(by) for by in (0, 1, 2, 4)] == [1, 0, 0, 1]
+
+
+def test_only_batches_that_one_work_group_ranks_are_ranked(rule):
+    """One thread a row: as many rows as the launch has room for, whatever the number of new tokens (0 among them)."""
+    assert [rule.orders(B, 8, 1, 8, 1) for B in (1, 4, 5, 64, 65, 130, 10**6)] == [0, 0, 1, 1, 0, 0, 0]
+    assert [rule.orders(B, 8, 0, 8, 1) for B in (1, 5, 64, 65, 130, 10**6)] == [0] * 6
+    assert [rule.orders(16, 8, S, 8, 1) for S in (-1, 0, 1, 4, 5)] == [0, 0, 1, 1, 0]
+    assert not rule.orders(16, 8, 1, 8, 0) and not rule.orders(16, 2, 1, 8, 1) and rule.orders(43, 2, 1, 3, 1)
 
 
 # --------------------------------------------------------------------------------------- the entry itself, on the GPU
@@ -179,3 +188,15 @@ def test_output_over_a_buffer_that_is_dead_before_the_merge(shared, window):
             place = _over_win_old if outs else place
         outs.append(_step(mgr, q, k, v, 2, place))
     assert torch.isfinite(outs[0]).all() and outs[0].abs().max() > 0 and torch.equal(*outs)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [33, 130])
+def test_step_without_new_tokens(batch):
+    """Attention over what is there, more rows than a work-group ranks among them."""
+    mgr, q, k, v = _filled(batch, 4, 2, 300)
+    got = _step(mgr, q, k, v, 2, S=0)
+    plans, cache = mgr._batched_args[0]["plans"], (mgr._k_packed[0], mgr._k_norms[0], mgr._v_packed[0], mgr._v_norms[0])
+    want = ops.decode_attention(plans, ops.rotate_q(plans, q[:, :, 0], 4), *cache, mgr.seq_len, seq_lens=mgr._seq_lens, n_splits=2,
+                                scale=mgr.scale, k_row_width=mgr._k_rows[0], v_row_width=mgr._vpb)
+    assert torch.isfinite(got).all() and got.abs().max() > 0 and torch.equal(got, want.view_as(got))
