@@ -569,9 +569,8 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         s = s0 + r;
         if (s >= a.S) { const unsigned q = (unsigned)s / (unsigned)a.S; b += (int)q; s -= (int)q * a.S; }
     };
-    // Raw rows, 16 lanes a row, 8 values each.  AHEAD: the first block's with the tables, the next one's before a block's
-    // records go out (8 heads of 128 tokens 14.0 -> 11.5 us, of 2001 17.5 -> 16.4; with a wave a block V's waves came to the
-    // matrix core together and the registers spilled: 31.4 -> 35.3)
+    // Raw rows, 16 lanes a row, 8 values each.  AHEAD: with the tables (8 heads of 128 tokens 14.0 -> 11.5 us, of 2001
+    // 17.5 -> 16.4; with a wave a block V's waves came to the matrix core together and the registers spilled: 31.4 -> 35.3)
     constexpr int PASS = 4 / CS;
     constexpr bool AHEAD = CS > 1;
     uint4 x4[PASS];
@@ -634,8 +633,9 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
             L.place[dim.w >> 8] = (uint16_t)(((tid & 3) * (D / 4) + (tid >> 2)) * 2);
             L.bin[tid] = bin;
         }
-        // The rotation, four rows interleaved on the way (as 256 loads of 16 columns of a row into LDS 0.4 us more).  A thread's columns leave in an order of its own, from column
-        // (tid / 4) % 4 of the four on: 16 lanes then write 256 bytes of 64 banks.
+        // The rotation, four rows interleaved on the way (as 256 loads of 16 columns of a row into LDS 0.4 us more).  A thread's
+        // columns leave in an order of its own, from column (tid / 4) % 4 of the four on: 16 lanes then write 256 bytes of 64
+        // banks.
         for (int at = tid;;) {
 #pragma unroll
             for (int n = 0; n < RT; n++) {
@@ -689,8 +689,9 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
         else __builtin_amdgcn_wave_barrier();                 // (a wave's LDS accesses keep their order)
         asm volatile("" ::: "memory");
     };
-    // (neighbouring blocks to the waves of one work-group; CS > 1: as many rounds for every wave of it, for the barriers'
-    // sake - rows past the last are zeros and stored nowhere)
+    // (neighbouring blocks to the waves of one work-group; CS > 1: launch_blocks() has a place for every block, so there is
+    // one round, with the rows fetched above, and every wave of it goes for the barriers' sake: rows past the last are zeros and
+    // stored nowhere.  Told so by a `break` at the end the compiler has K of 2001 tokens x 8 heads take 58 us for 16)
     for (int round = first * NB; CS == 1 ? round + slot < n_blocks : round < n_blocks; round += stride * NB) {
         const int blk = round + slot;
         // The oldest wave of a SIMD would run ahead, and the youngest end alone with a matrix core that it fills by half
@@ -1055,7 +1056,6 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
                 }
             }
         }
-        if (AHEAD && round + stride * NB < n_blocks) fetch_rows(round + stride * NB + slot);
         // ---- records
         if (a.codes_out) {
             for (int i = part * 64 + lane; i < 16 * (D / 4); i += 64 * CS) {
@@ -1126,7 +1126,7 @@ int launch_blocks(const EncodeArgs* k, const EncodeArgs* v, hipStream_t st) {
     const int64_t most = std::max<int64_t>(1, 256 / (any.n_kv * kinds));
     const int64_t share = (blocks + most - 1) / most, rounds = (share + 15) / 16;
     if (share <= 8) {
-        const int groups = (int)((blocks + share - 1) / share);
+        const int groups = (int)((blocks + share - 1) / share);      // (of at least `share` blocks at a time: one round)
         t.k_groups = k ? groups : 0;
         t.v_groups = v ? groups : 0;
         hipLaunchKernelGGL(encode_blocks_kernel<2>, dim3((unsigned)(groups * kinds * any.n_kv)), dim3((unsigned)std::max<int64_t>(4, 2 * share) * 64), 0, st, t);
