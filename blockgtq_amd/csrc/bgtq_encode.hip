@@ -1317,18 +1317,19 @@ __global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs a
 // buffer here, put there by those who read the one that leaves.
 // 32 rows x 8 heads x 4 queries over 132 buffered tokens: 4.9 (swap) + 11.1 + 13.3 us as launches of their own, 4.9 + 16.3
 // with K and V a work-group each and the swap ahead of them (1024 work-groups, two of them at a time on a compute unit), 14 here.
-template <bool SWAP, bool RANK>
+template <bool SWAP, class... Rank>
 __global__ __launch_bounds__(WINDOW_THREADS, 2) void prepare_window_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, WindowArgs w,
-                                                                        RingArgs rk, RingArgs rv, int rows, int n_window, RankArgs rank) {
+                                                                        RingArgs rk, RingArgs rv, int rows, int n_window, Rank... rank) {
     __shared__ __align__(16) float rot_s[D * D];
     static_assert(window_lds_floats<4>(WINDOW_RIDE_W) <= D * D, "a window's scores fit the rotation's place");
     static_assert(WINDOW_THREADS == 2 * NT, "");
     int bid = blockIdx.x;
     const int n_kv = ak.n_kv, tid = threadIdx.x;
-    if (RANK && bid == (int)gridDim.x - 1) {
-        rank_rows(rank, tid, (int*)rot_s);
-        return;
-    }
+    if constexpr (sizeof...(Rank) != 0)
+        if (bid == (int)gridDim.x - 1) {
+            rank_rows(rank..., tid, (int*)rot_s);
+            return;
+        }
     if (bid < n_window) {
         window_attn_block<4, SWAP>(w, bid % n_kv, bid / n_kv, rot_s);
         return;
@@ -1419,9 +1420,13 @@ int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, in
         const dim3 grid(blocks - (unsigned)(rows * n_kv) + (unsigned)(B * n_kv));
         const RingArgs rk{w.swap.slot, (uint16_t*)w.kbuf, w.w_sb, w.w_sh, w.w_st, w.W, w.swap.k, w.swap.k_sb, w.swap.k_sh, w.bf16};
         const RingArgs rv{w.swap.slot, (uint16_t*)w.vbuf, w.w_sb, w.w_sh, w.w_st, w.W, w.swap.v, w.swap.v_sb, w.swap.v_sh, w.bf16};
-        auto kern = w.swap.slot ? (rank.order ? prepare_window_kernel<true, true> : prepare_window_kernel<true, false>)
-                                : (rank.order ? prepare_window_kernel<false, true> : prepare_window_kernel<false, false>);
-        hipLaunchKernelGGL(kern, grid, dim3(WINDOW_THREADS), 0, st, ak, av, aq, w, rk, rv, rows, B * n_kv, rank);
+        if (rank.order) {
+            auto kern = w.swap.slot ? prepare_window_kernel<true, RankArgs> : prepare_window_kernel<false, RankArgs>;
+            hipLaunchKernelGGL(kern, grid, dim3(WINDOW_THREADS), 0, st, ak, av, aq, w, rk, rv, rows, B * n_kv, rank);
+        } else {
+            auto kern = w.swap.slot ? prepare_window_kernel<true> : prepare_window_kernel<false>;
+            hipLaunchKernelGGL(kern, grid, dim3(WINDOW_THREADS), 0, st, ak, av, aq, w, rk, rv, rows, B * n_kv);
+        }
     } else {
         const bool bf16 = ak.bf16 || av.bf16 || (q && q_bf16);
         if (rank.order) {
