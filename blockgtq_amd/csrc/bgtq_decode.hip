@@ -753,7 +753,7 @@ int bgtq_decode_step(const bgtq_step* step, void* stream) {
         s.k = old_k; s.v = old_v;
         s.k_sb = s.v_sb = (int64_t)s.n_kv * D; s.k_sh = s.v_sh = D; s.k_ss = s.v_ss = D;
     }
-    int32_t* order = bgtq_orders_rows(s.B, s.n_kv, s.S, s.n_splits, s.seq_lens != nullptr) && bgtq_order_fits(*step) ? (int32_t*)s.out : nullptr;
+    int32_t* order = bgtq_orders_rows(s.B, s.n_kv, s.S, s.T, s.n_splits, s.seq_lens != nullptr) && bgtq_order_fits(*step) ? (int32_t*)s.out : nullptr;
     int rc = bgtq_step_prepare(s, windowed && s.x_dtype == BGTQ_X_BF16, window.q ? &window : nullptr, order, st);
     if (rc != BGTQ_OK) return rc;
     const void* q = s.q_rot ? s.q_rot : s.q;

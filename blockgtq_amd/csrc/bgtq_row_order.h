@@ -11,14 +11,19 @@ constexpr int BGTQ_ONE_LAUNCH_ROWS = 64;
 
 // Whether a step sends rows of different lengths out by falling length (ranked in the launch that prepares the step): where
 // there is more than one round of work-groups, the long partitions first and the short ones into the places that come free.
-// The same partitions, the same results.  us a step, rows as they come and in order:
-//   20 rows x 8 heads, up to 8k:  48.3, 40.8 (3 partitions)    16 x 8, 16k: 64.4, 56.3 (6)
-//   24 rows x 4 heads, up to 16k: 55.6, 52.7 (8)               32 x 8, 16k: 96.2, 94.5 (4)
-// and with all rows equal after all 54.7, 54.8; 73.1, 73.5; 62.6, 63.3; 142.1, 141.4.  (Fewer partitions would do now, 90.2 us with
-// two for the last; other partitions mean other roundings.)
-inline bool bgtq_orders_rows(int B, int n_kv, int S, int n_splits, bool ragged) {
+// The same partitions, the same results.  us a step (captured), rows as they come and in order; lengths even from T / 16 to T, and all T:
+//   64 rows x 8 heads, T 3000, 1 partition:  65.3, 54.8; 68.5, 69.1     64 x 8, 1500, 1: 50.7, 48.4; 52.8, 53.4
+//   64 x 2, 12000, 4:                        51.7, 42.1; 56.1, 56.5     24 x 8, 6000, 4: 52.3, 50.0; 57.6, 58.2
+//   40 x 4, 3000, 3:                         33.0, 30.9; 34.6, 35.4     24 x 4, 6000, 5: 35.0, 32.8; 37.0, 37.8
+// The ranking and a dependent read at every work-group's start cost 0 to 1 us, which equal rows do not get back.  Short partitions
+// give too little for it: 40 x 8, 700 (11 tiles) 32.3, 31.6; 36.0, 36.3, but 40 x 8, 300 (5 tiles) 24.4, 24.6; 25.3, 25.6, so these
+// go as they come.  (Fewer partitions would do for rows in order, 32 x 8 of up to 16k 90.2 us with two for 94.5 with four; other
+// partitions mean other roundings.)
+inline bool bgtq_orders_rows(int B, int n_kv, int S, int T, int n_splits, bool ragged) {
+    constexpr int64_t SHORTEST = 8, TILE = 64;
     // (a step without new tokens is a launch of any number of rows)
-    return ragged && B > 1 && S >= 1 && (int64_t)B * S <= BGTQ_ONE_LAUNCH_ROWS && (int64_t)B * n_kv * n_splits > 256;
+    return ragged && B > 1 && S >= 1 && (int64_t)B * S <= BGTQ_ONE_LAUNCH_ROWS && (int64_t)B * n_kv * n_splits > 256 &&
+           T > (SHORTEST - 1) * TILE * n_splits;
 }
 
 // The order lies at the start of the step's output, which nothing else writes before the partitions are merged.  It is written

@@ -283,11 +283,12 @@ def test_buffered_step_with_a_new_token_that_nobody_sees(bad, n_q):
     assert torch.isfinite(slow).all() and slow.abs().max() > 0 and torch.equal(fast, slow)
 
 
-# more than one round of work-groups: rows go out by falling length.  Ties, equal rows, empty rows, all 64 rows a step ranks
+# more than one round of work-groups and partitions of eight tiles: rows go out by falling length.  Ties, equal rows, rows of a
+# few tokens, all 64 rows a step ranks and one more
 @pytest.mark.parametrize("batch,n_kv,splits,window,kind", [(33, 8, 1, 0, "mixed"), (64, 1, 5, 0, "mixed"), (64, 8, 2, 0, "equal"), (9, 2, 16, 0, "mixed"),
                                                            (33, 4, 2, 64, "mixed"), (65, 4, 1, 0, "mixed")])
 def test_rows_by_falling_length_change_nothing(batch, n_kv, splits, window, kind):
-    context = 700
+    context = max(700, 500 * splits)
     gen = torch.Generator().manual_seed(batch)
     lens = [context] * batch if kind == "equal" else torch.randint(window + 5 if window else 0, context + 1, (batch,), generator=gen).tolist()
     lens[0] = context

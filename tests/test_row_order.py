@@ -52,7 +52,7 @@ extern "C" int fits_without(void) {
     s.win_k = s.win_v = s.win_old = nullptr; s.win_slot = s.win_lens = nullptr; s.win_out = s.win_lse = nullptr;
     return bgtq_order_fits(s);
 }
-extern "C" int orders(int B, int n_kv, int S, int splits, int ragged) { return bgtq_orders_rows(B, n_kv, S, splits, ragged); }
+extern "C" int orders(int B, int n_kv, int S, int T, int splits, int ragged) { return bgtq_orders_rows(B, n_kv, S, T, splits, ragged); }
 extern "C" int64_t plan_bytes(void) { return sizeof(bgtq_head_plan); }
 """
 
@@ -101,10 +101,18 @@ def test_strides_that_run_backwards_and_unaligned_outputs_keep_rows_as_they_come
 
 def test_only_batches_that_one_work_group_ranks_are_ranked(rule):
     """One thread a row: as many rows as the launch has room for, whatever the number of new tokens (0 among them)."""
-    assert [rule.orders(B, 8, 1, 8, 1) for B in (1, 4, 5, 64, 65, 130, 10**6)] == [0, 0, 1, 1, 0, 0, 0]
-    assert [rule.orders(B, 8, 0, 8, 1) for B in (1, 5, 64, 65, 130, 10**6)] == [0] * 6
-    assert [rule.orders(16, 8, S, 8, 1) for S in (-1, 0, 1, 4, 5)] == [0, 0, 1, 1, 0]
-    assert not rule.orders(16, 8, 1, 8, 0) and not rule.orders(16, 2, 1, 8, 1) and rule.orders(43, 2, 1, 3, 1)
+    T = 8192
+    assert [rule.orders(B, 8, 1, T, 8, 1) for B in (1, 4, 5, 64, 65, 130, 10**6)] == [0, 0, 1, 1, 0, 0, 0]
+    assert [rule.orders(B, 8, 0, T, 8, 1) for B in (1, 5, 64, 65, 130, 10**6)] == [0] * 6
+    assert [rule.orders(16, 8, S, T, 8, 1) for S in (-1, 0, 1, 4, 5)] == [0, 0, 1, 1, 0]
+    assert not rule.orders(16, 8, 1, T, 8, 0) and not rule.orders(16, 2, 1, T, 8, 1) and rule.orders(43, 2, 1, T, 3, 1)
+
+
+def test_short_partitions_go_as_they_come(rule):
+    """Eight tiles of 64 tokens in the longest partition at least."""
+    assert [rule.orders(40, 8, 1, T, 1, 1) for T in (0, 1, 448, 449, 512, 2**31 - 1)] == [0, 0, 0, 1, 1, 1]
+    assert [rule.orders(40, 8, 1, T, 3, 1) for T in (1344, 1345)] == [0, 1]
+    assert [rule.orders(40, 8, 1, 8192, splits, 1) for splits in (0, 16, 19, 32)] == [0, 1, 0, 0]
 
 
 # --------------------------------------------------------------------------------------- the entry itself, on the GPU
@@ -183,7 +191,7 @@ def test_output_over_a_buffer_that_is_dead_before_the_merge(shared, window):
     """264 work-groups, ragged: rows by falling length where the output is apart, as they come where it is not."""
     outs = []
     for place in (lambda out, scratch: out, lambda out, scratch: scratch[shared].view_as(out)):
-        mgr, q, k, v = _filled(33, 4, 2, 700, window)
+        mgr, q, k, v = _filled(33, 4, 2, 1000, window)
         if shared == "win_old":
             place = _over_win_old if outs else place
         outs.append(_step(mgr, q, k, v, 2, place))
