@@ -1274,13 +1274,9 @@ struct RankArgs { const int32_t* lens; int32_t* order; int B; };      // order n
 static_assert(BGTQ_ONE_LAUNCH_ROWS <= NT, "a thread a row");
 
 __device__ __forceinline__ void rank_rows(const RankArgs& r, const int tid, int* lens_s) {
-    const int len = tid < r.B ? r.lens[tid] : 0;
-    if (tid < r.B) lens_s[tid] = len;
+    if (tid < r.B) lens_s[tid] = r.lens[tid];
     __syncthreads();
-    if (tid >= r.B) return;
-    int rank = 0;                                             // (equal rows stay in order)
-    for (int i = 0; i < r.B; i++) rank += lens_s[i] > len || (lens_s[i] == len && i < tid) ? 1 : 0;
-    r.order[rank] = tid;
+    if (tid < r.B) r.order[bgtq_row_rank(lens_s, r.B, tid)] = tid;
 }
 
 // ---- decode-step preparation: append-encode K and V and rotate the queries, one launch ----

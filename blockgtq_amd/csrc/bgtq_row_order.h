@@ -1,4 +1,4 @@
-// Rows of a decode step by falling length: when a step sends them out so, where the order lies meanwhile.
+// Rows of a decode step by falling length: when a step sends them out so, a row's place, where the order lies meanwhile.
 // No device types: it compiles for the CPU alone as well.
 #pragma once
 #include <stddef.h>
@@ -24,6 +24,13 @@ inline bool bgtq_orders_rows(int B, int n_kv, int S, int T, int n_splits, bool r
     // (a step without new tokens is a launch of any number of rows)
     return ragged && B > 1 && S >= 1 && (int64_t)B * S <= BGTQ_ONE_LAUNCH_ROWS && (int64_t)B * n_kv * n_splits > 256 &&
            T > (SHORTEST - 1) * TILE * n_splits;
+}
+
+// Place of row i of n by falling length, equal rows as they come
+__host__ __device__ inline int bgtq_row_rank(const int* lens, int n, int i) {
+    int rank = 0;
+    for (int j = 0; j < n; j++) rank += lens[j] > lens[i] || (lens[j] == lens[i] && j < i) ? 1 : 0;
+    return rank;
 }
 
 // The order lies at the start of the step's output, which nothing else writes before the partitions are merged.  It is written

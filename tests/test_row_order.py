@@ -53,6 +53,7 @@ extern "C" int fits_without(void) {
     return bgtq_order_fits(s);
 }
 extern "C" int orders(int B, int n_kv, int S, int T, int splits, int ragged) { return bgtq_orders_rows(B, n_kv, S, T, splits, ragged); }
+extern "C" int rank(const int* lens, int n, int i) { return bgtq_row_rank(lens, n, i); }
 extern "C" int64_t plan_bytes(void) { return sizeof(bgtq_head_plan); }
 """
 
@@ -115,6 +116,13 @@ def test_short_partitions_go_as_they_come(rule):
     assert [rule.orders(40, 8, 1, 8192, splits, 1) for splits in (0, 16, 19, 32)] == [0, 1, 0, 0]
 
 
+@pytest.mark.parametrize("lens", [[5], [0, 0], [3, 1, 2], [7] * 64, [0, 9, 0, 9, 4, -1, 4, 2**31 - 1], [i * 37 % 11 for i in range(64)]])
+def test_rank_is_the_stable_order_by_falling_length(rule, lens):
+    ranks = [rule.rank((ctypes.c_int * len(lens))(*lens), len(lens), i) for i in range(len(lens))]
+    assert sorted(range(len(lens)), key=lambda i: ranks[i]) == sorted(range(len(lens)), key=lambda i: -lens[i])
+    assert sorted(ranks) == list(range(len(lens)))
+
+
 # --------------------------------------------------------------------------------------- the entry itself, on the GPU
 _C = {"int32_t": ctypes.c_int32, "int64_t": ctypes.c_int64, "float": ctypes.c_float}
 
@@ -129,7 +137,7 @@ def _step_type():
     return type("Step", (ctypes.Structure,), {"_fields_": fields})
 
 
-def _filled(batch, n_kv, gqa, context, window=0, seed=41):
+def _filled(batch, n_kv, gqa, context, window=0, seed=41, dtype=torch.float16):
     gen = torch.Generator().manual_seed(seed)
     lens = torch.randint(window + 5 if window else 0, context + 1, (batch,), generator=gen).tolist()
     lens[0] = context
@@ -137,11 +145,12 @@ def _filled(batch, n_kv, gqa, context, window=0, seed=41):
     mgr, energies = wl.build_manager(w, DEV)
     wl.fill_cache(mgr, w, energies, DEV)
     k, v = wl.draw_kv(w, energies[0], 1, 321, DEV, pos0=context)
-    return mgr, wl.draw_q(w, 0, DEV, context).contiguous(), k.contiguous(), v.contiguous()
+    return mgr, *[t.to(dtype).contiguous() for t in (wl.draw_q(w, 0, DEV, context), k, v)]
 
 
-def _step(mgr, q, k, v, splits, place=lambda out, scratch: out, S=1):
-    """bgtq_decode_step on layer 0; `place` says where the output lies, given one of its own and the scratch buffers."""
+def _step(mgr, q, k, v, splits, place=lambda out, scratch: out, S=1, empty=()):
+    """bgtq_decode_step on layer 0; `place` says where the output lies, given one of its own and the scratch buffers; the rows of
+    `empty` see no record."""
     B, n_q, n_kv = q.shape[0], q.shape[1], k.shape[1]
     kp, kn, vp, vn = mgr._k_packed[0], mgr._k_norms[0], mgr._v_packed[0], mgr._v_norms[0]
     f32, f16 = dict(dtype=torch.float32, device=DEV), dict(dtype=torch.float16, device=DEV)
@@ -150,6 +159,7 @@ def _step(mgr, q, k, v, splits, place=lambda out, scratch: out, S=1):
     s = _step_type()()
     s.plans = mgr._batched_args[0]["plans"].data_ptr()
     s.B, s.n_kv, s.gqa, s.S, s.n_splits, s.scale = B, n_kv, n_q // n_kv, S, splits, mgr.scale
+    s.x_dtype = int(q.dtype == torch.bfloat16)
     s.q_sb, s.q_sh = q.stride(0), q.stride(1)
     s.k_sb, s.k_sh, s.k_ss = s.v_sb, s.v_sh, s.v_ss = k.stride()[:3]
     s.k_packed, s.kp_sb, s.kp_sh, s.kp_st = kp.data_ptr(), *kp.stride()[:3]
@@ -168,6 +178,8 @@ def _step(mgr, q, k, v, splits, place=lambda out, scratch: out, S=1):
     else:
         t_pos, lens = mgr._seq_lens, mgr._seq_lens + S
         s.T = mgr.seq_len + S
+    lens = lens.clone()
+    lens[list(empty)] = 0
     s.t_pos, s.seq_lens = t_pos.data_ptr(), lens.data_ptr()
     out = place(torch.zeros(B, n_q, 128, **f16), scratch)
     for name, t in dict(scratch, out=out).items():
@@ -208,3 +220,42 @@ def test_step_without_new_tokens(batch):
     want = ops.decode_attention(plans, ops.rotate_q(plans, q[:, :, 0], 4), *cache, mgr.seq_len, seq_lens=mgr._seq_lens, n_splits=2,
                                 scale=mgr.scale, k_row_width=mgr._k_rows[0], v_row_width=mgr._vpb)
     assert torch.isfinite(got).all() and got.abs().max() > 0 and torch.equal(got, want.view_as(got))
+
+
+# query heads a KV head (9 .. 16 are two launches over one order), types, buffer; new tokens off 16 bytes enter the buffer in a
+# launch of its own, and so does the buffer's attention with one query head a KV head
+@pytest.mark.gpu
+@pytest.mark.parametrize("gqa,dtype,window,off", [(7, torch.float16, 0, 0), (12, torch.bfloat16, 0, 0), (1, torch.bfloat16, 0, 0), (2, torch.bfloat16, 64, 0),
+                                                  (12, torch.float16, 64, 0), (4, torch.float16, 64, 1), (1, torch.float16, 64, 0)])
+def test_rows_by_falling_length_and_as_they_come_are_the_same(gqa, dtype, window, off):
+    """Rows that see nothing and rows of one length among them; the cache as well."""
+    steps = []
+    for place in (lambda out, scratch: out, lambda out, scratch: scratch["q_rot"]):
+        mgr, q, k, v = _filled(33, 4, gqa, 1000, window, dtype=dtype)
+        if off:
+            k, v = [torch.cat([t.new_zeros(off), t.flatten()])[off:].view_as(t) for t in (k, v)]
+        out = _step(mgr, q, k, v, 2, place, empty=(3, 4, 32))
+        steps.append([out, mgr._k_packed[0], mgr._k_norms[0], mgr._v_packed[0], mgr._v_norms[0]] + ([mgr._buf_k, mgr._buf_v] if window else []))
+    assert torch.isfinite(steps[0][0]).all() and all(torch.equal(a, b) for a, b in zip(*steps))
+    assert (steps[0][0].flatten(1).abs().amax(1) > 0).tolist() == [window > 0 or b not in (3, 4, 32) for b in range(33)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("window", [0, 64])
+def test_captured_step_replays_by_falling_length(window):
+    """Every replay against a step of the general path (rows as they come), inputs held."""
+    (mgr, q, k, v), (general, *_) = _filled(33, 4, 2, 1000, window), _filled(33, 4, 2, 1000, window)
+    mgr.n_splits = general.n_splits = 2
+    general._native = lambda li: general._ensure_storage()
+    assert torch.equal(mgr.append_and_attend(0, q, k, v), general.append_and_attend(0, q, k, v))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = mgr.append_and_attend(0, q, k, v)
+    for turn in range(4):
+        q.add_(0.125), k.mul_(1.25), v.mul_(-0.75)
+        want = general.append_and_attend(0, q, k, v)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.isfinite(out).all() and torch.equal(out, want), turn
