@@ -833,8 +833,9 @@ __device__ __forceinline__ void encode_blocks(const EncodeArgs& a, const int h, 
 #pragma unroll
             for (int q = 0; q < D / 32; q++) {
                 load_a(q);
-                // (addresses and masks that are the same for every block would be worked out ahead of the loop: 560 instructions
-                // a wave there, half of them moves of masks to lanes and back; 18.4 -> 17.5 us for K of 8 heads of 2001 tokens)
+                // (addresses and masks that are the same for every block would be worked out ahead of the loop and spilled: with two
+                // waves a block 166 moves of masks to lanes and back and 43 scratch accesses in the kernel, 42 and 2 this way;
+                // 18.4 -> 17.5 us for K of 8 heads of 2001 tokens)
                 uint32_t segs = seg_of[q];
                 asm volatile("" : "+v"(segs));
 #pragma unroll
