@@ -294,9 +294,13 @@ __device__ __forceinline__ int grid_row(const int32_t* order) { return order[blo
 // HEADS: query heads per KV head the MFMA layout serves (4 or 8)
 // VBW: bits per V code; VST: bytes from one V record to the next (the record itself is
 // 16 * VBW bytes; a padded stride keeps the rows of a tile on different LDS banks)
+// NIB: the V records are nibbles (VBW 4), of codes of at most 3 bits as a rule.  Their pair table is the bit-packed one: a byte
+// indexes 256 entries that cannot be replicated, and reads of it are what bounds this layout (a read by 64 lanes takes a CU 2.8 ns,
+// one of 64 entries x 32 replicas 1.1 ns; with the shift and mask in front of them 2.8 and 1.3).  So a nibble pair is brought to
+// the 64-entry index by one dot product of nibbles: 4 layers of 8 rows x 2 heads of 32k, K3V3, 153.0 -> 146.3 us.
 // Order: the batch row of each grid row, or nothing.  (Asked at run time, here and in the preparation, it cost steps without an
 // order 0.6 us a layer, 2 to 3 %; as a member of DecodeArgs 0.5 %.)
-template <int HEADS, int VBW, int VST, class... Order>
+template <int HEADS, int VBW, int VST, bool NIB, class... Order>
 __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a, Order... order) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -308,7 +312,6 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a
     const int gqa = a.gqa;
     const int li = lane & 15, lg = lane >> 4;           // MFMA row/col index, lane group (value product)
     const int kl = a.k_layout;
-    const bool vnib = a.v_layout == BGTQ_V_NIBBLE;
     constexpr int WAVES_OFF = waves_off(HEADS);
 
     // ---- this partition's tiles: the tiles of the row are dealt to the partitions as evenly as
@@ -341,6 +344,10 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a
         const uint32_t* src = &P.swalk[kl][min(lane, BGTQ_MAX_WALK - 1)][0];
         asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(seg_w) : "v"(src) : "memory");
     }
+    // (bits a V code: whether the nibbles hold codes of at most 3 bits)
+    constexpr bool V_UNREP = VBW == 4;                        // 4-bit codes and every nibble record (VBW 4 by construction)
+    uint32_t v_bits = 4;
+    if constexpr (NIB) asm volatile("global_load_dword %0, %1, off" : "=v"(v_bits) : "v"(&P.v_bits) : "memory");
     // Set-up jobs: job j < (HEADS + 1) * MAX_UNITS fills one 16-byte query slot (head j / MAX_UNITS, the
     // last struct is the zero row) from the plan's unit map: a slot holds the unit's up to 8 query values,
     // zero where the unit has no dim.  The first N_QJOBS threads take one job each.
@@ -449,7 +456,7 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a
         constexpr int VCH = BGTQ_VLUT_BYTES / 1024, NCH = VCH + (BGTQ_LUT_IMAGE_BYTES + 1023) / 1024;
         constexpr int LAST_PIECES = (BGTQ_LUT_IMAGE_BYTES - (NCH - VCH - 1) * 1024) / 16;
         static_assert(BGTQ_VLUT_BYTES % 1024 == 0 && VTAB_BYTES == BGTQ_VLUT_BYTES && LAST_PIECES >= 1 && LAST_PIECES <= 64, "");
-        const uint8_t* vimg = (const uint8_t*)P.vlut_image[vnib ? 1 : 0];
+        const uint8_t* vimg = (const uint8_t*)P.vlut_image[BGTQ_V_BITPACKED];     // (of either layout: nibbles are brought to its index)
         const uint8_t* kimg_m = (const uint8_t*)P.lut_image[kl] - VCH * 1024;
         for (int cc = nw - 1 - wave; cc < NCH; cc += nw) {
             const uint8_t* src = (cc < VCH ? vimg : kimg_m) + cc * 1024;
@@ -497,7 +504,6 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a
     uint32_t qs_l = QS_OFF + (q_head >= 0 ? q_head : HEADS) * QSTRUCT;
     // PV operands: V table replica (the table sits at LDS address 0, so field bits OR-ed in never meet the
     // base; the 256-entry tables are not replicated), raw codes, P rows
-    constexpr bool V_UNREP = VBW == 4;                        // also every nibble record (VBW 4 by construction)
     constexpr int VWIN = V_UNREP ? 0 : 8;                     // replicated tables: codes fetched with the byte in front of them
     uint32_t vbank = V_UNREP ? 0u : rep;
     constexpr int vshift = V_UNREP ? 2 : 7;
@@ -525,6 +531,17 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a
     wait_loads(k_loads);
     asm volatile("" : "+v"(seg_w) :: "memory");
     const uint32_t seg_w0 = seg_w[0], seg_w1 = seg_w[1], seg_w2 = seg_w[2];
+    // Nibble records of codes of at most 3 bits: the fields' bits, and the factors that bring a nibble pair to its index
+    // c0 | c1 << bits (one dot product of nibbles a pair)
+    uint32_t v_field = 0, v_pair = 0;
+    if constexpr (NIB) {
+        asm volatile("" : "+v"(v_bits) :: "memory");
+        const uint32_t bits = __builtin_amdgcn_readfirstlane(v_bits);
+        if (bits >= 1 && bits <= 3) {
+            v_field = 0x11111111u * ((1u << bits) - 1u);
+            v_pair = 1u | (16u << bits);
+        }
+    }
     const int n_walk = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < BGTQ_MAX_WALK && seg_w1 != 0));
     if (job_wave) {
         asm volatile("" : "+v"(job_w[0]), "+v"(job_w[1]), "+v"(job_w[2]), "+v"(job_w[3]) :: "memory");
@@ -668,45 +685,61 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a
             // comes, and the 8 head rows that would repeat rows 0..7 carry the odd dims instead.
             // Lane (c = li, lg) decodes unit c of tokens 4lg .. 4lg+3 of every 16-token block; raw
             // codes are fetched one block ahead.
-            uint32_t vlo[4], vhi[4];
+            auto values = [&](auto compact_c) {
+                constexpr bool COMPACT = decltype(compact_c)::value;
+                uint32_t vlo[4], vhi[4];
 #pragma unroll
-            for (int i = 0; i < 4; i++) lds_read2(vbase + (uint32_t)i * vrow, vlo[i], vhi[i]);
+                for (int i = 0; i < 4; i++) lds_read2(vbase + (uint32_t)i * vrow, vlo[i], vhi[i]);
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const uint4v pw = lds_at<uint4v>(p_rd + k * 64);
-                uint4v W[4];                                  // [pair of the unit][token]
-                uint32_t raw[4];
+                for (int k = 0; k < 4; k++) {
+                    const uint4v pw = lds_at<uint4v>(p_rd + k * 64);
+                    uint4v W[4];                                  // [pair of the unit][token]
+                    uint32_t raw[4];
 #pragma unroll
-                for (int i = 0; i < 4; i++) raw[i] = __builtin_amdgcn_alignbyte(vhi[i], vlo[i], v_sh);
-                __builtin_amdgcn_sched_barrier(0);
-                uint32_t ad[4][4];
+                    for (int i = 0; i < 4; i++) raw[i] = __builtin_amdgcn_alignbyte(vhi[i], vlo[i], v_sh);
+                    if constexpr (COMPACT) {
 #pragma unroll
-                for (int e = 0; e < 4; e++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        constexpr uint32_t fmask = ((1u << (2 * VBW)) - 1u) << vshift;
-                        const int fp = VWIN + e * 2 * VBW;
-                        ad[e][i] = and_or(fp <= vshift ? raw[i] << (vshift - fp) : raw[i] >> (fp - vshift), fmask, vbank);
+                        for (int i = 0; i < 4; i++) raw[i] &= v_field;        // (rows past the last record hold anything)
                     }
-                __builtin_amdgcn_sched_barrier(0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    uint32_t ad[4][4];
 #pragma unroll
-                for (int e = 0; e < 4; e++)
+                    for (int e = 0; e < 4; e++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++) W[e][i] = lds_at<uint32_t>(ad[e][i]);
-                __builtin_amdgcn_sched_barrier(0);
-                if (k + 1 < 4) {
+                        for (int i = 0; i < 4; i++) {
+                            if constexpr (COMPACT) {
+                                ad[e][i] = (__builtin_amdgcn_udot8(raw[i], v_pair << (8 * e), 0u, false) << 7) | rep;
+                                continue;
+                            }
+                            constexpr uint32_t fmask = ((1u << (2 * VBW)) - 1u) << vshift;
+                            const int fp = VWIN + e * 2 * VBW;
+                            ad[e][i] = and_or(fp <= vshift ? raw[i] << (vshift - fp) : raw[i] >> (fp - vshift), fmask, vbank);
+                        }
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int i = 0; i < 4; i++) lds_read2(vbase + (uint32_t)((k + 1) * 16 + i) * vrow, vlo[i], vhi[i]);
+                    for (int e = 0; e < 4; e++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) W[e][i] = lds_at<uint32_t>(ad[e][i]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (k + 1 < 4) {
+#pragma unroll
+                        for (int i = 0; i < 4; i++) lds_read2(vbase + (uint32_t)((k + 1) * 16 + i) * vrow, vlo[i], vhi[i]);
+                    }
+                    uint4v Pa;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) Pa[i] = __builtin_amdgcn_perm(pw[i], pw[i], p_sel);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int jb = 0; jb < 4; jb++)
+                        acc[jb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, Pa),
+                                                                         __builtin_bit_cast(half8, W[jb]), acc[jb], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                uint4v Pa;
-#pragma unroll
-                for (int i = 0; i < 4; i++) Pa[i] = __builtin_amdgcn_perm(pw[i], pw[i], p_sel);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int jb = 0; jb < 4; jb++)
-                    acc[jb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, Pa),
-                                                                     __builtin_bit_cast(half8, W[jb]), acc[jb], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
+            };
+            if constexpr (NIB) {
+                if (v_pair) values(std::true_type{}); else values(std::false_type{});     // (uniform)
+            } else {
+                values(std::false_type{});
             }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -817,7 +850,7 @@ size_t seg_smem_bytes(const TileLayout& tl, int nw, bool p_over_k) {
     return (size_t)waves_off(HEADS) + (size_t)nw * wave_lds_bytes(tl, p_over_k);
 }
 
-template <int HEADS, int VBW, int VST>
+template <int HEADS, int VBW, int VST, bool NIB>
 int launch_kernel(DecodeArgs a, const int32_t* order, hipStream_t st) {
     a.tl = tile_layout(a.k_row_width, VST, (int)a.kn_st);
     // no more waves than the longest partition has tiles
@@ -850,8 +883,8 @@ int launch_kernel(DecodeArgs a, const int32_t* order, hipStream_t st) {
     }
     a.per_tiles = tiles / a.n_splits;
     a.rem_tiles = tiles - a.per_tiles * a.n_splits;
-    auto kern = decode_seg_kernel<HEADS, VBW, VST>;
-    auto ordered = decode_seg_kernel<HEADS, VBW, VST, const int32_t*>;
+    auto kern = decode_seg_kernel<HEADS, VBW, VST, NIB>;
+    auto ordered = decode_seg_kernel<HEADS, VBW, VST, NIB, const int32_t*>;
     // 1: usable, -1: not usable.  Two threads racing through the first call both run the idempotent
     // set-up below and store the same value.
     static std::atomic<int> ready{0};
@@ -876,9 +909,9 @@ int launch_kernel(DecodeArgs a, const int32_t* order, hipStream_t st) {
     return bgtq_launch_status();
 }
 
-template <int VBW, int VST>
+template <int VBW, int VST, bool NIB = false>
 int launch(const DecodeArgs& a, const int32_t* order, hipStream_t st) {
-    return a.gqa > 4 ? launch_kernel<8, VBW, VST>(a, order, st) : launch_kernel<4, VBW, VST>(a, order, st);
+    return a.gqa > 4 ? launch_kernel<8, VBW, VST, NIB>(a, order, st) : launch_kernel<4, VBW, VST, NIB>(a, order, st);
 }
 
 }  // namespace
@@ -925,6 +958,8 @@ static int launch_group(const DecodeArgs& a, const int32_t* row_order, hipStream
     // V records follow each other directly, or 4 bytes apart where the record width itself
     // (32 or 64 bytes) would put the rows of a tile on the same LDS banks
     const int64_t pad = a.vp_st - a.v_row_width;
+    if (a.v_layout == BGTQ_V_NIBBLE)
+        return pad == 0 ? launch<4, 64, true>(a, row_order, stream) : pad == 4 ? launch<4, 68, true>(a, row_order, stream) : BGTQ_EUNSUPPORTED;
     switch (a.v_row_width) {
     case 16: return pad == 0 ? launch<1, 16>(a, row_order, stream) : BGTQ_EUNSUPPORTED;
     case 32: return pad == 0 ? launch<2, 32>(a, row_order, stream) : pad == 4 ? launch<2, 36>(a, row_order, stream) : BGTQ_EUNSUPPORTED;

@@ -451,6 +451,26 @@ def test_with_buffer_manager_at_the_full_ragged_shape(oracle_lib, decode_path):
             assert np.abs(got - ref).max() < TOL, (step, b, h, np.abs(got - ref).max())
 
 
+@pytest.mark.parametrize("vb", [1, 2, 3, 4])
+@pytest.mark.parametrize("stride", [64, 68])
+def test_nibble_records_of_every_code_width(oracle_lib, vb, stride, decode_path):
+    """Nibble V records, together and 4 bytes apart, whole tiles and remainders; what lies behind the last record, nibbles that
+    no code has and not-a-number norms among it, is not looked at."""
+    args, qs, q_rot, kp, kn, vp, vn = _build(192, 1, 8, vb, 2, 8, 2, 200, seed=60 + vb, k_layout=1, v_layout=1)
+    wide = torch.full((2, 2, 202, stride), 255, dtype=torch.uint8, device=DEV)
+    wide[..., :64] = vp
+    for T in (1, 63, 64, 129, 200):
+        kp2, kn2, vp2, vn2 = kp.clone(), kn.clone(), wide.clone(), vn.clone()
+        kp2[:, :, T:], vp2[:, :, T:], kn2[:, :, T:], vn2[:, :, T:] = 255, 255, float("nan"), float("nan")
+        ref, ref_lse = _reference(oracle_lib, args['plans_np'], qs, kp.cpu().numpy(), kn.cpu().numpy(), vp.cpu().numpy(),
+                                  vn.cpu().numpy(), q_rot.cpu().numpy(), [T, T], 8, 1, 1, vb)
+        out, lse = ops.decode_attention(args['plans'], q_rot, kp2, kn2, vp2[..., :64], vn2, T, n_splits=2, k_layout=1, v_layout=1,
+                                        return_lse=True)
+        assert np.abs(out.float().cpu().numpy() - ref).max() < TOL, T
+        assert np.abs(lse.cpu().numpy() - ref_lse).max() < LSE_TOL
+        assert ops.last_decode_path() == (ops.MFMA_PATH if decode_path == "auto" else ops.GENERIC_PATH)
+
+
 @pytest.mark.parametrize("k_layout,v_layout,vb", [(0, 0, 3), (1, 1, 3), (1, 0, 4), (0, 1, 2), (1, 1, 4)])
 def test_mfma_kernel_takes_every_record_layout(oracle_lib, k_layout, v_layout, vb):
     """With the layout-agnostic kernel switched off, the MFMA kernel must accept bit-packed
