@@ -19,7 +19,9 @@ HOST_PATH = os.path.join(LIB_DIR, "_bgtq_host.so")       # CPython extension nex
 ARCH = "gfx950"
 COMMON = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-std=c++17",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-          "-fhip-fp32-correctly-rounded-divide-sqrt"]
+          "-fhip-fp32-correctly-rounded-divide-sqrt",
+          # leading scalar arguments of a kernel are in registers when its waves start, instead of a trip to memory away
+          "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 # source file -> extra flags.  The encoders promise a fixed floating-point
 # evaluation order, so nothing in that file may be contracted into an fma
 # behind the author's back.
