@@ -1250,15 +1250,18 @@ __device__ __forceinline__ void rotate_q_group(const RotQArgs& a, const int64_t 
             a.q_rot[row * a.qr_sr + (int64_t)(h * gqa + h_first + r) * a.qr_sh + j] = bgtq_f2h(acc[r]);
 }
 
-// Work-group `bid` of the query part: a.group heads of one (row, KV head).  One head per
+// Query heads [part * a.group, ..) of one (row, KV head).  One head per
 // work-group where that still leaves the chip partly idle (every work-group fetches the 64 KB
 // rotation), four where the rows are many.
+__device__ __forceinline__ void rotate_q_block(const RotQArgs& a, const int row, const int h, const int part, float* rot_s) {
+    if (a.group == 1) rotate_q_group<1>(a, row, h, part, rot_s);
+    else              rotate_q_group<4>(a, row, h, part * 4, rot_s);
+}
 __device__ __forceinline__ void rotate_q_block(const RotQArgs& a, const int bid, float* rot_s) {
     const int n_kv = a.n_q / a.gqa;
     const int per = (a.gqa + a.group - 1) / a.group;            // work-groups per (row, KV head)
     const int rowh = bid / per, part = bid - rowh * per;
-    if (a.group == 1) rotate_q_group<1>(a, rowh / n_kv, rowh % n_kv, part, rot_s);
-    else              rotate_q_group<4>(a, rowh / n_kv, rowh % n_kv, part * 4, rot_s);
+    rotate_q_block(a, rowh / n_kv, rowh % n_kv, part, rot_s);
 }
 __host__ inline int rotate_q_group_size(int64_t n_rows, int n_q) { return n_rows * n_q > 256 ? 4 : 1; }
 __host__ inline unsigned rotate_q_blocks(int64_t n_rows, int n_kv, int gqa, int group) {
@@ -1296,19 +1299,37 @@ __device__ __forceinline__ void prepare_part(const EncodeArgs& ak, const EncodeA
     }
 }
 // (BF16: some input is; asking at run time costs the chains of fp16 inputs 0.2 of 5.0 us)
-// Rank: RankArgs of a first work-group that ranks the rows, or nothing.  (Behind the others it started when a place came free
-// and ended last: 64 equal rows x 8 heads of 700 tokens 43.1 us a step as they come, 45.5 with a last one, 43.9 with a first.)
-template <bool BF16, class... Rank>
-__global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, int rows, Rank... rank) {
-    if (!BF16) ak.bf16 = av.bf16 = aq.bf16 = 0;
+// Steps of one token whose rows need no rank, which is nearly all: the grid is (rows, KV heads, 2 + query parts), with no division
+// on the way to a work-group's rows, and what the first loads need (plans, K and V rows) comes as arguments of its own ahead of
+// the blocks: they are in scalar registers when a wave starts (kernarg preload), the blocks a trip to memory behind it.  With
+// the attention's and the merge's arguments taken the same way: one row x 8 heads of 4k tokens 66.8 -> 63.0 us (4 layers), 4 rows x
+// 2 heads of 8k 152.3 -> 146.7 (8), 12 ragged rows of 7-head groups 88.4 -> 85.2 (4), 8 x 2 of 32k 201.9 -> 195.1 (6); 65.2,
+// 151.2 and 87.3 of them with the merge alone.
+template <bool BF16>
+__global__ __launch_bounds__(NT) void prepare_token_kernel(const bgtq_head_plan* plans, const uint16_t* v, const uint16_t* k, uint32_t v_sb, uint32_t v_sh,
+                                                           uint32_t k_sb, uint32_t k_sh, EncodeArgs ak, EncodeArgs av, RotQArgs aq) {
     __shared__ __align__(16) float rot_s[D * D];       // the work-group's rotation, whatever its role
-    int bid = blockIdx.x;
-    if constexpr (sizeof...(Rank) != 0)
-        if (bid-- == 0) {                              // (uniform)
-            rank_rows(rank..., threadIdx.x, (int*)rot_s);
-            return;
-        }
-    prepare_part(ak, av, aq, rows, bid, rot_s);
+    if (!BF16) ak.bf16 = av.bf16 = aq.bf16 = 0;
+    ak.plans = av.plans = aq.plans = plans;
+    av.x = v; av.x_sb = v_sb; av.x_sh = v_sh;
+    ak.x = k; ak.x_sb = k_sb; ak.x_sh = k_sh;
+    ak.S = av.S = 1;
+    const int row = blockIdx.x, h = blockIdx.y, role = blockIdx.z;
+    if (role == 0) encode_row<true>(av, row, h, threadIdx.x, rot_s);
+    else if (role == 1) encode_row<false>(ak, row, h, threadIdx.x, rot_s);
+    else rotate_q_block(aq, row, h, role - 2, rot_s);
+}
+// All others.  A first work-group ranks the rows, if any are to be ranked.  (Behind the others it started when a place came free
+// and ended last: 64 equal rows x 8 heads of 700 tokens 43.1 us a step as they come, 45.5 with a last one, 43.9 with a first.)
+template <bool BF16>
+__global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, int rows, RankArgs rank) {
+    if (!BF16) ak.bf16 = av.bf16 = aq.bf16 = 0;
+    __shared__ __align__(16) float rot_s[D * D];
+    if (blockIdx.x == 0) {                             // (uniform)
+        rank_rows(rank, threadIdx.x, (int*)rot_s);
+        return;
+    }
+    prepare_part(ak, av, aq, rows, blockIdx.x - 1, rot_s);
 }
 // The same with the attention over the buffered tokens, which depends on none of it: the longer work-groups first, in
 // the LDS that is a rotation's otherwise; then the token that leaves the buffer, K and V by the two halves of a
@@ -1413,7 +1434,7 @@ int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, in
     const int group = rotate_q_group_size(B, n_kv * gqa);
     RotQArgs aq{ak.plans, (const uint16_t*)q, q_sr, q_sh, (uint16_t*)q_rot, qr_sr, qr_sh, B, n_kv * gqa, gqa, group, q_bf16};
     const int rows = (int)N;
-    const unsigned blocks = (unsigned)(2 * rows * n_kv) + (q ? rotate_q_blocks(B, n_kv, gqa, group) : 0u) + (rank.order ? 1u : 0u);
+    const unsigned blocks = (unsigned)(2 * rows * n_kv) + (q ? rotate_q_blocks(B, n_kv, gqa, group) : 0u) + (rank.order || !window ? 1u : 0u);
     if (window) {
         const WindowArgs& w = *window;
         const dim3 grid(blocks - (unsigned)(rows * n_kv) + (unsigned)(B * n_kv));
@@ -1428,12 +1449,18 @@ int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, in
         }
     } else {
         const bool bf16 = ak.bf16 || av.bf16 || (q && q_bf16);
-        if (rank.order) {
-            auto kern = bf16 ? prepare_kernel<true, RankArgs> : prepare_kernel<false, RankArgs>;
-            hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows, rank);
+        const int64_t strides[] = {av.x_sb, av.x_sh, ak.x_sb, ak.x_sh};
+        bool token = !rank.order && ak.S == 1;
+        for (int64_t each : strides) token = token && each >= 0 && each < (int64_t)1 << 32;
+        if (token) {
+            auto kern = bf16 ? prepare_token_kernel<true> : prepare_token_kernel<false>;
+            const dim3 grid((unsigned)rows, (unsigned)n_kv, 2u + (q ? (unsigned)((gqa + group - 1) / group) : 0u));
+            hipLaunchKernelGGL(kern, grid, dim3(NT), 0, st, ak.plans, av.x, ak.x, (uint32_t)av.x_sb, (uint32_t)av.x_sh,
+                               (uint32_t)ak.x_sb, (uint32_t)ak.x_sh, ak, av, aq);
         } else {
+            // (no rows are ranked where rank.order is null)
             auto kern = bf16 ? prepare_kernel<true> : prepare_kernel<false>;
-            hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows);
+            hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows, rank.order ? rank : RankArgs{});
         }
     }
     return bgtq_launch_status();

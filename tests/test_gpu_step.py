@@ -305,3 +305,25 @@ def test_rows_by_falling_length_change_nothing(batch, n_kv, splits, window, kind
     general._native = lambda li: general._ensure_storage()          # (rows as they come)
     for _ in range(2):
         assert torch.equal(mgrs[0].append_and_attend(0, q, k, v), general.append_and_attend(0, q, k, v))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_token_rows_at_strides_beyond_32_bits(dtype):
+    """New rows whose batch stride leaves 32 bits (one batch row: it is never used) take the general preparation, others the one
+    of single tokens: the same step, also with heads that share a row of K and lie apart in V."""
+    w, e, caches = _pair()
+    one = lambda t: t[:1].expand(2, -1, -1, -1)
+    q, k, v = [t.contiguous() for t in _inputs(w, [e], 90, dtype)]
+    outs = [caches[0].encode_and_attend(0, one(q), k[:1, :1].expand(2, 4, 1, 128), one(v)),
+            caches[1].encode_and_attend(0, one(q).contiguous(), k[:1, :1].expand(2, 4, 1, 128).contiguous(), one(v).contiguous())]
+    assert outs[0].abs().max() > 0 and torch.equal(*outs)
+    w1 = wl.Workload("t", 1, 8, 2, 1, 90, 1e6, seed=38)
+    got = []
+    for far in (False, True):
+        mgr, energies = wl.build_manager(w1, DEV)
+        wl.fill_cache(mgr, w1, energies, DEV)
+        q, k, v = [t.contiguous() for t in _inputs(w1, energies, 90, dtype)]
+        if far:
+            k, v = [t.as_strided((1, 2, 1, 128), (2 ** 33, 128, 128, 1)) for t in (k, v)]
+        got.append((mgr.append_and_attend(0, q, k, v), mgr._k_packed[0], mgr._k_norms[0], mgr._v_packed[0], mgr._v_norms[0]))
+    assert got[0][0].abs().max() > 0 and all(torch.equal(a, b) for a, b in zip(*got))
