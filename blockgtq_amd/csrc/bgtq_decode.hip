@@ -765,7 +765,7 @@ int bgtq_decode_step(const bgtq_step* step, void* stream) {
 
 size_t bgtq_plan_sizeof(void) { return sizeof(bgtq_head_plan); }
 int bgtq_abi_version(void) { return 8; }
-int bgtq_decode_kernel_revision(void) { return 10; }
+int bgtq_decode_kernel_revision(void) { return 11; }
 
 const char* bgtq_strerror(int code) {
     switch (code) {

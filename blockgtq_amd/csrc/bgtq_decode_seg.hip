@@ -298,10 +298,15 @@ __device__ __forceinline__ int grid_row(const int32_t* order) { return order[blo
 // indexes 256 entries that cannot be replicated, and reads of it are what bounds this layout (a read by 64 lanes takes a CU 2.8 ns,
 // one of 64 entries x 32 replicas 1.1 ns; with the shift and mask in front of them 2.8 and 1.3).  So a nibble pair is brought to
 // the 64-entry index by one dot product of nibbles: 4 layers of 8 rows x 2 heads of 32k, K3V3, 153.0 -> 146.3 us.
+// plans .. rem_tiles: members of the argument block that the first requests need, in front of it, where they are in scalar
+// registers when a wave starts (kernarg preload, 14 dwords at most): walk words and tables do not wait for the block.
 // Order: the batch row of each grid row, or nothing.  (Asked at run time, here and in the preparation, it cost steps without an
 // order 0.6 us a layer, 2 to 3 %; as a member of DecodeArgs 0.5 %.)
 template <int HEADS, int VBW, int VST, bool NIB, class... Order>
-__global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(DecodeArgs a, Order... order) {
+__global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(const bgtq_head_plan* plans, const int32_t* seq_lens, int k_layout, int waves, int tile_waves,
+                                                                      int T_max, int n_splits, int per_tiles, int rem_tiles, DecodeArgs a, Order... order) {
+    a.plans = plans, a.seq_lens = seq_lens, a.k_layout = k_layout, a.nw = waves, a.nw_tiles = tile_waves;
+    a.T = T_max, a.n_splits = n_splits, a.per_tiles = per_tiles, a.rem_tiles = rem_tiles;
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -904,8 +909,10 @@ int launch_kernel(DecodeArgs a, const int32_t* order, hipStream_t st) {
     }
     if (ready.load(std::memory_order_acquire) < 0) return BGTQ_EUNSUPPORTED;
     dim3 grid((unsigned)a.n_splits, (unsigned)a.n_kv, (unsigned)a.B);
-    if (order) hipLaunchKernelGGL(ordered, grid, dim3(a.nw * 64), smem, st, a, order);
-    else hipLaunchKernelGGL(kern, grid, dim3(a.nw * 64), smem, st, a);
+    if (order) hipLaunchKernelGGL(ordered, grid, dim3(a.nw * 64), smem, st, a.plans, a.seq_lens, a.k_layout, a.nw, a.nw_tiles, a.T,
+                                  a.n_splits, a.per_tiles, a.rem_tiles, a, order);
+    else hipLaunchKernelGGL(kern, grid, dim3(a.nw * 64), smem, st, a.plans, a.seq_lens, a.k_layout, a.nw, a.nw_tiles, a.T,
+                            a.n_splits, a.per_tiles, a.rem_tiles, a);
     return bgtq_launch_status();
 }
 
