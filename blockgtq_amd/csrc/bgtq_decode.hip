@@ -278,9 +278,6 @@ __global__ __launch_bounds__(RT_THREADS) void lse_reduce_kernel(
     constexpr int RT_CLASSES = RT_THREADS / 32;
     __shared__ __align__(16) float cls_sum[RT_CLASSES][D];
     __shared__ float vec[D];
-    __shared__ float wgt[BGTQ_MAX_SPLITS];
-    __shared__ float red[RT_THREADS / 64];
-    __shared__ float dsum[RT_CLASSES];
     const int j = threadIdx.x;
     const int cls = j >> 5, c4 = (j & 31) * 4;
     const int h = blockIdx.y, hq = h * gqa + blockIdx.x, b = blockIdx.z;
@@ -291,56 +288,60 @@ __global__ __launch_bounds__(RT_THREADS) void lse_reduce_kernel(
     const float* po = part_out + row * n_splits * D + c4;
 
     // loads land in issue order: the partitions' log-sum-exps go first, so that the maximum and
-    // the weights are worked out while the vectors and the un-rotation are still on their way
-    const float l_first = j < n_splits ? pl[j] : -INFINITY;
+    // the weights are worked out while the vectors and the un-rotation are still on their way.  Every wave works out
+    // maximum and denominator by itself, 16 lanes beside each other over all partitions, and a thread the weights of its
+    // own row class: no trip through LDS and two barriers less (one row x 32 heads of 4k tokens 63.0 -> 61.5 us for 4 layers, 4 x 16
+    // of 8k 146.7 -> 144.3 for 8, 12 x 28 ragged 85.2 -> 84.4 for 4).
     constexpr int NB = 16 / RT_CLASSES;        // rounds of partial vectors fetched before anything else (16 vectors)
+    constexpr int NL = 4;                      // log-sum-exps a lane holds of all of them
+    const int s16 = j & 15;
+    float l_all[NL], l_own[NB];
+#pragma unroll
+    for (int i = 0; i < NL; i++) l_all[i] = s16 + 16 * i < n_splits ? pl[s16 + 16 * i] : -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NB; i++) l_own[i] = RT_CLASSES * i + cls < n_splits ? pl[RT_CLASSES * i + cls] : -INFINITY;
     float4 pv[NB];
 #pragma unroll
     for (int i = 0; i < NB; i++) pv[i] = *(const float4*)(po + (size_t)min(RT_CLASSES * i + cls, n_splits - 1) * D);
+    const float x0 = n_extra && j < D ? extra_out[row * n_extra * D + j] : 0.f;
     float4 rv[D / RT_CLASSES];                 // rows 16 i + cls of the un-rotation, this thread's four columns
     if (unrotate) {
 #pragma unroll
         for (int i = 0; i < D / RT_CLASSES; i++) rv[i] = *(const float4*)(R + (RT_CLASSES * i + cls) * D + c4);
     }
 
-    float m = l_first;
-    if (j < n_splits) wgt[j] = l_first;
-    for (int c = j + RT_THREADS; c < n_splits; c += RT_THREADS) { float l = pl[c]; wgt[c] = l; m = fmaxf(m, l); }
-    for (int c = j; c < n_extra; c += RT_THREADS) m = fmaxf(m, el[c]);
-    m = wave_max(m);
-    if ((j & 63) == 0) red[j >> 6] = m;
-    __syncthreads();
-    m = red[0];
-#pragma unroll
-    for (int i = 1; i < RT_THREADS / 64; i++) m = fmaxf(m, red[i]);
-    if (m == -INFINITY) {                      // nothing visible at all
+    float m = fmaxf(fmaxf(l_all[0], l_all[1]), fmaxf(l_all[2], l_all[3]));
+    for (int c = s16 + 16 * NL; c < n_splits; c += 16) m = fmaxf(m, pl[c]);
+    m = row16_max(m);
+    for (int e = 0; e < n_extra; e++) m = fmaxf(m, el[e]);
+    if (m == -INFINITY) {                      // nothing visible at all (the same in every thread)
         if (j < D) out[b * o_sb + hq * o_sh + j] = 0;
         if (lse_out && j == 0) lse_out[row] = -INFINITY;
         return;
     }
     // weights: exp(lse - m), 0 for empty partitions (their vectors are undefined)
-    for (int c = j; c < n_splits; c += RT_THREADS) { float l = wgt[c]; wgt[c] = (l == -INFINITY) ? 0.f : __expf(l - m); }
-    __syncthreads();
-    float dcl = 0.f;                           // weight sum of this thread's row class
+    auto weight = [&](float l) { return l == -INFINITY ? 0.f : __expf(l - m); };
+    float den = 0.f;
+#pragma unroll
+    for (int i = 0; i < NL; i++) den += weight(l_all[i]);
+    for (int c = s16 + 16 * NL; c < n_splits; c += 16) den += weight(pl[c]);
+    den = row16_sum(den);
     float4 a4 = {0.f, 0.f, 0.f, 0.f};
     auto add = [&](float w, const float4& v) {
-        dcl += w;
         if (w != 0.f) { a4.x += w * v.x; a4.y += w * v.y; a4.z += w * v.z; a4.w += w * v.w; }
     };
 #pragma unroll
-    for (int i = 0; i < NB; i++)
-        if (RT_CLASSES * i + cls < n_splits) add(wgt[RT_CLASSES * i + cls], pv[i]);
-    for (int c = RT_CLASSES * NB + cls; c < n_splits; c += RT_CLASSES) add(wgt[c], *(const float4*)(po + (size_t)c * D));
+    for (int i = 0; i < NB; i++) add(weight(l_own[i]), pv[i]);
+    for (int c = RT_CLASSES * NB + cls; c < n_splits; c += RT_CLASSES) add(weight(pl[c]), *(const float4*)(po + (size_t)c * D));
     *(float4*)&cls_sum[cls][c4] = a4;
-    if ((j & 31) == 0) dsum[cls] = dcl;
-    float acce = 0.f, den = 0.f;
+    float acce = 0.f;
     if (j < D)
         for (int e = 0; e < n_extra; e++) {
             float l = el[e];
             if (l == -INFINITY) continue;
             float w = __expf(l - m);
             den += w;
-            acce += w * extra_out[(row * n_extra + e) * D + j];
+            acce += w * (e == 0 ? x0 : extra_out[(row * n_extra + e) * D + j]);
         }
     __syncthreads();
     // the classes are added pairwise in a fixed order
@@ -355,17 +356,7 @@ __global__ __launch_bounds__(RT_THREADS) void lse_reduce_kernel(
         return s[0];
     };
     float res = 0.f;
-    if (j < D) {
-        float ds[RT_CLASSES];
-#pragma unroll
-        for (int i = 0; i < RT_CLASSES; i++) ds[i] = dsum[i];
-#pragma unroll
-        for (int w = RT_CLASSES / 2; w >= 1; w >>= 1)
-#pragma unroll
-            for (int i = 0; i < w; i++) ds[i] = ds[2 * i] + ds[2 * i + 1];
-        den += ds[0];
-        res = fold(cls_sum, j);
-    }
+    if (j < D) res = fold(cls_sum, j);
     if (unrotate) {
         if (j < D) vec[j] = res;
         __syncthreads();                       // also: every read of cls_sum above is done

@@ -27,6 +27,14 @@ __device__ __forceinline__ float row16_sum(float x) {
     return x;
 }
 
+__device__ __forceinline__ float row16_max(float x) {
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x128, 0xf, 0xf, false)));
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x124, 0xf, 0xf, false)));
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x122, 0xf, 0xf, false)));
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x121, 0xf, 0xf, false)));
+    return x;
+}
+
 // The token that enters the buffer in this step (slot[b], nothing where that lies outside [0, W)), where the launch itself
 // puts it there: the attention takes that row from the new tokens whatever the slot holds by then.
 struct WindowSwap {

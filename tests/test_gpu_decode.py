@@ -718,6 +718,40 @@ def test_merge_entry_point_refuses_what_its_kernel_cannot_take():
         _capi.check(call(_capi.ptr(part[1:]), 4), "bgtq_lse_reduce")
 
 
+@pytest.mark.parametrize("B", [1, 70])                       # 512 threads a row, and 128 from 257 rows on
+@pytest.mark.parametrize("n_splits,n_extra", [(1, 0), (3, 1), (15, 0), (16, 2), (17, 1), (63, 0), (64, 1), (65, 0), (200, 3), (512, 1)])
+def test_merge_over_partition_counts(B, n_splits, n_extra):
+    """Weighted mean of partials by exp(lse), un-rotated, plus partials that are not; empty ones hold anything.  fp16 output of
+    fp32 sums of values near 1: half an fp16 step and 1e-5 of the terms' sum (128 products of a rotation row)."""
+    from blockgtq_amd import _capi
+    args = _build(192, 1, 5, 3, 2, 2, 1, 4, seed=3)[0]
+    n_kv, gqa = 2, 2
+    gen = torch.Generator(device=DEV).manual_seed(n_splits)
+    part = torch.randn(B, 4, n_splits, 128, generator=gen, device=DEV)
+    lse = torch.randn(B, 4, n_splits, generator=gen, device=DEV) * 3
+    empty = torch.rand(B, 4, n_splits, generator=gen, device=DEV) < 0.3
+    empty[0, 1] = True                                       # (a row that sees nothing, or the extra partials alone)
+    part[empty], lse[empty] = float("nan"), -float("inf")
+    xo = torch.randn(B, 4, max(n_extra, 1), 128, generator=gen, device=DEV)
+    xl = torch.randn(B, 4, max(n_extra, 1), generator=gen, device=DEV)
+    xl[..., 1:] = -float("inf")
+    out, tot = torch.zeros(B, 4, 128, dtype=torch.float16, device=DEV), torch.zeros(B, 4, device=DEV)
+    _capi.check(_capi.lib().bgtq_lse_reduce(
+        _capi.ptr(args['plans']), _capi.ptr(part), _capi.ptr(lse), n_splits, _capi.ptr(xo) if n_extra else None,
+        _capi.ptr(xl) if n_extra else None, n_extra, B, n_kv, gqa, 1, _capi.ptr(out), 512, 128, _capi.ptr(tot),
+        _capi.stream_ptr(out.device)), "bgtq_lse_reduce")
+    R = torch.tensor(np.stack([args['plans_np']['v_rot'][h] for h in range(n_kv)])).to(DEV).double().reshape(n_kv, 1, 128, 128)
+    every = torch.cat([lse, xl], -1) if n_extra else lse
+    want_lse = every.double().logsumexp(-1)
+    w = torch.where(torch.isinf(want_lse), torch.zeros_like(want_lse), want_lse).unsqueeze(-1)
+    acc = (torch.where(empty, 0.0, (lse.double() - w).exp()).unsqueeze(-1) * part.nan_to_num().double()).sum(-2)
+    want = (acc.reshape(B, n_kv, gqa, 1, 128) @ R).reshape(B, 4, 128)
+    if n_extra:
+        want += ((xl.double() - w).exp().unsqueeze(-1) * xo.double()).sum(-2)
+    torch.testing.assert_close(out.double(), want, rtol=6e-4, atol=2e-5)
+    torch.testing.assert_close(tot.double(), want_lse, rtol=1e-5, atol=2e-5)
+
+
 def test_window_swap_equals_indexed_copies():
     """The one-launch ring update of the with-buffer append against the tensor operations it
     replaces, bit for bit, on strided buffers (a layer slice of a larger tensor)."""
