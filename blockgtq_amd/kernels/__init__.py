@@ -45,9 +45,11 @@ def _quantizer_of(codebook_flat):
     return entry[1]()
 
 
-def _plan_from_args(codebook_flat, segments, v_lut, v_rotation, v_bits, device):
+def _plan_from_args(codebook_flat, segments, v_lut, v_rotation, v_bits, v_nibble, device):
     """Decode-only plan assembled from the loose arguments of the fused entry
-    (used when the codebook was not produced by this package's quantizer)."""
+    (used when the codebook was not produced by this package's quantizer).
+    Nibble records do not need ``v_bits`` (callers leave it 0): every entry of
+    ``v_lut`` is a code then."""
     p = np.zeros((), dtype=_plan.PLAN_DTYPE)
     segs = [s for s in segments if s[2] > 0]
     p['n_seg'] = len(segs)
@@ -73,7 +75,9 @@ def _plan_from_args(codebook_flat, segments, v_lut, v_rotation, v_bits, device):
                                  else nib + (start - int(p['nopack_start'])))
     p['k_row_bytes'] = tot
     p['k_mixed_bytes'] = nib + nopack_len
-    p['v_bits'] = v_bits
+    if v_nibble:
+        v_bits = min(4, max(int(v_bits), 1, (v_lut.numel() - 1).bit_length()))
+    p['v_bits'] = int(v_bits)
     lut = v_lut.detach().cpu().to(torch.float16).numpy().view(np.uint16)
     p['v_lut_f16'][:lut.size] = lut
     if v_rotation is not None:
@@ -123,8 +127,7 @@ def fused_blockgtq_decode_attention(
     if quant is not None:
         plans = quant.device_plan()
     else:
-        plans = _plan_from_args(codebook_flat, segments, v_lut, v_rotation,
-                                int(v_bits) if not v_nibble else max(int(v_bits), 1), q.device)
+        plans = _plan_from_args(codebook_flat, segments, v_lut, v_rotation, v_bits, v_nibble, q.device)
     if v_norms.dim() == 4:
         v_norms = v_norms[..., 0]
     n_splits = max(1, min(int(t_splits), 512))
@@ -178,8 +181,7 @@ def fused_blockgtq_prefill_attention(
     if quant is not None:
         plans = quant.device_plan()
     else:
-        plans = _plan_from_args(codebook_flat, segments, v_lut, v_rotation,
-                                int(v_bits) if not v_nibble else max(int(v_bits), 1), q.device)
+        plans = _plan_from_args(codebook_flat, segments, v_lut, v_rotation, v_bits, v_nibble, q.device)
     if v_norms.dim() == 4:
         v_norms = v_norms[..., 0]
     kl = _plan.K_MIXED if k_nibble else _plan.K_BITPACKED

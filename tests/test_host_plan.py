@@ -686,3 +686,27 @@ def test_v_encoder_tables(v_bits):
     vt = p['v_rot_T'].reshape(128, 128)
     for r in (0, 1, 5, 66, 127):
         assert np.array_equal(p['v_rot_T4'][r // 4, :, r % 4], vt[r])
+
+
+@pytest.mark.parametrize("entry", ["fused_blockgtq_decode_attention", "fused_blockgtq_prefill_attention"])
+@pytest.mark.parametrize("bits", [1, 2, 3, 4])
+@pytest.mark.parametrize("given", [0, None])                  # (the argument's default and the width itself)
+def test_nibble_records_of_foreign_tensors_hold_every_code_of_the_v_table(entry, bits, given, monkeypatch):
+    from blockgtq_amd import kernels
+    q8, _ = make_quantizer(seed=bits, v_bits=bits)
+    a, plans = q8.build_kernel_args(), []
+
+    def upload(p, device):
+        plans.append(p)
+        raise InterruptedError                                # (the plan is all there is to see off the GPU)
+
+    monkeypatch.setattr(kernels._plan, "upload_plans", upload)
+    rows = torch.zeros(1, 1, 4, 64, dtype=torch.uint8)
+    norms = torch.zeros(1, 1, 4, 5, dtype=torch.float16)
+    with pytest.raises(InterruptedError):
+        getattr(kernels, entry)(torch.zeros(1, 4, 1, 128, dtype=torch.float16), rows, norms, a['codebook_flat'].clone(), a['lut_offset'],
+                                a['norm_group'], a['segments_b'], rows, norms[..., 0], q8.v_lut, v_bits=bits if given is None else given,
+                                k_nibble=True, v_nibble=True)
+    own = q8.plan()
+    assert plans[0]['v_bits'][0] == bits
+    assert np.array_equal(plans[0]['vlut_image'], own['vlut_image'])
