@@ -257,21 +257,31 @@ int launch_generic(const DecodeArgs& a, hipStream_t st) {
 }
 
 // ---- partition merge + V un-rotation ------------------------------------------
-// One work-group of NTHR threads per (batch row, query head).  Its loads are 16 bytes a lane
+// One work-group of RT_THREADS threads per (batch row, query head).  Its loads are 16 bytes a lane
 // and contiguous across the wave: thread t holds columns 4(t & 31) .. +3 of the rows
-// r = t >> 5 (mod NTHR / 32) of the partial vectors and of the un-rotation, sums over its own
-// rows, and the NTHR / 32 row classes are added through LDS (in a fixed order, so the result
-// does not depend on timing).  Every load that does not depend on a computed value
-// (the first round of partial vectors, the whole un-rotation) is issued up front, so the
-// kernel pays for about one memory round trip.  512 threads (16 classes: 8 rows of the
-// un-rotation a thread instead of 32) where the launch has at most one work-group per compute
-// unit, 128 threads where work-groups queue up.
-// Grid (heads of a group, KV heads, rows): no division on the way to the un-rotation.  The arguments up to n_extra fill the 14
-// scalar registers that hold them when a wave starts (kernarg preload): the first loads go out at once.  One row x 32 heads of
+// r = t >> 5 (mod RT_THREADS / 32) of the partial vectors and of the un-rotation, sums over its own
+// rows, and the RT_THREADS / 32 row classes are added through LDS (in a fixed order, so the result
+// does not depend on timing).  What depends on no computed value is asked for up front: the log-sum-exps,
+// 16 partial vectors and the whole un-rotation.  Partitions behind the first 16 cost a round of loads each
+// RT_THREADS / 32 of them.  512 threads (16 classes: 8 rows of the un-rotation a thread instead of 32) where the
+// launch has at most one work-group per compute unit, 128 threads where work-groups queue up.
+// Grid (heads of a group, KV heads, rows): no division on the way to the un-rotation.  The arguments up to n_extra fill 13 of the
+// 14 scalar registers that hold them when a wave starts (kernarg preload): the first loads go out at once.  One row x 32 heads of
 // 4k tokens 66.8 -> 65.2 us (4 layers), 4 x 16 of 8k 152.8 -> 151.2 (8), 12 x 28 ragged 88.2 -> 87.3 (4).
+// MANY: how the weights of the partitions come about.  Up to merge_held() of them every wave works out maximum and denominator by
+// itself, 16 lanes beside each other over log-sum-exps that they hold, and a thread the weights of its own row class: no trip through
+// LDS and two barriers less.  Behind the first round of vectors it reads a log-sum-exp and then a vector, two trips; more partitions
+// are therefore weighed once by the whole work-group, in LDS.  us a launch (repeated in a graph), held and by the work-group:
+//   512 threads, 1 row x 4 heads: 24 partitions 2.74, 3.22; 48 3.20, 3.46; 64 3.52, 3.64; 85 4.27, 3.94; 128 5.33, 4.37; 256 8.62, 5.80
+//                1 row x 32 heads: 24 2.82, 3.27; 64 3.60, 3.71; 85 4.41, 4.03; 128 5.48, 4.44 (past 64 with loops over the rest)
+//   128 threads, 9 rows x 32 heads: 18 4.17, 4.22; 20 4.19, 4.25; 22 4.64, 4.63; 24 4.88, 4.71; 32 6.08, 5.46
+//                32 rows x 32 heads: 18 6.19, 6.28; 20 6.39, 6.29; 22 6.83, 6.73; 24 6.90, 6.77; 32 7.97, 7.19; 64 16.2, 12.5
+// (one row x 32 heads of 4k tokens, 32 partitions: 63.0 -> 61.5 us for 4 layers, 4 x 16 of 8k 146.7 -> 144.3 for 8, 12 x 28 ragged
+// 85.2 -> 84.4 for 4; one row x 4 heads of 65k, 256 partitions, a layer: 25.9 us held, 20.1 by the work-group)
+constexpr int merge_held(int threads) { return threads == 512 ? 64 : 20; }
 static_assert(offsetof(bgtq_head_plan, v_rot) % 16 == 0 && sizeof(bgtq_head_plan) % 16 == 0,
               "the un-rotation is read 16 bytes at a time");
-template <int RT_THREADS>
+template <int RT_THREADS, bool MANY>
 __global__ __launch_bounds__(RT_THREADS) void lse_reduce_kernel(
     const bgtq_head_plan* plans, const float* part_out, const float* part_lse, const float* extra_lse, int n_splits, int n_q,
     int gqa, int unrotate, int n_extra, const float* extra_out, uint16_t* out, int64_t o_sb, int64_t o_sh, float* lse_out) {
@@ -287,19 +297,20 @@ __global__ __launch_bounds__(RT_THREADS) void lse_reduce_kernel(
     const float* R = plans[h].v_rot;
     const float* po = part_out + row * n_splits * D + c4;
 
-    // loads land in issue order: the partitions' log-sum-exps go first, so that the maximum and
-    // the weights are worked out while the vectors and the un-rotation are still on their way.  Every wave works out
-    // maximum and denominator by itself, 16 lanes beside each other over all partitions, and a thread the weights of its
-    // own row class: no trip through LDS and two barriers less (one row x 32 heads of 4k tokens 63.0 -> 61.5 us for 4 layers, 4 x 16
-    // of 8k 146.7 -> 144.3 for 8, 12 x 28 ragged 85.2 -> 84.4 for 4).
+    // loads land in issue order: the partitions' log-sum-exps go first
     constexpr int NB = 16 / RT_CLASSES;        // rounds of partial vectors fetched before anything else (16 vectors)
-    constexpr int NL = 4;                      // log-sum-exps a lane holds of all of them
+    constexpr int NL = MANY ? 1 : (merge_held(RT_THREADS) + 15) / 16;      // log-sum-exps a lane holds of all of them
     const int s16 = j & 15;
     float l_all[NL], l_own[NB];
+    __shared__ float wgt[MANY ? BGTQ_MAX_SPLITS : 1], red[RT_THREADS / 64], dsum[RT_CLASSES];
+    if constexpr (MANY) {
+        l_all[0] = j < n_splits ? pl[j] : -INFINITY;
+    } else {
 #pragma unroll
-    for (int i = 0; i < NL; i++) l_all[i] = s16 + 16 * i < n_splits ? pl[s16 + 16 * i] : -INFINITY;
+        for (int i = 0; i < NL; i++) l_all[i] = s16 + 16 * i < n_splits ? pl[s16 + 16 * i] : -INFINITY;
 #pragma unroll
-    for (int i = 0; i < NB; i++) l_own[i] = RT_CLASSES * i + cls < n_splits ? pl[RT_CLASSES * i + cls] : -INFINITY;
+        for (int i = 0; i < NB; i++) l_own[i] = RT_CLASSES * i + cls < n_splits ? pl[RT_CLASSES * i + cls] : -INFINITY;
+    }
     float4 pv[NB];
 #pragma unroll
     for (int i = 0; i < NB; i++) pv[i] = *(const float4*)(po + (size_t)min(RT_CLASSES * i + cls, n_splits - 1) * D);
@@ -310,9 +321,23 @@ __global__ __launch_bounds__(RT_THREADS) void lse_reduce_kernel(
         for (int i = 0; i < D / RT_CLASSES; i++) rv[i] = *(const float4*)(R + (RT_CLASSES * i + cls) * D + c4);
     }
 
-    float m = fmaxf(fmaxf(l_all[0], l_all[1]), fmaxf(l_all[2], l_all[3]));
-    for (int c = s16 + 16 * NL; c < n_splits; c += 16) m = fmaxf(m, pl[c]);
-    m = row16_max(m);
+    float m;
+    if constexpr (MANY) {
+        m = l_all[0];
+        if (j < n_splits) wgt[j] = m;
+        for (int c = j + RT_THREADS; c < n_splits; c += RT_THREADS) { const float l = pl[c]; wgt[c] = l; m = fmaxf(m, l); }
+        m = wave_max(m);
+        if ((j & 63) == 0) red[j >> 6] = m;
+        __syncthreads();
+        m = red[0];
+#pragma unroll
+        for (int i = 1; i < RT_THREADS / 64; i++) m = fmaxf(m, red[i]);
+    } else {
+        m = l_all[0];
+#pragma unroll
+        for (int i = 1; i < NL; i++) m = fmaxf(m, l_all[i]);
+        m = row16_max(m);
+    }
     for (int e = 0; e < n_extra; e++) m = fmaxf(m, el[e]);
     if (m == -INFINITY) {                      // nothing visible at all (the same in every thread)
         if (j < D) out[b * o_sb + hq * o_sh + j] = 0;
@@ -321,18 +346,27 @@ __global__ __launch_bounds__(RT_THREADS) void lse_reduce_kernel(
     }
     // weights: exp(lse - m), 0 for empty partitions (their vectors are undefined)
     auto weight = [&](float l) { return l == -INFINITY ? 0.f : __expf(l - m); };
-    float den = 0.f;
-#pragma unroll
-    for (int i = 0; i < NL; i++) den += weight(l_all[i]);
-    for (int c = s16 + 16 * NL; c < n_splits; c += 16) den += weight(pl[c]);
-    den = row16_sum(den);
+    float den = 0.f, dcl = 0.f;                // (dcl: weights of this thread's row class)
     float4 a4 = {0.f, 0.f, 0.f, 0.f};
     auto add = [&](float w, const float4& v) {
+        if constexpr (MANY) dcl += w;
         if (w != 0.f) { a4.x += w * v.x; a4.y += w * v.y; a4.z += w * v.z; a4.w += w * v.w; }
     };
+    if constexpr (MANY) {
+        for (int c = j; c < n_splits; c += RT_THREADS) wgt[c] = weight(wgt[c]);
+        __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NB; i++) add(weight(l_own[i]), pv[i]);
-    for (int c = RT_CLASSES * NB + cls; c < n_splits; c += RT_CLASSES) add(weight(pl[c]), *(const float4*)(po + (size_t)c * D));
+        for (int i = 0; i < NB; i++) add(wgt[RT_CLASSES * i + cls], pv[i]);      // (more than 16 partitions)
+        for (int c = RT_CLASSES * NB + cls; c < n_splits; c += RT_CLASSES) add(wgt[c], *(const float4*)(po + (size_t)c * D));
+        if ((j & 31) == 0) dsum[cls] = dcl;
+    } else {
+#pragma unroll
+        for (int i = 0; i < NL; i++) den += weight(l_all[i]);
+        den = row16_sum(den);
+#pragma unroll
+        for (int i = 0; i < NB; i++) add(weight(l_own[i]), pv[i]);
+        for (int c = RT_CLASSES * NB + cls; c < n_splits; c += RT_CLASSES) add(weight(pl[c]), *(const float4*)(po + (size_t)c * D));
+    }
     *(float4*)&cls_sum[cls][c4] = a4;
     float acce = 0.f;
     if (j < D)
@@ -356,7 +390,19 @@ __global__ __launch_bounds__(RT_THREADS) void lse_reduce_kernel(
         return s[0];
     };
     float res = 0.f;
-    if (j < D) res = fold(cls_sum, j);
+    if (j < D) {
+        if constexpr (MANY) {
+            float ds[RT_CLASSES];
+#pragma unroll
+            for (int i = 0; i < RT_CLASSES; i++) ds[i] = dsum[i];
+#pragma unroll
+            for (int w = RT_CLASSES / 2; w >= 1; w >>= 1)
+#pragma unroll
+                for (int i = 0; i < w; i++) ds[i] = ds[2 * i] + ds[2 * i + 1];
+            den += ds[0];
+        }
+        res = fold(cls_sum, j);
+    }
     if (unrotate) {
         if (j < D) vec[j] = res;
         __syncthreads();                       // also: every read of cls_sum above is done
@@ -634,8 +680,10 @@ int bgtq_lse_reduce(const bgtq_head_plan* plans,
     BGTQ_CHECK_ARG(((uintptr_t)partial_out & 15) == 0 && ((uintptr_t)plans & 15) == 0);
     if (n_splits > BGTQ_MAX_SPLITS) return BGTQ_ELIMIT;
     if (B == 0 || n_kv == 0) return BGTQ_OK;
-    const bool few = (int64_t)B * n_kv * gqa <= 256;
-    hipLaunchKernelGGL(few ? lse_reduce_kernel<512> : lse_reduce_kernel<128>, dim3((unsigned)gqa, (unsigned)n_kv, (unsigned)B),
+    const bool few = (int64_t)B * n_kv * gqa <= 256, many = n_splits > merge_held(few ? 512 : 128);
+    auto kern = few ? (many ? lse_reduce_kernel<512, true> : lse_reduce_kernel<512, false>)
+                    : (many ? lse_reduce_kernel<128, true> : lse_reduce_kernel<128, false>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)gqa, (unsigned)n_kv, (unsigned)B),
                        dim3(few ? 512 : 128), 0, (hipStream_t)stream, plans, partial_out, partial_lse, n_extra ? extra_lse : nullptr,
                        n_splits, n_kv * gqa, gqa, unrotate, n_extra, n_extra ? extra_out : nullptr, (uint16_t*)out, o_sb, o_sh, lse_out);
     return bgtq_launch_status();

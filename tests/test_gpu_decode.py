@@ -718,8 +718,8 @@ def test_merge_entry_point_refuses_what_its_kernel_cannot_take():
         _capi.check(call(_capi.ptr(part[1:]), 4), "bgtq_lse_reduce")
 
 
-@pytest.mark.parametrize("B", [1, 70])                       # 512 threads a row, and 128 from 257 rows on
-@pytest.mark.parametrize("n_splits,n_extra", [(1, 0), (3, 1), (15, 0), (16, 2), (17, 1), (63, 0), (64, 1), (65, 0), (200, 3), (512, 1)])
+@pytest.mark.parametrize("B", [1, 70])                       # 512 threads a row, 128 from 257 rows on; weights held by lanes up to 64 and 20 partitions
+@pytest.mark.parametrize("n_splits,n_extra", [(1, 0), (3, 1), (15, 0), (16, 2), (17, 1), (20, 0), (21, 1), (63, 0), (64, 1), (65, 0), (200, 3), (512, 1)])
 def test_merge_over_partition_counts(B, n_splits, n_extra):
     """Weighted mean of partials by exp(lse), un-rotated, plus partials that are not; empty ones hold anything.  fp16 output of
     fp32 sums of values near 1: half an fp16 step and 1e-5 of the terms' sum (128 products of a rotation row)."""
