@@ -1301,10 +1301,9 @@ __device__ __forceinline__ void prepare_part(const EncodeArgs& ak, const EncodeA
 // (BF16: some input is; asking at run time costs the chains of fp16 inputs 0.2 of 5.0 us)
 // Steps of one token whose rows need no rank, which is nearly all: the grid is (rows, KV heads, 2 + query parts), with no division
 // on the way to a work-group's rows, and what the first loads need (plans, K and V rows) comes as arguments of its own ahead of
-// the blocks: they are in scalar registers when a wave starts (kernarg preload), the blocks a trip to memory behind it.  With
-// the attention's and the merge's arguments taken the same way: one row x 8 heads of 4k tokens 66.8 -> 63.0 us (4 layers), 4 rows x
-// 2 heads of 8k 152.3 -> 146.7 (8), 12 ragged rows of 7-head groups 88.4 -> 85.2 (4), 8 x 2 of 32k 201.9 -> 195.1 (6); 65.2,
-// 151.2 and 87.3 of them with the merge alone.
+// the blocks: they are in scalar registers when a wave starts (kernarg preload), the blocks a trip to memory behind it.
+// One row x 8 heads of 4k tokens 65.2 -> 63.0 us (4 layers), 4 rows x 2 heads of 8k 151.3 -> 146.7 (8), 12 ragged rows of 7-head
+// groups 87.8 -> 86.1 (4), 8 x 2 of 32k 205.1 -> 202.2 (6).
 template <bool BF16>
 __global__ __launch_bounds__(NT) void prepare_token_kernel(const bgtq_head_plan* plans, const uint16_t* v, const uint16_t* k, uint32_t v_sb, uint32_t v_sh,
                                                            uint32_t k_sb, uint32_t k_sh, EncodeArgs ak, EncodeArgs av, RotQArgs aq) {
@@ -1319,17 +1318,20 @@ __global__ __launch_bounds__(NT) void prepare_token_kernel(const bgtq_head_plan*
     else if (role == 1) encode_row<false>(ak, row, h, threadIdx.x, rot_s);
     else rotate_q_block(aq, row, h, role - 2, rot_s);
 }
-// All others.  A first work-group ranks the rows, if any are to be ranked.  (Behind the others it started when a place came free
-// and ended last: 64 equal rows x 8 heads of 700 tokens 43.1 us a step as they come, 45.5 with a last one, 43.9 with a first.)
-template <bool BF16>
-__global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, int rows, RankArgs rank) {
+// All others.  Rank: RankArgs of a first work-group that ranks the rows, or nothing.  (Behind the others it started when a place
+// came free and ended last: 64 equal rows x 8 heads of 700 tokens 43.1 us a step as they come, 45.5 with a last one, 43.9 with a
+// first.  One that finds nothing to rank and its arguments cost two new tokens of one row x 8 heads of 4k 1.1 %: 79.6 -> 80.6 us, 4
+// layers; eight of 8 x 2 and four of 12 x 4 rows nothing.)
+template <bool BF16, class... Rank>
+__global__ __launch_bounds__(NT) void prepare_kernel(EncodeArgs ak, EncodeArgs av, RotQArgs aq, int rows, Rank... rank) {
     if (!BF16) ak.bf16 = av.bf16 = aq.bf16 = 0;
     __shared__ __align__(16) float rot_s[D * D];
-    if (blockIdx.x == 0) {                             // (uniform)
-        rank_rows(rank, threadIdx.x, (int*)rot_s);
-        return;
-    }
-    prepare_part(ak, av, aq, rows, blockIdx.x - 1, rot_s);
+    if constexpr (sizeof...(Rank) != 0)
+        if (blockIdx.x == 0) {                         // (uniform)
+            rank_rows(rank..., threadIdx.x, (int*)rot_s);
+            return;
+        }
+    prepare_part(ak, av, aq, rows, (int)blockIdx.x - (int)sizeof...(Rank), rot_s);
 }
 // The same with the attention over the buffered tokens, which depends on none of it: the longer work-groups first, in
 // the LDS that is a rotation's otherwise; then the token that leaves the buffer, K and V by the two halves of a
@@ -1434,7 +1436,7 @@ int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, in
     const int group = rotate_q_group_size(B, n_kv * gqa);
     RotQArgs aq{ak.plans, (const uint16_t*)q, q_sr, q_sh, (uint16_t*)q_rot, qr_sr, qr_sh, B, n_kv * gqa, gqa, group, q_bf16};
     const int rows = (int)N;
-    const unsigned blocks = (unsigned)(2 * rows * n_kv) + (q ? rotate_q_blocks(B, n_kv, gqa, group) : 0u) + (rank.order || !window ? 1u : 0u);
+    const unsigned blocks = (unsigned)(2 * rows * n_kv) + (q ? rotate_q_blocks(B, n_kv, gqa, group) : 0u) + (rank.order ? 1u : 0u);
     if (window) {
         const WindowArgs& w = *window;
         const dim3 grid(blocks - (unsigned)(rows * n_kv) + (unsigned)(B * n_kv));
@@ -1457,10 +1459,14 @@ int launch_prepare(const EncodeArgs& ak, const EncodeArgs& av, const void* q, in
             const dim3 grid((unsigned)rows, (unsigned)n_kv, 2u + (q ? (unsigned)((gqa + group - 1) / group) : 0u));
             hipLaunchKernelGGL(kern, grid, dim3(NT), 0, st, ak.plans, av.x, ak.x, (uint32_t)av.x_sb, (uint32_t)av.x_sh,
                                (uint32_t)ak.x_sb, (uint32_t)ak.x_sh, ak, av, aq);
+        } else if (blocks == 0) {
+            return BGTQ_OK;                            // (no tokens and no queries)
+        } else if (rank.order) {
+            auto kern = bf16 ? prepare_kernel<true, RankArgs> : prepare_kernel<false, RankArgs>;
+            hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows, rank);
         } else {
-            // (no rows are ranked where rank.order is null)
             auto kern = bf16 ? prepare_kernel<true> : prepare_kernel<false>;
-            hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows, rank.order ? rank : RankArgs{});
+            hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), 0, st, ak, av, aq, rows);
         }
     }
     return bgtq_launch_status();

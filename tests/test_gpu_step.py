@@ -327,3 +327,23 @@ def test_token_rows_at_strides_beyond_32_bits(dtype):
             k, v = [t.as_strided((1, 2, 1, 128), (2 ** 33, 128, 128, 1)) for t in (k, v)]
         got.append((mgr.append_and_attend(0, q, k, v), mgr._k_packed[0], mgr._k_norms[0], mgr._v_packed[0], mgr._v_norms[0]))
     assert got[0][0].abs().max() > 0 and all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("S", [1, 2, 5, 33])                 # (66 new rows leave the one launch)
+def test_steps_of_several_new_tokens(S, dtype):
+    """The preparation of any number of new tokens leaves the records that appends of one token each leave."""
+    w, e, caches = _pair()
+    for c in caches:                                         # room for 33
+        for name in ("k_packed", "k_norms", "v_packed", "v_norms"):
+            t = getattr(c, name)
+            setattr(c, name, torch.cat([t, torch.zeros_like(t)], 3))
+        c.max_T *= 2
+    q, _, _ = _inputs(w, [e], 90, dtype)
+    k, v = [t.to(dtype) for t in wl.draw_kv(w, e, S, 322, DEV, pos0=90)]
+    fast, slow = [c.encode_and_attend(0, q, k, v) for c in caches]
+    assert fast.abs().max() > 0 and torch.equal(fast, slow)
+    for s in range(S):
+        caches[1]._encode_batched(0, k[:, :, s:s + 1], v[:, :, s:s + 1], 90 + s)
+    for name in ("k_packed", "k_norms", "v_packed", "v_norms"):
+        assert torch.equal(getattr(caches[0], name), getattr(caches[1], name)), name
