@@ -294,7 +294,8 @@ __device__ __forceinline__ int grid_row(const int32_t* order) { return order[blo
 // HEADS: query heads per KV head the MFMA layout serves (4 or 8)
 // VBW: bits per V code; VST: bytes from one V record to the next (the record itself is
 // 16 * VBW bytes; a padded stride keeps the rows of a tile on different LDS banks)
-// NIB: the V records are nibbles (VBW 4), of codes of at most 3 bits as a rule.  Their pair table is the bit-packed one: a byte
+// NIB: the V records are nibbles (VBW 4), of codes of at most 3 bits as a rule (4-bit ones are bit-packed records as well, and
+// come as such where the host knows the width).  Their pair table is the bit-packed one: a byte
 // indexes 256 entries that cannot be replicated, and reads of it are what bounds this layout (a read by 64 lanes takes a CU 2.8 ns,
 // one of 64 entries x 32 replicas 1.1 ns; with the shift and mask in front of them 2.8 and 1.3).  So a nibble pair is brought to
 // the 64-entry index by one dot product of nibbles: 4 layers of 8 rows x 2 heads of 32k, K3V3, 153.0 -> 146.3 us.

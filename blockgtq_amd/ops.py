@@ -110,6 +110,7 @@ def decode_attention(plans: torch.Tensor, q_rot: torch.Tensor,
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
     k_row_width = k_packed.shape[-1] if k_row_width is None else k_row_width
     v_row_width = v_packed.shape[-1] if v_row_width is None else v_row_width
+    v_layout = _plan.attended_v_layout(plans, v_layout, v_row_width)
     L = _capi.lib()
     if n_splits <= 0:
         pick = L.bgtq_default_splits if seq_lens is None else L.bgtq_ragged_splits

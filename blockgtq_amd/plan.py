@@ -373,9 +373,22 @@ def stack_plans(quantizers) -> np.ndarray:
 
 
 def upload_plans(plans: np.ndarray, device) -> torch.Tensor:
-    """Copy a structured plan array to ``device`` as a flat uint8 tensor."""
-    raw = torch.from_numpy(np.ascontiguousarray(plans).view(np.uint8).copy())
-    return raw.to(device)
+    """Copy a structured plan array to ``device`` as a flat uint8 tensor.  ``v_code_bits`` of the tensor: bits of
+    every head's V codes (0 where heads differ), for host code that chooses a kernel by them."""
+    raw = torch.from_numpy(np.ascontiguousarray(plans).view(np.uint8).copy()).to(device)
+    bits = np.unique(plans['v_bits'])
+    raw.v_code_bits = int(bits[0]) if bits.size == 1 else 0
+    return raw
+
+
+def attended_v_layout(plans: torch.Tensor, v_layout: int, v_row_width: int) -> int:
+    """Layout under which attention reads V records.  Nibble records of 4-bit codes are bit-packed records of 4-bit
+    codes, byte for byte.  The kernel of nibble records must take narrower codes too, and the device alone knows the
+    width there: the second body cost 4-bit codes 2 to 4 % (four layers of 8 x 2 x 32k K4V4 157.6 us as nibbles, 153.9 as
+    bit-packed; 8 x 8 x 4k 123.0 and 118.7, 1 x 8 x 4k 72.9 and 71.7).  Plans of unknown origin stay with it."""
+    if v_layout == V_NIBBLE and v_row_width == HEAD_DIM // 2 and getattr(plans, 'v_code_bits', 0) == 4:
+        return V_BITPACKED
+    return v_layout
 
 
 def cache_row_bytes(record_bytes: int) -> int:

@@ -347,3 +347,32 @@ def test_steps_of_several_new_tokens(S, dtype):
         caches[1]._encode_batched(0, k[:, :, s:s + 1], v[:, :, s:s + 1], 90 + s)
     for name in ("k_packed", "k_norms", "v_packed", "v_norms"):
         assert torch.equal(getattr(caches[0], name), getattr(caches[1], name)), name
+
+
+@pytest.mark.parametrize("bits", [3, 4])
+@pytest.mark.parametrize("n_q", [8, 16, 24])                 # 4 and 8 query heads a KV head, and two launches
+def test_nibble_records_with_and_without_a_known_code_width(bits, n_q):
+    """Plans that say how wide V's codes are and copies that do not: the same records and outputs, native, general and the attention alone."""
+    from blockgtq_amd import ops, plan as P
+    w = wl.Workload("t", 1, n_q, 2, 2, 200, 1e6, k_bits=float(bits), v_bits=bits, seed=39)
+    qs, e = wl.calibrate_layer(w, 0, DEV)
+    k0, v0 = wl.draw_kv(w, e, 200, 5, DEV)
+    q, k, v = _inputs(w, [e], 200, torch.float16)
+    got = []
+    for known in (True, False):
+        c = BlockGTQProductionCache([qs], [build_batched_encode_args(qs, device=DEV)], [[q8.build_kernel_args() for q8 in qs]],
+                                    1, 2, n_q, 128, 210, v_bits=bits, device=DEV, batch_size=2)
+        plans = c.batched_args[0]['plans']
+        assert plans.v_code_bits == bits
+        if not known:
+            plans = c.batched_args[0]['plans'] = plans.clone()
+        assert P.attended_v_layout(plans, c._v_layout, c.vpb) == (P.V_BITPACKED if known and bits == 4 else P.V_NIBBLE)
+        c._encode_batched(0, k0, v0, 0)
+        c.seq_len = 200
+        outs = [c.encode_and_attend(0, q, k, v), c._encode_and_attend_general(0, q, k, v)]
+        outs.append(ops.decode_attention(plans, ops.rotate_q(plans, q[:, :, 0].contiguous(), 2), c.k_packed[0], c.k_norms[0],
+                                         c.v_packed[0], c.v_norms[0], 201, k_layout=c._k_layout, v_layout=c._v_layout).unsqueeze(2))
+        assert ops.last_decode_path() == ops.MFMA_PATH
+        assert outs[0].abs().max() > 0 and all(torch.equal(outs[0], o) for o in outs)
+        got.append([outs[0], c.k_packed, c.k_norms, c.v_packed, c.v_norms])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
