@@ -90,7 +90,7 @@ __global__ __launch_bounds__(GT) void decode_generic_kernel(DecodeArgs a) {
     const int n_seg = P.n_seg;
     const int kbytes = min((a.k_layout == BGTQ_K_MIXED) ? P.k_mixed_bytes : P.k_row_bytes,
                            a.k_row_width);
-    const int vbw = (a.v_layout == BGTQ_V_NIBBLE) ? 4 : P.v_bits;
+    const int vbw = (a.v_layout == BGTQ_V_BITPACKED) ? P.v_bits : 4;
     const int vbytes = min(bgtq_seg_bytes(vbw, D), a.v_row_width);
 
     const uint8_t* kp_base = a.kp + b * a.kp_sb + h * a.kp_sh;
@@ -601,7 +601,7 @@ int decode_attn(const bgtq_head_plan* plans,
     BGTQ_CHECK_ARG(B >= 0 && n_kv >= 0 && T >= 0);
     BGTQ_CHECK_ARG(gqa >= 1 && gqa <= BGTQ_MAX_GQA);
     BGTQ_CHECK_ARG(k_layout == BGTQ_K_BITPACKED || k_layout == BGTQ_K_MIXED);
-    BGTQ_CHECK_ARG(v_layout == BGTQ_V_BITPACKED || v_layout == BGTQ_V_NIBBLE);
+    BGTQ_CHECK_ARG(v_layout == BGTQ_V_BITPACKED || v_layout == BGTQ_V_NIBBLE || v_layout == BGTQ_V_NIBBLE4);
     if (n_splits > BGTQ_MAX_SPLITS) return BGTQ_ELIMIT;
     BGTQ_CHECK_ARG(n_splits >= 1);
     if (B == 0 || n_kv == 0) return BGTQ_OK;
@@ -804,7 +804,7 @@ int bgtq_decode_step(const bgtq_step* step, void* stream) {
 
 size_t bgtq_plan_sizeof(void) { return sizeof(bgtq_head_plan); }
 int bgtq_abi_version(void) { return 8; }
-int bgtq_decode_kernel_revision(void) { return 11; }
+int bgtq_decode_kernel_revision(void) { return 12; }
 
 const char* bgtq_strerror(int code) {
     switch (code) {

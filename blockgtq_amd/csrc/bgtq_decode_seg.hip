@@ -294,8 +294,8 @@ __device__ __forceinline__ int grid_row(const int32_t* order) { return order[blo
 // HEADS: query heads per KV head the MFMA layout serves (4 or 8)
 // VBW: bits per V code; VST: bytes from one V record to the next (the record itself is
 // 16 * VBW bytes; a padded stride keeps the rows of a tile on different LDS banks)
-// NIB: the V records are nibbles (VBW 4), of codes of at most 3 bits as a rule (4-bit ones are bit-packed records as well, and
-// come as such where the host knows the width).  Their pair table is the bit-packed one: a byte
+// NIB: the V records are nibbles (VBW 4), of codes of at most 3 bits as a rule (4-bit ones take the kernel without it where the
+// caller knows the width, BGTQ_V_NIBBLE4: nibbles are its records whatever they hold, through the byte-indexed table).  Their pair table is the bit-packed one: a byte
 // indexes 256 entries that cannot be replicated, and reads of it are what bounds this layout (a read by 64 lanes takes a CU 2.8 ns,
 // one of 64 entries x 32 replicas 1.1 ns; with the shift and mask in front of them 2.8 and 1.3).  So a nibble pair is brought to
 // the 64-entry index by one dot product of nibbles: 4 layers of 8 rows x 2 heads of 32k, K3V3, 153.0 -> 146.3 us.
@@ -462,7 +462,9 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void decode_seg_kernel(const bgtq_h
         constexpr int VCH = BGTQ_VLUT_BYTES / 1024, NCH = VCH + (BGTQ_LUT_IMAGE_BYTES + 1023) / 1024;
         constexpr int LAST_PIECES = (BGTQ_LUT_IMAGE_BYTES - (NCH - VCH - 1) * 1024) / 16;
         static_assert(BGTQ_VLUT_BYTES % 1024 == 0 && VTAB_BYTES == BGTQ_VLUT_BYTES && LAST_PIECES >= 1 && LAST_PIECES <= 64, "");
-        const uint8_t* vimg = (const uint8_t*)P.vlut_image[BGTQ_V_BITPACKED];     // (of either layout: nibbles are brought to its index)
+        // NIB brings nibbles to the bit-packed table's index.  The byte-indexed table serves nibbles of any width, and for 4-bit codes
+        // it is the bit-packed one (chosen by a layout that the argument block holds: 8 x 8 x 4k 107.0 us for four layers, 106.3 without).
+        const uint8_t* vimg = (const uint8_t*)P.vlut_image[VBW == 4 && !NIB ? BGTQ_V_NIBBLE : BGTQ_V_BITPACKED];
         const uint8_t* kimg_m = (const uint8_t*)P.lut_image[kl] - VCH * 1024;
         for (int cc = nw - 1 - wave; cc < NCH; cc += nw) {
             const uint8_t* src = (cc < VCH ? vimg : kimg_m) + cc * 1024;
@@ -961,7 +963,7 @@ static int launch_group(const DecodeArgs& a, const int32_t* row_order, hipStream
     if (a.k_row_width < 4 || a.k_row_width > 128) return BGTQ_EUNSUPPORTED;
     if (a.vn_st != 1 || a.kn_st < 1 || a.kn_st > MAX_KN) return BGTQ_EUNSUPPORTED;
     if ((a.q_sb & 1) || (a.q_sh & 1) || ((uintptr_t)a.q & 3)) return BGTQ_EUNSUPPORTED;
-    if (a.v_layout == BGTQ_V_NIBBLE && a.v_row_width != 64) return BGTQ_EUNSUPPORTED;
+    if (a.v_layout != BGTQ_V_BITPACKED && a.v_row_width != 64) return BGTQ_EUNSUPPORTED;
     // a bit-packed V record of 128 dims is 16 bytes per bit of code width, a nibble record 64
     // V records follow each other directly, or 4 bytes apart where the record width itself
     // (32 or 64 bytes) would put the rows of a tile on the same LDS banks

@@ -1479,7 +1479,8 @@ int fill_step_args(const bgtq_step& s, EncodeArgs& ak, EncodeArgs& av) {
                          s.k_layout, s.quant_mode);
     if (rc != BGTQ_OK) return rc;
     rc = fill_v_args(av, s.plans, s.v, s.v_sb, s.v_sh, s.v_ss, s.B, s.n_kv, s.S, s.v_packed, s.vp_sb, s.vp_sh, s.vp_st,
-                     s.v_row_width, s.v_norms, s.vn_sb, s.vn_sh, s.vn_st, s.t_pos, s.t_pos_scalar, s.max_T, s.v_layout);
+                     s.v_row_width, s.v_norms, s.vn_sb, s.vn_sh, s.vn_st, s.t_pos, s.t_pos_scalar, s.max_T,
+                     s.v_layout == BGTQ_V_NIBBLE4 ? BGTQ_V_NIBBLE : s.v_layout);
     ak.bf16 = av.bf16 = s.x_dtype == BGTQ_X_BF16;
     return rc;
 }

@@ -17,7 +17,7 @@ MAX_WALK = 12
 ROT_COL = 48
 
 K_BITPACKED, K_MIXED = 0, 1
-V_BITPACKED, V_NIBBLE = 0, 1
+V_BITPACKED, V_NIBBLE, V_NIBBLE4 = 0, 1, 2
 QUANT_LUT256, QUANT_EXACT = 0, 1
 
 _S, _D, _C = MAX_SEGMENTS, HEAD_DIM, MAX_CENTROIDS
@@ -374,7 +374,7 @@ def stack_plans(quantizers) -> np.ndarray:
 
 def upload_plans(plans: np.ndarray, device) -> torch.Tensor:
     """Copy a structured plan array to ``device`` as a flat uint8 tensor.  ``v_code_bits`` of the tensor: bits of
-    every head's V codes (0 where heads differ), for host code that chooses a kernel by them."""
+    every head's V codes at the upload (0 where heads differ); nothing but speed may hang on it."""
     raw = torch.from_numpy(np.ascontiguousarray(plans).view(np.uint8).copy()).to(device)
     bits = np.unique(plans['v_bits'])
     raw.v_code_bits = int(bits[0]) if bits.size == 1 else 0
@@ -382,12 +382,12 @@ def upload_plans(plans: np.ndarray, device) -> torch.Tensor:
 
 
 def attended_v_layout(plans: torch.Tensor, v_layout: int, v_row_width: int) -> int:
-    """Layout under which attention reads V records.  Nibble records of 4-bit codes are bit-packed records of 4-bit
-    codes, byte for byte.  The kernel of nibble records must take narrower codes too, and the device alone knows the
-    width there: the second body cost 4-bit codes 2 to 4 % (four layers of 8 x 2 x 32k K4V4 157.6 us as nibbles, 153.9 as
-    bit-packed; 8 x 8 x 4k 123.0 and 118.7, 1 x 8 x 4k 72.9 and 71.7).  Plans of unknown origin stay with it."""
+    """Layout under which attention reads V records: nibble records of 4-bit codes by the kernel of 4-bit codes.  The one
+    of nibble records must take narrower codes too, and the device alone knows the width there: the second body cost 4-bit
+    codes 2 to 4 % (four layers of 8 x 2 x 32k K4V4 157.6 us, 153.9 by the other; 8 x 8 x 4k 123.0 and 118.7, 1 x 8 x 4k 72.9
+    and 71.7).  Both read codes of every width, so plans of unknown origin, or written over since, cost time alone."""
     if v_layout == V_NIBBLE and v_row_width == HEAD_DIM // 2 and getattr(plans, 'v_code_bits', 0) == 4:
-        return V_BITPACKED
+        return V_NIBBLE4
     return v_layout
 
 

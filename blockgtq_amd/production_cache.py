@@ -66,7 +66,7 @@ class BlockGTQProductionCache:
         """The layer's native handle (None off the GPU), made anew when something it was made from has changed."""
         h = self._layers[li]
         plans = self.batched_args[li]['plans']
-        v_layout = _plan.attended_v_layout(plans, self._v_layout, self.vpb)     # (records are written alike)
+        v_layout = _plan.attended_v_layout(plans, self._v_layout, self.vpb)
         args = (li, plans, self.k_packed, self.k_norms, self.v_packed, self.v_norms,
                 self.k_bytes_per_tok, self.max_ng, self.vpb, self.nq, self._k_layout, v_layout, self.scale,
                 self.quantizers[li][0]._q_perm_baked, None, None)

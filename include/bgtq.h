@@ -79,6 +79,9 @@ extern "C" {
 /* V record layouts (blockgtq/v_packing.py:17-28, blockgtq/quantizer.py:2096-2099) */
 #define BGTQ_V_BITPACKED   0     /* v_bits per code, LSB first */
 #define BGTQ_V_NIBBLE      1     /* 4 bits per code whatever v_bits is */
+/* The same records, for bgtq_decode_attn, bgtq_decode_attend_static, bgtq_decode_step and bgtq_encode_kv: attended by the
+ * kernel of 4-bit codes.  Codes of every width are read and written as with BGTQ_V_NIBBLE, only the speed differs. */
+#define BGTQ_V_NIBBLE4     2
 /* K scalar quantisation rule */
 #define BGTQ_QUANT_LUT256  0     /* 256-bin table, blockgtq/quantizer.py:841-850 */
 #define BGTQ_QUANT_EXACT   1     /* count of boundaries below y, blockgtq/block_gtq_pipeline.py:337-341 */

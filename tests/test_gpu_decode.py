@@ -730,11 +730,15 @@ def test_merge_over_partition_counts(B, n_splits, n_extra):
     part = torch.randn(B, 4, n_splits, 128, generator=gen, device=DEV)
     lse = torch.randn(B, 4, n_splits, generator=gen, device=DEV) * 3
     empty = torch.rand(B, 4, n_splits, generator=gen, device=DEV) < 0.3
-    empty[0, 1] = True                                       # (a row that sees nothing, or the extra partials alone)
+    empty[0, 1:3] = True                                     # (rows that see the extra partials alone, or nothing)
     part[empty], lse[empty] = float("nan"), -float("inf")
     xo = torch.randn(B, 4, max(n_extra, 1), 128, generator=gen, device=DEV)
-    xl = torch.randn(B, 4, max(n_extra, 1), generator=gen, device=DEV)
-    xl[..., 1:] = -float("inf")
+    xl = torch.randn(B, 4, max(n_extra, 1), generator=gen, device=DEV) * 3
+    no_extra = torch.rand(B, 4, max(n_extra, 1), generator=gen, device=DEV) < 0.3
+    no_extra[0, 0], no_extra[0, 2] = False, True
+    no_extra[0, 1] = torch.arange(max(n_extra, 1), device=DEV) < n_extra - 1      # (the last one alone)
+    no_extra[0, 3] = torch.arange(max(n_extra, 1), device=DEV) == 0               # (all but the first)
+    xo[no_extra], xl[no_extra] = float("nan"), -float("inf")
     out, tot = torch.zeros(B, 4, 128, dtype=torch.float16, device=DEV), torch.zeros(B, 4, device=DEV)
     _capi.check(_capi.lib().bgtq_lse_reduce(
         _capi.ptr(args['plans']), _capi.ptr(part), _capi.ptr(lse), n_splits, _capi.ptr(xo) if n_extra else None,
@@ -747,7 +751,7 @@ def test_merge_over_partition_counts(B, n_splits, n_extra):
     acc = (torch.where(empty, 0.0, (lse.double() - w).exp()).unsqueeze(-1) * part.nan_to_num().double()).sum(-2)
     want = (acc.reshape(B, n_kv, gqa, 1, 128) @ R).reshape(B, 4, 128)
     if n_extra:
-        want += ((xl.double() - w).exp().unsqueeze(-1) * xo.double()).sum(-2)
+        want += (torch.where(no_extra, 0.0, (xl.double() - w).exp()).unsqueeze(-1) * xo.nan_to_num().double()).sum(-2)
     torch.testing.assert_close(out.double(), want, rtol=6e-4, atol=2e-5)
     torch.testing.assert_close(tot.double(), want_lse, rtol=1e-5, atol=2e-5)
 

@@ -309,24 +309,32 @@ def test_rows_by_falling_length_change_nothing(batch, n_kv, splits, window, kind
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_token_rows_at_strides_beyond_32_bits(dtype):
-    """New rows whose batch stride leaves 32 bits (one batch row: it is never used) take the general preparation, others the one
-    of single tokens: the same step, also with heads that share a row of K and lie apart in V."""
+    """New rows whose batch stride leaves 32 bits take the general preparation, others the one of single tokens (its last stride
+    among them): the same step, also with heads that share a row of K and lie apart in V.  Cut to 32 bits, a stride of 2 ** 32
+    would give the second row the tokens of the first."""
     w, e, caches = _pair()
     one = lambda t: t[:1].expand(2, -1, -1, -1)
     q, k, v = [t.contiguous() for t in _inputs(w, [e], 90, dtype)]
     outs = [caches[0].encode_and_attend(0, one(q), k[:1, :1].expand(2, 4, 1, 128), one(v)),
             caches[1].encode_and_attend(0, one(q).contiguous(), k[:1, :1].expand(2, 4, 1, 128).contiguous(), one(v).contiguous())]
     assert outs[0].abs().max() > 0 and torch.equal(*outs)
-    w1 = wl.Workload("t", 1, 8, 2, 1, 90, 1e6, seed=38)
+    w2 = wl.Workload("t", 1, 8, 2, 2, 90, 1e6, seed=38)
+    memory = torch.empty(2 ** 32 + 1024, dtype=dtype, device=DEV)           # (8.6 GB, touched at both ends alone)
     got = []
-    for far in (False, True):
-        mgr, energies = wl.build_manager(w1, DEV)
-        wl.fill_cache(mgr, w1, energies, DEV)
-        q, k, v = [t.contiguous() for t in _inputs(w1, energies, 90, dtype)]
-        if far:
-            k, v = [t.as_strided((1, 2, 1, 128), (2 ** 33, 128, 128, 1)) for t in (k, v)]
+    for stride in (None, 2 ** 32 - 128, 2 ** 32):
+        mgr, energies = wl.build_manager(w2, DEV)
+        wl.fill_cache(mgr, w2, energies, DEV)
+        q, k, v = [t.contiguous() for t in _inputs(w2, energies, 90, dtype)]
+        assert not torch.equal(k[0], k[1]) and not torch.equal(v[0], v[1])
+        if stride:
+            far = [memory.as_strided((2, 2, 1, 128), (stride, 128, 128, 1), at) for at in (0, 512)]
+            k, v = [f.copy_(t) for f, t in zip(far, (k, v))]
         got.append((mgr.append_and_attend(0, q, k, v), mgr._k_packed[0], mgr._k_norms[0], mgr._v_packed[0], mgr._v_norms[0]))
-    assert got[0][0].abs().max() > 0 and all(torch.equal(a, b) for a, b in zip(*got))
+    del memory, far, k, v
+    torch.cuda.empty_cache()
+    assert got[0][0].abs().max() > 0
+    for other in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got[0], other))
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
@@ -366,7 +374,7 @@ def test_nibble_records_with_and_without_a_known_code_width(bits, n_q):
         assert plans.v_code_bits == bits
         if not known:
             plans = c.batched_args[0]['plans'] = plans.clone()
-        assert P.attended_v_layout(plans, c._v_layout, c.vpb) == (P.V_BITPACKED if known and bits == 4 else P.V_NIBBLE)
+        assert P.attended_v_layout(plans, c._v_layout, c.vpb) == (P.V_NIBBLE4 if known and bits == 4 else P.V_NIBBLE)
         c._encode_batched(0, k0, v0, 0)
         c.seq_len = 200
         outs = [c.encode_and_attend(0, q, k, v), c._encode_and_attend_general(0, q, k, v)]
@@ -376,3 +384,38 @@ def test_nibble_records_with_and_without_a_known_code_width(bits, n_q):
         assert outs[0].abs().max() > 0 and all(torch.equal(outs[0], o) for o in outs)
         got.append([outs[0], c.k_packed, c.k_norms, c.v_packed, c.v_norms])
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("bits", [1, 2, 3, 4])
+def test_nibble_records_behind_plans_written_over(bits):
+    """Plans of 4-bit codes that other ones were copied over since: records and outputs of those, by every kernel."""
+    from blockgtq_amd import _capi, ops, plan as P
+    made = []
+    for b in (4, bits):
+        w = wl.Workload("t", 1, 8, 2, 2, 200, 1e6, k_bits=3.0, v_bits=b, seed=40)
+        made.append((w,) + wl.calibrate_layer(w, 0, DEV))
+    (_, q4, _), (w, qs, e) = made
+    k0, v0 = wl.draw_kv(w, e, 200, 5, DEV)
+    q, k, v = _inputs(w, [e], 200, torch.float16)
+    want = build_batched_encode_args(qs, device=DEV)['plans']
+    got = []
+    for over in (False, True):
+        c = BlockGTQProductionCache([qs], [build_batched_encode_args(q4 if over else qs, device=DEV)], [[q8.build_kernel_args() for q8 in qs]],
+                                    1, 2, 8, 128, 210, v_bits=bits, device=DEV, batch_size=2)
+        plans = c.batched_args[0]['plans']
+        if over:
+            assert P.attended_v_layout(plans, c._v_layout, c.vpb) == P.V_NIBBLE4
+            plans.copy_(want)
+        assert torch.equal(plans, want)
+        c._encode_batched(0, k0, v0, 0)
+        c.seq_len = 200
+        outs = [c.encode_and_attend(0, q, k, v)]
+        for path in (2, 1):                                  # matrix cores, any layout
+            assert _capi.lib().bgtq_set_decode_path(path) == 0
+            try:
+                outs.append(ops.decode_attention(plans, ops.rotate_q(plans, q[:, :, 0].contiguous(), 2), c.k_packed[0], c.k_norms[0],
+                                                 c.v_packed[0], c.v_norms[0], 201, k_layout=c._k_layout, v_layout=c._v_layout))
+            finally:
+                _capi.lib().bgtq_set_decode_path(0)
+        got.append(outs + [c.k_packed, c.k_norms, c.v_packed, c.v_norms])
+    assert got[0][0].abs().max() > 0 and all(torch.equal(a, b) for a, b in zip(*got))

@@ -712,13 +712,13 @@ def test_nibble_records_of_foreign_tensors_hold_every_code_of_the_v_table(entry,
     assert np.array_equal(plans[0]['vlut_image'], own['vlut_image'])
 
 
-def test_nibble_records_of_4_bit_codes_are_attended_as_bit_packed_ones():
-    """Only where every head's width is known to be 4, and only records a nibble record wide."""
+def test_nibble_records_of_4_bit_codes_take_the_kernel_of_4_bit_codes():
+    """Only where every head's width is known to be 4, and only records a nibble record wide; never as bit-packed records."""
     plans = {bits: make_quantizer(seed=bits, v_bits=bits)[0].plan() for bits in (1, 2, 3, 4)}
     for bits, p in plans.items():
         t = P.upload_plans(np.concatenate([p, p]), 'cpu')
         assert t.v_code_bits == bits
-        assert P.attended_v_layout(t, P.V_NIBBLE, 64) == (P.V_BITPACKED if bits == 4 else P.V_NIBBLE)
+        assert P.attended_v_layout(t, P.V_NIBBLE, 64) == (P.V_NIBBLE4 if bits == 4 else P.V_NIBBLE)
         assert P.attended_v_layout(t, P.V_BITPACKED, 64) == P.V_BITPACKED
         for other in (48, 63, 68, 128):
             assert P.attended_v_layout(t, P.V_NIBBLE, other) == P.V_NIBBLE
@@ -726,6 +726,5 @@ def test_nibble_records_of_4_bit_codes_are_attended_as_bit_packed_ones():
             assert P.attended_v_layout(unknown, P.V_NIBBLE, 64) == P.V_NIBBLE
     mixed = P.upload_plans(np.concatenate([plans[4], plans[3]]), 'cpu')
     assert mixed.v_code_bits == 0 and P.attended_v_layout(mixed, P.V_NIBBLE, 64) == P.V_NIBBLE
-    p = plans[4][0]                                              # what the two layouts' kernels go by
-    assert np.array_equal(p['enc_vbyte'][P.V_BITPACKED], p['enc_vbyte'][P.V_NIBBLE])
+    p = plans[4][0]                                              # (one table serves both layouts in that kernel)
     assert np.array_equal(p['vlut_image'][P.V_BITPACKED][:256], p['vlut_image'][P.V_NIBBLE][:256])
