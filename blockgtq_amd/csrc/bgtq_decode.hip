@@ -561,7 +561,9 @@ int scratch_of_current_device(void** out) {
 // Partitions per (row, KV head).  A work-group keeps a compute unit busy, so what a launch takes is its rounds of 256
 // work-groups times (set-up and merge + tiles of a partition), in units of one tile at a work-group's full rate
 // (0.4 to 0.5 us); set-up and merge are worth 12 of them.  Only counts that just fill some number of rounds are
-// looked at, and a partition has at least 128 tokens.  One work-group too many costs a round:
+// looked at, and a partition has at least 128 tokens.  The merge takes 0.01 to 0.02 us a partition (512 threads), 0.1 to 0.2 where
+// 128-thread work-groups queue up; two fifths or two thirds of MERGE choose alike for all but 15 of 24 000 shapes.  One work-group too
+// many costs a round:
 //   12 rows x 4 heads, 3001 tokens: 6 partitions (288 work-groups) 32.6 us a step, 5 (240) 26.0
 //   20 rows x 8 heads, 8k tokens:   2 (320) 105 us, 3 (480, two full rounds) 81
 // Rows of different lengths (the lengths are on the device): half of the longest on average, and where there are several

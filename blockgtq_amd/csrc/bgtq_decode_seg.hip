@@ -300,7 +300,9 @@ __device__ __forceinline__ int grid_row(const int32_t* order) { return order[blo
 // one of 64 entries x 32 replicas 1.1 ns; with the shift and mask in front of them 2.8 and 1.3).  So a nibble pair is brought to
 // the 64-entry index by one dot product of nibbles: 4 layers of 8 rows x 2 heads of 32k, K3V3, 153.0 -> 146.3 us.
 // plans .. rem_tiles: members of the argument block that the first requests need, in front of it, where they are in scalar
-// registers when a wave starts (kernarg preload, 14 dwords at most): walk words and tables do not wait for the block.
+// registers when a wave starts (kernarg preload, 14 dwords at most): walk words and tables do not wait for the block.  Alone it is
+// worth 0.4 to 1.2 % of a replayed step (6 layers of 8 x 2 x 32k 194.2 -> 193.1 us, 8 of 4 x 2 x 8k 143.3 -> 142.0, 2 of 32 ragged x 8
+// with a window 211.5 -> 208.9) and nothing of an eager one of few rows (one row of 4k 61.3 -> 61.4, 12 ragged 84.6 -> 84.8).
 // Order: the batch row of each grid row, or nothing.  (Asked at run time, here and in the preparation, it cost steps without an
 // order 0.6 us a layer, 2 to 3 %; as a member of DecodeArgs 0.5 %.)
 template <int HEADS, int VBW, int VST, bool NIB, class... Order>
