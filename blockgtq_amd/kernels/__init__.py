@@ -132,8 +132,7 @@ def fused_blockgtq_decode_attention(
         v_norms = v_norms[..., 0]
     n_splits = max(1, min(int(t_splits), 512))
     k_layout = _plan.K_MIXED if k_nibble else _plan.K_BITPACKED
-    v_layout = _plan.V_NIBBLE if v_nibble else _plan.V_BITPACKED
-    v_layout = _plan.attended_v_layout(plans, v_layout, v_codes.shape[-1])
+    v_layout = _plan.attended_v_layout(plans, _plan.V_NIBBLE, v_codes.shape[-1]) if v_nibble else _plan.V_BITPACKED
     scale = (1.0 / math.sqrt(D)) if scale is None else float(scale)
     if not return_lse:
         out = _host.module().attend(plans, q, k_packed, k_norms, v_codes, v_norms, T, n_splits, k_layout, v_layout,

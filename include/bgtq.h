@@ -180,7 +180,8 @@ typedef struct bgtq_head_plan {
      * raw tables at BGTQ_LUTM_KRAW + (bw - 5) * 512.
      * vlut_image[v]: V pair table for V layout v (BGTQ_V_BITPACKED: entry (c0 | c1 <<
      * v_bits), 32 replicas for v_bits <= 3, unreplicated for 4; BGTQ_V_NIBBLE: 256
-     * byte-indexed entries, unreplicated).
+     * byte-indexed entries, unreplicated, for 4-bit codes the same ones).  Both are filled
+     * whatever layout the records have: nibbles may be read through either, by v_bits.
      */
     int32_t  n_units[2];
     int32_t  n_pair_units[2];
